@@ -20,13 +20,6 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 # -packed-fp32-ops off: hipcc must not emit packed FP32 instructions.
 HIP_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Xclang", "-target-feature", "-Xclang",
              "-packed-fp32-ops", "-Wno-unused-result"]
-# Per-source flags.  The integrator kernel is one loop around the whole RHS;
-# machine-level loop-invariant code motion hoists the RHS's 64-bit constants
-# (polynomial coefficients of exp/log and the like) out of it and holds them
-# in registers for the whole integration, which spills live values to
-# scratch memory.  Materialising a constant where it is used costs the same
-# two moves and no register.
-SOURCE_FLAGS = {"gal_ode.hip": ["-mllvm", "-disable-machine-licm"]}
 
 
 def build(verbose: bool = False) -> str:
@@ -37,7 +30,7 @@ def build(verbose: bool = False) -> str:
     procs, objs = [], []
     for s in srcs:
         obj = os.path.join(objdir, s + ".o")
-        cmd = [HIPCC, *HIP_FLAGS, *SOURCE_FLAGS.get(s, []), "-c", "-o", obj, os.path.join(CSRC, s)]
+        cmd = [HIPCC, *HIP_FLAGS, "-c", "-o", obj, os.path.join(CSRC, s)]
         if verbose:
             print(" ".join(cmd), flush=True)
         procs.append((s, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))

@@ -28,10 +28,6 @@ struct gal_ode_batch {
   double* d_params = nullptr;
   double* d_table = nullptr;
   unsigned int* d_work = nullptr;
-  double* d_ywork = nullptr;  // lane-private state/scales for two workgroups per CU
-  int ywork_lanes = 0;
-  double* d_kwork = nullptr;  // lane-private stage derivatives for four workgroups per CU
-  int kwork_lanes = 0;
   int* d_order = nullptr;
   // claim order planned by gal_ode_batch_plan_d in d_order, for the next
   // gal_ode_batch_evolve_planned_d of the same y, n and ld

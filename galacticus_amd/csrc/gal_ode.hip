@@ -1,10 +1,11 @@
 // gal_ode.hip -- batched node-ODE evolution on MI355X (gfx950) and its C ABI.
 //
-// One lane owns one node.  A persistent grid of workgroups claims nodes from
-// a global counter (one atomic per wave per refill) and integrates each from
-// t_start to t_end with the Cash-Karp (4,5) pair, the scaled error norm and
-// step controller, the driver loop and the node-evolver trial loop of the
-// reference:
+// A group of 64 nodes is served by one workgroup of four waves, one wave on
+// each SIMD of a CU and one lane position per node.  A persistent grid of
+// groups claims nodes from a global counter (one atomic per refill) and
+// integrates each from t_start to t_end with the Cash-Karp (4,5) pair, the
+// scaled error norm and step controller, the driver loop and the node-evolver
+// trial loop of the reference:
 //   trial loop    node_evolver/standard.F90:587-740
 //   solve         numerical/ODE_solver/solver.F90:492-691
 //   driver        external/gslODEInitVal2/driver2.c:148-250
@@ -13,27 +14,16 @@
 // When a lane's node finishes it claims the next one, so lanes stay busy
 // while step counts differ by two orders of magnitude between nodes.
 //
-// Schedule.  The lanes of a wave advance in lockstep through a six-phase
-// loop, one Cash-Karp attempt per trip:
-//   phases 0-4  stage inputs for k2..k6, RHS, store (phase 4: combine,
-//               error norm, controller, accept / reject / fail)
-//   phase 5     claim nodes for lanes that finished, then one shared RHS
-//               slot at (t, y): dydt at the new point (the reference's
-//               dydt_out, reused as the next k1), or k1 of a freshly claimed
-//               node, or k1 after a trial restart.
-// There is a single RHS call site, every lane spends six RHS evaluations per
-// trip whatever it is doing, and the RHS never diverges by phase.
+// Schedule.  The lanes of a group advance in lockstep, one Cash-Karp attempt
+// per trip: the derivative at (t, y) -- dydt at the new point (the reference's
+// dydt_out, reused as the next k1), k1 of a freshly claimed node, or k1 after a
+// trial restart -- then the five stages of k2..k6, the solution, its error norm
+// and the controller.  Every lane spends six RHS evaluations per trip whatever
+// it is doing, and the RHS never diverges by stage.
 //
 // Memory.  State is structure-of-arrays in HBM (y[v*ld + i]); it is read once
-// when a node is claimed and written once when it finishes.  Within a node,
-// the RHS input and output stay in registers, and the five stage
-// derivatives k1..k5, the state y and the error scales live in a
-// lane-private, bank-conflict-free layout L[(vec*30 + v)*BLOCK + lane]
-// (7*30*8 = 1680 bytes per lane): all in LDS (105 KiB per 64-lane
-// workgroup), or part of them in an HBM workspace of the same layout so that
-// two or four workgroups share a CU (see evolve_kernel).  Nothing is
-// addressable private memory, so the long dependent chain of a node never
-// waits on scratch.
+// when a node is claimed and written once when it finishes.  In between the
+// integrator's state is in registers and in the group's LDS (see group_wave).
 #include <hip/hip_runtime.h>
 #include <cstddef>
 #include <cstdint>
@@ -50,15 +40,13 @@
 #include "integrator.hpp"
 #include "batch.hpp"
 #include "events.hpp"
+#include "group_rhs.hpp"
 
 #include <hipcub/device/device_radix_sort.hpp>
 
 using namespace gal;
 
 namespace {
-
-constexpr int kStages = 5;  // k1..k5 kept; k6 is consumed as it is produced
-constexpr int kLdsVectors = kStages + 2;  // k1..k5, y, scales
 
 struct EvolveArgs {
   int n, ld;
@@ -74,9 +62,6 @@ struct EvolveArgs {
   long long* counters;
   const int* order;
   unsigned int* work;
-  double* ywork;  // per-lane state and scales in HBM (variant without them in LDS)
-  int ystride;    // lanes in the grid (ywork holds 2*30 doubles per lane)
-  double* kwork;  // per-lane stage derivatives in HBM (variant without them in LDS)
   const double* P;
   const double* tab;
   DerivedConstants D;
@@ -124,593 +109,557 @@ __device__ __forceinline__ void write_counters(const EvolveArgs& a, int node, lo
   }
 }
 
-// Three placements of the lane-private vectors (each [vector][variable][lane]
-// per workgroup, so a wave touches 64 consecutive doubles per variable):
-//  YLDS && KLDS:  stage derivatives, state and error scales in LDS (105 KiB
-//                 per 64 lanes: one workgroup per CU);
-//  !YLDS && KLDS: state and scales in an HBM workspace, stages in LDS
-//                 (75 KiB: two workgroups per CU);
-//  YLDS && !KLDS: stages in an HBM workspace, state and scales in LDS
-//                 (30 KiB: four workgroups per CU, one wave on every SIMD).
-// The arithmetic is the same in all three; only where the operands wait
-// between phases differs.
-//
-// WAVES = 2 gives each group of BLOCK nodes a second wave, on another SIMD of
-// the CU, that computes the hot-halo half of every RHS while the first wave
-// computes the galaxy half and runs the integrator.  One wave64 instruction
-// costs the same issue time however many of its lanes are active, so a
-// node's chain of RHS evaluations -- which sets the launch time when a few
-// stiff nodes take thousands of attempts -- shortens by the share of the
-// RHS the second wave takes.  Per RHS the first wave publishes the stage
-// state in LDS and a command (compute, skip, quit); barrier; both halves;
-// barrier; the first wave adds the second's derivatives.  Only the first
-// wave touches the integrator's state; the exchange area is written by one
-// wave and read by the other on opposite sides of a barrier.
-constexpr int kXchgVectors = kNV + 1 + 7 + kNV;   // stage state and time, node parameters, hot-half derivatives
-enum : int { kCmdCompute = 1, kCmdSkip = 2, kCmdQuit = 3 };
-
-template <int BLOCK, bool YLDS, bool KLDS>
-constexpr size_t lds_vector_bytes() {
-  return sizeof(double) * ((YLDS ? 2 : 0) + (KLDS ? kStages : 0)) * kNV * BLOCK;
-}
-
-// The kernel's one argument starts the kernarg segment: the derived constants
-// and table descriptor are read from there through an offset the compiler
-// cannot prove constant, so their scalar loads stay inside each RHS instead
-// of being hoisted and held (and spilled) across the whole integration.
-struct UniformRefs {
-  const double* P;
-  const DerivedConstants* D;
-  const CoolingDesc* C;
+// What a lane of the cooling wave keeps about the node it claimed last.
+struct ClaimState {
+  int op = -1, pend = -1;              // graph mode: operation in hand, claimed ready-list entry
+  unsigned int wait_tail = ~0u;        // graph mode: appends seen while waiting on the entry
+  unsigned long long wait_since = 0ull;
 };
-__device__ __forceinline__ UniformRefs uniform_refs(const double* P) {
-  int opaque = 0;
-  asm volatile("" : "+s"(opaque));
-  opaque = __builtin_amdgcn_readfirstlane(opaque);
-  const char* kargs = (const char*)__builtin_amdgcn_kernarg_segment_ptr() + opaque;
-  return UniformRefs{P + opaque, (const DerivedConstants*)(kargs + offsetof(EvolveArgs, D)),
-                     (const CoolingDesc*)(kargs + offsetof(EvolveArgs, cd))};
-}
+// Rounds of an attempt: the time part alone (new nodes), the derivative at its
+// start, then the stages 0-4 that give k2-k6.
+enum : int { kTimeOnly = -2, kFirst = -1, kLast = 4 };
+enum : int { kNoClaim = -1, kExhausted = -2 };   // codes of the claim vector beside a node index
 
-template <int BLOCK>
-__device__ __forceinline__ void rhs_coprocessor(const double* P, const double* __restrict__ tab, int mode,
-                                                double* __restrict__ xchg, volatile int* cmd) {
-  const int lane = threadIdx.x - BLOCK;
-  double* __restrict__ X = xchg + lane;
-  for (;;) {
-    __syncthreads();   // stage state published
-    const int c = __builtin_amdgcn_readfirstlane(*cmd);
-    if (c == kCmdQuit) break;
-    if (c == kCmdCompute) {
-      double yy[kNV], fh[kNV];
+// Claim a node's interval for each lane that wants one (cooling wave) and
+// publish it, or why there is none, in the claim vectors of the exchange
+// area.
+template <bool GRAPH>
+__device__ __forceinline__ void claim_nodes(const EvolveArgs& a, int n_claim, bool want, ClaimState& c,
+                                            double* __restrict__ C) {
+  auto publish = [&](int node, double t0, double t1, const double* np, size_t stride) {
+    C[kXClaimNode * kGroupNodes] = (double)node;
+    C[kXClaimT0 * kGroupNodes] = t0;
+    C[kXClaimT1 * kGroupNodes] = t1;
+    C[kXClaimStep * kGroupNodes] = a.h_step[node];
 #pragma unroll
-      for (int v = 0; v < kNV; ++v) yy[v] = X[v * BLOCK];
-      const double ts = X[kNV * BLOCK];
-      NodePar np;
-      np.t_ref = X[(kNV + 1) * BLOCK];
-      np.m_ref = X[(kNV + 2) * BLOCK];
-      np.m_rate = X[(kNV + 3) * BLOCK];
-      np.spin_rate = X[(kNV + 4) * BLOCK];
-      np.ram_force = X[(kNV + 5) * BLOCK];
-      np.v_host = X[(kNV + 6) * BLOCK];
-      np.satellite = X[(kNV + 7) * BLOCK] != 0.0;
-      const UniformRefs u = uniform_refs(P);
-      rhs_part<kRhsHalo>(u.P, *u.D, tab, *u.C, mode, np, ts, yy, fh);
-#pragma unroll
-      for (int v = 0; v < kNV; ++v) X[(kNV + 8 + v) * BLOCK] = fh[v];
+    for (int k = 0; k < GAL_NPARAM_NODE; ++k) C[(kXClaimPar + k) * kGroupNodes] = np[k * stride];
+  };
+  C[kXClaimNode * kGroupNodes] = (double)kNoClaim;
+  if constexpr (GRAPH) {
+    // claim an entry of the ready list, then wait for it to be written;
+    // events are applied on the spot and their successors released
+    bool again = true;
+    while (again) {
+      const bool need = want && c.pend < 0;
+      if (__any(need)) {
+        const int j = wave_claim(need, a.work, a.g.n, nullptr);
+        if (need) {
+          if (j < 0) {
+            want = false;
+            C[kXClaimNode * kGroupNodes] = (double)kExhausted;
+          } else {
+            c.pend = j;
+            c.wait_tail = ~0u;
+          }
+        }
+      }
+      if (want && c.pend >= 0) {
+        const int k = graph_ready_entry(a.g, c.pend);
+        if (k >= 0) {
+          c.pend = -1;
+          const gal_schedule_op* o = a.g.ops + k;
+          const int kind = o->kind;
+          if (kind != GAL_OP_EVOLVE) {
+            apply_event(kind, (size_t)o->a, (size_t)o->b, a.ld, a.y, a.h_step, a.g.major_ratio);
+            graph_release(a.g, k);
+          } else {
+            c.op = k;
+            publish(o->a, o->t0, o->t1, o->node_par, 1);
+            want = false;
+          }
+        } else {
+          const unsigned int tl = __hip_atomic_load(a.g.tail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          const unsigned long long now = wall_clock64();
+          if (tl != c.wait_tail) {
+            c.wait_tail = tl;
+            c.wait_since = now;
+          } else if (now - c.wait_since > a.stall_ticks) {
+            __hip_atomic_store(a.graph_error, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            want = false;
+            c.pend = -1;
+            C[kXClaimNode * kGroupNodes] = (double)kExhausted;
+          }
+        }
+      }
+      again = __any(want && c.pend < 0);
     }
-    __syncthreads();   // hot-half derivatives published
+  } else {
+    // an order entry outside the batch (a plan the caller did not let finish)
+    // ends this lane's claims instead of addressing past it
+    const int claimed = wave_claim(want, a.work, n_claim, a.order);
+    if (want) {
+      if (claimed < 0 || claimed >= a.n) C[kXClaimNode * kGroupNodes] = (double)kExhausted;
+      else publish(claimed, a.t_start[claimed], a.t_end[claimed], a.np + claimed, (size_t)a.ld);
+    }
   }
 }
 
-template <int BLOCK, bool YLDS, bool KLDS, int WAVES = 1, bool GRAPH = false>
-__global__ __launch_bounds__(BLOCK * WAVES, 1) void evolve_kernel(EvolveArgs a) {
-  extern __shared__ double lds_k[];
-  __shared__ int xchg_cmd;
-  double* __restrict__ xchg = lds_k + lds_vector_bytes<BLOCK, YLDS, KLDS>() / sizeof(double);
-  if constexpr (WAVES == 2) {
-    if (threadIdx.x >= BLOCK) {
-      rhs_coprocessor<BLOCK>(a.P, a.tab, a.mode, xchg, &xchg_cmd);
-      return;
-    }
-  }
-  double* __restrict__ XC = xchg + threadIdx.x;    // this lane's column of the exchange area
-  double* __restrict__ K = lds_k + threadIdx.x;   // K[(s*kNV + v)*BLOCK] when KLDS
-  // In the HBM workspace the stage vectors are reached through a buffer
-  // resource over the workgroup's slab: the lane offset sits in one VGPR and
-  // the per-vector offsets in SGPRs, so 150 addresses cost no registers.
-  const __amdgpu_buffer_rsrc_t krs = __builtin_amdgcn_make_buffer_rsrc(
-      KLDS ? nullptr : a.kwork + (size_t)blockIdx.x * (kStages * kNV * BLOCK), (short)0,
-      (int)(sizeof(double) * kStages * kNV * BLOCK), 0x00020000);
-  const int k_lane = (int)(threadIdx.x * sizeof(double));
-  using B64 = decltype(__builtin_amdgcn_raw_buffer_load_b64(krs, 0, 0, 0));
-  auto kget = [&](int st, int v) -> double {
-    if constexpr (KLDS) {
-      return K[(st * kNV + v) * BLOCK];
-    } else {
-      return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(
-                                            krs, k_lane, (int)sizeof(double) * (st * kNV + v) * BLOCK, 0));
-    }
-  };
-  auto kset = [&](int st, int v, double x) {
-    if constexpr (KLDS) {
-      K[(st * kNV + v) * BLOCK] = x;
-    } else {
-      const int su = __builtin_amdgcn_readfirstlane(st);   // the phase is uniform over the wave
-      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(B64, x), krs, k_lane,
-                                            (int)sizeof(double) * (su * kNV + v) * BLOCK, 0);
-    }
-  };
-  const double* __restrict__ P = a.P;
+// Persistent integrator: a workgroup of four waves serves 64 nodes, one per
+// lane position, and group_rhs.hpp deals the RHS out over the waves.  The
+// integrator's state is in registers, split by variable: wave w (of the first
+// three) owns variables [10 w, 10 w + 10) of every node -- state, stage
+// derivatives and error scales -- and forms their stage inputs, solution and
+// error norm; LDS only carries what waves exchange.  What steers a node
+// (times, step size, trial, flags) is held by all four waves alike: each runs
+// the same code on the same published values, so they agree without a
+// message.  The cooling wave owns no variables and does what needs one wave:
+// claims, statuses, counters, the wall clock.
+//
+// The step controller's pow is not on the path: whether a step is accepted
+// follows from the error norm alone, and the derivative at the new point does
+// not depend on the step size, so the time wave computes the next step size
+// during that evaluation (which also decides a step-size underflow).
+//
+// Measured on the stiffest node of 100,000 isolated halos (3701 attempts): 22.6
+// us an attempt, against 43 us with one wave for the whole RHS and its stage
+// vectors in LDS, or two waves that split it in halves; evolving all 100,000
+// takes 44.8 ms instead of 85.6.
+//
+// One instance of this per wave of the group: a lone wave issues one
+// instruction every 4.6 cycles whatever it is (a dependent FP64 FMA costs no
+// more than an independent one, and a move of half a constant as much as
+// either), so the instruction count of each wave is what there is to save.
+// With a loop of its own a wave keeps the constants of its own transcendental
+// functions in registers across the integration.
+template <int WAVE, bool GRAPH>
+__device__ __forceinline__ void group_wave(const EvolveArgs& a, double* __restrict__ X,
+                                           const GroupConstants& constants, int* __restrict__ norm_flags,
+                                           int* __restrict__ flags, int& wall_expired) {
+  // in registers for the whole integration, as far as this wave uses them
+  const GroupConstants G = constants;
+  constexpr int wave = WAVE;
+  constexpr bool owner = wave < kOwnerWaves;
+  constexpr int v0 = owner ? wave * kOwned : 0;    // first owned variable
+  const int lane = threadIdx.x & (kGroupNodes - 1);
+  double* __restrict__ XY = X + (kXState + v0) * kGroupNodes;   // owned rows (owners only)
+  double* __restrict__ XG = X + (kXGalaxy + v0) * kGroupNodes;
+  double* __restrict__ XH = X + (kXHalo + v0) * kGroupNodes;
+  double* __restrict__ XK = X + (kXStage + v0) * kGroupNodes;
   const int mode = a.mode;
+  const int ops = mode == GAL_PHYSICS_STANDARD ? (int)a.P[GAL_P_OPERATORS] : 0;
   const bool reuse = (a.flags & GAL_FLAG_REUSE_STEP_SIZE) != 0;
   const bool enforce = (a.flags & GAL_FLAG_ENFORCE_NON_NEGATIVITY) != 0;
   const bool scales_given = (a.flags & GAL_FLAG_SCALES_PROVIDED) != 0;
-#define KS(s, v) kget((s), (v))
+  // owned variables that may not be negative, and those the post-step fixes
+  constexpr unsigned nonneg = kNonNegative >> v0;
+  const bool galaxy_fix = a.P[GAL_P_POST_STEP_ZERO_NEGATIVE_MASSES] != 0.0;
+  const unsigned fixable =
+      (mode == GAL_PHYSICS_TEST ? 0u : kPostStepHalo | (galaxy_fix ? kPostStepGalaxy : 0u)) >> v0;
 
-  // Both layouts are [vector][variable][lane] per workgroup: a wave reads
-  // 64 consecutive doubles per variable.
-  constexpr int ys = BLOCK;
-  double* __restrict__ YL = YLDS ? lds_k + (KLDS ? kStages * kNV * BLOCK : 0) + threadIdx.x
-                                 : a.ywork + (size_t)blockIdx.x * (2 * kNV * BLOCK) + threadIdx.x;
-  double* __restrict__ SL = YL + kNV * BLOCK;
-#define Y(v) YL[(v) * ys]
-#define SC(v) SL[(v) * ys]
-  // Partial sums over the stage derivatives already in memory, formed while
-  // an RHS is in flight: for phases 0-3 the next stage's input sum without
-  // its newest term; for phase 4 the fifth-order solution's sum without k6.
-  // Each is completed, in the order of the full sum, once the newest
-  // derivative is known.
-  // Coefficients of the newest term of the stage input that follows phase ph (0-3).
-  auto stage_b_new = [](int ph) {
-    return ph == 0 ? ck::b32 : (ph == 1 ? ck::b43 : (ph == 2 ? ck::b54 : ck::b65));
-  };
-  auto stage_a_new = [](int ph) { return ph == 0 ? ck::a3 : (ph == 1 ? ck::a4 : (ph == 2 ? ck::a5 : ck::a6)); };
-  // The LDS operands are gathered ten variables at a time before the
-  // arithmetic, so that their reads are in flight together rather than one
-  // read-and-wait per variable.
-  constexpr int kChunk = 10;
-  static_assert(kNV % kChunk == 0, "chunks must tile the state");
-  auto stage_partials = [&](double (&sp)[kNV], int ph, bool act) {
-    if (!act) return;
-#pragma unroll
-    for (int c = 0; c < kNV; c += kChunk) {
-      double g0[kChunk], g1[kChunk], g2[kChunk], g3[kChunk];
-      switch (ph) {
-        case 0:
-#pragma unroll
-          for (int i = 0; i < kChunk; ++i) g0[i] = KS(0, c + i);
-#pragma unroll
-          for (int i = 0; i < kChunk; ++i) sp[c + i] = ck::b31 * g0[i];
-          break;
-        case 1:
-#pragma unroll
-          for (int i = 0; i < kChunk; ++i) { g0[i] = KS(0, c + i); g1[i] = KS(1, c + i); }
-#pragma unroll
-          for (int i = 0; i < kChunk; ++i) sp[c + i] = ck::b41 * g0[i] + ck::b42 * g1[i];
-          break;
-        case 2:
-#pragma unroll
-          for (int i = 0; i < kChunk; ++i) { g0[i] = KS(0, c + i); g1[i] = KS(1, c + i); g2[i] = KS(2, c + i); }
-#pragma unroll
-          for (int i = 0; i < kChunk; ++i) sp[c + i] = ck::b51 * g0[i] + ck::b52 * g1[i] + ck::b53 * g2[i];
-          break;
-        case 3:
-#pragma unroll
-          for (int i = 0; i < kChunk; ++i) {
-            g0[i] = KS(0, c + i); g1[i] = KS(1, c + i); g2[i] = KS(2, c + i); g3[i] = KS(3, c + i);
-          }
-#pragma unroll
-          for (int i = 0; i < kChunk; ++i)
-            sp[c + i] = ck::b61 * g0[i] + ck::b62 * g1[i] + ck::b63 * g2[i] + ck::b64 * g3[i];
-          break;
-        case 4:
-#pragma unroll
-          for (int i = 0; i < kChunk; ++i) { g0[i] = KS(0, c + i); g2[i] = KS(2, c + i); g3[i] = KS(3, c + i); }
-#pragma unroll
-          for (int i = 0; i < kChunk; ++i) sp[c + i] = ck::c1 * g0[i] + ck::c3 * g2[i] + ck::c4 * g3[i];
-          break;
-        default:
-          break;
-      }
-    }
-  };
+  // steering, alike in all four waves
   NodePar np{};
-  int node = -1;
-  int op = -1, pend = -1;                  // graph mode: operation in hand, claimed ready-list entry
-  unsigned int wait_tail = ~0u;            // graph mode: appends seen while waiting on the entry
-  unsigned long long wait_since = 0ull;
-  bool active = false, want = true, eval_pending = false, post_pending = false, final_step = false;
+  int node = -1, trial = 0;
+  bool active = false, want = true, eval = false, post = false, decide = false, final_step = false;
   double t = 0.0, t0 = 0.0, t1 = 0.0, h = 0.0, h0 = 0.0, h_node = 0.0, sign = 1.0;
-  int trial = 0;
+  ErrorNorm en;
+  int need_fix = 0;
+  bool time_stale = false;
+  int round = 0;
+  int tb = 0;              // time part of the coming stage: kXTime + tb * kTimeVectors
+  // owners
+  double y[kOwned], sc[kOwned];
+#pragma unroll
+  for (int i = 0; i < kOwned; ++i) y[i] = sc[i] = 0.0;
+  auto K = [&](int stage, int i) -> double& { return XK[(stage * kNV + i) * kGroupNodes]; };
+  // cooling wave
+  ClaimState claim;
   long long n_attempt = 0, n_accept = 0, n_rhs = 0;
   const int n_claim = a.n_claim_dev ? *a.n_claim_dev : a.n_claim;
-
-  int phase = 5;
-  double ts = 0.0;   // time of the stage input ytmp (carried over for phases 1-4)
   const unsigned long long t_launch = a.wall_ticks ? wall_clock64() : 0ull;
-  for (;;) {
-    // Stage input, stage derivative and partial sums: rewritten before every
-    // use within an iteration, so nothing of them is carried round the loop.
-    double ytmp[kNV], kout[kNV], sp[kNV];
-    bool do_rhs = false;
-    if (phase == 5) {
-      // ---- claim nodes for lanes that need one (convergent point) ------
-      bool again = true;
-      while (again) {
-        bool begun = false;   // this lane takes a node's interval
-        if constexpr (GRAPH) {
-          // claim an entry of the ready list, then wait for it to be written;
-          // events are applied on the spot and their successors released
-          const bool need = want && pend < 0;
-          if (__any(need)) {
-            const int j = wave_claim(need, a.work, a.g.n, nullptr);
-            if (need) {
-              if (j < 0) {
-                want = false;
-                active = false;
-              } else {
-                pend = j;
-                wait_tail = ~0u;
-              }
-            }
-          }
-          if (want && pend >= 0) {
-            const int k = graph_ready_entry(a.g, pend);
-            if (k >= 0) {
-              pend = -1;
-              const gal_schedule_op* o = a.g.ops + k;
-              const int kind = o->kind;
-              if (kind != GAL_OP_EVOLVE) {
-                apply_event(kind, (size_t)o->a, (size_t)o->b, a.ld, a.y, a.h_step, a.g.major_ratio);
-                graph_release(a.g, k);
-              } else {
-                op = k;
-                node = o->a;
-                np = load_node_par(o->node_par, 1, 0);
-                t0 = o->t0;
-                t1 = o->t1;
-                begun = true;
-              }
-            } else {
-              const unsigned int tl = __hip_atomic_load(a.g.tail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-              const unsigned long long now = wall_clock64();
-              if (tl != wait_tail) {
-                wait_tail = tl;
-                wait_since = now;
-              } else if (now - wait_since > a.stall_ticks) {
-                __hip_atomic_store(a.graph_error, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                want = false;
-                pend = -1;
-              }
-            }
-          }
-        } else {
-          // an order entry outside the batch (a plan the caller did not let
-          // finish) ends this lane's claims instead of addressing past it
-          const int claimed = wave_claim(want, a.work, n_claim, a.order);
-          const int idx = claimed < a.n ? claimed : -1;
-          if (want) {
-            if (idx < 0) {
-              want = false;
-              active = false;
-            } else {
-              node = idx;
-              np = load_node_par(a.np, a.ld, node);
-              t0 = a.t_start[node];
-              t1 = a.t_end[node];
-              begun = true;
-            }
-          }
-        }
-        if (begun) {
-          if constexpr (WAVES == 2) {
-            XC[(kNV + 1) * BLOCK] = np.t_ref;
-            XC[(kNV + 2) * BLOCK] = np.m_ref;
-            XC[(kNV + 3) * BLOCK] = np.m_rate;
-            XC[(kNV + 4) * BLOCK] = np.spin_rate;
-            XC[(kNV + 5) * BLOCK] = np.ram_force;
-            XC[(kNV + 6) * BLOCK] = np.v_host;
-            XC[(kNV + 7) * BLOCK] = np.satellite ? 1.0 : 0.0;
-          }
-          h_node = a.h_step[node];
+
+  // The first step of a trial (solver.F90:537-555)
+  auto start_trial = [&](double step_size) {
+    double xs = t1 - t0;
+    if (step_size > 0.0) xs = fmin(step_size, xs);
+    h = xs;
+    h0 = xs;
+    t = t0;
+    eval = true;
+  };
+  // Results of a lane's interval (cooling wave); its state is stored by the
+  // owners beforehand, and in graph mode its successors are released.
+  auto finish = [&](bool done, double h_out, bool write_h, int status) {
+    if (wave == kCoolingWave && done) {
+      if (write_h) a.h_step[node] = h_out;
+      a.status[node] = status;
+      write_counters(a, node, n_attempt, n_accept, n_rhs);
+    }
+    if constexpr (GRAPH) {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+      __syncthreads();
+      if (wave == kCoolingWave && done) graph_release(a.g, claim.op);
+    }
+    if (done) {
+      active = false;
+      want = true;
+    }
+  };
+  auto store_state = [&](bool done) {
+    if (owner && done) {
 #pragma unroll
-          for (int v = 0; v < kNV; ++v) ytmp[v] = a.y[v * (size_t)a.ld + node];
+      for (int i = 0; i < kOwned; ++i) a.y[(size_t)(v0 + i) * a.ld + node] = y[i];
+    }
+  };
+  // The reference's negative-value fixes on the published state of the given
+  // lanes (rare): one wave fixes, the owners take their variables back.
+  auto fix_published = [&](bool lanes) {
+    if (wave == kCoolingWave && lanes) post_step(constants.P, constants.D, np, mode, t, X + kXState * kGroupNodes, kGroupNodes);
+    __syncthreads();
+    if (owner && lanes) {
+#pragma unroll
+      for (int i = 0; i < kOwned; ++i) y[i] = XY[i * kGroupNodes];
+    }
+  };
+
+  // The sums over the older stage derivatives, formed beside the RHS; each is
+  // completed once the newest derivative is known.
+  double sp[kOwned];
+  auto older_terms = [&](int ph) {
+    if constexpr (owner) {
+#pragma clang fp contract(off)
+#pragma unroll
+      for (int i = 0; i < kOwned; ++i) sp[i] = 0.0;
+      if (ph == 0) {
+#pragma unroll
+        for (int i = 0; i < kOwned; ++i) sp[i] = ck::b31 * K(0, i);
+      } else if (ph == 1) {
+#pragma unroll
+        for (int i = 0; i < kOwned; ++i) sp[i] = fma(ck::b41, K(0, i), ck::b42 * K(1, i));
+      } else if (ph == 2) {
+#pragma unroll
+        for (int i = 0; i < kOwned; ++i) sp[i] = fma(ck::b53, K(2, i), fma(ck::b52, K(1, i), ck::b51 * K(0, i)));
+      } else if (ph == 3) {
+#pragma unroll
+        for (int i = 0; i < kOwned; ++i)
+          sp[i] = fma(ck::b64, K(3, i), fma(ck::b63, K(2, i), fma(ck::b61, K(0, i), ck::b62 * K(1, i))));
+      } else if (ph == kLast) {
+#pragma unroll
+        for (int i = 0; i < kOwned; ++i) sp[i] = fma(ck::c4, K(3, i), fma(ck::c1, K(0, i), ck::c3 * K(2, i)));
+      }
+    }
+  };
+
+  for (;;) {
+    // ---- claims ------------------------------------------------------------
+    bool begun = false, zero_length = false;
+    if (__any(want)) {
+      double* C = X + (kXTime + (tb ^ 1) * kTimeVectors) * kGroupNodes;
+      if (wave == kCoolingWave) claim_nodes<GRAPH>(a, n_claim, want, claim, C);
+      __syncthreads();
+      const int code = (int)C[kXClaimNode * kGroupNodes];
+      if (want && code == kExhausted) want = false;
+      begun = want && code >= 0;
+      if (begun) {
+        node = code;
+        t0 = C[kXClaimT0 * kGroupNodes];
+        t1 = C[kXClaimT1 * kGroupNodes];
+        h_node = C[kXClaimStep * kGroupNodes];
+        np = load_node_par(C + kXClaimPar * kGroupNodes, kGroupNodes, 0);
+        want = false;
+        active = true;
+        trial = 0;
+        post = decide = false;
+        n_attempt = n_accept = n_rhs = 0;
+        zero_length = t0 == t1;
+        start_trial(reuse ? h_node : -1.0);
+        sign = h > 0.0 ? 1.0 : -1.0;
+        eval = !zero_length;
+        if (owner) {
+#pragma unroll
+          for (int i = 0; i < kOwned; ++i) y[i] = a.y[(size_t)(v0 + i) * a.ld + node];
           if (scales_given) {
 #pragma unroll
-            for (int v = 0; v < kNV; ++v) kout[v] = a.scale[v * (size_t)a.ld + node];
-          } else if (mode == GAL_PHYSICS_TEST) {
-#pragma unroll
-            for (int v = 0; v < kNV; ++v) kout[v] = 1.0;
-          } else {
-            scales(P, a.D, np, t0, ytmp, kout);
+            for (int i = 0; i < kOwned; ++i) sc[i] = a.scale[(size_t)(v0 + i) * a.ld + node];
           }
-          if (!scales_given && a.scale) {
-#pragma unroll
-            for (int v = 0; v < kNV; ++v) a.scale[v * (size_t)a.ld + node] = kout[v];
-          }
-#pragma unroll
-          for (int v = 0; v < kNV; ++v) {
-            Y(v) = ytmp[v];
-            SC(v) = kout[v];
-          }
-          n_attempt = n_accept = n_rhs = 0;
-          trial = 0;
-          if (t0 == t1) {
-            // nothing to integrate (standard.F90:580): success, timeStep -1
-            a.h_step[node] = -1.0;
-            a.status[node] = GAL_STATUS_SUCCESS;
-            write_counters(a, node, 0, 0, 0);
-            if constexpr (GRAPH) graph_release(a.g, op);
-          } else {
-            want = false;
-            active = true;
-            // odeSolverSolve initial step (solver.F90:537-555)
-            const double step_size = reuse ? h_node : -1.0;
-            double xs = t1 - t0;
-            if (step_size > 0.0) xs = fmin(step_size, xs);
-            h = xs;
-            h0 = h;
-            sign = h > 0.0 ? 1.0 : -1.0;
-            t = t0;
-            eval_pending = true;
-          }
-        }
-        if constexpr (GRAPH) again = __any(want && pend < 0);
-        else again = __any(want);
-      }
-      if (eval_pending) {
-        do_rhs = true;
-        ts = t;
-#pragma unroll
-        for (int v = 0; v < kNV; ++v) ytmp[v] = Y(v);
-      }
-    } else if (active) {
-      do_rhs = true;
-      switch (phase) {
-        case 0: {
-          // Wall-time limit (node_evolver/standard.F90:693-705 and the RHS's
-          // own check, standard.F90:860-866): the node returns
-          // errorStatusXCPU with its state as it came in.
-          if (a.wall_ticks && wall_clock64() - t_launch > a.wall_ticks) {
-            a.status[node] = GAL_STATUS_XCPU;
-            write_counters(a, node, n_attempt, n_accept, n_rhs);
-            if constexpr (GRAPH) graph_release(a.g, op);
-            active = false;
-            want = true;
-            do_rhs = false;
-            break;
-          }
-          // gsl_odeiv2_evolve_apply: clip the step to reach t1 exactly
-          const double dt = t1 - t;
-          final_step = false;
-          if ((dt >= 0.0 && h0 > dt) || (dt < 0.0 && h0 < dt)) {
-            h0 = dt;
-            final_step = true;
-          }
-          ++n_attempt;
-          ts = t + ck::a2 * h0;
-#pragma unroll
-          for (int c = 0; c < kNV; c += kChunk) {
-            double gy[kChunk], gk[kChunk];
-#pragma unroll
-            for (int i = 0; i < kChunk; ++i) { gy[i] = Y(c + i); gk[i] = KS(0, c + i); }
-#pragma unroll
-            for (int i = 0; i < kChunk; ++i) ytmp[c + i] = gy[i] + h0 * (ck::b21 * gk[i]);
-          }
-          break;
-        }
-        default:
-          // phases 1-4: y + h (sum of the older stage terms + the newest)
-          if constexpr (WAVES == 2) {
-            // formed at the end of the previous iteration, in the exchange area
-            ts = XC[kNV * BLOCK];
-#pragma unroll
-            for (int v = 0; v < kNV; ++v) ytmp[v] = XC[v * BLOCK];
-          } else {
-            stage_partials(sp, phase - 1, true);
-            const double b_new = stage_b_new(phase - 1);
-            ts = t + stage_a_new(phase - 1) * h0;
-#pragma unroll
-            for (int c = 0; c < kNV; c += kChunk) {
-              double gy[kChunk], gk[kChunk];
-#pragma unroll
-              for (int i = 0; i < kChunk; ++i) { gy[i] = Y(c + i); gk[i] = KS(phase, c + i); }
-#pragma unroll
-              for (int i = 0; i < kChunk; ++i) ytmp[c + i] = gy[i] + h0 * (sp[c + i] + b_new * gk[i]);
-            }
-          }
-          break;
-      }
-    }
-
-    if constexpr (WAVES == 2) {
-      const bool any_rhs = __any(do_rhs);
-      if (phase == 0 || phase == 5) {
-#pragma unroll
-        for (int v = 0; v < kNV; ++v) XC[v * BLOCK] = ytmp[v];
-        XC[kNV * BLOCK] = ts;
-      }
-      if (threadIdx.x == 0) xchg_cmd = any_rhs ? kCmdCompute : kCmdSkip;
-      __syncthreads();   // stage state published
-      if (do_rhs) {
-        const UniformRefs u = uniform_refs(P);
-        rhs_part<kRhsGalaxy>(u.P, *u.D, a.tab, *u.C, mode, np, ts, ytmp, kout);
-        ++n_rhs;
-      }
-      stage_partials(sp, phase, active);   // while the hot half is still in flight
-      __syncthreads();   // hot-half derivatives published
-      if (do_rhs) {
-        double kh[kNV];
-#pragma unroll
-        for (int v = 0; v < kNV; ++v) kh[v] = XC[(kNV + 8 + v) * BLOCK];
-#pragma unroll
-        for (int v = 0; v < kNV; ++v) kout[v] += kh[v];
-      }
-    } else {
-      if (do_rhs) {
-        const UniformRefs u = uniform_refs(P);
-        rhs(u.P, *u.D, a.tab, *u.C, mode, np, ts, ytmp, kout);
-        ++n_rhs;
-      }
-      if (phase == 4) stage_partials(sp, phase, active);
-    }
-
-    if (phase < 4) {
-      if (active) {
-#pragma unroll
-        for (int v = 0; v < kNV; ++v) kset(phase + 1, v, kout[v]);
-        if constexpr (WAVES == 2) {
-          // the next stage's input, straight into the exchange area (the
-          // other wave is past its reads and waits for the next publish)
-          const double b_new = stage_b_new(phase);
-          XC[kNV * BLOCK] = t + stage_a_new(phase) * h0;
-#pragma unroll
-          for (int c = 0; c < kNV; c += kChunk) {
-            double gy[kChunk];
-#pragma unroll
-            for (int i = 0; i < kChunk; ++i) gy[i] = Y(c + i);
-#pragma unroll
-            for (int i = 0; i < kChunk; ++i) XC[(c + i) * BLOCK] = gy[i] + h0 * (sp[c + i] + b_new * kout[c + i]);
-          }
-        }
-      }
-      ++phase;
-      continue;
-    }
-    if (phase == 5) {
-      if (eval_pending) {
-#pragma unroll
-        for (int v = 0; v < kNV; ++v) kset(0, v, kout[v]);
-        eval_pending = false;
-        if (post_pending) {
-          post_step(P, a.D, np, mode, t, &Y(0), ys);   // GSL_CONTINUE: no evolver reset
-          post_pending = false;
         }
       }
       if (!__any(active)) {
-        if constexpr (GRAPH) {
-          // lanes wait on ready-list entries: poll again after a pause
-          if (__any(want)) {
-            __builtin_amdgcn_s_sleep(8);
-            continue;
+        __syncthreads();   // the claim vectors are free again
+        if (!__any(want)) break;
+        // graph mode: lanes wait on ready-list entries; poll again after a pause
+        __builtin_amdgcn_s_sleep(8);
+        continue;
+      }
+    } else if (!__any(active)) {
+      break;
+    }
+    // ---- the derivative at (t, y), and one Cash-Karp attempt ------------------
+    if (owner) {
+#pragma unroll
+      for (int i = 0; i < kOwned; ++i) XY[i * kGroupNodes] = y[i];
+    }
+    // The time part of the first derivative was computed ahead for lanes that
+    // go on; for new ones an extra round computes it (all lanes; the others'
+    // comes out as it was).
+    const bool stale = time_stale || __any(begun);
+    time_stale = false;
+    bool stepping = false;
+    for (int ph = stale ? kTimeOnly : kFirst; ph <= kLast; ++ph) {
+      const int xt = kXTime + tb * kTimeVectors;
+      ++round;
+      __syncthreads();   // stage state and time part published
+      if (ph == kFirst && !scales_given && owner && __any(begun)) {
+        double ys[kNV], s30[kNV];
+        load_state(X, ys);
+        const TimePart T = load_time_part(X + xt * kGroupNodes);
+        scales_of_halo(G.P, G.D, T.mass, T.r_vir, T.v_vir, galaxy_radius(T, ys[GAL_V_SPIN_ANGULAR_MOMENTUM]).r, ys, s30);
+        if (begun) {
+#pragma unroll
+          for (int i = 0; i < kOwned; ++i) sc[i] = mode == GAL_PHYSICS_TEST ? 1.0 : s30[v0 + i];
+          if (a.scale) {
+#pragma unroll
+            for (int i = 0; i < kOwned; ++i) a.scale[(size_t)(v0 + i) * a.ld + node] = sc[i];
           }
         }
-        if constexpr (WAVES == 2) {
-          if (threadIdx.x == 0) xchg_cmd = kCmdQuit;
+      }
+      if constexpr (wave == kTimeWave) {
+        older_terms(ph);   // its own work waits for nobody, so these come first
+        // the time of the next stage, or after the last one of the point that
+        // the step leads to if it is accepted
+        double tn = t;
+        if (ph == kFirst) {
+          const double hn = decide ? hadjust_step(en, kRkckOrder, h0) : h0;
+          X[kXStep * kGroupNodes] = hn;
+          const double dt = t1 - t;
+          const double hs = ((dt >= 0.0 && hn > dt) || (dt < 0.0 && hn < dt)) ? dt : hn;
+          tn = t + ck::a2 * hs;
+        } else if (ph == kLast) {
+          if (!eval) tn = final_step ? t1 : t + h0;
+        } else if (ph != kTimeOnly) {
+          const double an = ph == 0 ? ck::a3 : (ph == 1 ? ck::a4 : (ph == 2 ? ck::a5 : ck::a6));
+          tn = t + an * h0;
+        }
+        store_time_part(time_part(G.P, G.D, G.C, np, tn),
+                        X + (kXTime + (tb ^ 1) * kTimeVectors) * kGroupNodes);
+      } else if (ph != kTimeOnly) {
+        if constexpr (wave == kGalaxyWave) {
+          galaxy_wave_rhs(G, mode, ops, np, X, xt, flags, round);
+        } else if (mode == GAL_PHYSICS_STANDARD) {
+          if constexpr (wave == kProfileWave) profile_wave_rhs(G, ops, X, xt, flags, round);
+          if constexpr (wave == kCoolingWave) cooling_wave_rhs(G, a.tab, np, X, xt, flags, round);
+        }
+        if constexpr (wave == kCoolingWave) {
+          if (ph == kFirst ? eval : stepping) ++n_rhs;
+          if (ph == kFirst && a.wall_ticks && lane == 0) wall_expired = wall_clock64() - t_launch > a.wall_ticks;
+        }
+      }
+      if constexpr (wave != kTimeWave) older_terms(ph);
+      __syncthreads();   // derivatives published
+      tb ^= 1;
+      if (ph == kTimeOnly) continue;
+      double kn[kOwned];
+      if (owner) {
+#pragma unroll
+        for (int i = 0; i < kOwned; ++i) kn[i] = XG[i * kGroupNodes] + XH[i * kGroupNodes];
+      }
+      if (ph >= 0 && ph < kLast) {
+        // the next stage's input y + h (older terms + newest)
+        if (owner) {
+#pragma clang fp contract(off)
+          const double bn = ph == 0 ? ck::b32 : (ph == 1 ? ck::b43 : (ph == 2 ? ck::b54 : ck::b65));
+#pragma unroll
+          for (int i = 0; i < kOwned; ++i) XY[i * kGroupNodes] = fma(h0, fma(bn, kn[i], sp[i]), y[i]);
+#pragma unroll
+          for (int i = 0; i < kOwned; ++i) K(ph + 1, i) = kn[i];
+        }
+        continue;
+      }
+      if (ph == kFirst) {
+        if (owner && eval) {
+#pragma unroll
+          for (int i = 0; i < kOwned; ++i) K(0, i) = kn[i];
+        }
+        eval = false;
+        // GSL_CONTINUE: the post-step fixes leave the derivative as it is
+        const bool fix = post && need_fix != 0;
+        post = false;
+        if (__any(fix)) fix_published(fix);
+        const double hn = X[kXStep * kGroupNodes];
+        bool failed = false;
+        if (decide) {
+          if (hadjust_kind(en) == kHadjDec) {
+            const double t_adv = final_step ? t1 : t + h0;
+            if (fabs(hn) < fabs(h0) && t_adv + hn != t_adv) h0 = hn;   // rejected: retry, same k1
+            else failed = true;                                         // step size underflow
+          } else {
+            h = hn;
+            h0 = hn;
+          }
+          decide = false;
+        }
+        if (__any(zero_length)) {
+          // nothing to integrate (standard.F90:580): success, timeStep -1
+          finish(zero_length, -1.0, true, GAL_STATUS_SUCCESS);
+          zero_length = false;
+        }
+        if (__any(failed)) {
+          // node-evolver trial loop (standard.F90:657-692)
+          bool rescued = false;
+          if (enforce) {
+            if (owner) {
+              bool any = false;
+#pragma unroll
+              for (int i = 0; i < kOwned; ++i) any |= y[i] < 0.0 && ((nonneg >> i) & 1u);
+              norm_flags[wave * kGroupNodes + lane] = any ? 4 : 0;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int w = 0; w < kOwnerWaves; ++w) rescued |= (norm_flags[w * kGroupNodes + lane] & 4) != 0;
+            rescued = rescued && failed;
+            if (owner && rescued) {
+#pragma unroll
+              for (int i = 0; i < kOwned; ++i)
+                if (y[i] < 0.0 && ((nonneg >> i) & 1u)) y[i] = 0.0;
+            }
+            store_state(rescued);
+            if (__any(rescued)) finish(rescued, h_node / (double)(1 << trial), true, GAL_STATUS_SUCCESS);
+          }
+          const bool retry = failed && !rescued;
+          bool spent = false;
+          if (retry) {
+            spent = ++trial >= 8;
+            if (!spent) {
+              if (owner) {
+#pragma unroll
+                for (int i = 0; i < kOwned; ++i) y[i] = a.y[(size_t)(v0 + i) * a.ld + node];
+              }
+              start_trial(reuse ? h_node / (double)(1 << trial) : -1.0);
+            }
+          }
+          // all trials failed: state restored, errorStatusUnderflow (standard.F90:715-718)
+          if (__any(spent)) finish(spent, 0.0, false, GAL_STATUS_UNDERFLOW);
+        }
+        // Wall-time limit (node_evolver/standard.F90:693-705 and the RHS's own
+        // check, standard.F90:860-866): the nodes return errorStatusXCPU with
+        // their state as it came in.
+        if (a.wall_ticks && wall_expired && __any(active)) {
+          finish(active, 0.0, false, GAL_STATUS_XCPU);
+          eval = false;
+        }
+        stepping = active && !eval;
+        if (!__any(stepping)) {
+          time_stale = true;
+          break;
+        }
+        // gsl_odeiv2_evolve_apply: clip the step to reach t1 exactly
+        const double dt = t1 - t;
+        final_step = false;
+        if (stepping && ((dt >= 0.0 && h0 > dt) || (dt < 0.0 && h0 < dt))) {
+          h0 = dt;
+          final_step = true;
+        }
+        if (stepping) ++n_attempt;
+        if (owner) {
+#pragma clang fp contract(off)
+#pragma unroll
+          for (int i = 0; i < kOwned; ++i) XY[i * kGroupNodes] = fma(h0, ck::b21 * K(0, i), y[i]);
+        }
+        continue;
+      }
+      // ---- k6 is in kn: solution, error norm, controller ----------------------
+      double yn[kOwned];
+      if (owner) {
+        ErrorNorm e;
+        unsigned negative = 0u;
+#pragma unroll
+        for (int i = 0; i < kOwned; ++i) {
+#pragma clang fp contract(off)
+          yn[i] = fma(h0, fma(ck::c6, kn[i], sp[i]), y[i]);
+          const double ye =
+              h0 * fma(ck::ec6, kn[i],
+                       fma(ck::ec5, K(4, i), fma(ck::ec4, K(3, i), fma(ck::ec3, K(2, i), ck::ec1 * K(0, i)))));
+          error_norm_add(e, a.eps_abs, a.eps_rel, 1.0, 0.0, h0, yn[i], ye, 0.0, sc[i],
+                         enforce && ((nonneg >> i) & 1u));
+          negative |= yn[i] < 0.0 ? 1u << i : 0u;
+        }
+        X[(kXNorm + wave) * kGroupNodes] = e.rmax;
+        norm_flags[wave * kGroupNodes + lane] = (e.forbidden ? 1 : 0) | ((negative & fixable) ? 2 : 0);
+      }
+      __syncthreads();   // error norms published
+      en = ErrorNorm{};
+      need_fix = 0;
+#pragma unroll
+      for (int w = 0; w < kOwnerWaves; ++w) {
+        const double r = X[(kXNorm + w) * kGroupNodes];
+        en.rmax = r > en.rmax ? r : en.rmax;
+        const int fl = norm_flags[w * kGroupNodes + lane];
+        en.forbidden = en.forbidden || (fl & 1) != 0;
+        need_fix |= fl & 2;
+      }
+      decide = stepping;
+      const bool accepted = stepping && hadjust_kind(en) != kHadjDec;
+      bool done = false;
+      if (accepted) {
+        ++n_accept;
+        t = final_step ? t1 : t + h0;
+        if (owner) {
+#pragma unroll
+          for (int i = 0; i < kOwned; ++i) y[i] = yn[i];
+        }
+        done = !(sign * (t1 - t) > 0.0);
+        eval = post = !done;
+        if (done) decide = false;
+      }
+      if (__any(done)) {
+        if (__any(done && need_fix != 0)) {
+          if (owner && done) {
+#pragma unroll
+            for (int i = 0; i < kOwned; ++i) XY[i * kGroupNodes] = y[i];
+          }
           __syncthreads();
+          fix_published(done && need_fix != 0);
         }
-        break;
-      }
-      phase = 0;
-      continue;
-    }
-
-    // ---- phase 4: k6 is in kout; combine, error norm, controller --------
-    phase = 5;
-    if (!active) continue;
-    ErrorNorm en;
-#pragma unroll
-    for (int c = 0; c < kNV; c += kChunk) {
-      double gy[kChunk], g1[kChunk], g3[kChunk], g4[kChunk], g5[kChunk], gs[kChunk];
-#pragma unroll
-      for (int i = 0; i < kChunk; ++i) {
-        gy[i] = Y(c + i); g1[i] = KS(0, c + i); g3[i] = KS(2, c + i); g4[i] = KS(3, c + i); g5[i] = KS(4, c + i);
-        gs[i] = SC(c + i);
-      }
-#pragma unroll
-      for (int i = 0; i < kChunk; ++i) {
-        const int v = c + i;
-        const double yn = gy[i] + h0 * (sp[v] + ck::c6 * kout[v]);
-        const double ye = h0 * (ck::ec1 * g1[i] + ck::ec3 * g3[i] + ck::ec4 * g4[i] + ck::ec5 * g5[i] +
-                                ck::ec6 * kout[v]);
-        ytmp[v] = yn;
-        error_norm_add(en, a.eps_abs, a.eps_rel, 1.0, 0.0, h0, yn, ye, 0.0, gs[i], enforce && var_non_negative(v));
-      }
-    }
-    double h_adj = h0;
-    const int decision = hadjust_decide(en, kRkckOrder, h_adj);
-    const double t_adv = final_step ? t1 : t + h0;
-    bool failed = false;
-    if (decision == kHadjDec) {
-      if (fabs(h_adj) < fabs(h0) && t_adv + h_adj != t_adv) h0 = h_adj;  // reject: retry, same k1
-      else failed = true;                                                 // step size underflow
-    } else {
-      ++n_accept;
-      t = t_adv;
-      if (!final_step) h = h_adj;
-      h0 = h;
-#pragma unroll
-      for (int v = 0; v < kNV; ++v) Y(v) = ytmp[v];
-      if (sign * (t1 - t) > 0.0) {
-        eval_pending = true;   // dydt at the new point, then the post-step
-        post_pending = true;
-      } else {
-        post_step(P, a.D, np, mode, t, &Y(0), ys);
+        store_state(done);
         // odeSolverSolve returns xStep = driver h (solver.F90:593)
-#pragma unroll
-        for (int v = 0; v < kNV; ++v) a.y[v * (size_t)a.ld + node] = Y(v);
-        a.h_step[node] = h;
-        a.status[node] = GAL_STATUS_SUCCESS;
-        write_counters(a, node, n_attempt, n_accept, n_rhs);
-        if constexpr (GRAPH) graph_release(a.g, op);
-        active = false;
-        want = true;
-      }
-    }
-    if (failed) {
-      // node-evolver trial loop (standard.F90:657-692)
-      bool rescued = false;
-      if (enforce) {
-        bool any = false;
-#pragma unroll
-        for (int v = 0; v < kNV; ++v) any |= (Y(v) < 0.0 && var_non_negative(v));
-        if (any) {
-#pragma unroll
-          for (int v = 0; v < kNV; ++v)
-            if (Y(v) < 0.0 && var_non_negative(v)) Y(v) = 0.0;
-          rescued = true;
-        }
-      }
-      if (rescued) {
-#pragma unroll
-        for (int v = 0; v < kNV; ++v) a.y[v * (size_t)a.ld + node] = Y(v);
-        a.h_step[node] = h_node / (double)(1 << trial);
-        a.status[node] = GAL_STATUS_SUCCESS;
-        write_counters(a, node, n_attempt, n_accept, n_rhs);
-        if constexpr (GRAPH) graph_release(a.g, op);
-        active = false;
-        want = true;
-      } else if (++trial < 8) {
-#pragma unroll
-        for (int v = 0; v < kNV; ++v) Y(v) = a.y[v * (size_t)a.ld + node];
-        const double step_size = reuse ? h_node / (double)(1 << trial) : -1.0;
-        double xs = t1 - t0;
-        if (step_size > 0.0) xs = fmin(step_size, xs);
-        h = xs;
-        h0 = h;
-        t = t0;
-        eval_pending = true;
-      } else {
-        // all trials failed: state restored, errorStatusUnderflow (standard.F90:715-718)
-        a.status[node] = GAL_STATUS_UNDERFLOW;
-        write_counters(a, node, n_attempt, n_accept, n_rhs);
-        if constexpr (GRAPH) graph_release(a.g, op);
-        active = false;
-        want = true;
+        double h_out = h;
+        if (wave == kCoolingWave && done && !final_step) h_out = hadjust_step(en, kRkckOrder, h0);
+        finish(done, h_out, true, GAL_STATUS_SUCCESS);
       }
     }
   }
-#undef KS
-#undef Y
-#undef SC
+}
+
+template <bool GRAPH>
+__global__ __launch_bounds__(kGroupNodes * kGroupWaves, 1) void evolve_kernel(EvolveArgs a) {
+  extern __shared__ double exchange[];
+  __shared__ GroupConstants constants;
+  __shared__ int norm_flags[kOwnerWaves * kGroupNodes];   // bit 0: forbidden, bit 1: post-step needed, bit 2: rescue
+  __shared__ int wall_expired;
+  __shared__ int flags[kSignals];
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kGroupNodes));
+  double* X = exchange + (threadIdx.x & (kGroupNodes - 1));
+  if (threadIdx.x < kSignals) flags[threadIdx.x] = 0;
+  for (int k = wave; k < 2 * kNV; k += kGroupWaves) X[(kXGalaxy + k) * kGroupNodes] = 0.0;
+  {
+    // the derived constants and the table's grid are read from the kernel's
+    // argument segment, which its one argument starts
+    const char* args = (const char*)__builtin_amdgcn_kernarg_segment_ptr();
+    const double* d = (const double*)(args + offsetof(EvolveArgs, D));
+    const double* c = (const double*)(args + offsetof(EvolveArgs, cd));
+    constexpr int threads = kGroupNodes * kGroupWaves;
+    for (int k = threadIdx.x; k < GAL_NPARAM; k += threads) constants.P[k] = a.P[k];
+    for (int k = threadIdx.x; k < (int)(sizeof(constants.D) / 8); k += threads) ((double*)&constants.D)[k] = d[k];
+    for (int k = threadIdx.x; k < (int)(sizeof(constants.C) / 8); k += threads) ((double*)&constants.C)[k] = c[k];
+  }
+  __syncthreads();
+  if (wave == kGalaxyWave) group_wave<kGalaxyWave, GRAPH>(a, X, constants, norm_flags, flags, wall_expired);
+  else if (wave == kProfileWave) group_wave<kProfileWave, GRAPH>(a, X, constants, norm_flags, flags, wall_expired);
+  else if (wave == kTimeWave) group_wave<kTimeWave, GRAPH>(a, X, constants, norm_flags, flags, wall_expired);
+  else group_wave<kCoolingWave, GRAPH>(a, X, constants, norm_flags, flags, wall_expired);
 }
 
 __global__ void reset_counter_kernel(unsigned int* w) {
   if (threadIdx.x == 0 && blockIdx.x == 0) *w = 0u;
 }
 
-__global__ void rhs_kernel(int n, int ld, const double* __restrict__ t, const double* __restrict__ y,
+// One lane per node and some 3500 instructions a node with 60 doubles in and
+// out: a million nodes take 116 us, 4.8 TB/s, and 100,000 17 us.  The whole RHS
+// in one lane wants more than 200 registers, so two waves share a SIMD: with
+// 128 registers a wave (four to a SIMD) it spills and takes 210 us, with 168
+// 149 us.  Single waves as workgroups spread a small batch over more CUs than
+// groups of four do (123 us and 17 us).
+constexpr int kRhsThreads = 64, kRhsWavesPerSimd = 2;
+__global__ __launch_bounds__(kRhsThreads, kRhsWavesPerSimd) void rhs_kernel(int n, int ld, const double* __restrict__ t, const double* __restrict__ y,
                            const double* __restrict__ npa, double* __restrict__ dydt, const double* __restrict__ P,
                            const double* __restrict__ tab, DerivedConstants D, CoolingDesc cd, int mode) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -745,7 +694,7 @@ __global__ void hadjust_kernel(int n, int dim, int ord, double eps_abs, double e
 // start point; cost key = |t_end - t_start| / sqrt(tau), tau = the shortest
 // e-folding time min_v (|y_v| + scale_v) / |dy_v/dt|.  Only the order in
 // which lanes claim nodes depends on it, never a result.
-__global__ void cost_probe_kernel(int n_items, const int* __restrict__ subset, int ld, const double* __restrict__ y,
+__global__ __launch_bounds__(kRhsThreads, kRhsWavesPerSimd) void cost_probe_kernel(int n_items, const int* __restrict__ subset, int ld, const double* __restrict__ y,
                                   const double* __restrict__ npa, const double* __restrict__ t_start,
                                   const double* __restrict__ t_end, const double* __restrict__ scale_in,
                                   const double* __restrict__ P, const double* __restrict__ tab, DerivedConstants D,
@@ -787,29 +736,17 @@ __global__ void cost_probe_kernel(int n_items, const int* __restrict__ subset, i
   index[j] = i;
 }
 
-template <int BLOCK, bool YLDS, bool KLDS, int WAVES = 1>
-constexpr size_t lds_bytes() {
-  return lds_vector_bytes<BLOCK, YLDS, KLDS>() + (WAVES == 2 ? sizeof(double) * kXchgVectors * BLOCK : 0);
-}
+// LDS of a group of nodes: one group fills a CU's 160 KiB.
+constexpr size_t kExchangeBytes = sizeof(double) * kXVectors * kGroupNodes;
+static_assert(kExchangeBytes + sizeof(GroupConstants) + 1024 <= 163840, "a group must fit 160 KiB");
 
-// The dynamic LDS of every launch shape of the evolve kernel, in node mode
-// and in operation-graph mode.
-template <bool GRAPH>
 hipError_t set_lds_attributes() {
-  const struct { const void* f; size_t bytes; } shapes[] = {
-      {(const void*)evolve_kernel<64, true, true, 2, GRAPH>, lds_bytes<64, true, true, 2>()},
-      {(const void*)evolve_kernel<64, true, false, 2, GRAPH>, lds_bytes<64, true, false, 2>()},
-      {(const void*)evolve_kernel<64, true, true, 1, GRAPH>, lds_bytes<64, true, true>()},
-      {(const void*)evolve_kernel<64, false, true, 1, GRAPH>, lds_bytes<64, false, true>()},
-      {(const void*)evolve_kernel<64, true, false, 1, GRAPH>, lds_bytes<64, true, false>()},
-  };
-  for (const auto& sh : shapes) {
-    const hipError_t e = hipFuncSetAttribute(sh.f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh.bytes);
+  for (const void* f : {(const void*)evolve_kernel<false>, (const void*)evolve_kernel<true>}) {
+    const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kExchangeBytes);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
 }
-
 
 }  // namespace
 
@@ -939,26 +876,12 @@ int gal_ode_batch_create(int n_max, double tol_abs, double tol_rel, int flags, g
     gal_ode_batch_destroy(h);
     return GAL_E_NOMEM;
   }
-  h->ywork_lanes = ncu * 2 * 64;
-  h->kwork_lanes = ncu * 4 * 64;
-  if (hipMalloc(&h->d_ywork, sizeof(double) * 2 * kNV * (size_t)h->ywork_lanes) != hipSuccess ||
-      hipMalloc(&h->d_kwork, sizeof(double) * kStages * kNV * (size_t)h->kwork_lanes) != hipSuccess) {
-    gal_ode_batch_destroy(h);
-    return GAL_E_NOMEM;
-  }
   // Set on every handle creation (on the current device): no process-wide
   // state, and cheap.
-  {
-    static_assert(lds_bytes<64, true, true>() <= 163840, "lane-private LDS vectors must fit 160 KiB");
-    static_assert(2 * lds_bytes<64, false, true>() <= 163840, "two workgroups per CU must fit 160 KiB");
-    static_assert(4 * lds_bytes<64, true, false>() <= 163840, "four workgroups per CU must fit 160 KiB");
-    static_assert(lds_bytes<64, true, true, 2>() + 16 <= 163840, "two-wave groups with LDS stages must fit 160 KiB");
-    static_assert(2 * (lds_bytes<64, true, false, 2>() + 16) <= 163840, "two two-wave groups per CU must fit");
-    if (set_lds_attributes<false>() != hipSuccess || set_lds_attributes<true>() != hipSuccess) {
-      (void)hipGetLastError();
-      gal_ode_batch_destroy(h);
-      return GAL_E_HIP;
-    }
+  if (set_lds_attributes() != hipSuccess) {
+    (void)hipGetLastError();
+    gal_ode_batch_destroy(h);
+    return GAL_E_HIP;
   }
   *out = h;
   return GAL_OK;
@@ -977,8 +900,6 @@ int gal_ode_batch_destroy(gal_ode_batch* h) {
   hipFree(h->d_params);
   hipFree(h->d_table);
   hipFree(h->d_work);
-  hipFree(h->d_ywork);
-  hipFree(h->d_kwork);
   hipFree(h->d_order);
   hipFree(h->d_index);
   hipFree(h->d_key);
@@ -1084,41 +1005,12 @@ int gal_ode_batch_get_launch(gal_ode_batch* h, int* nodes_per_block, int* blocks
 extern "C++" {
 template <bool GRAPH = false>
 static int launch_evolve(gal_ode_batch* h, const EvolveArgs& args, hipStream_t s) {
-  const int blocks = std::max(1, h->n_cus * h->blocks_per_cu);
   if (h->rhs_waves == 2 && h->blocks_per_cu > 2) return GAL_E_INVALID;
+  // one group of nodes fills a CU, and a lone group per CU is claimed from
+  // until the last node is out
+  const int blocks = std::max(1, h->n_cus);
   hipLaunchKernelGGL(reset_counter_kernel, dim3(1), dim3(64), 0, s, args.work);
-  if (h->rhs_waves == 2) {
-    // two waves per group of 64 nodes: one group per CU with the stage
-    // derivatives in LDS, or two with them in the HBM workspace
-    if (h->blocks_per_cu == 1) {
-      constexpr size_t lds = lds_bytes<64, true, true, 2>();
-      hipLaunchKernelGGL((evolve_kernel<64, true, true, 2, GRAPH>), dim3(blocks), dim3(128), lds, s, args);
-    } else {
-      EvolveArgs b = args;
-      b.kwork = h->d_kwork;
-      if (blocks * 64 > h->kwork_lanes) return GAL_E_INVALID;
-      constexpr size_t lds = lds_bytes<64, true, false, 2>();
-      hipLaunchKernelGGL((evolve_kernel<64, true, false, 2, GRAPH>), dim3(blocks), dim3(128), lds, s, b);
-    }
-    HIP_TRY(hipGetLastError());
-    return GAL_OK;
-  }
-  constexpr size_t lds_all = lds_bytes<64, true, true>(), lds_k = lds_bytes<64, false, true>(),
-                   lds_y = lds_bytes<64, true, false>();
-  if (h->blocks_per_cu == 1) {
-    hipLaunchKernelGGL((evolve_kernel<64, true, true, 1, GRAPH>), dim3(blocks), dim3(64), lds_all, s, args);
-  } else if (h->blocks_per_cu == 2) {
-    EvolveArgs b = args;
-    b.ywork = h->d_ywork;
-    b.ystride = blocks * 64;
-    if (b.ystride > h->ywork_lanes) return GAL_E_INVALID;
-    hipLaunchKernelGGL((evolve_kernel<64, false, true, 1, GRAPH>), dim3(blocks), dim3(64), lds_k, s, b);
-  } else {
-    EvolveArgs b = args;
-    b.kwork = h->d_kwork;
-    if (blocks * 64 > h->kwork_lanes) return GAL_E_INVALID;
-    hipLaunchKernelGGL((evolve_kernel<64, true, false, 1, GRAPH>), dim3(blocks), dim3(64), lds_y, s, b);
-  }
+  hipLaunchKernelGGL((evolve_kernel<GRAPH>), dim3(blocks), dim3(kGroupNodes * kGroupWaves), kExchangeBytes, s, args);
   HIP_TRY(hipGetLastError());
   return GAL_OK;
 }
@@ -1145,9 +1037,6 @@ static int make_args(gal_ode_batch* h, int n, int ld, double* y, const double* n
   a.order = nullptr;
   a.n_claim_dev = nullptr;
   a.work = h->d_work;
-  a.ywork = nullptr;
-  a.ystride = 0;
-  a.kwork = nullptr;
   a.P = h->d_params;
   a.tab = h->d_table;
   a.D = h->D;
@@ -1213,7 +1102,7 @@ int gal_ode_rhs_d(gal_ode_batch* h, int n, int ld, const double* t, const double
   if (!h || n < 0 || ld < n || !h->have_physics || !h->have_table) return GAL_E_INVALID;
   if (n == 0) return GAL_OK;
   if (!t || !y || !node_par || !dydt) return GAL_E_INVALID;
-  const int threads = 256;
+  const int threads = kRhsThreads;
   hipLaunchKernelGGL(rhs_kernel, dim3((n + threads - 1) / threads), dim3(threads), 0, (hipStream_t)stream, n, ld, t,
                      y, node_par, dydt, (const double*)h->d_params, (const double*)h->d_table, h->D, h->cd,
                      (int)h->params[GAL_P_PHYSICS_MODE]);
@@ -1251,8 +1140,9 @@ int gal_ode_batch_autotune(gal_ode_batch* h, int n, int ld, double* y, const dou
     hipFree(wy); hipFree(wh); hipFree(wsc); hipFree(wst);
     return GAL_E_NOMEM;
   }
-  // (nodes per workgroup, workgroups per CU, waves per group of nodes)
-  const int shapes[][3] = {{64, 1, 1}, {64, 2, 1}, {64, 4, 1}, {64, 1, 2}, {64, 2, 2}};
+  // (nodes per workgroup, workgroups per CU, waves per group of nodes); the
+  // kernel runs alike at every admitted shape, so one stands for all
+  const int shapes[][3] = {{64, 1, 2}};
   float best = 1e30f;
   int bn = h->nodes_per_block, bb = h->blocks_per_cu, bw = h->rhs_waves;
   hipEvent_t e0, e1;
@@ -1334,8 +1224,7 @@ static int static_scratch(int device, void** ptr, int* n_cus) {
     int cus = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || cus < 1)
       return GAL_E_HIP;
-    if (hipFuncSetAttribute((const void*)evolve_kernel<64, true, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)lds_bytes<64, true, true>()) != hipSuccess) {
+    if (set_lds_attributes() != hipSuccess) {
       (void)hipGetLastError();
       return GAL_E_HIP;
     }
@@ -1400,10 +1289,9 @@ extern "C" int gal_ode_evolve_static_d(const double* params, int n_params, const
   a.flags = flags;
   a.mode = (int)params[GAL_P_PHYSICS_MODE];
   a.wall_ticks = 0;
-  // every lane vector in LDS, one workgroup per CU: no workspace beyond the scratch
-  constexpr size_t lds_all = lds_bytes<64, true, true>();
+  // one group of nodes per CU; no workspace beyond the scratch
   hipLaunchKernelGGL(reset_counter_kernel, dim3(1), dim3(64), 0, s, work);
-  hipLaunchKernelGGL((evolve_kernel<64, true, true>), dim3(n_cus), dim3(64), lds_all, s, a);
+  hipLaunchKernelGGL((evolve_kernel<false>), dim3(n_cus), dim3(kGroupNodes * kGroupWaves), kExchangeBytes, s, a);
   HIP_TRY(hipGetLastError());
   return GAL_OK;
 }
@@ -1414,7 +1302,7 @@ extern "C" int gal_ode_evolve_static_d(const double* params, int n_params, const
 static int plan_claim_order(gal_ode_batch* h, int n_subset, const int* subset, int ld, const double* y,
                             const double* node_par, const double* t_start, const double* t_end, const double* scale,
                             const int* n_subset_dev, hipStream_t s) {
-  const int threads = 256;
+  const int threads = kRhsThreads;
   hipLaunchKernelGGL(cost_probe_kernel, dim3((n_subset + threads - 1) / threads), dim3(threads), 0, s, n_subset,
                      subset, ld, y, node_par, t_start, t_end, scale, (const double*)h->d_params,
                      (const double*)h->d_table, h->D, h->cd, (int)h->params[GAL_P_PHYSICS_MODE],

@@ -1,0 +1,245 @@
+// group_rhs.hpp -- the RHS of a group of 64 nodes computed by the four waves
+// of a workgroup, one wave on each SIMD of a CU.  Internal.
+//
+// A node's Cash-Karp attempts are a serial chain of RHS evaluations, and a
+// wave64 FP64 instruction takes its issue cycles whether one lane or all 64
+// are active, so the time of a stiff node -- and of every launch, which lasts
+// as long as its stiffest node -- is the number of instructions in the
+// longest wave's share of an RHS.  The blocks of physics.hpp are dealt out by
+// what they wait for:
+//   galaxy wave   the galaxy half, then the CGM outer radius;
+//   profile wave  hot-halo profile, ISCO, spheroid accretion, then the mean
+//                 radius of the hot gas and its radiated energy, then the
+//                 black hole's rates and winds;
+//   time wave     the part that depends on the time alone, of the *next*
+//                 stage (its time is known ahead of its state), and the step
+//                 controller's pow;
+//   cooling wave  cooling function and time, then cooling radius, hot-mode
+//                 accretion and jet power, then net cooling: the serial chain
+//                 that nothing takes off the path.
+// They meet in a barrier when the stage state is published and when the
+// derivatives are.  In between a value goes from the wave that computes it to
+// the ones that need it by a flag in LDS (Signal below): barriers there made
+// every wave wait for the slowest at each of them, 8800 cycles an evaluation
+// for 6300 cycles of work in the busiest wave.
+//
+// All exchange goes through LDS vectors of 64 doubles, one per lane
+// (conflict-free); a vector is written by one wave and read by the others on
+// the far side of a barrier.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include "physics.hpp"
+
+namespace gal {
+
+constexpr int kGroupNodes = 64;
+enum : int { kGalaxyWave = 0, kProfileWave = 1, kTimeWave = 2, kCoolingWave = 3, kGroupWaves = 4 };
+
+// The integrator's variables are owned by three of the waves, ten each; the
+// cooling wave, the longest of an RHS, owns none.
+constexpr int kOwnerWaves = 3, kOwned = kNV / kOwnerWaves;
+static_assert(kOwned * kOwnerWaves == kNV, "owners must tile the state");
+
+constexpr int kTimeVectors = (int)(sizeof(TimePart) / sizeof(double));
+constexpr int kMidVectors = 11;
+
+// Stages whose derivatives are kept (the sixth is consumed as it is produced).
+constexpr int kStages = 5;
+
+// LDS of a group, in vectors of 64 doubles.
+enum : int {
+  kXState = 0,                              // stage state
+  kXGalaxy = kXState + kNV,                 // galaxy half of the derivative
+  kXHalo = kXGalaxy + kNV,                  // hot-halo half
+  kXStage = kXHalo + kNV,                   // stage derivatives k1..k5, each kNV vectors
+  kXTime = kXStage + kStages * kNV,         // TimePart of this stage and of the next
+  kXMid = kXTime + 2 * kTimeVectors,        // published at the pauses
+  kXNorm = kXMid + kMidVectors,             // each owner's error norm
+  kXStep = kXNorm + kOwnerWaves,            // step size chosen by the controller
+  kXVectors = kXStep + 1,
+  // published at the pauses
+  kMidRho0 = kXMid, kMidRhoOut, kMidEffThin, kMidEddCap, kMidMdotSph, kMidInvRMean,   // profile wave
+  kMidLambda, kMidNhPerRho, kMidNallPerNh, kMidMdot, kMidJet,                         // cooling wave
+  kMidEnd,
+  // claimed nodes, in the time part that is not in use
+  kXClaimNode = 0, kXClaimT0, kXClaimT1, kXClaimStep, kXClaimPar
+};
+static_assert(kMidEnd - kXMid == kMidVectors, "count the published values");
+static_assert(kXClaimPar + GAL_NPARAM_NODE <= kTimeVectors, "a claim must fit a time part");
+
+// The copy of the parameters that the RHS reads.
+struct GroupConstants {
+  double P[GAL_NPARAM];
+  DerivedConstants D;
+  CoolingDesc C;
+};
+
+// Variables whose derivative has a part in each half; the other entries of
+// the exchange area stay zero.
+constexpr unsigned var_bits(std::initializer_list<int> vars) {
+  unsigned m = 0;
+  for (int v : vars) m |= 1u << v;
+  return m;
+}
+constexpr unsigned kGalaxyVars =
+    var_bits({GAL_V_HOT_MASS, GAL_V_HOT_ABUNDANCES, GAL_V_HOT_ANGULAR_MOMENTUM, GAL_V_HOT_OUTFLOWED_MASS,
+              GAL_V_HOT_OUTFLOWED_ANGULAR_MOMENTUM, GAL_V_HOT_OUTFLOWED_ABUNDANCES, GAL_V_HOT_UNACCRETED_MASS,
+              GAL_V_HOT_UNACCRETED_ABUNDANCES, GAL_V_HOT_OUTER_RADIUS, GAL_V_HOT_STRIPPED_MASS,
+              GAL_V_HOT_STRIPPED_ABUNDANCES, GAL_V_DISK_MASS_STELLAR, GAL_V_DISK_MASS_STELLAR_FORMED,
+              GAL_V_DISK_ABUNDANCES_STELLAR, GAL_V_DISK_MASS_GAS, GAL_V_DISK_ABUNDANCES_GAS,
+              GAL_V_DISK_ANGULAR_MOMENTUM, GAL_V_SPHEROID_MASS_STELLAR, GAL_V_SPHEROID_MASS_STELLAR_FORMED,
+              GAL_V_SPHEROID_ABUNDANCES_STELLAR, GAL_V_SPHEROID_MASS_GAS, GAL_V_SPHEROID_ABUNDANCES_GAS,
+              GAL_V_SPHEROID_ANGULAR_MOMENTUM, GAL_V_SPIN_ANGULAR_MOMENTUM, GAL_V_SATELLITE_BOUND_MASS});
+constexpr unsigned kHaloVars =
+    var_bits({GAL_V_HOT_MASS, GAL_V_HOT_ABUNDANCES, GAL_V_HOT_ANGULAR_MOMENTUM, GAL_V_HOT_OUTFLOWED_MASS,
+              GAL_V_HOT_OUTFLOWED_ANGULAR_MOMENTUM, GAL_V_HOT_OUTFLOWED_ABUNDANCES, GAL_V_HOT_STRIPPED_MASS,
+              GAL_V_HOT_STRIPPED_ABUNDANCES, GAL_V_HOT_ENERGY_RADIATED, GAL_V_DISK_MASS_GAS,
+              GAL_V_DISK_ABUNDANCES_GAS, GAL_V_DISK_ANGULAR_MOMENTUM, GAL_V_SPHEROID_MASS_GAS,
+              GAL_V_SPHEROID_ABUNDANCES_GAS, GAL_V_SPHEROID_ANGULAR_MOMENTUM, GAL_V_BH_MASS, GAL_V_BH_SPIN});
+
+// What one wave tells others within an evaluation, as the number of the
+// evaluation (a round counts up alike in all waves).  A wave publishes its
+// vectors, then the flag; LDS keeps one wave's operations in order, and the
+// fences keep the compiler to it.  Every wait ends: a flag is set by a wave of
+// the same workgroup that runs the same rounds, and the waits form no cycle
+// (profile -> cooling -> profile's last part, profile -> galaxy).
+enum Signal : int { kProfileReady = 0, kAccretorReady, kMeanRadiusReady, kCoolingFunctionReady, kAccretionReady, kSignals };
+
+__device__ __forceinline__ void signal(int* __restrict__ flags, Signal s, int round) {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  if ((threadIdx.x & (kGroupNodes - 1)) == 0)
+    __hip_atomic_store(flags + s, round, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+__device__ __forceinline__ void await(int* __restrict__ flags, Signal s, int round) {
+  while (__builtin_amdgcn_readfirstlane(
+             __hip_atomic_load(flags + s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) != round) {
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// Work that follows a signal stays behind it: without this the compiler
+// mixes later arithmetic in before the signal and delays who waits for it.
+__device__ __forceinline__ double after_signal(double x) {
+  asm volatile("" : "+v"(x) : : "memory");
+  return x;
+}
+
+__device__ __forceinline__ TimePart load_time_part(const double* __restrict__ X) {
+  double v[kTimeVectors];
+#pragma unroll
+  for (int k = 0; k < kTimeVectors; ++k) v[k] = X[k * kGroupNodes];
+  return __builtin_bit_cast(TimePart, v);
+}
+
+__device__ __forceinline__ void store_time_part(const TimePart& T, double* __restrict__ X) {
+  struct Values { double v[kTimeVectors]; };
+  const Values w = __builtin_bit_cast(Values, T);
+#pragma unroll
+  for (int k = 0; k < kTimeVectors; ++k) X[k * kGroupNodes] = w.v[k];
+}
+
+__device__ __forceinline__ void load_state(const double* __restrict__ X, double (&y)[kNV]) {
+#pragma unroll
+  for (int v = 0; v < kNV; ++v) y[v] = X[(kXState + v) * kGroupNodes];
+}
+
+// X: this lane's column of the group's LDS; xt, the vector at which this
+// stage's time part starts.
+__device__ __forceinline__ void galaxy_wave_rhs(const GroupConstants& G, int mode, int ops, const NodePar& np,
+                                                double* __restrict__ X, int xt, int* __restrict__ flags, int round) {
+  double y[kNV], f[kNV];
+  load_state(X, y);
+#pragma unroll
+  for (int v = 0; v < kNV; ++v) f[v] = 0.0;
+  const TimePart T = load_time_part(X + xt * kGroupNodes);
+  if (mode == GAL_PHYSICS_TEST) {
+    test_rates(T.time, y, f);
+  } else {
+    const bool box = mode == GAL_PHYSICS_BOX;
+    galaxy_rates(G.P, G.D, ops, box, np, T, y, f);
+    if (!box && (ops & GAL_OPERATOR_CGM_OUTER_RADIUS)) {
+      await(flags, kProfileReady, round);
+      outer_radius_rates(G.P, np, T, X[kMidRho0 * kGroupNodes], X[kMidRhoOut * kGroupNodes], y, f);
+    }
+  }
+#pragma unroll
+  for (int v = 0; v < kNV; ++v)
+    if ((kGalaxyVars >> v) & 1u) X[(kXGalaxy + v) * kGroupNodes] = f[v];
+}
+
+// Of the hot-halo half, the profile wave writes the variables of the black
+// hole, its spheroid and the outflow, the cooling wave the others.
+constexpr unsigned kBlackHoleVars =
+    var_bits({GAL_V_HOT_OUTFLOWED_MASS, GAL_V_HOT_OUTFLOWED_ANGULAR_MOMENTUM, GAL_V_HOT_OUTFLOWED_ABUNDANCES,
+              GAL_V_HOT_ENERGY_RADIATED, GAL_V_SPHEROID_MASS_GAS, GAL_V_SPHEROID_ABUNDANCES_GAS,
+              GAL_V_SPHEROID_ANGULAR_MOMENTUM, GAL_V_BH_MASS, GAL_V_BH_SPIN});
+constexpr unsigned kCoolingVars = kHaloVars & ~kBlackHoleVars;
+
+__device__ __forceinline__ void profile_wave_rhs(const GroupConstants& G, int ops, double* __restrict__ X, int xt,
+                                                 int* __restrict__ flags, int round) {
+  auto Y = [&](int v) { return X[(kXState + v) * kGroupNodes]; };
+  const TimePart T = load_time_part(X + xt * kGroupNodes);
+  const double m_hot = Y(GAL_V_HOT_MASS), r_out = Y(GAL_V_HOT_OUTER_RADIUS), m_bh = Y(GAL_V_BH_MASS);
+  const double mg_s = Y(GAL_V_SPHEROID_MASS_GAS), ms_s = Y(GAL_V_SPHEROID_MASS_STELLAR);
+  const double j_s = Y(GAL_V_SPHEROID_ANGULAR_MOMENTUM), zg_s = Y(GAL_V_SPHEROID_ABUNDANCES_GAS);
+  const double y_spin = Y(GAL_V_BH_SPIN), r_bh = Y(GAL_V_BH_RADIAL_POSITION);
+  const GalaxyRadius galaxy = galaxy_radius(T, Y(GAL_V_SPIN_ANGULAR_MOMENTUM));
+  HotProfile p = hot_profile(T, m_hot, r_out);
+  X[kMidRho0 * kGroupNodes] = p.rho0;
+  X[kMidRhoOut * kGroupNodes] = p.rho_out;
+  signal(flags, kProfileReady, round);
+  const BlackHole b = black_hole(G.P, G.D, galaxy, m_bh, after_signal(y_spin), after_signal(r_bh), mg_s);
+  X[kMidEffThin * kGroupNodes] = b.eff_thin;
+  X[kMidEddCap * kGroupNodes] = b.edd_cap;
+  X[kMidMdotSph * kGroupNodes] = b.mdot_sph;
+  signal(flags, kAccretorReady, round);
+  p.uo = after_signal(p.uo);
+  X[kMidInvRMean * kGroupNodes] = hot_inv_mean_radius(T, p);
+  signal(flags, kMeanRadiusReady, round);
+  double f[kNV];
+#pragma unroll
+  for (int v = 0; v < kNV; ++v) f[v] = 0.0;
+  await(flags, kCoolingFunctionReady, round);
+  f[GAL_V_HOT_ENERGY_RADIATED] += radiated_energy(X[kMidLambda * kGroupNodes], X[kMidNhPerRho * kGroupNodes],
+                                                  X[kMidNallPerNh * kGroupNodes], m_hot, r_out);
+  await(flags, kAccretionReady, round);
+  black_hole_rates(G.P, G.D, ops, T, b, X[kMidMdot * kGroupNodes], X[kMidJet * kGroupNodes], m_bh, mg_s, ms_s, j_s,
+                   zg_s, galaxy.r, f);
+#pragma unroll
+  for (int v = 0; v < kNV; ++v)
+    if ((kBlackHoleVars >> v) & 1u) X[(kXHalo + v) * kGroupNodes] = f[v];
+}
+
+__device__ __forceinline__ void cooling_wave_rhs(const GroupConstants& G, const double* __restrict__ tab,
+                                                 const NodePar& np, double* __restrict__ X, int xt,
+                                                 int* __restrict__ flags, int round) {
+  auto Y = [&](int v) { return X[(kXState + v) * kGroupNodes]; };
+  const TimePart T = load_time_part(X + xt * kGroupNodes);
+  const double m_hot = Y(GAL_V_HOT_MASS), r_out = Y(GAL_V_HOT_OUTER_RADIUS), z_hot = Y(GAL_V_HOT_ABUNDANCES);
+  const double j_hot = Y(GAL_V_HOT_ANGULAR_MOMENTUM), m_bh = Y(GAL_V_BH_MASS), y_spin = Y(GAL_V_BH_SPIN);
+  const CoolingTime c = cooling_time(G.D, tab, G.C, T, m_hot, z_hot, r_out);
+  X[kMidLambda * kGroupNodes] = c.lambda_cool;
+  X[kMidNhPerRho * kGroupNodes] = c.nh_per_rho;
+  X[kMidNallPerNh * kGroupNodes] = c.nall_per_nh;
+  signal(flags, kCoolingFunctionReady, round);
+  await(flags, kAccretorReady, round);   // and with it the profile
+  const double rho0 = X[kMidRho0 * kGroupNodes];
+  const HotAccretion s = hot_accretion(G.P, G.D, T, c, X[kMidEffThin * kGroupNodes], X[kMidEddCap * kGroupNodes],
+                                       X[kMidMdotSph * kGroupNodes], rho0, X[kMidRhoOut * kGroupNodes], m_hot, r_out,
+                                       m_bh, y_spin);
+  X[kMidMdot * kGroupNodes] = s.mdot;
+  X[kMidJet * kGroupNodes] = s.p_jet;
+  signal(flags, kAccretionReady, round);
+  double f[kNV];
+#pragma unroll
+  for (int v = 0; v < kNV; ++v) f[v] = 0.0;
+  await(flags, kMeanRadiusReady, round);
+  cooling_rates(G.P, np, T, s, c.inv_m_hot, rho0, X[kMidInvRMean * kGroupNodes], m_hot, z_hot, j_hot, r_out, m_bh, f);
+#pragma unroll
+  for (int v = 0; v < kNV; ++v)
+    if ((kCoolingVars >> v) & 1u) X[(kXHalo + v) * kGroupNodes] = f[v];
+}
+
+}  // namespace gal

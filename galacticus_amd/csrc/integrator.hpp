@@ -51,27 +51,36 @@ __device__ __forceinline__ void error_norm_add(ErrorNorm& e, double eps_abs, dou
   if (non_negative && y < 0.0) e.forbidden = true;
 }
 
-// Step decision from the accumulated norm (cscal2.c:127-168).
-__device__ __forceinline__ int hadjust_decide(const ErrorNorm& e, int ord, double& h) {
+// Step decision from the accumulated norm (cscal2.c:127-168): whether the
+// step is repeated, kept or kept with a longer one next, and the step size
+// that follows (a pow, which callers may leave to another wave).
+__device__ __forceinline__ int hadjust_kind(const ErrorNorm& e) {
+  if (e.rmax > 1.1 || e.forbidden) return kHadjDec;
+  return e.rmax < 0.5 ? kHadjInc : kHadjNil;
+}
+
+__device__ __forceinline__ double hadjust_step(const ErrorNorm& e, int ord, double h_old) {
 #pragma clang fp contract(off)
   const double S = 0.9;
-  const double h_old = h;
-  if (e.rmax > 1.1) {
-    double r = S / pow(e.rmax, 1.0 / ord);
-    if (r < 0.2) r = 0.2;
+  const bool shrink = e.rmax > 1.1, grow = !shrink && !e.forbidden && e.rmax < 0.5;
+  double h = (!shrink && e.forbidden) ? 0.5 * h_old : h_old;
+  if (shrink || grow) {
+    // one pow for the lanes of a wave that shrink and those that grow
+    double r = S / pow(e.rmax, shrink ? 1.0 / ord : 1.0 / (ord + 1.0));
+    if (shrink) {
+      if (r < 0.2) r = 0.2;
+    } else {
+      if (r > 4.9) r = 4.9;
+      if (r < 1.0) r = 1.0;
+    }
     h = r * h_old;
-    return kHadjDec;
-  } else if (e.forbidden) {
-    h = 0.5 * h_old;
-    return kHadjDec;
-  } else if (e.rmax < 0.5) {
-    double r = S / pow(e.rmax, 1.0 / (ord + 1.0));
-    if (r > 4.9) r = 4.9;
-    if (r < 1.0) r = 1.0;
-    h = r * h_old;
-    return kHadjInc;
   }
-  return kHadjNil;
+  return h;
+}
+
+__device__ __forceinline__ int hadjust_decide(const ErrorNorm& e, int ord, double& h) {
+  h = hadjust_step(e, ord, h);
+  return hadjust_kind(e);
 }
 
 }  // namespace gal

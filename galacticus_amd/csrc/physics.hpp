@@ -78,6 +78,15 @@ __device__ __forceinline__ double rcp(double x) {
   return fma(r, e, r);
 }
 
+// A value that later arithmetic must take as it was rounded.  The compiler
+// contracts a product and the sum that consumes it into one fused operation
+// when it sees both; whether it sees both would otherwise depend on whether
+// the two sit in one wave's code or either side of an exchange.
+__device__ __forceinline__ double rounded(double x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
+
 // Cooling table descriptor (table itself in global memory).
 struct CoolingDesc {
   int n_t, n_z;
@@ -106,13 +115,21 @@ __device__ __forceinline__ NodePar load_node_par(const double* __restrict__ np, 
 }
 
 // isNonNegative attributes of the state variables (component _class.F90 XML).
-__device__ __forceinline__ bool var_non_negative(int v) {
-  return !(v == GAL_V_HOT_ANGULAR_MOMENTUM || v == GAL_V_HOT_OUTFLOWED_ANGULAR_MOMENTUM ||
-           v == GAL_V_HOT_ENERGY_RADIATED || v == GAL_V_BH_RADIAL_POSITION || v == GAL_V_SPIN_ANGULAR_MOMENTUM);
+
+constexpr unsigned non_negative_bits() {
+  unsigned m = 0;
+  for (int v = 0; v < kNV; ++v)
+    if (!(v == GAL_V_HOT_ANGULAR_MOMENTUM || v == GAL_V_HOT_OUTFLOWED_ANGULAR_MOMENTUM ||
+          v == GAL_V_HOT_ENERGY_RADIATED || v == GAL_V_BH_RADIAL_POSITION || v == GAL_V_SPIN_ANGULAR_MOMENTUM))
+      m |= 1u << v;
+  return m;
 }
+constexpr unsigned kNonNegative = non_negative_bits();
+__device__ __forceinline__ bool var_non_negative(int v) { return (kNonNegative >> v) & 1u; }
 
 // x^(n2/2) for integer n2 given sqrt(x); wave-uniform n2.
-__device__ __forceinline__ double pow_half(double x, double sqrt_x, int n2) {
+__device__ __forceinline__ double pow_half(double x, double sqrt_x, int n2_of_lane) {
+  const int n2 = __builtin_amdgcn_readfirstlane(n2_of_lane);
   const int m = n2 < 0 ? -n2 : n2;
   double r = (m & 1) ? sqrt_x : 1.0;
   double b = x;
@@ -125,7 +142,7 @@ __device__ __forceinline__ double pow_half(double x, double sqrt_x, int n2) {
 
 // x^alpha: half-integer fast path, else exp(alpha ln x).
 __device__ __forceinline__ double pow_param(double x, double sqrt_x, double ln_x_fn_arg, int n2, double alpha) {
-  if (n2 != kNoHalfPower) return pow_half(x, sqrt_x, n2);
+  if (__builtin_amdgcn_readfirstlane(n2) != kNoHalfPower) return pow_half(x, sqrt_x, n2);
   return exp(alpha * ln_x_fn_arg);
 }
 
@@ -141,48 +158,64 @@ __device__ __forceinline__ double clamp_temperature(const CoolingDesc& c, double
 __device__ __forceinline__ double clamp_metallicity(const CoolingDesc& c, double z_solar) {
   return fmin(fmax(z_solar, c.z_min), c.z_max);
 }
-__device__ __forceinline__ double cooling_function_ln(const double* __restrict__ tab, const CoolingDesc& c, double lt,
-                                                      double lz) {
+// Row of the table and weight within it of a temperature's logarithm; the row
+// is a whole number held in a double.
+__device__ __forceinline__ void cooling_temperature_index(const CoolingDesc& c, double lt, double& row, double& ht) {
   int it = (int)((lt - c.ln_t_min) * c.inv_d_ln_t);
-  int iz = (int)((lz - c.ln_z_min) * c.inv_d_ln_z);
   it = it < 0 ? 0 : (it > c.n_t - 2 ? c.n_t - 2 : it);
-  iz = iz < 0 ? 0 : (iz > c.n_z - 2 ? c.n_z - 2 : iz);
   const double t0 = c.ln_t_min + c.d_ln_t * it, t1 = c.ln_t_min + c.d_ln_t * (it + 1);
+  row = it;
+  ht = rounded((lt - t0) / (t1 - t0));
+}
+__device__ __forceinline__ double cooling_function_ln(const double* __restrict__ tab, const CoolingDesc& c, double row,
+                                                      double ht, double lz) {
+  const int it = (int)row;
+  int iz = (int)((lz - c.ln_z_min) * c.inv_d_ln_z);
+  iz = iz < 0 ? 0 : (iz > c.n_z - 2 ? c.n_z - 2 : iz);
   const double z0 = c.ln_z_min + c.d_ln_z * iz, z1 = c.ln_z_min + c.d_ln_z * (iz + 1);
-  const double ht = (lt - t0) / (t1 - t0);
   const double hz = (lz - z0) / (z1 - z0);
   const double* r0 = tab + iz * c.n_t + it;
   const double* r1 = r0 + c.n_t;
-  const double v = r0[0] * (1.0 - ht) * (1.0 - hz) + r1[0] * (1.0 - ht) * hz + r0[1] * ht * (1.0 - hz) +
-                   r1[1] * ht * hz;
+  const double v = fma(r1[1] * ht, hz, fma(r0[1] * ht, 1.0 - hz,
+                                           fma(r0[0] * (1.0 - ht), 1.0 - hz, rounded(r1[0] * (1.0 - ht) * hz))));
   return exp(v);
 }
 
 // ISCO specific energy and angular momentum, prograde, gravitational units
-// (black_holes/fundamentals.F90; Bardeen, Press & Teukolsky 1972).
-__device__ __forceinline__ void isco(double a, double& energy, double& ang_mom) {
+// (black_holes/fundamentals.F90; Bardeen, Press & Teukolsky 1972), as
+// numerators over a common denominator.
+struct Isco {
+  double energy, ang_mom, inv_den;
+};
+__device__ __forceinline__ Isco isco(double a) {
   const double cp = cbrt(1.0 + a), cm = cbrt(1.0 - a);
   const double a1 = 1.0 + cp * cm * (cp + cm);
-  const double a2 = sqrt(3.0 * a * a + a1 * a1);
+  const double a2 = sqrt(fma(3.0 * a, a, rounded(a1 * a1)));
   // A1 <= 3 for |a| <= 1; rounding can push it just above 3 for tiny spins
   const double r = 3.0 + a2 - sqrt(fmax(3.0 - a1, 0.0) * (3.0 + a1 + 2.0 * a2));
   const double sr = sqrt(r);
   const double inv_den = rcp(r) * rsqrt(r * r - 3.0 * r + 2.0 * a * sr);
-  energy = (r * r - 2.0 * r + a * sr) * inv_den;
-  ang_mom = (r * r - 2.0 * a * sr + a * a) * sr * inv_den;
+  return Isco{r * r - 2.0 * r + a * sr, (rounded(r * r) - rounded(2.0 * a * sr) + a * a) * sr, inv_den};
 }
 
-// Hernquist density of mass M with scale radius a at r (zero for
+// The galaxy's radius, factor * r_vir * lambda (fixed.F90:318-325), with its
+// factors.
+struct GalaxyRadius {
+  double per_lambda, lambda, r;
+};
+
+// Hernquist density of mass M with the galaxy's radius as scale at r (zero for
 // non-positive arguments).
-__device__ __forceinline__ double hernquist_density(double mass, double scale, double r) {
-  const double rs = r + scale;
-  const double rho = mass * scale * (1.0 / (2.0 * kPi)) * rcp(r * rs * rs * rs);
-  return (mass > 0.0 && scale > 0.0 && r > 0.0) ? rho : 0.0;
+__device__ __forceinline__ double hernquist_density(double mass, const GalaxyRadius& g, double r) {
+  const double rs = fma(g.per_lambda, g.lambda, r);
+  const double rho = mass * g.r * (1.0 / (2.0 * kPi)) * rcp(r * rs * rs * rs);
+  return (mass > 0.0 && g.r > 0.0 && r > 0.0) ? rho : 0.0;
 }
 
 // Halo quantities shared by the RHS, the scale rules and the post-step.
 struct Halo {
   double mass, a3, r_vir, inv_r_vir, v_vir, inv_v, t_dyn, inv_t_dyn, lambda, r_gal;
+  double inv_j_scale;  // 1 / (M V r), 0 for a halo without mass
   double r_vir_rate;   // darkMatterHaloScale%radiusVirialGrowthRate
 };
 
@@ -213,118 +246,239 @@ __device__ __forceinline__ Halo halo(const double* __restrict__ P, const Derived
   h.t_dyn = kMpcPerKmsToGyr * h.r_vir * h.inv_v;
   h.inv_t_dyn = h.v_vir * h.inv_r_vir * (1.0 / kMpcPerKmsToGyr);
   const double jscale = h.mass * h.v_vir * h.r_vir;
-  h.lambda = jscale > 0.0 ? spin_j * rcp(jscale) : 0.0;
+  const double inv_jscale = rcp(jscale);
+  h.inv_j_scale = jscale > 0.0 ? inv_jscale : 0.0;
+  h.lambda = jscale > 0.0 ? spin_j * h.inv_j_scale : 0.0;
   h.r_gal = P[GAL_P_RADIUS_FACTOR] * h.r_vir * h.lambda;  // fixed.F90:318-325
   // radiusVirialGrowthRate (virial_density_contrast.F90:338-354):
   // (r_vir/3)(Mdot/M - dln(Delta_c E^2)/dt), dln E^2/dt = -3 H Omega_m(a),
   // dOmega_m(a)/dt = -3 H Omega_m(a)(1 - Omega_m(a)); zero for satellites.
   const double hub = D.h0_gyr * sqrt(e2);
-  const double dx = -3.0 * hub * om_a * (1.0 - om_a);
-  const double dln = (82.0 - 78.0 * x) * dx * rcp(delta_c) - 3.0 * hub * om_a;
-  h.r_vir_rate = np.satellite ? 0.0 : h.r_vir * (1.0 / 3.0) * (mrate * rcp(h.mass) - dln);
+  const double dx = -3.0 * hub * om_a * (1.0 - rounded(om_a));
+  const double dln = fma((82.0 - 78.0 * x) * dx, rcp(delta_c), -rounded(3.0 * hub * om_a));
+  const double rv_rate = h.r_vir * (1.0 / 3.0) * (mrate * rcp(h.mass) - dln);
+  h.r_vir_rate = np.satellite ? 0.0 : rv_rate;
   return h;
 }
 
 // ---- the RHS -------------------------------------------------------------
 // Written as straight-line dataflow: every process rate is computed and
 // then selected by its applicability condition, so that the independent
-// chains (halo scales, ISCO, metallicity, star formation, hot-halo
-// structure) can be interleaved by the scheduler.  A rate that does not
-// apply is exactly zero, which leaves the accumulated sums unchanged.
+// chains can be interleaved by the scheduler.  A rate that does not apply is
+// exactly zero, which leaves the accumulated sums unchanged.
 //
-// The operators fall into two halves that share only the halo scales, the
-// hot halo's density profile and the state: the galaxy half (spin growth,
-// satellite mass loss, star formation, stellar feedback, bar instability,
-// CGM accretion, outflow reincorporation and the CGM outer radius) and the
-// hot-halo half (ISCO, cooling function and radius, black-hole accretion,
-// jet and winds, cooling and heating, radiated energy).  The outer radius
-// needs only the density profile, and sits in the galaxy half because the
-// hot-halo half is the longer of the two.  rhs_part<PART> computes one
-// half (or both); every path forms the derivative as f_galaxy + f_halo, so a
-// wave that computes one half while another wave computes the other gets the
-// same bits as one lane computing both.
-enum : int { kRhsGalaxy = 1, kRhsHalo = 2 };
+// The RHS is cut into blocks that different waves of a workgroup can compute
+// at the same time (group_rhs.hpp); rhs() runs them one after the other in a
+// lane.  The cuts follow what each block waits for:
+//   TimePart       what depends on the time and the halo alone: the virial
+//                  scales, the power laws of the virial velocity, the
+//                  cooling table's temperature index;
+//   HotProfile     the hot halo's density profile (its outer radius and mass);
+//   BlackHole      ISCO, Eddington cap and accretion from the spheroid;
+//   CoolingTime    the cooling function and time of the hot gas;
+//   galaxy_rates, outer_radius_rates    the galaxy half of the derivative:
+//                  spin growth, satellite mass loss, star formation, stellar
+//                  feedback, bar instability, CGM accretion, outflow
+//                  reincorporation and the CGM outer radius;
+//   hot_accretion, black_hole_rates, radiated_energy, cooling_rates    the
+//                  hot-halo half: black-hole accretion, jet and winds, cooling
+//                  and heating, radiated energy.
+// The derivative is f_galaxy + f_halo in every caller, and a block is the
+// same code wherever it runs: one lane computing all of them and four waves
+// computing some each give the same bits.
 
-template <int PART>
-__device__ __forceinline__ void rhs_part(const double* __restrict__ P, const DerivedConstants& D,
-                                         const double* __restrict__ tab, const CoolingDesc& cd, int mode,
-                                         const NodePar& np, double t, const double (&y)[kNV], double (&f)[kNV]) {
-  constexpr bool GAL = (PART & kRhsGalaxy) != 0, HOT = (PART & kRhsHalo) != 0;
-#pragma unroll
-  for (int i = 0; i < kNV; ++i) f[i] = 0.0;
-  if (mode == GAL_PHYSICS_TEST) {
-    // source/tests/ODE_solver/functions.F90:37-80
-    if constexpr (GAL) {
-      f[0] = sin(t);
-      f[1] = y[2];
-      f[2] = -1.0 * y[1];
-    }
-    return;
-  }
-  const bool box = mode == GAL_PHYSICS_BOX;
-  // closed-box mode has no hot halo, black hole or CGM
-  if constexpr (!GAL) {
-    if (box) return;
-  }
-  // ---- chains that do not depend on the halo scales ---------------------
-  const double m_bh = y[GAL_V_BH_MASS];
-  const double spin = fmin(fmax(y[GAL_V_BH_SPIN], 0.0), 0.998);
-  double e_isco, l_isco;
-  isco(spin, e_isco, l_isco);
-  const double m_hot = y[GAL_V_HOT_MASS], r_out = y[GAL_V_HOT_OUTER_RADIUS];
-  const bool hot_ok = m_hot > 0.0 && r_out > 0.0;
-  // Reciprocal masses for the ratios of a reservoir (metallicity, specific
-  // angular momentum).  Below kRatioMassMin the ratio is taken as zero: rcp()
-  // of a subnormal mass overflows (NaN after the Newton steps), and a
-  // reservoir that enforceNonNegativity lets decay towards zero by halved
-  // steps reaches subnormal values; every flow such a ratio multiplies scales
-  // with the reservoir itself, so the flows dropped are below 1e-100 Msun/Gyr.
-  constexpr double kRatioMassMin = 1.0e-100;
-  const double inv_m_hot = (hot_ok && m_hot > kRatioMassMin) ? rcp(m_hot) : 0.0;
-  const double zf = fmin(fmax(y[GAL_V_HOT_ABUNDANCES] * inv_m_hot, 0.0), 1.0);
-  const double lz = log(clamp_metallicity(cd, zf * (1.0 / kMetallicitySolar)));
-  const double mg_d = y[GAL_V_DISK_MASS_GAS], ms_d = y[GAL_V_DISK_MASS_STELLAR];
-  const double j_d = y[GAL_V_DISK_ANGULAR_MOMENTUM], zg_d = y[GAL_V_DISK_ABUNDANCES_GAS];
-  const double mg_s = y[GAL_V_SPHEROID_MASS_GAS], ms_s = y[GAL_V_SPHEROID_MASS_STELLAR];
-  const double j_s = y[GAL_V_SPHEROID_ANGULAR_MOMENTUM], zg_s = y[GAL_V_SPHEROID_ABUNDANCES_GAS];
-  const double inv_mg_d = mg_d > kRatioMassMin ? rcp(mg_d) : 0.0;
-  const double inv_mg_s = mg_s > kRatioMassMin ? rcp(mg_s) : 0.0;
-  const double mt_d = mg_d + ms_d, mt_s = mg_s + ms_s;
-  const double inv_mt_d = mt_d > kRatioMassMin ? rcp(mt_d) : 0.0;
-  const double inv_mt_s = mt_s > kRatioMassMin ? rcp(mt_s) : 0.0;
+// Reciprocal masses for the ratios of a reservoir (metallicity, specific
+// angular momentum).  Below kRatioMassMin the ratio is taken as zero: rcp()
+// of a subnormal mass overflows (NaN after the Newton steps), and a
+// reservoir that enforceNonNegativity lets decay towards zero by halved
+// steps reaches subnormal values; every flow such a ratio multiplies scales
+// with the reservoir itself, so the flows dropped are below 1e-100 Msun/Gyr.
+constexpr double kRatioMassMin = 1.0e-100;
+// Written, like the other conditional reciprocals here, as a value and a
+// select: a branch around five instructions costs more than they do and keeps
+// the scheduler from filling their latency with other chains.
+__device__ __forceinline__ double rcp_ratio(double mass) {
+  const double r = rcp(mass);
+  return mass > kRatioMassMin ? r : 0.0;
+}
 
-  // ---- halo analytics ----------------------------------------------------
-  const Halo H = halo(P, D, np, t, y[GAL_V_SPIN_ANGULAR_MOMENTUM]);
-  const double v_gal = H.v_vir, r_gal = H.r_gal;
+// Test ODEs (source/tests/ODE_solver/functions.F90:37-80).
+__device__ __forceinline__ void test_rates(double t, const double (&y)[kNV], double (&f)[kNV]) {
+  f[0] = sin(t);
+  f[1] = y[2];
+  f[2] = -1.0 * y[1];
+}
+
+struct TimePart {
+  double time;
+  double mass, inv_mass, r_vir, inv_r_vir, v_vir, inv_v, t_dyn, inv_t_dyn;
+  double inv_j_scale;        // 1 / (M V r), 0 for a halo without mass
+  double r_gal_per_lambda;   // galacticStructureSolver factor * r_vir (fixed.F90:318-325)
+  double r_vir_rate;
+  double failed;             // accretion suppressed by reionization (1 or 0)
+  double pow_sf_d, pow_sf_s, pow_fb_d, pow_fb_s;   // the four power laws of the virial velocity
+  double t_vir, table_t, table_ht;                 // virial temperature, its table row and weight
+  double r_core, inv_r_core;
+  double cs, inv_cs2;        // sound speed of the hot gas
+  double bind, profile_vir, profile_small, rho_min;   // font2008 binding scale, profile shape at r_vir and 1e-6 r_vir
+};
+
+__device__ __forceinline__ TimePart time_part(const double* __restrict__ P, const DerivedConstants& D,
+                                              const CoolingDesc& cd, const NodePar& np, double t) {
+  TimePart T;
+  T.time = t;
+  const Halo H = halo(P, D, np, t, 0.0);
+  T.mass = H.mass;
+  T.r_vir = H.r_vir;
+  T.inv_r_vir = H.inv_r_vir;
+  T.v_vir = H.v_vir;
+  T.inv_v = H.inv_v;
+  T.t_dyn = H.t_dyn;
+  T.inv_t_dyn = H.inv_t_dyn;
+  T.inv_j_scale = H.inv_j_scale;
+  T.r_gal_per_lambda = P[GAL_P_RADIUS_FACTOR] * H.r_vir;
+  T.r_vir_rate = H.r_vir_rate;
+  T.inv_mass = rcp(H.mass);
+  T.failed = (H.a3 > D.a3_reion && H.v_vir < P[GAL_P_VELOCITY_SUPPRESSION_REIONIZATION]) ? 1.0 : 0.0;
+  const double v_gal = H.v_vir;
   const double inv_sqrt_v = rsqrt(v_gal);
   const double sqrt_v = v_gal * inv_sqrt_v;
   const bool generic_pow = D.n2_sf_disk == kNoHalfPower || D.n2_sf_sph == kNoHalfPower ||
                            D.n2_fb_disk == kNoHalfPower || D.n2_fb_sph == kNoHalfPower;
-  const double ln_v = generic_pow ? log(v_gal) : 0.0;
-  const double tdyn_gal = kMpcPerKmsToGyr * r_gal * H.inv_v;
-  const double inv_tdyn_gal = H.v_vir * rcp(r_gal) * (1.0 / kMpcPerKmsToGyr);
-  const double t_vir = D.t_vir_per_v2 * H.v_vir * H.v_vir;
-  const double lt = log(clamp_temperature(cd, t_vir));
+  const double ln_v = __builtin_amdgcn_readfirstlane((int)generic_pow) ? log(v_gal) : 0.0;
+  const double x_sf = v_gal * D.inv_200, sqrt_x_sf = sqrt_v * D.inv_sqrt_200;
+  T.pow_sf_d = pow_param(x_sf, sqrt_x_sf, ln_v - D.ln_200, D.n2_sf_disk, P[GAL_P_SF_DISK_EXPONENT_VELOCITY]);
+  T.pow_sf_s = pow_param(x_sf, sqrt_x_sf, ln_v - D.ln_200, D.n2_sf_sph, P[GAL_P_SF_SPHEROID_EXPONENT_VELOCITY]);
+  T.pow_fb_d = pow_param(D.v_fb_disk * H.inv_v, D.sqrt_v_fb_disk * inv_sqrt_v, D.ln_v_fb_disk - ln_v, D.n2_fb_disk,
+                         P[GAL_P_FB_DISK_EXPONENT]);
+  T.pow_fb_s = pow_param(D.v_fb_sph * H.inv_v, D.sqrt_v_fb_sph * inv_sqrt_v, D.ln_v_fb_sph - ln_v, D.n2_fb_sph,
+                         P[GAL_P_FB_SPHEROID_EXPONENT]);
+  T.t_vir = D.t_vir_per_v2 * H.v_vir * H.v_vir;
+  cooling_temperature_index(cd, log(clamp_temperature(cd, T.t_vir)), T.table_t, T.table_ht);
+  T.r_core = P[GAL_P_CORE_RADIUS_OVER_VIRIAL] * H.r_vir;
+  T.inv_r_core = H.inv_r_vir * D.inv_core;
+  const double cs2 = D.cs2_per_t * T.t_vir;
+  T.cs = sqrt(cs2);
+  T.inv_cs2 = rcp(cs2);
+  T.bind = P[GAL_P_RAM_PRESSURE_FORM_FACTOR] * H.v_vir * H.v_vir;
+  const double x_v = H.r_vir * T.inv_r_core, x_s = 1.0e-6 * H.r_vir * T.inv_r_core;
+  T.profile_vir = rcp(1.0 + x_v * x_v);
+  T.profile_small = rcp(1.0 + x_s * x_s);
+  T.rho_min = D.f_baryon * H.mass * (H.inv_r_vir * H.inv_r_vir * H.inv_r_vir) * (1.0 / (4.0 * kPi));
+  return T;
+}
 
-  // ---- hot-halo structure (both halves: the galaxy half strips it) ------
-  // beta=2/3 profile, core coreRadiusOverVirialRadius*r_vir, truncated at
-  // outerRadius (hot_halo/mass_distribution/beta_profile.F90); virial
-  // (isothermal) temperature (hot_halo/temperature_profile/virial.F90).
-  const double r_core = P[GAL_P_CORE_RADIUS_OVER_VIRIAL] * H.r_vir;
-  const double inv_r_core = H.inv_r_vir * D.inv_core;
-  const double xo = r_out * inv_r_core;
-  // shape integrals S = x - atan x and N = (x^2 - ln(1 + x^2))/2, by their
-  // Taylor series below x = 0.01 where the differences cancel
-  const double uo = xo * xo;
-  const bool small_xo = xo < 0.01;
-  const double shape_m = small_xo ? xo * uo * (1.0 / 3.0 - uo * (1.0 / 5.0 - uo * (1.0 / 7.0 - uo * (1.0 / 9.0))))
-                                  : xo - atan(xo);
-  const double inv_shape = hot_ok ? rcp(shape_m) : 0.0;
-  const double rho0 = m_hot * inv_shape * (1.0 / (4.0 * kPi)) * inv_r_core * inv_r_core * inv_r_core;
-  const double rho_out = rho0 * rcp(1.0 + xo * xo);
+__device__ __forceinline__ GalaxyRadius galaxy_radius(const TimePart& T, double spin_j) {
+  const double lambda = T.inv_j_scale != 0.0 ? spin_j * T.inv_j_scale : 0.0;
+  return GalaxyRadius{T.r_gal_per_lambda, lambda, rounded(T.r_gal_per_lambda * lambda)};
+}
 
-  const int ops = box ? 0 : (int)P[GAL_P_OPERATORS];
-  if constexpr (GAL) {
+// Hot-halo structure: beta=2/3 profile, core coreRadiusOverVirialRadius*r_vir,
+// truncated at outerRadius (hot_halo/mass_distribution/beta_profile.F90).
+// Shape integrals S = x - atan x and N = (x^2 - ln(1 + x^2))/2, by their
+// Taylor series below x = 0.01 where the differences cancel.
+struct HotProfile {
+  double xo, uo, inv_shape, rho0, rho_out;
+};
+
+__device__ __forceinline__ HotProfile hot_profile(const TimePart& T, double m_hot, double r_out) {
+  HotProfile p;
+  p.xo = rounded(r_out * T.inv_r_core);
+  p.uo = rounded(p.xo * p.xo);
+  const double uo = p.uo;
+  const bool hot_ok = m_hot > 0.0 && r_out > 0.0;
+  const double series = p.xo * uo * (1.0 / 3.0 - uo * (1.0 / 5.0 - uo * (1.0 / 7.0 - uo * (1.0 / 9.0))));
+  const double closed = p.xo - atan(p.xo);
+  const double shape = p.xo < 0.01 ? series : closed;
+  const double inv_shape = rcp(shape);
+  p.inv_shape = hot_ok ? inv_shape : 0.0;
+  p.rho0 = rounded(m_hot * p.inv_shape * (1.0 / (4.0 * kPi)) * T.inv_r_core * T.inv_r_core * T.inv_r_core);
+  p.rho_out = rounded(p.rho0 * rcp(1.0 + p.uo));
+  return p;
+}
+
+// 1 / <r> of the hot gas, for the specific angular momentum at a radius.
+__device__ __forceinline__ double hot_inv_mean_radius(const TimePart& T, const HotProfile& p) {
+  const double uo = p.uo;
+  const double series = uo * uo * (1.0 / 4.0 - uo * (1.0 / 6.0 - uo * (1.0 / 8.0 - uo * (1.0 / 10.0))));
+  const double closed = 0.5 * uo - 0.5 * log1p(uo);
+  const double shape_r = p.xo < 0.01 ? series : closed;
+  return rounded(rcp(T.r_core * shape_r * p.inv_shape));
+}
+
+// What black-hole accretion needs beside the hot gas (blackHolesAccretion,
+// black_holes/accretion.F90:113-170; accretion_rates/standard.F90:236-440;
+// Bondi-Hoyle-Lyttleton: accretion/Bondi_Hoyle_Lyttleton.F90:34-78; thin disk:
+// accretion_disks/Shakura_Sunyaev.F90:70-179).
+struct BlackHole {
+  double eff_thin, edd_cap, spin_up, mdot_sph;
+};
+
+__device__ __forceinline__ double black_hole_spin(double y_spin) { return fmin(fmax(y_spin, 0.0), 0.998); }
+
+__device__ __forceinline__ BlackHole black_hole(const double* __restrict__ P, const DerivedConstants& D,
+                                                const GalaxyRadius& galaxy, double m_bh, double y_spin, double r_bh, double mg_s) {
+  BlackHole b;
+  const double spin = black_hole_spin(y_spin);
+  const Isco is = isco(spin);
+  b.eff_thin = fma(-is.energy, is.inv_den, 1.0);
+  b.edd_cap = rounded(D.m_edd_per_mass * m_bh * rcp(b.eff_thin));
+  b.spin_up = fma(is.ang_mom, is.inv_den, -(2.0 * spin * rounded(is.energy * is.inv_den)));
+  double racc = P[GAL_P_BH_TEMPERATURE_SPHEROID] > 0.0 ? kGravity * m_bh * D.inv_cs2_sph : HUGE_VAL;
+  racc = fmax(racc, r_bh);
+  const double rho_a = hernquist_density(mg_s, galaxy, racc);
+  const double lj = fmin(rsqrt(D.jeans_coeff * rho_a), galaxy.r);
+  const double rho_j = hernquist_density(mg_s, galaxy, lj);
+  const double rho = lj > racc ? rho_j : rho_a;
+  double m = fmax(D.bhl_sph_coeff * m_bh * m_bh * rho, 0.0);
+  m = (m > 0.0 && b.eff_thin > 0.0) ? fmin(m, b.edd_cap) : m;
+  b.mdot_sph = (m_bh > 0.0 && rho_a > 1.0) ? m : 0.0;
+  return b;
+}
+
+// Cooling function and time of the hot gas: virial (isothermal) temperature
+// (hot_halo/temperature_profile/virial.F90), composition of metallicity-only
+// abundances with fully ionized H and He, simpleTime
+// (cooling_time/simple.F90:128-181): t_cool = K / rho.
+struct CoolingTime {
+  double inv_m_hot, lambda_cool, nall_per_nh, nh_per_rho, k, inv_k;
+};
+
+__device__ __forceinline__ CoolingTime cooling_time(const DerivedConstants& D, const double* __restrict__ tab,
+                                                    const CoolingDesc& cd, const TimePart& T, double m_hot,
+                                                    double z_hot, double r_out) {
+  CoolingTime c;
+  const bool hot_ok = m_hot > 0.0 && r_out > 0.0;
+  const double inv_m = rcp(m_hot);
+  c.inv_m_hot = (hot_ok && m_hot > kRatioMassMin) ? inv_m : 0.0;
+  const double zf = fmin(fmax(z_hot * c.inv_m_hot, 0.0), 1.0);
+  const double lz = log(clamp_metallicity(cd, zf * (1.0 / kMetallicitySolar)));
+  c.lambda_cool = cooling_function_ln(tab, cd, T.table_t, T.table_ht, lz);
+  constexpr double kNorm = 1.0 / (kHydrogenPrimordial + kHeliumPrimordial);
+  const double X = (1.0 - zf) * kHydrogenPrimordial * kNorm;
+  const double Yh = (1.0 - zf) * kHeliumPrimordial * kNorm;
+  const double nh_n = X / kAtomicMassHydrogen, nhe_n = Yh / kAtomicMassHelium;
+  c.nh_per_rho = rounded(X * D.nh_coeff);
+  const double inv_nh_n = rcp(nh_n);
+  c.nall_per_nh = (nh_n + nhe_n) * inv_nh_n + (1.0 + 2.0 * nhe_n * inv_nh_n);
+  c.k = rounded(D.cool_k_pre * T.t_vir * c.nall_per_nh * rcp(c.lambda_cool * c.nh_per_rho));
+  c.inv_k = rcp(c.k);
+  return c;
+}
+
+__device__ __forceinline__ void galaxy_rates(const double* __restrict__ P, const DerivedConstants& D, int ops, bool box,
+                                             const NodePar& np, const TimePart& T, const double (&y)[kNV],
+                                             double (&f)[kNV]) {
+  const double mg_d = y[GAL_V_DISK_MASS_GAS], ms_d = y[GAL_V_DISK_MASS_STELLAR];
+  const double j_d = y[GAL_V_DISK_ANGULAR_MOMENTUM], zg_d = y[GAL_V_DISK_ABUNDANCES_GAS];
+  const double mg_s = y[GAL_V_SPHEROID_MASS_GAS], ms_s = y[GAL_V_SPHEROID_MASS_STELLAR];
+  const double j_s = y[GAL_V_SPHEROID_ANGULAR_MOMENTUM], zg_s = y[GAL_V_SPHEROID_ABUNDANCES_GAS];
+  const double inv_mg_d = rcp_ratio(mg_d), inv_mg_s = rcp_ratio(mg_s);
+  const double mt_d = mg_d + ms_d, mt_s = mg_s + ms_s;
+  const double inv_mt_d = rcp_ratio(mt_d), inv_mt_s = rcp_ratio(mt_s);
+  const double v_gal = T.v_vir, r_gal = galaxy_radius(T, y[GAL_V_SPIN_ANGULAR_MOMENTUM]).r;
+  const double tdyn_gal = kMpcPerKmsToGyr * r_gal * T.inv_v;
+  const double inv_tdyn_gal = T.v_vir * rcp(r_gal) * (1.0 / kMpcPerKmsToGyr);
   // spin%angularMomentum growth (halo_angular_momentum_interpolate.F90)
   f[GAL_V_SPIN_ANGULAR_MOMENTUM] += np.satellite ? 0.0 : np.spin_rate;
   // satelliteMassLoss (satellite/mass_loss/_class.F90:176-200): an isolated
@@ -338,15 +492,14 @@ __device__ __forceinline__ void rhs_part(const double* __restrict__ P, const Der
   // timescaleRate (star_formation/rates/disks/timescale.F90:109-130),
   // instantaneousRates (stellar_populations/properties/instantaneous.F90:133-182)
   const bool disk_ok = !(j_d < 0.0 || r_gal < 0.0 || mg_d < 0.0);
-  const double x_sf = v_gal * D.inv_200, sqrt_x_sf = sqrt_v * D.inv_sqrt_200;
   double tau_d;
   {
     const double eff = P[GAL_P_SF_DISK_EFFICIENCY];
-    const double pw = pow_param(x_sf, sqrt_x_sf, ln_v - D.ln_200, D.n2_sf_disk, P[GAL_P_SF_DISK_EXPONENT_VELOCITY]);
-    tau_d = (v_gal <= 0.0 || eff == 0.0) ? 0.0 : fmax(tdyn_gal * pw * D.inv_eff_sf_disk, P[GAL_P_SF_DISK_TIMESCALE_MINIMUM]);
+    tau_d = (v_gal <= 0.0 || eff == 0.0) ? 0.0 : fmax(tdyn_gal * T.pow_sf_d * D.inv_eff_sf_disk, P[GAL_P_SF_DISK_TIMESCALE_MINIMUM]);
     if (box) tau_d = P[GAL_P_BOX_TIMESCALE];  // starFormationTimescale fixed
   }
-  const double sfr_d = (disk_ok && tau_d > 0.0) ? mg_d * rcp(tau_d) : 0.0;
+  const double sfr_of_tau_d = mg_d * rcp(tau_d);
+  const double sfr_d = (disk_ok && tau_d > 0.0) ? sfr_of_tau_d : 0.0;
   {
     const double zfuel = zg_d * inv_mg_d;
     const double rs = (1.0 - R) * sfr_d;
@@ -361,11 +514,11 @@ __device__ __forceinline__ void rhs_part(const double* __restrict__ P, const Der
   double tau_s;
   {
     const double eff = P[GAL_P_SF_SPHEROID_EFFICIENCY];
-    const double pw = pow_param(x_sf, sqrt_x_sf, ln_v - D.ln_200, D.n2_sf_sph, P[GAL_P_SF_SPHEROID_EXPONENT_VELOCITY]);
-    tau_s = (v_gal <= 0.0 || eff == 0.0) ? 0.0 : fmax(tdyn_gal * pw * D.inv_eff_sf_sph, P[GAL_P_SF_SPHEROID_TIMESCALE_MINIMUM]);
+    tau_s = (v_gal <= 0.0 || eff == 0.0) ? 0.0 : fmax(tdyn_gal * T.pow_sf_s * D.inv_eff_sf_sph, P[GAL_P_SF_SPHEROID_TIMESCALE_MINIMUM]);
     if (box) tau_s = P[GAL_P_BOX_TIMESCALE];  // starFormationTimescale fixed
   }
-  const double sfr_s = (sph_ok && tau_s > 0.0) ? mg_s * rcp(tau_s) : 0.0;
+  const double sfr_of_tau_s = mg_s * rcp(tau_s);
+  const double sfr_s = (sph_ok && tau_s > 0.0) ? sfr_of_tau_s : 0.0;
   {
     const double zfuel = zg_s * inv_mg_s;
     const double rs = (1.0 - R) * sfr_s;
@@ -383,9 +536,7 @@ __device__ __forceinline__ void rhs_part(const double* __restrict__ P, const Der
   const double inv_tdyn_fb = (v_gal <= 0.0 || r_gal <= 0.0) ? 1.0 : inv_tdyn_gal;
   double out_d, out_s;
   {
-    const double w = D.v_fb_disk * H.inv_v;
-    double o = pow_param(w, D.sqrt_v_fb_disk * inv_sqrt_v, D.ln_v_fb_disk - ln_v, D.n2_fb_disk,
-                         P[GAL_P_FB_DISK_EXPONENT]) * sfr_d;
+    double o = T.pow_fb_d * sfr_d;
     o = v_gal <= 0.0 ? 0.0 : o;
     if (box) o = P[GAL_P_BOX_OUTFLOW_FRACTION] * sfr_d;  // stellarFeedbackOutflows fixed
     const double omax = fmax(mg_d * inv_tdyn_fb * D.inv_tmin_fb_disk, 0.0);
@@ -393,9 +544,7 @@ __device__ __forceinline__ void rhs_part(const double* __restrict__ P, const Der
     out_d = (disk_ok && o > 0.0) ? o : 0.0;
   }
   {
-    const double w = D.v_fb_sph * H.inv_v;
-    double o = pow_param(w, D.sqrt_v_fb_sph * inv_sqrt_v, D.ln_v_fb_sph - ln_v, D.n2_fb_sph,
-                         P[GAL_P_FB_SPHEROID_EXPONENT]) * sfr_s;
+    double o = T.pow_fb_s * sfr_s;
     o = v_gal <= 0.0 ? 0.0 : o;
     if (box) o = P[GAL_P_BOX_OUTFLOW_FRACTION_SPHEROID] * sfr_s;  // stellarFeedbackOutflows fixed
     const double omax = fmax(mg_s * inv_tdyn_fb * D.inv_tmin_fb_sph, 0.0);
@@ -435,8 +584,8 @@ __device__ __forceinline__ void rhs_part(const double* __restrict__ P, const Der
   // NaN gas fraction and, as in the reference, no instability.
   {
     constexpr double kEpsIso = 0.6221297315, kBoost = 1.1800237580, kDimMax = 1.0e10;
-    const double fgas = mg_d * rcp(mt_d);
-    const double thr = P[GAL_P_BAR_THRESHOLD_STELLAR] * (1.0 - fgas) + P[GAL_P_BAR_THRESHOLD_GASEOUS] * fgas;
+    const double inv_mt_d = rcp(mt_d), fgas = rounded(mg_d * inv_mt_d);
+    const double thr = fma(P[GAL_P_BAR_THRESHOLD_STELLAR], fma(-mg_d, inv_mt_d, 1.0), rounded(P[GAL_P_BAR_THRESHOLD_GASEOUS] * fgas));
     const double v_self2 = kGravity * mt_d * rcp(r_gal);
     double est = fmax(kEpsIso, kBoost * v_gal * rsqrt(v_self2));
     est = (mt_d >= 0.0 && v_self2 > 0.0) ? est : HUGE_VAL;
@@ -467,9 +616,8 @@ __device__ __forceinline__ void rhs_part(const double* __restrict__ P, const Der
   // ---- CGMAccretion (circumgalactic_medium/accretion.F90:517) with
   //      accretionHalo simple (accretion/halo/simple.F90:281-378) ---------
   {
-    const bool acc = !np.satellite && H.mass > 0.0;
-    const double failed = (H.a3 > D.a3_reion && H.v_vir < P[GAL_P_VELOCITY_SUPPRESSION_REIONIZATION]) ? 1.0 : 0.0;
-    const double inv_mass = rcp(H.mass);
+    const bool acc = !np.satellite && T.mass > 0.0;
+    const double failed = T.failed, inv_mass = T.inv_mass;
     const double growth = np.m_rate * inv_mass;
     const double m_un = y[GAL_V_HOT_UNACCRETED_MASS], z_un = y[GAL_V_HOT_UNACCRETED_ABUNDANCES];
     const double rate_acc = D.f_baryon * np.m_rate * (1.0 - failed) + m_un * growth * (1.0 - failed);
@@ -486,7 +634,7 @@ __device__ __forceinline__ void rhs_part(const double* __restrict__ P, const Der
   {
     const double m_o = y[GAL_V_HOT_OUTFLOWED_MASS];
     const bool ok = m_o > 0.0;
-    const double q = P[GAL_P_REINCORPORATION_MULTIPLIER] * H.inv_t_dyn;
+    const double q = P[GAL_P_REINCORPORATION_MULTIPLIER] * T.inv_t_dyn;
     const double r = m_o * q;
     const double rr = ok ? r : 0.0;
     const double rj = ok ? y[GAL_V_HOT_OUTFLOWED_ANGULAR_MOMENTUM] * q : 0.0;
@@ -498,116 +646,99 @@ __device__ __forceinline__ void rhs_part(const double* __restrict__ P, const Der
     f[GAL_V_HOT_ANGULAR_MOMENTUM] += rj;
     f[GAL_V_HOT_ABUNDANCES] += rz;
   }
-  // ---- CGMOuterRadiusRamPressureStripping
-  //      (circumgalactic_medium/outer_radius/ram_pressure_stripping.F90:111-242)
-  // Returning outflows push the outer radius out when it lies inside the
-  // virial radius; a central's follows the virial radius; a satellite's
-  // shrinks towards the font2008 stripping radius
-  // (hot_halo/ram_pressure_stripping/Font2008.F90:115-267) on the
-  // ram-pressure acceleration time (timescale/ram_pressure_acceleration.F90:79-134).
-  // The stripping radius is the closed form of the binding condition
-  // formFactor G M(<r) rho_hot(r) / r = F for the isothermal halo
-  // M(<r) = M_vir r / r_vir: formFactor V_vir^2 rho_hot(r) = F.
-  if (ops & GAL_OPERATOR_CGM_OUTER_RADIUS) {
-    const double rv = H.r_vir;
-    const double rho_ro = hot_ok ? rho_out : 0.0;
-    const double m_return = y[GAL_V_HOT_OUTFLOWED_MASS] * P[GAL_P_REINCORPORATION_MULTIPLIER] * H.inv_t_dyn;
-    const double rho_min = D.f_baryon * H.mass * (H.inv_r_vir * H.inv_r_vir * H.inv_r_vir) * (1.0 / (4.0 * kPi));
-    const double ret_a = m_return * (1.0 / (4.0 * kPi)) * rcp(r_out * r_out * fmax(rho_ro, rho_min));
-    const double ret_b = m_return * rcp(H.mass) * rv;
-    double ret = (r_out > 0.0 && rho_ro > 0.0) ? ret_a : (m_return > 0.0 ? ret_b : 0.0);
-    // the outer radius starts at the virial radius, an exact tie in the
-    // reference; a last-place difference between the caller's value and the
-    // recomputed virial radius is judged a tie (1e-12 relative)
-    const bool at_rv = r_out >= rv * (1.0 - 1.0e-12);
-    ret = at_rv ? 0.0 : ret;
-    // stripping radius and timescale
-    const double force = np.ram_force;
-    const double bind = P[GAL_P_RAM_PRESSURE_FORM_FACTOR] * H.v_vir * H.v_vir;
-    const double x_v = rv * inv_r_core, r_small = 1.0e-6 * rv, x_s = r_small * inv_r_core;
-    const double rho_rv = (hot_ok && at_rv) ? rho0 * rcp(1.0 + x_v * x_v) : 0.0;
-    const double rho_small = (hot_ok && r_small <= r_out) ? rho0 * rcp(1.0 + x_s * x_s) : 0.0;
-    const double r_star = fmin(r_core * sqrt(fmax(bind * rho0 * rcp(force) - 1.0, 0.0)), r_out);
-    const double r_rp = bind * rho_rv - force >= 0.0 ? rv : (bind * rho_small - force <= 0.0 ? 0.0 : r_star);
-    const double sigma = r_out * rho_ro;
-    const double t_floor = np.v_host > 0.0 ? r_out * 0.1 * rcp(np.v_host) : HUGE_VAL;
-    double tau = kMpcPerKmsToGyr * fmax(sqrt(2.0 * r_out * sigma * rcp(force)), t_floor);
-    tau = (r_out <= 0.0 || sigma <= 0.0) ? H.t_dyn : tau;
-    tau = force <= 0.0 ? kDoubleMax : tau;
-    const double dr = (r_rp < r_out && y[GAL_V_HOT_ANGULAR_MOMENTUM] > 0.0) ? (r_rp - r_out) / tau : 0.0;
-    const bool strip = np.satellite && dr != 0.0 && m_hot > 0.0 && r_out > 1.0e-3 * rv;
-    const double loss = strip ? 4.0 * kPi * rho_ro * r_out * r_out * dr : 0.0;
-    const double lm = loss * inv_m_hot;
-    f[GAL_V_HOT_OUTER_RADIUS] += ret + (np.satellite ? (strip ? dr : 0.0) : H.r_vir_rate);
-    f[GAL_V_HOT_MASS] += loss;
-    f[GAL_V_HOT_ANGULAR_MOMENTUM] += y[GAL_V_HOT_ANGULAR_MOMENTUM] * lm;
-    f[GAL_V_HOT_ABUNDANCES] += y[GAL_V_HOT_ABUNDANCES] * lm;
-    f[GAL_V_HOT_STRIPPED_MASS] -= loss;
-    f[GAL_V_HOT_STRIPPED_ABUNDANCES] -= y[GAL_V_HOT_ABUNDANCES] * lm;
-  }
-  }  // galaxy half
-  if constexpr (!HOT) return;
-  // ---- cooling radius ------------------------------------------------------
-  const double shape_r = small_xo ? uo * uo * (1.0 / 4.0 - uo * (1.0 / 6.0 - uo * (1.0 / 8.0 - uo * (1.0 / 10.0))))
-                                  : 0.5 * uo - 0.5 * log1p(uo);
-  const double r_mean = r_core * shape_r * inv_shape;
-  // composition of metallicity-only abundances, fully ionized H and He
-  constexpr double kNorm = 1.0 / (kHydrogenPrimordial + kHeliumPrimordial);
-  const double X = (1.0 - zf) * kHydrogenPrimordial * kNorm;
-  const double Yh = (1.0 - zf) * kHeliumPrimordial * kNorm;
-  const double nh_n = X / kAtomicMassHydrogen, nhe_n = Yh / kAtomicMassHelium;
-  const double nh_per_rho = X * D.nh_coeff;
-  const double inv_nh_n = rcp(nh_n);
-  const double nall_per_nh = (nh_n + nhe_n) * inv_nh_n + (1.0 + 2.0 * nhe_n * inv_nh_n);
-  const double lambda_cool = cooling_function_ln(tab, cd, lt, lz);
-  // simpleTime (cooling_time/simple.F90:128-181): t_cool = K / rho;
+}
+
+// ---- CGMOuterRadiusRamPressureStripping
+//      (circumgalactic_medium/outer_radius/ram_pressure_stripping.F90:111-242)
+// Returning outflows push the outer radius out when it lies inside the
+// virial radius; a central's follows the virial radius; a satellite's
+// shrinks towards the font2008 stripping radius
+// (hot_halo/ram_pressure_stripping/Font2008.F90:115-267) on the
+// ram-pressure acceleration time (timescale/ram_pressure_acceleration.F90:79-134).
+// The stripping radius is the closed form of the binding condition
+// formFactor G M(<r) rho_hot(r) / r = F for the isothermal halo
+// M(<r) = M_vir r / r_vir: formFactor V_vir^2 rho_hot(r) = F.
+__device__ __forceinline__ void outer_radius_rates(const double* __restrict__ P, const NodePar& np, const TimePart& T,
+                                                   double rho0, double rho_out, const double (&y)[kNV],
+                                                   double (&f)[kNV]) {
+  const double m_hot = y[GAL_V_HOT_MASS], r_out = y[GAL_V_HOT_OUTER_RADIUS];
+  const bool hot_ok = m_hot > 0.0 && r_out > 0.0;
+  const double rv = T.r_vir;
+  const double rho_ro = hot_ok ? rho_out : 0.0;
+  const double m_return = y[GAL_V_HOT_OUTFLOWED_MASS] * P[GAL_P_REINCORPORATION_MULTIPLIER] * T.inv_t_dyn;
+  const double ret_a = m_return * (1.0 / (4.0 * kPi)) * rcp(r_out * r_out * fmax(rho_ro, T.rho_min));
+  const double ret_b = m_return * rcp(T.mass) * rv;
+  double ret = (r_out > 0.0 && rho_ro > 0.0) ? ret_a : (m_return > 0.0 ? ret_b : 0.0);
+  // the outer radius starts at the virial radius, an exact tie in the
+  // reference; a last-place difference between the caller's value and the
+  // recomputed virial radius is judged a tie (1e-12 relative)
+  const bool at_rv = r_out >= rv * (1.0 - 1.0e-12);
+  ret = at_rv ? 0.0 : ret;
+  // stripping radius and timescale
+  const double force = np.ram_force;
+  const double bind = T.bind;
+  const double r_small = 1.0e-6 * rv;
+  const double rho_rv = (hot_ok && at_rv) ? rho0 * T.profile_vir : 0.0;
+  const double rho_small = (hot_ok && r_small <= r_out) ? rho0 * T.profile_small : 0.0;
+  const double r_star = fmin(T.r_core * sqrt(fmax(bind * rho0 * rcp(force) - 1.0, 0.0)), r_out);
+  const double r_rp = bind * rho_rv - force >= 0.0 ? rv : (bind * rho_small - force <= 0.0 ? 0.0 : r_star);
+  const double sigma = r_out * rho_ro;
+  const double t_cross = r_out * 0.1 * rcp(np.v_host);
+  const double t_floor = np.v_host > 0.0 ? t_cross : HUGE_VAL;
+  double tau = kMpcPerKmsToGyr * fmax(sqrt(2.0 * r_out * sigma * rcp(force)), t_floor);
+  tau = (r_out <= 0.0 || sigma <= 0.0) ? T.t_dyn : tau;
+  tau = force <= 0.0 ? kDoubleMax : tau;
+  const double dr = (r_rp < r_out && y[GAL_V_HOT_ANGULAR_MOMENTUM] > 0.0) ? (r_rp - r_out) / tau : 0.0;
+  const bool strip = np.satellite && dr != 0.0 && m_hot > 0.0 && r_out > 1.0e-3 * rv;
+  const double loss = strip ? 4.0 * kPi * rho_ro * r_out * r_out * dr : 0.0;
+  const double inv_m = rcp(m_hot);
+  const double inv_m_hot = (hot_ok && m_hot > kRatioMassMin) ? inv_m : 0.0;
+  const double lm = loss * inv_m_hot;
+  f[GAL_V_HOT_OUTER_RADIUS] += ret + (np.satellite ? (strip ? dr : 0.0) : T.r_vir_rate);
+  f[GAL_V_HOT_MASS] += loss;
+  f[GAL_V_HOT_ANGULAR_MOMENTUM] += y[GAL_V_HOT_ANGULAR_MOMENTUM] * lm;
+  f[GAL_V_HOT_ABUNDANCES] += y[GAL_V_HOT_ABUNDANCES] * lm;
+  f[GAL_V_HOT_STRIPPED_MASS] -= loss;
+  f[GAL_V_HOT_STRIPPED_ABUNDANCES] -= y[GAL_V_HOT_ABUNDANCES] * lm;
+}
+
+// ---- the hot-halo half -----------------------------------------------------
+// hot_accretion: cooling radius, hot-mode accretion and jet power, the serial
+// chain of the RHS; black_hole_rates: what the accretion and its winds do to
+// the black hole, the spheroid and the outflow; cooling_rates: cooling against
+// heating of the hot gas.
+struct HotAccretion {
+  double r_cool, xc, mdot_hot, mdot, p_jet;
+};
+
+__device__ __forceinline__ HotAccretion hot_accretion(const double* __restrict__ P, const DerivedConstants& D,
+                                                      const TimePart& T, const CoolingTime& c, double eff_thin,
+                                                      double edd_cap, double mdot_sph, double rho0, double rho_out,
+                                                      double m_hot, double r_out, double m_bh, double y_spin) {
+  const bool hot_ok = m_hot > 0.0 && r_out > 0.0;
+  const double lambda_cool = c.lambda_cool, K = c.k, inv_k = c.inv_k;
   // simpleRadius (cooling_radius/simple.F90:313-387) with t_available = t_dyn
   // (time_available/White-Frenk.F90:144-146, ageFactor = 0)
-  const double t_avail = H.t_dyn;
-  const double K = D.cool_k_pre * t_vir * nall_per_nh * rcp(lambda_cool * nh_per_rho);
-  const double inv_k = rcp(K);
-  double r_cool = fmin(r_core * sqrt(fmax(rho0 * t_avail * inv_k - 1.0, 0.0)), r_out);
+  const double t_avail = T.t_dyn;
+  double r_cool = fmin(T.r_core * sqrt(fmax(rho0 * t_avail * inv_k - 1.0, 0.0)), r_out);
   r_cool = (K - t_avail * rho0 > 0.0) ? 0.0 : r_cool;
   r_cool = (K - t_avail * rho_out < 0.0) ? r_out : r_cool;
   r_cool = (lambda_cool > 0.0 && hot_ok) ? r_cool : 0.0;
-  // simpleRadiusGrowthRate (cooling_radius/simple.F90:229-309); the
-  // time-available growth rate is 1 (White-Frenk.F90:161-168)
-  const double xc = r_cool * inv_r_core;
-  const double slope = 2.0 * xc * xc / (1.0 + xc * xc);
-  double r_cool_rate = r_cool * H.inv_t_dyn * rcp(slope);
-  r_cool_rate = (r_cool < r_out && r_cool > 0.0 && slope != 0.0) ? r_cool_rate : 0.0;
-
-  // ---- blackHolesAccretion (black_holes/accretion.F90:113-170) ----------
-  // rates: accretion_rates/standard.F90:236-440; Bondi-Hoyle-Lyttleton:
-  // accretion/Bondi_Hoyle_Lyttleton.F90:34-78; thin disk:
-  // accretion_disks/Shakura_Sunyaev.F90:70-179.
+  const double xc = rounded(r_cool * T.inv_r_core);
+  // ---- blackHolesAccretion, hot mode -------------------------------------
+  const double spin = black_hole_spin(y_spin);
   const bool bh_ok = m_bh > 0.0;
-  const double eff_thin = 1.0 - e_isco;
-  const double edd_cap = D.m_edd_per_mass * m_bh * rcp(eff_thin);
   constexpr double kBhlUnit = kKilo * kGigaYear / kMegaParsec * 4.0 * kPi;
-  double mdot_sph;
-  {
-    double racc = P[GAL_P_BH_TEMPERATURE_SPHEROID] > 0.0 ? kGravity * m_bh * D.inv_cs2_sph : HUGE_VAL;
-    racc = fmax(racc, y[GAL_V_BH_RADIAL_POSITION]);
-    const double rho_a = hernquist_density(mg_s, r_gal, racc);
-    const double lj = fmin(rsqrt(D.jeans_coeff * rho_a), r_gal);
-    const double rho_j = hernquist_density(mg_s, r_gal, lj);
-    const double rho = lj > racc ? rho_j : rho_a;
-    double m = fmax(D.bhl_sph_coeff * m_bh * m_bh * rho, 0.0);
-    m = (m > 0.0 && eff_thin > 0.0) ? fmin(m, edd_cap) : m;
-    mdot_sph = (bh_ok && rho_a > 1.0) ? m : 0.0;
-  }
   double mdot_hot;
   {
-    const double cs2 = D.cs2_per_t * t_vir;
-    const double cs = sqrt(cs2);
-    const double r2 = fmin(kGravity * m_bh * rcp(cs2), r_out);
-    const double q = r_cool * H.inv_r_vir;
+    const double cs = T.cs;
+    const double r2 = fmin(kGravity * m_bh * T.inv_cs2, r_out);
+    const double q = r_cool * T.inv_r_vir;
     // standardHotModeFraction (accretion_rates/standard.F90:442-466)
     const double xq = (q - 0.9) * 10.0;
     double fhot = xq * xq * (2.0 * xq - 3.0) + 1.0;
     fhot = q < 0.9 ? 1.0 : (q > 1.0 ? 0.0 : fhot);
-    const double rho2 = fhot * (rho0 * rcp(1.0 + sq(r2 * inv_r_core)));
+    const double rho2 = fhot * (rho0 * rcp(1.0 + sq(r2 * T.inv_r_core)));
     double m = fmax(P[GAL_P_BH_ENHANCEMENT_HOT_HALO] * kBhlUnit * r2 * r2 * rho2 * cs, 0.0);
     m = fmin(m, fmax(m_hot * cs * rcp(r_out) * (1.0 / kMpcPerKmsToGyr), 0.0));
     m = (m > 0.0 && eff_thin > 0.0) ? fmin(m, edd_cap) : m;
@@ -619,24 +750,31 @@ __device__ __forceinline__ void rhs_part(const double* __restrict__ P, const Der
   // M^-0.3 Mdot^1.2 = (Mdot^4 / M)^0.3
   const double inv_m_bh = rcp(m_bh);
   const double lm = 0.3 * log(mdot * mdot * mdot * mdot * inv_m_bh);
-  const double p_jet_k = exp(D.ln_jet_kerr + lm) * (1.0 + 1.1 * spin + 0.29 * spin * spin);
-  const double p_jet_s = exp(D.ln_jet_schw + lm + 3.785 * spin);
-  const double p_jet = acc_ok ? (spin > 0.8 ? p_jet_k : p_jet_s) : 0.0;
+  const bool kerr = spin > 0.8;
+  const double e_jet = exp(kerr ? D.ln_jet_kerr + lm : D.ln_jet_schw + lm + 3.785 * spin);
+  const double p_jet_k = e_jet * (1.0 + 1.1 * spin + 0.29 * spin * spin);
+  const double p_jet = acc_ok ? (kerr ? p_jet_k : e_jet) : 0.0;
+  return HotAccretion{r_cool, xc, mdot_hot, mdot, rounded(p_jet)};
+}
+
+__device__ __forceinline__ void black_hole_rates(const double* __restrict__ P, const DerivedConstants& D, int ops,
+                                                 const TimePart& T, const BlackHole& b, double mdot, double p_jet,
+                                                 double m_bh, double mg_s, double ms_s, double j_s, double zg_s,
+                                                 double r_gal, double (&f)[kNV]) {
+  const bool acc_ok = m_bh > 0.0 && mdot > 0.0;
+  const double mt_s = mg_s + ms_s, v_gal = T.v_vir;
+  const double inv_mg_s = rcp_ratio(mg_s), inv_mt_s = rcp_ratio(mt_s), inv_m_bh = rcp(m_bh);
+  const double eff_thin = b.eff_thin, mdot_sph = b.mdot_sph;
   {
     constexpr double kInvC2 = 1.0 / ((kSpeedLight / kKilo) * (kSpeedLight / kKilo));
     const double eff_jet = p_jet * rcp(mdot) * kInvC2;
     const double reduced = mdot * (1.0 - eff_thin - eff_jet);
-    const double spin_up = (l_isco - 2.0 * spin * e_isco) * mdot * inv_m_bh;
+    const double spin_up = b.spin_up * mdot * inv_m_bh;
     f[GAL_V_BH_MASS] += acc_ok ? reduced : 0.0;
     // spheroid%massGasSinkRate: gas, metals and angular momentum in proportion
     f[GAL_V_SPHEROID_MASS_GAS] -= acc_ok ? mdot_sph : 0.0;
     f[GAL_V_SPHEROID_ABUNDANCES_GAS] -= acc_ok ? mdot_sph * (zg_s * inv_mg_s) : 0.0;
     f[GAL_V_SPHEROID_ANGULAR_MOMENTUM] -= acc_ok ? mdot_sph * (j_s * inv_mt_s) : 0.0;
-    // hotHalo%massSinkRate: mass, metals and angular momentum in proportion
-    const bool hs = acc_ok && hot_ok;
-    f[GAL_V_HOT_MASS] -= hs ? mdot_hot : 0.0;
-    f[GAL_V_HOT_ABUNDANCES] -= hs ? mdot_hot * (y[GAL_V_HOT_ABUNDANCES] * inv_m_hot) : 0.0;
-    f[GAL_V_HOT_ANGULAR_MOMENTUM] -= hs ? mdot_hot * (y[GAL_V_HOT_ANGULAR_MOMENTUM] * inv_m_hot) : 0.0;
     f[GAL_V_BH_SPIN] += acc_ok ? spin_up : 0.0;
   }
   // ---- blackHolesWinds (black_holes/winds.F90:102-133) with ciotti2009
@@ -652,7 +790,7 @@ __device__ __forceinline__ void rhs_part(const double* __restrict__ P, const Der
     constexpr double kC2 = (kSpeedLight / kKilo) * (kSpeedLight / kKilo);
     const double power = eff * coupled * mdot * kC2;
     const bool drive = on && power > 0.0 && mg_s > 0.0 && mt_s > 0.0 && v_gal > 0.0;
-    const double mo = drive ? P[GAL_P_SPHEROID_ENERGETIC_OUTFLOW] * power * H.inv_v * H.inv_v : 0.0;
+    const double mo = drive ? P[GAL_P_SPHEROID_ENERGETIC_OUTFLOW] * power * T.inv_v * T.inv_v : 0.0;
     const double jo = mo * inv_mt_s * j_s;
     const double zo = mo * inv_mg_s * zg_s;
     f[GAL_V_SPHEROID_MASS_GAS] -= mo;
@@ -662,27 +800,60 @@ __device__ __forceinline__ void rhs_part(const double* __restrict__ P, const Der
     f[GAL_V_HOT_OUTFLOWED_ANGULAR_MOMENTUM] += jo * D.inv_one_minus_j_loss;
     f[GAL_V_HOT_OUTFLOWED_ABUNDANCES] += zo;
   }
+}
+
+// coolingEnergyRadiated (cooling_energy_radiated.F90:200-260)
+__device__ __forceinline__ double radiated_energy(double lambda_cool, double nh_per_rho, double nall_per_nh,
+                                                  double m_hot, double r_out) {
+  const bool hot_ok = m_hot > 0.0 && r_out > 0.0;
+  const double rho = m_hot * (3.0 / (4.0 * kPi)) * rcp(r_out * r_out * r_out);
+  const double nh = rho * nh_per_rho;
+  const double rcm = r_out * (kMegaParsec / kCenti);
+  const double count = nh * nall_per_nh * (4.0 * kPi / 3.0) * rcm * rcm * rcm;
+  return hot_ok ? lambda_cool * nh * count : 0.0;
+}
+
+__device__ __forceinline__ void cooling_rates(const double* __restrict__ P, const NodePar& np, const TimePart& T,
+                                              const HotAccretion& s, double inv_m_hot, double rho0, double inv_r_mean,
+                                              double m_hot, double z_of_hot, double j_of_hot, double r_out,
+                                              double m_bh, double (&f)[kNV]) {
+  const bool hot_ok = m_hot > 0.0 && r_out > 0.0;
+  const double r_cool = s.r_cool, xc = s.xc, mdot_hot = s.mdot_hot;
+  const bool acc_ok = m_bh > 0.0 && s.mdot > 0.0;
+  {
+    // hotHalo%massSinkRate: mass, metals and angular momentum in proportion
+    const bool hs = acc_ok && hot_ok;
+    f[GAL_V_HOT_MASS] -= hs ? mdot_hot : 0.0;
+    f[GAL_V_HOT_ABUNDANCES] -= hs ? mdot_hot * (z_of_hot * inv_m_hot) : 0.0;
+    f[GAL_V_HOT_ANGULAR_MOMENTUM] -= hs ? mdot_hot * (j_of_hot * inv_m_hot) : 0.0;
+  }
+  // simpleRadiusGrowthRate (cooling_radius/simple.F90:229-309); the
+  // time-available growth rate is 1 (White-Frenk.F90:161-168)
+  const double slope = 2.0 * xc * xc / (1.0 + xc * xc);
+  double r_cool_rate = r_cool * T.inv_t_dyn * rcp(slope);
+  r_cool_rate = (r_cool < r_out && r_cool > 0.0 && slope != 0.0) ? r_cool_rate : 0.0;
+
   // ---- CGMCoolingHeating (circumgalactic_medium/cooling_heating.F90:216-381)
   //      whiteFrenk1991Rate (cooling_rate/White-Frenk.F90:132-185) ---------
   {
-    const bool ok = hot_ok && y[GAL_V_HOT_ANGULAR_MOMENTUM] > 0.0;
+    const bool ok = hot_ok && j_of_hot > 0.0;
     double cool = 4.0 * kPi * r_cool * r_cool * (rho0 * rcp(1.0 + xc * xc)) * r_cool_rate;
-    cool = r_cool >= r_out ? m_hot * H.inv_t_dyn : cool;
-    cool = H.v_vir > P[GAL_P_COOLING_VELOCITY_CUTOFF] ? 0.0 : cool;
-    const double heat = P[GAL_P_EFFICIENCY_RADIO_MODE] * p_jet * sq(H.inv_v);
+    cool = r_cool >= r_out ? m_hot * T.inv_t_dyn : cool;
+    cool = T.v_vir > P[GAL_P_COOLING_VELOCITY_CUTOFF] ? 0.0 : cool;
+    const double heat = rounded(P[GAL_P_EFFICIENCY_RADIO_MODE] * s.p_jet * sq(T.inv_v));
     const bool heating = ok && heat > cool;
     const bool cooling = ok && cool > heat;
     // excess heating expels gas from the node (excessHeatDrivesOutflow); a
     // satellite's joins its stripped reservoir (outflow_stripping/standard.F90:120-131)
     const bool expel = heating && P[GAL_P_EXCESS_HEAT_DRIVES_OUTFLOW] != 0.0;
-    const double out = expel ? fmin(heat - cool, P[GAL_P_RATE_MAXIMUM_EXPULSION] * m_hot * H.inv_t_dyn) : 0.0;
+    const double out = expel ? fmin(heat - cool, P[GAL_P_RATE_MAXIMUM_EXPULSION] * m_hot * T.inv_t_dyn) : 0.0;
     // net cooling onto the disk; constantRotation j(r) = (J/M) r / <r>
     const double c = cooling ? fmax(cool - heat, 0.0) : 0.0;
-    const double j_hot = y[GAL_V_HOT_ANGULAR_MOMENTUM] * inv_m_hot;
-    const double z_hot = y[GAL_V_HOT_ABUNDANCES] * inv_m_hot;
-    const double oz = y[GAL_V_HOT_ABUNDANCES] * (out * inv_m_hot);
-    const double oj = y[GAL_V_HOT_ANGULAR_MOMENTUM] * (out * inv_m_hot);
-    const double cj = cooling ? c * (j_hot * r_cool * rcp(r_mean)) : 0.0;
+    const double j_hot = j_of_hot * inv_m_hot;
+    const double z_hot = z_of_hot * inv_m_hot;
+    const double oz = z_of_hot * (out * inv_m_hot);
+    const double oj = j_of_hot * (out * inv_m_hot);
+    const double cj = cooling ? c * (j_hot * r_cool * inv_r_mean) : 0.0;
     const double cz = c * z_hot;
     f[GAL_V_HOT_MASS] -= heating ? out : c;
     f[GAL_V_HOT_ABUNDANCES] -= heating ? oz : cz;
@@ -693,23 +864,41 @@ __device__ __forceinline__ void rhs_part(const double* __restrict__ P, const Der
     f[GAL_V_DISK_ABUNDANCES_GAS] += cz;
     f[GAL_V_DISK_ANGULAR_MOMENTUM] += cj * (1.0 - P[GAL_P_FRACTION_LOSS_ANGULAR_MOMENTUM]);
   }
-  // ---- coolingEnergyRadiated (cooling_energy_radiated.F90:200-260) -------
-  {
-    const double rho = m_hot * (3.0 / (4.0 * kPi)) * rcp(r_out * r_out * r_out);
-    const double nh = rho * nh_per_rho;
-    const double rcm = r_out * (kMegaParsec / kCenti);
-    const double count = nh * nall_per_nh * (4.0 * kPi / 3.0) * rcm * rcm * rcm;
-    f[GAL_V_HOT_ENERGY_RADIATED] += hot_ok ? lambda_cool * nh * count : 0.0;
-  }
 }
 
-// The whole RHS: both halves, summed as f_galaxy + f_halo.
+// The whole RHS of one node in one lane: the blocks one after the other,
+// summed as f_galaxy + f_halo.
 __device__ __forceinline__ void rhs(const double* __restrict__ P, const DerivedConstants& D,
                                     const double* __restrict__ tab, const CoolingDesc& cd, int mode,
                                     const NodePar& np, double t, const double (&y)[kNV], double (&f)[kNV]) {
   double fh[kNV];
-  rhs_part<kRhsGalaxy>(P, D, tab, cd, mode, np, t, y, f);
-  rhs_part<kRhsHalo>(P, D, tab, cd, mode, np, t, y, fh);
+#pragma unroll
+  for (int i = 0; i < kNV; ++i) f[i] = fh[i] = 0.0;
+  if (mode == GAL_PHYSICS_TEST) {
+    test_rates(t, y, f);
+    return;
+  }
+  const bool box = mode == GAL_PHYSICS_BOX;
+  const int ops = box ? 0 : (int)P[GAL_P_OPERATORS];
+  const TimePart T = time_part(P, D, cd, np, t);
+  galaxy_rates(P, D, ops, box, np, T, y, f);
+  if (!box) {
+    // closed-box mode has no hot halo, black hole or CGM
+    const double m_hot = y[GAL_V_HOT_MASS], r_out = y[GAL_V_HOT_OUTER_RADIUS], z_hot = y[GAL_V_HOT_ABUNDANCES];
+    const double m_bh = y[GAL_V_BH_MASS], y_spin = y[GAL_V_BH_SPIN], mg_s = y[GAL_V_SPHEROID_MASS_GAS];
+    const GalaxyRadius galaxy = galaxy_radius(T, y[GAL_V_SPIN_ANGULAR_MOMENTUM]);
+    const HotProfile p = hot_profile(T, m_hot, r_out);
+    if (ops & GAL_OPERATOR_CGM_OUTER_RADIUS) outer_radius_rates(P, np, T, p.rho0, p.rho_out, y, f);
+    const CoolingTime c = cooling_time(D, tab, cd, T, m_hot, z_hot, r_out);
+    const BlackHole b = black_hole(P, D, galaxy, m_bh, y_spin, y[GAL_V_BH_RADIAL_POSITION], mg_s);
+    const HotAccretion s = hot_accretion(P, D, T, c, b.eff_thin, b.edd_cap, b.mdot_sph, p.rho0, p.rho_out, m_hot,
+                                         r_out, m_bh, y_spin);
+    black_hole_rates(P, D, ops, T, b, s.mdot, s.p_jet, m_bh, mg_s, y[GAL_V_SPHEROID_MASS_STELLAR],
+                     y[GAL_V_SPHEROID_ANGULAR_MOMENTUM], y[GAL_V_SPHEROID_ABUNDANCES_GAS], galaxy.r, fh);
+    fh[GAL_V_HOT_ENERGY_RADIATED] += radiated_energy(c.lambda_cool, c.nh_per_rho, c.nall_per_nh, m_hot, r_out);
+    cooling_rates(P, np, T, s, c.inv_m_hot, p.rho0, hot_inv_mean_radius(T, p), m_hot, z_hot,
+                  y[GAL_V_HOT_ANGULAR_MOMENTUM], r_out, m_bh, fh);
+  }
 #pragma unroll
   for (int i = 0; i < kNV; ++i) f[i] += fh[i];
 }
@@ -717,10 +906,9 @@ __device__ __forceinline__ void rhs(const double* __restrict__ P, const DerivedC
 // Component scale-set rules at the start of an evolve (hot_halo/standard/_class.F90:804-840,
 // disk/standard/_class.F90:735-828, spheroid/standard/_class.F90:804-860,
 // black_hole/standard/_class.F90:195-240, cooling_energy_radiated.F90:150-185).
-__device__ __forceinline__ void scales(const double* __restrict__ P, const DerivedConstants& D, const NodePar& np,
-                                       double t, const double (&y)[kNV], double (&sc)[kNV]) {
-  const Halo H = halo(P, D, np, t, y[GAL_V_SPIN_ANGULAR_MOMENTUM]);
-  const double mass = H.mass, r_vir = H.r_vir, v_vir = H.v_vir;
+__device__ __forceinline__ void scales_of_halo(const double* __restrict__ P, const DerivedConstants& D, double mass,
+                                               double r_vir, double v_vir, double r_gal, const double (&y)[kNV],
+                                               double (&sc)[kNV]) {
   constexpr double mrel = 1.0e-3, rrel = 1.0e-1;
 #pragma unroll
   for (int i = 0; i < kNV; ++i) sc[i] = 1.0;
@@ -759,9 +947,15 @@ __device__ __forceinline__ void scales(const double* __restrict__ P, const Deriv
   sc[GAL_V_SPHEROID_ABUNDANCES_STELLAR] = zsc;
   sc[GAL_V_BH_MASS] = fmax(fmax(1.0, 1.0e-4 * y[GAL_V_SPHEROID_MASS_STELLAR]), y[GAL_V_BH_MASS]);
   sc[GAL_V_BH_SPIN] = 1.0;
-  sc[GAL_V_BH_RADIAL_POSITION] = fmax(1.0e-4 * H.r_gal, 1.0e-6);
+  sc[GAL_V_BH_RADIAL_POSITION] = fmax(1.0e-4 * r_gal, 1.0e-6);
   sc[GAL_V_SPIN_ANGULAR_MOMENTUM] = mass * r_vir * v_vir * mrel;
   sc[GAL_V_SATELLITE_BOUND_MASS] = mass * mrel;
+}
+
+__device__ __forceinline__ void scales(const double* __restrict__ P, const DerivedConstants& D, const NodePar& np,
+                                       double t, const double (&y)[kNV], double (&sc)[kNV]) {
+  const Halo H = halo(P, D, np, t, y[GAL_V_SPIN_ANGULAR_MOMENTUM]);
+  scales_of_halo(P, D, H.mass, H.r_vir, H.v_vir, H.r_gal, y, sc);
 }
 
 // Post-step: standardPostStepProcessing (node_evolver/standard.F90:1160-1185)
@@ -815,6 +1009,12 @@ __device__ __noinline__ void post_step_fix(const double* __restrict__ P, HaloCon
   if (y[GAL_V_HOT_MASS * stride] < 0.0) y[GAL_V_HOT_MASS * stride] = 0.0;
   if (y[GAL_V_HOT_OUTER_RADIUS * stride] < 0.0) y[GAL_V_HOT_OUTER_RADIUS * stride] = 0.0;
 }
+
+// The variables whose sign the post-step looks at.
+constexpr unsigned kPostStepHalo = 1u << GAL_V_HOT_MASS | 1u << GAL_V_HOT_OUTER_RADIUS;
+constexpr unsigned kPostStepGalaxy = 1u << GAL_V_DISK_MASS_GAS | 1u << GAL_V_DISK_MASS_STELLAR |
+                                     1u << GAL_V_DISK_ANGULAR_MOMENTUM | 1u << GAL_V_SPHEROID_MASS_GAS |
+                                     1u << GAL_V_SPHEROID_MASS_STELLAR | 1u << GAL_V_SPHEROID_ANGULAR_MOMENTUM;
 
 __device__ __forceinline__ void post_step(const double* __restrict__ P, const DerivedConstants& D, const NodePar& np,
                                           int mode, double t, double* __restrict__ y, int stride) {

@@ -102,7 +102,9 @@ class NodeEvolverBatched:
 
     def set_launch(self, nodes_per_block: int, blocks_per_cu: int, rhs_waves: Optional[int] = None):
         """Launch shape: nodes per workgroup, workgroups per CU and, if given,
-        waves per group of nodes (2 splits every RHS over two SIMDs)."""
+        waves per group of nodes.  Kept on the handle and reported by
+        :meth:`launch`; the integrator runs four waves per group of 64 nodes
+        and one group per CU at every admitted shape."""
         _lib.check(self.L.gal_ode_batch_set_launch(self.handle, nodes_per_block, blocks_per_cu),
                    "gal_ode_batch_set_launch")
         if rhs_waves is not None:

@@ -1,10 +1,9 @@
 """Static algorithmic FLOP count of the device RHS and of one Cash-Karp attempt.
 
-The count is taken from the source text of ``rhs_part()`` in
-``galacticus_amd/csrc/physics.hpp`` (both halves of the RHS, plus the sum
-that joins them, and the inlined helpers), so it moves with the code.  The
-halo scales, which a two-wave launch computes once per half, count once.
-Weights:
+The count is taken from the source text of the blocks of the RHS in
+``galacticus_amd/csrc/physics.hpp`` (plus the sum that joins its two halves
+and the inlined helpers), so it moves with the code.  Each block counts once,
+whichever wave of a group computes it.  Weights:
 
 * ``+ - * /`` on doubles, ``sqrt``, ``rsqrt``, ``fmin``, ``fmax``, ``fabs``: 1
 * ``exp``, ``log``, ``log1p``, ``cbrt``, ``atan``, ``pow``, ``sinh``: 20 each
@@ -31,6 +30,10 @@ NVAR = 30
 TRANSCENDENTAL_WEIGHT = 20
 TRANSCENDENTALS = ("exp", "log", "log1p", "cbrt", "atan", "pow", "sinh")
 UNIT_CALLS = ("sqrt", "rsqrt", "fmin", "fmax", "fabs")
+# The functions an evaluation goes through once.
+BLOCKS = ("halo", "time_part", "cooling_temperature_index", "cooling_function_ln", "isco", "galaxy_radius",
+          "hot_profile", "hot_inv_mean_radius", "black_hole", "cooling_time", "galaxy_rates", "outer_radius_rates",
+          "hot_accretion", "black_hole_rates", "radiated_energy", "cooling_rates")
 
 
 def _function_body(src: str, signature_start: str) -> str:
@@ -55,9 +58,7 @@ def _strip(body: str) -> str:
 
 def _count_ops(body: str) -> int:
     b = _strip(body)
-    # drop the test-mode branch and the zero-initialisation loop
-    b = re.sub(r"if \(mode == GAL_PHYSICS_TEST\) \{.*?return;\s*\}", "", b, flags=re.S)
-    b = re.sub(r"for \(int i = 0; i < kNV; \+\+i\) f\[i\] = 0\.0;", "", b)
+    b = re.sub(r"\bfma\(", "fma(+*", b)              # a product and a sum
     b = re.sub(r"\[[^\]]*\]", "", b)                 # array indices are not flops
     b = re.sub(r"\+\+|--", "", b)
     b = re.sub(r"<=|>=|==|!=|&&|\|\||->", " ", b)
@@ -69,13 +70,13 @@ def _count_ops(body: str) -> int:
 
 def rhs_flops() -> int:
     src = open(PHYSICS, encoding="utf-8").read()
-    total = _count_ops(_function_body(src, "__device__ __forceinline__ void rhs_part("))
+    def ops(name: str) -> int:
+        return _count_ops(_function_body(src, re.search(
+            r"__device__ __forceinline__ \w+ %s\(" % name, src).group(0)))
+
+    total = sum(ops(name) for name in BLOCKS)
+    total += 2 * ops("hernquist_density")   # at the accretion radius and at the Jeans length
     total += NVAR    # f = f_galaxy + f_halo
-    # helpers inlined once per evaluation
-    total += _count_ops(_function_body(src, "__device__ __forceinline__ Halo halo("))
-    total += _count_ops(_function_body(src, "__device__ __forceinline__ void isco("))
-    total += _count_ops(_function_body(src, "__device__ __forceinline__ double cooling_function_ln("))
-    total += 2 * _count_ops(_function_body(src, "__device__ __forceinline__ double hernquist_density("))
     total += 4 * 3   # pow_half: three multiplies (and one divide) per power law
     return total
 

@@ -232,16 +232,10 @@ int gal_ode_batch_set_cooling_table(gal_ode_batch *h, const double *ln_lambda,
                                     int n_t, double ln_t_min, double d_ln_t,
                                     int n_z, double ln_z_min, double d_ln_z);
 
-/* Launch geometry of the persistent grid: nodes_per_block lanes per
-   workgroup and blocks_per_cu workgroups per CU.  Admitted: 64 lanes (one
-   wave) and 1 to 4 workgroups per CU.  One keeps every lane vector (stage
-   derivatives, state, error scales) in LDS (105 KiB); two keep state and
-   scales in an HBM workspace (75 KiB of LDS each); three or four keep the
-   stage derivatives there (30 KiB each).  Results are identical bit for bit.
-   Defaults: 64 and 1 (with two waves per group of nodes, see
-   gal_ode_batch_set_rhs_waves); gal_ode_batch_autotune measures the shapes
-   (64,1), (64,2) and (64,4) with one wave per group of nodes and (64,1) and
-   (64,2) with two. */
+/* Launch geometry, validated and kept on the handle: 64 nodes per workgroup
+   and 1 to 4 workgroups per CU are admitted.  The integrator has one shape: a
+   group of 64 nodes takes four waves and the LDS of a whole CU, and the grid is
+   one such group per CU, whatever is set here.  Defaults: 64 and 1. */
 int gal_ode_batch_set_launch(gal_ode_batch *h, int nodes_per_block, int blocks_per_cu);
 
 /* Evolve n nodes (device pointers, SoA with leading dimension ld).
@@ -355,12 +349,10 @@ int gal_ode_batch_set_wall_limit(gal_ode_batch *h, double seconds);
    from holding the GPU, and a tiny value forces that failure path in tests. */
 int gal_ode_batch_set_graph_stall_limit(gal_ode_batch *h, double seconds);
 
-/* Waves per group of 64 nodes: 1 (one lane per node computes the whole RHS)
-   or 2, the default (a second wave, on another SIMD, computes the hot-halo
-   half of every RHS while the first computes the galaxy half and integrates;
-   with 2 the launch takes one or two workgroups per CU).  Results are
-   identical bit for bit.  No counterpart in the reference (launch shape of
-   the GPU kernel). */
+/* Waves per group of 64 nodes, validated and kept on the handle: 1 or 2, the
+   default; an evolve with 2 needs one or two workgroups per CU.  The integrator
+   uses four waves per group whatever is set here.  No counterpart in the
+   reference (launch shape of the GPU kernel). */
 int gal_ode_batch_set_rhs_waves(gal_ode_batch *h, int waves);
 
 /* The launch currently set on the handle (by set_launch, set_rhs_waves or

@@ -1,0 +1,54 @@
+"""The integrator's groups of 64 nodes, partial and full.  The nodes of a
+group share barriers, flags and LDS but no arithmetic, so a node's results are
+the same to the last bit in any lane and beside any other nodes."""
+import numpy as np
+import pytest
+
+from galacticus_amd import params as gp, workloads as wl
+from galacticus_amd.cooling import synthetic_cie_table
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def torch_cuda():
+    torch = pytest.importorskip("torch")
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    return torch
+
+
+def _evolve(torch, physics, options, y, node_par, t0, t1, h):
+    from galacticus_amd.evolver import NodeEvolverBatched
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    n = len(t0)
+    ev = NodeEvolverBatched(n, physics, synthetic_cie_table(), **options)
+    y, h = d(y), d(h)
+    scale = torch.zeros((30, n), dtype=torch.float64, device="cuda")
+    counters = torch.zeros(3 * n, dtype=torch.int64, device="cuda")
+    status = ev.evolve_device(y, d(node_par), d(t0), d(t1), h, scale=scale, counters=counters)
+    torch.cuda.synchronize()
+    return y.cpu(), h.cpu(), status.cpu(), scale.cpu(), counters.cpu().view(3, n)
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 200])
+@pytest.mark.parametrize("kind,operators,options", [
+    ("isolated", None, {}), ("isolated", 0, {}), ("isolated", 2, {"enforceNonNegativity": True}),
+    ("satellite", None, {"odeToleranceRelative": 1.0e-4})])
+def test_results_do_not_depend_on_the_group(torch_cuda, n, kind, operators, options):
+    physics = gp.physics_params()
+    make = wl.isolated_halos if kind == "isolated" else wl.satellite_halos
+    b = make(n, seed=43, params=physics)
+    if operators is not None:
+        physics[gp.P["nodeOperators"]] = operators
+    t1 = b.t_start + 0.1 * (b.t_end - b.t_start)
+    t1[5::11] = b.t_start[5::11]          # intervals of zero length among them
+    run = lambda i: _evolve(torch_cuda, physics, options, b.y[:, i], b.node_par[:, i], b.t_start[i], t1[i],
+                            b.h_step[i])
+    together = run(np.arange(n))
+    order = np.random.Generator(np.random.PCG64(n)).permutation(n)
+    alone = int(order[n // 2])
+    for i in (order, np.array([alone]), np.concatenate([order, order])):
+        for whole, part in zip(together, run(i)):
+            assert torch_cuda.equal(whole[..., torch_cuda.from_numpy(i)], part)
+    assert (together[2] == 0).all()
