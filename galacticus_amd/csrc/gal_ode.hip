@@ -82,6 +82,12 @@ struct EvolveArgs {
   unsigned long long stall_ticks;
 };
 
+// An index the compiler computes addresses from but does not fold.
+__device__ __forceinline__ int opaque(int index) {
+  asm volatile("" : "+v"(index));
+  return index;
+}
+
 // Claim one node index per requesting lane with a single atomic per wave.
 __device__ __forceinline__ int wave_claim(bool want, unsigned int* work, int n, const int* order) {
   const unsigned long long mask = __ballot(want);
@@ -115,9 +121,32 @@ struct ClaimState {
   unsigned int wait_tail = ~0u;        // graph mode: appends seen while waiting on the entry
   unsigned long long wait_since = 0ull;
 };
-// Rounds of an attempt: the time part alone (new nodes), the derivative at its
+// Claims, then the rounds of an attempt: the time part alone (new nodes), the derivative at its
 // start, then the stages 0-4 that give k2-k6.
-enum : int { kTimeOnly = -2, kFirst = -1, kLast = 4 };
+enum : int { kClaims = -3, kTimeOnly = -2, kFirst = -1, kLast = 4 };
+// By stage 0-3: the next stage's time.
+__constant__ const double kNextTime[kLast] = {ck::a3, ck::a4, ck::a5, ck::a6};
+// What steers a lane, as bits of one register: booleans of their own cost three
+// scalar instructions each wherever two paths of the round meet.
+struct LaneFlags {
+  enum : unsigned {
+    kActive = 1u,        // has a node
+    kWant = 2u,          // wants one
+    kEval = 4u,          // the coming derivative is one it needs
+    kPost = 8u,          // an accepted state awaits the post-step fixes
+    kDecide = 16u,       // an attempt awaits the controller
+    kFinalStep = 32u,    // its step ends the interval
+    kFetch = 64u,        // its state is to be loaded
+    kFresh = 128u,       // its node was claimed just now
+    kStepping = 256u,    // in an attempt
+    kForbidden = 512u,   // the attempt's state is negative where it may not be
+    kNeedFix = 1024u     // and where the post-step fixes apply
+  };
+  unsigned bits;
+  __device__ __forceinline__ bool has(unsigned f) const { return (bits & f) != 0u; }
+  __device__ __forceinline__ void set(unsigned f) { bits |= f; }
+  __device__ __forceinline__ void clear(unsigned f) { bits &= ~f; }
+};
 enum : int { kNoClaim = -1, kExhausted = -2 };   // codes of the claim vector beside a node index
 
 // Claim a node's interval for each lane that wants one (cooling wave) and
@@ -196,31 +225,35 @@ __device__ __forceinline__ void claim_nodes(const EvolveArgs& a, int n_claim, bo
 
 // Persistent integrator: a workgroup of four waves serves 64 nodes, one per
 // lane position, and group_rhs.hpp deals the RHS out over the waves.  The
-// integrator's state is in registers, split by variable: wave w (of the first
-// three) owns variables [10 w, 10 w + 10) of every node -- state, stage
-// derivatives and error scales -- and forms their stage inputs, solution and
-// error norm; LDS only carries what waves exchange.  What steers a node
-// (times, step size, trial, flags) is held by all four waves alike: each runs
-// the same code on the same published values, so they agree without a
-// message.  The cooling wave owns no variables and does what needs one wave:
-// claims, statuses, counters, the wall clock.
+// integrator's state is split by variable: wave w (of the first three) owns
+// variables [10 w, 10 w + 10) of every node -- state, stage derivatives and
+// error scales -- and forms their stage inputs, solution and error norm.  What
+// steers a node (times, step size, trial, flags) is held by all four waves
+// alike: each runs the same code on the same published values, so they agree
+// without a message.  The cooling wave owns no variables and does what needs
+// one wave: claims, statuses, counters, the wall clock.
 //
 // The step controller's pow is not on the path: whether a step is accepted
 // follows from the error norm alone, and the derivative at the new point does
 // not depend on the step size, so the time wave computes the next step size
 // during that evaluation (which also decides a step-size underflow).
 //
-// Measured on the stiffest node of 100,000 isolated halos (3701 attempts): 22.6
-// us an attempt, against 43 us with one wave for the whole RHS and its stage
-// vectors in LDS, or two waves that split it in halves; evolving all 100,000
-// takes 44.8 ms instead of 85.6.
-//
 // One instance of this per wave of the group: a lone wave issues one
 // instruction every 4.6 cycles whatever it is (a dependent FP64 FMA costs no
 // more than an independent one, and a move of half a constant as much as
 // either), so the instruction count of each wave is what there is to save.
 // With a loop of its own a wave keeps the constants of its own transcendental
-// functions in registers across the integration.
+// functions in registers across the integration.  Between two evaluations
+// every value that is carried round the loop and set on more than one path
+// costs a move on each: the state at the start of the step is therefore kept
+// in LDS, a lane's booleans share one register, and there is one loop with one
+// evaluation in it and one exit.
+//
+// Measured on the stiffest node of 100,000 isolated halos (3701 attempts): 20.3
+// us an attempt, 22.6 us with the state in registers and nested loops, and 43
+// us with one wave for the whole RHS, or two waves that split it in halves.
+// Evolving 100,000 of them takes 44.7 ms, and 88.2 ms that way.
+//
 template <int WAVE, bool GRAPH>
 __device__ __forceinline__ void group_wave(const EvolveArgs& a, double* __restrict__ X,
                                            const GroupConstants& constants, int* __restrict__ norm_flags,
@@ -234,7 +267,11 @@ __device__ __forceinline__ void group_wave(const EvolveArgs& a, double* __restri
   double* __restrict__ XY = X + (kXState + v0) * kGroupNodes;   // owned rows (owners only)
   double* __restrict__ XG = X + (kXGalaxy + v0) * kGroupNodes;
   double* __restrict__ XH = X + (kXHalo + v0) * kGroupNodes;
-  double* __restrict__ XK = X + (kXStage + v0) * kGroupNodes;
+  // bases of their own: an offset past 64 KiB would cost an addition per access
+  double* __restrict__ XK = X + opaque((kXStage + v0) * kGroupNodes);
+  double* __restrict__ X0 = X + opaque((kXStart + v0) * kGroupNodes);
+  double* __restrict__ F = X + opaque(kXFar * kGroupNodes);
+  auto time_vectors = [&](int which) { return F + (kFarTime + which * kTimeVectors) * kGroupNodes; };
   const int mode = a.mode;
   const int ops = mode == GAL_PHYSICS_STANDARD ? (int)a.P[GAL_P_OPERATORS] : 0;
   const bool reuse = (a.flags & GAL_FLAG_REUSE_STEP_SIZE) != 0;
@@ -249,18 +286,19 @@ __device__ __forceinline__ void group_wave(const EvolveArgs& a, double* __restri
   // steering, alike in all four waves
   NodePar np{};
   int node = -1, trial = 0;
-  bool active = false, want = true, eval = false, post = false, decide = false, final_step = false;
+  LaneFlags s{LaneFlags::kWant};
   double t = 0.0, t0 = 0.0, t1 = 0.0, h = 0.0, h0 = 0.0, h_node = 0.0, sign = 1.0;
-  ErrorNorm en;
-  int need_fix = 0;
+  double rmax = 0.0;       // error norm of the attempt
   bool time_stale = false;
   int round = 0;
-  int tb = 0;              // time part of the coming stage: kXTime + tb * kTimeVectors
+  int tb = 0;              // which time part is the coming stage's
   // owners
-  double y[kOwned], sc[kOwned];
+  double sc[kOwned];
 #pragma unroll
-  for (int i = 0; i < kOwned; ++i) y[i] = sc[i] = 0.0;
-  auto K = [&](int stage, int i) -> double& { return XK[(stage * kNV + i) * kGroupNodes]; };
+  for (int i = 0; i < kOwned; ++i) sc[i] = 0.0;
+  // derivative of a stage, and the state at the start of the step
+  auto K = [&](int stage, int i) -> double& { return XK[((stage == 4 ? 1 : stage) * kNV + i) * kGroupNodes]; };
+  auto Y0 = [&](int i) -> double& { return X0[i * kGroupNodes]; };
   // cooling wave
   ClaimState claim;
   long long n_attempt = 0, n_accept = 0, n_rhs = 0;
@@ -274,7 +312,7 @@ __device__ __forceinline__ void group_wave(const EvolveArgs& a, double* __restri
     h = xs;
     h0 = xs;
     t = t0;
-    eval = true;
+    s.set(LaneFlags::kEval);
   };
   // Results of a lane's interval (cooling wave); its state is stored by the
   // owners beforehand, and in graph mode its successors are released.
@@ -290,273 +328,281 @@ __device__ __forceinline__ void group_wave(const EvolveArgs& a, double* __restri
       if (wave == kCoolingWave && done) graph_release(a.g, claim.op);
     }
     if (done) {
-      active = false;
-      want = true;
-    }
-  };
-  auto store_state = [&](bool done) {
-    if (owner && done) {
-#pragma unroll
-      for (int i = 0; i < kOwned; ++i) a.y[(size_t)(v0 + i) * a.ld + node] = y[i];
+      s.clear(LaneFlags::kActive);
+      s.set(LaneFlags::kWant);
     }
   };
   // The reference's negative-value fixes on the published state of the given
   // lanes (rare): one wave fixes, the owners take their variables back.
-  auto fix_published = [&](bool lanes) {
+  auto fix_published = [&](bool lanes, auto&& take) {
     if (wave == kCoolingWave && lanes) post_step(constants.P, constants.D, np, mode, t, X + kXState * kGroupNodes, kGroupNodes);
     __syncthreads();
     if (owner && lanes) {
 #pragma unroll
-      for (int i = 0; i < kOwned; ++i) y[i] = XY[i * kGroupNodes];
+      for (int i = 0; i < kOwned; ++i) take(i, XY[i * kGroupNodes]);
     }
   };
 
+  auto norm = [&]() {
+    ErrorNorm e;
+    e.rmax = rmax;
+    e.forbidden = s.has(LaneFlags::kForbidden);
+    return e;
+  };
   // The sums over the older stage derivatives, formed beside the RHS; each is
-  // completed once the newest derivative is known.
-  double sp[kOwned];
-  auto older_terms = [&](int ph) {
+  // completed once the newest derivative is known, with its coefficient bn.
+  auto older_terms = [&](int ph, double (&y)[kOwned], double (&sp)[kOwned], double& bn) {
     if constexpr (owner) {
 #pragma clang fp contract(off)
+      bn = 0.0;
 #pragma unroll
-      for (int i = 0; i < kOwned; ++i) sp[i] = 0.0;
+      for (int i = 0; i < kOwned; ++i) y[i] = Y0(i);
       if (ph == 0) {
+        bn = ck::b32;
 #pragma unroll
         for (int i = 0; i < kOwned; ++i) sp[i] = ck::b31 * K(0, i);
       } else if (ph == 1) {
+        bn = ck::b43;
 #pragma unroll
         for (int i = 0; i < kOwned; ++i) sp[i] = fma(ck::b41, K(0, i), ck::b42 * K(1, i));
       } else if (ph == 2) {
+        bn = ck::b54;
 #pragma unroll
         for (int i = 0; i < kOwned; ++i) sp[i] = fma(ck::b53, K(2, i), fma(ck::b52, K(1, i), ck::b51 * K(0, i)));
       } else if (ph == 3) {
+        bn = ck::b65;
 #pragma unroll
         for (int i = 0; i < kOwned; ++i)
           sp[i] = fma(ck::b64, K(3, i), fma(ck::b63, K(2, i), fma(ck::b61, K(0, i), ck::b62 * K(1, i))));
       } else if (ph == kLast) {
 #pragma unroll
         for (int i = 0; i < kOwned; ++i) sp[i] = fma(ck::c4, K(3, i), fma(ck::c1, K(0, i), ck::c3 * K(2, i)));
+      } else {
+        // not used, and set so that nothing is carried from round to round
+#pragma unroll
+        for (int i = 0; i < kOwned; ++i) sp[i] = 0.0;
       }
     }
   };
 
+  // One RHS evaluation per trip.  What follows an evaluation of the stages 0-3,
+  // four of an attempt's six, touches none of the steering; everything rarer
+  // sits in branches that leave the state in the registers where it was.
+  int ph = kClaims;
   for (;;) {
-    // ---- claims ------------------------------------------------------------
-    bool begun = false, zero_length = false;
-    if (__any(want)) {
-      double* C = X + (kXTime + (tb ^ 1) * kTimeVectors) * kGroupNodes;
-      if (wave == kCoolingWave) claim_nodes<GRAPH>(a, n_claim, want, claim, C);
-      __syncthreads();
-      const int code = (int)C[kXClaimNode * kGroupNodes];
-      if (want && code == kExhausted) want = false;
-      begun = want && code >= 0;
-      if (begun) {
-        node = code;
-        t0 = C[kXClaimT0 * kGroupNodes];
-        t1 = C[kXClaimT1 * kGroupNodes];
-        h_node = C[kXClaimStep * kGroupNodes];
-        np = load_node_par(C + kXClaimPar * kGroupNodes, kGroupNodes, 0);
-        want = false;
-        active = true;
-        trial = 0;
-        post = decide = false;
-        n_attempt = n_accept = n_rhs = 0;
-        zero_length = t0 == t1;
-        start_trial(reuse ? h_node : -1.0);
-        sign = h > 0.0 ? 1.0 : -1.0;
-        eval = !zero_length;
-        if (owner) {
-#pragma unroll
-          for (int i = 0; i < kOwned; ++i) y[i] = a.y[(size_t)(v0 + i) * a.ld + node];
-          if (scales_given) {
+    if (ph == kClaims) {
+      // ---- claims, and the state the next derivative is taken at -------------
+      bool begun = false;
+      while (__any(s.has(LaneFlags::kWant))) {
+        double* C = time_vectors(tb ^ 1);
+        if (wave == kCoolingWave) claim_nodes<GRAPH>(a, n_claim, s.has(LaneFlags::kWant), claim, C);
+        __syncthreads();
+        const int code = (int)C[kXClaimNode * kGroupNodes];
+        begun = s.has(LaneFlags::kWant) && code >= 0;
+        if (code == kExhausted) s.clear(LaneFlags::kWant);
+        if (begun) {
+          node = code;
+          t0 = C[kXClaimT0 * kGroupNodes];
+          t1 = C[kXClaimT1 * kGroupNodes];
+          h_node = C[kXClaimStep * kGroupNodes];
+          np = load_node_par(C + kXClaimPar * kGroupNodes, kGroupNodes, 0);
+          s = LaneFlags{LaneFlags::kActive | LaneFlags::kFetch | LaneFlags::kFresh};
+          trial = 0;
+          n_attempt = n_accept = n_rhs = 0;
+          start_trial(reuse ? h_node : -1.0);
+          sign = h > 0.0 ? 1.0 : -1.0;
+          if (t0 == t1) s.clear(LaneFlags::kEval);
+          if (owner && scales_given) {
 #pragma unroll
             for (int i = 0; i < kOwned; ++i) sc[i] = a.scale[(size_t)(v0 + i) * a.ld + node];
           }
         }
-      }
-      if (!__any(active)) {
+        if (__any(s.has(LaneFlags::kActive))) break;
         __syncthreads();   // the claim vectors are free again
-        if (!__any(want)) break;
         // graph mode: lanes wait on ready-list entries; poll again after a pause
-        __builtin_amdgcn_s_sleep(8);
-        continue;
+        if (__any(s.has(LaneFlags::kWant))) __builtin_amdgcn_s_sleep(8);
       }
-    } else if (!__any(active)) {
-      break;
+      if (!__any(s.has(LaneFlags::kActive))) break;
+      if (owner && s.has(LaneFlags::kFetch)) {
+#pragma unroll
+        for (int i = 0; i < kOwned; ++i) XY[i * kGroupNodes] = Y0(i) = a.y[(size_t)(v0 + i) * a.ld + node];
+      }
+      s.clear(LaneFlags::kFetch);
+      // The time part of the derivative was computed ahead for lanes that go
+      // on; for new ones an extra round computes it (all lanes; the others'
+      // comes out as it was).
+      ph = time_stale || __any(begun) ? kTimeOnly : kFirst;
+      time_stale = false;
     }
-    // ---- the derivative at (t, y), and one Cash-Karp attempt ------------------
-    if (owner) {
+    ++round;
+    __syncthreads();   // stage state and time part published
+    if (ph == kFirst && !scales_given && owner && __any(s.has(LaneFlags::kFresh))) {
+      double ys[kNV], s30[kNV];
+      load_state(X, ys);
+      const TimePart T = load_time_part(time_vectors(tb));
+      scales_of_halo(G.P, G.D, T.mass, T.r_vir, T.v_vir, galaxy_radius(T, ys[GAL_V_SPIN_ANGULAR_MOMENTUM]).r, ys, s30);
+      if (s.has(LaneFlags::kFresh)) {
 #pragma unroll
-      for (int i = 0; i < kOwned; ++i) XY[i * kGroupNodes] = y[i];
+        for (int i = 0; i < kOwned; ++i) sc[i] = mode == GAL_PHYSICS_TEST ? 1.0 : s30[v0 + i];
+        if (a.scale) {
+#pragma unroll
+          for (int i = 0; i < kOwned; ++i) a.scale[(size_t)(v0 + i) * a.ld + node] = sc[i];
+        }
+      }
     }
-    // The time part of the first derivative was computed ahead for lanes that
-    // go on; for new ones an extra round computes it (all lanes; the others'
-    // comes out as it was).
-    const bool stale = time_stale || __any(begun);
-    time_stale = false;
-    bool stepping = false;
-    for (int ph = stale ? kTimeOnly : kFirst; ph <= kLast; ++ph) {
-      const int xt = kXTime + tb * kTimeVectors;
-      ++round;
-      __syncthreads();   // stage state and time part published
-      if (ph == kFirst && !scales_given && owner && __any(begun)) {
-        double ys[kNV], s30[kNV];
-        load_state(X, ys);
-        const TimePart T = load_time_part(X + xt * kGroupNodes);
-        scales_of_halo(G.P, G.D, T.mass, T.r_vir, T.v_vir, galaxy_radius(T, ys[GAL_V_SPIN_ANGULAR_MOMENTUM]).r, ys, s30);
-        if (begun) {
-#pragma unroll
-          for (int i = 0; i < kOwned; ++i) sc[i] = mode == GAL_PHYSICS_TEST ? 1.0 : s30[v0 + i];
-          if (a.scale) {
-#pragma unroll
-            for (int i = 0; i < kOwned; ++i) a.scale[(size_t)(v0 + i) * a.ld + node] = sc[i];
-          }
-        }
-      }
-      if constexpr (wave == kTimeWave) {
-        older_terms(ph);   // its own work waits for nobody, so these come first
-        // the time of the next stage, or after the last one of the point that
-        // the step leads to if it is accepted
-        double tn = t;
-        if (ph == kFirst) {
-          const double hn = decide ? hadjust_step(en, kRkckOrder, h0) : h0;
-          X[kXStep * kGroupNodes] = hn;
-          const double dt = t1 - t;
-          const double hs = ((dt >= 0.0 && hn > dt) || (dt < 0.0 && hn < dt)) ? dt : hn;
-          tn = t + ck::a2 * hs;
-        } else if (ph == kLast) {
-          if (!eval) tn = final_step ? t1 : t + h0;
-        } else if (ph != kTimeOnly) {
-          const double an = ph == 0 ? ck::a3 : (ph == 1 ? ck::a4 : (ph == 2 ? ck::a5 : ck::a6));
-          tn = t + an * h0;
-        }
-        store_time_part(time_part(G.P, G.D, G.C, np, tn),
-                        X + (kXTime + (tb ^ 1) * kTimeVectors) * kGroupNodes);
-      } else if (ph != kTimeOnly) {
-        if constexpr (wave == kGalaxyWave) {
-          galaxy_wave_rhs(G, mode, ops, np, X, xt, flags, round);
-        } else if (mode == GAL_PHYSICS_STANDARD) {
-          if constexpr (wave == kProfileWave) profile_wave_rhs(G, ops, X, xt, flags, round);
-          if constexpr (wave == kCoolingWave) cooling_wave_rhs(G, a.tab, np, X, xt, flags, round);
-        }
-        if constexpr (wave == kCoolingWave) {
-          if (ph == kFirst ? eval : stepping) ++n_rhs;
-          if (ph == kFirst && a.wall_ticks && lane == 0) wall_expired = wall_clock64() - t_launch > a.wall_ticks;
-        }
-      }
-      if constexpr (wave != kTimeWave) older_terms(ph);
-      __syncthreads();   // derivatives published
-      tb ^= 1;
-      if (ph == kTimeOnly) continue;
-      double kn[kOwned];
-      if (owner) {
-#pragma unroll
-        for (int i = 0; i < kOwned; ++i) kn[i] = XG[i * kGroupNodes] + XH[i * kGroupNodes];
-      }
-      if (ph >= 0 && ph < kLast) {
-        // the next stage's input y + h (older terms + newest)
-        if (owner) {
-#pragma clang fp contract(off)
-          const double bn = ph == 0 ? ck::b32 : (ph == 1 ? ck::b43 : (ph == 2 ? ck::b54 : ck::b65));
-#pragma unroll
-          for (int i = 0; i < kOwned; ++i) XY[i * kGroupNodes] = fma(h0, fma(bn, kn[i], sp[i]), y[i]);
-#pragma unroll
-          for (int i = 0; i < kOwned; ++i) K(ph + 1, i) = kn[i];
-        }
-        continue;
-      }
+    double y[kOwned], sp[kOwned], bn;
+    if constexpr (wave == kTimeWave) {
+      older_terms(ph, y, sp, bn);   // its own work waits for nobody, so these come first
+      // the time of the next stage, or after the last one of the point that
+      // the step leads to if it is accepted
+      double tn = t;
       if (ph == kFirst) {
-        if (owner && eval) {
+        const double hn = s.has(LaneFlags::kDecide) ? hadjust_step(norm(), kRkckOrder, h0) : h0;
+        F[kFarStep * kGroupNodes] = hn;
+        const double dt = t1 - t;
+        const double hs = ((dt >= 0.0 && hn > dt) || (dt < 0.0 && hn < dt)) ? dt : hn;
+        tn = t + ck::a2 * hs;
+      } else if (ph == kLast) {
+        if (!s.has(LaneFlags::kEval)) tn = s.has(LaneFlags::kFinalStep) ? t1 : t + h0;
+      } else if (ph != kTimeOnly) {
+        tn = t + kNextTime[ph] * h0;
+      }
+      store_time_part(time_part(G.P, G.D, G.C, np, tn), time_vectors(tb ^ 1));
+    } else if (ph != kTimeOnly) {
+      if constexpr (wave == kGalaxyWave) {
+        galaxy_wave_rhs(G, mode, ops, np, X, F, time_vectors(tb), flags, round);
+      } else if (mode == GAL_PHYSICS_STANDARD) {
+        if constexpr (wave == kProfileWave) profile_wave_rhs(G, ops, X, F, time_vectors(tb), flags, round);
+        if constexpr (wave == kCoolingWave) cooling_wave_rhs(G, a.tab, np, X, F, time_vectors(tb), flags, round);
+      }
+      if constexpr (wave == kCoolingWave) {
+        if (ph == kFirst && a.wall_ticks && lane == 0) wall_expired = wall_clock64() - t_launch > a.wall_ticks;
+      }
+    }
+    if constexpr (wave != kTimeWave) older_terms(ph, y, sp, bn);
+    __syncthreads();   // derivatives published
+    tb ^= 1;
+    double kn[kOwned];
+    if (owner) {
+      // all reads in flight before the first sum; a half that has no part of a
+      // variable's derivative is not read
+      double fh[kOwned];
 #pragma unroll
-          for (int i = 0; i < kOwned; ++i) K(0, i) = kn[i];
+      for (int i = 0; i < kOwned; ++i) kn[i] = (kGalaxyVars >> (v0 + i)) & 1u ? XG[i * kGroupNodes] : 0.0;
+#pragma unroll
+      for (int i = 0; i < kOwned; ++i) fh[i] = (kHaloVars >> (v0 + i)) & 1u ? XH[i * kGroupNodes] : 0.0;
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < kOwned; ++i) {
+        if (!((kGalaxyVars >> (v0 + i)) & 1u)) kn[i] = fh[i];
+        else if ((kHaloVars >> (v0 + i)) & 1u) kn[i] += fh[i];
+      }
+    }
+    if (ph >= 0 && ph < kLast) {
+      // the next stage's input y + h (older terms + newest)
+      if (owner) {
+#pragma clang fp contract(off)
+#pragma unroll
+        for (int i = 0; i < kOwned; ++i) XY[i * kGroupNodes] = fma(h0, fma(bn, kn[i], sp[i]), y[i]);
+#pragma unroll
+        for (int i = 0; i < kOwned; ++i) K(ph + 1, i) = kn[i];
+      }
+      ++ph;
+    } else if (ph == kTimeOnly) {
+      ph = kFirst;
+    } else if (ph == kFirst) {
+      const bool evaluated = s.has(LaneFlags::kEval), zero_length = s.has(LaneFlags::kFresh) && !evaluated;
+      if (owner && evaluated) {
+#pragma unroll
+        for (int i = 0; i < kOwned; ++i) K(0, i) = kn[i];
+      }
+      if (wave == kCoolingWave && evaluated) ++n_rhs;
+      // GSL_CONTINUE: the post-step fixes leave the derivative as it is
+      const bool fix = s.has(LaneFlags::kPost) && s.has(LaneFlags::kNeedFix);
+      if (__any(fix)) fix_published(fix, [&](int i, double v) { Y0(i) = v; });
+      const double hn = F[kFarStep * kGroupNodes];
+      bool failed = false;
+      if (s.has(LaneFlags::kDecide)) {
+        if (hadjust_kind(norm()) == kHadjDec) {
+          const double t_adv = s.has(LaneFlags::kFinalStep) ? t1 : t + h0;
+          if (fabs(hn) < fabs(h0) && t_adv + hn != t_adv) h0 = hn;   // rejected: retry, same k1
+          else failed = true;                                         // step size underflow
+        } else {
+          h = hn;
+          h0 = hn;
         }
-        eval = false;
-        // GSL_CONTINUE: the post-step fixes leave the derivative as it is
-        const bool fix = post && need_fix != 0;
-        post = false;
-        if (__any(fix)) fix_published(fix);
-        const double hn = X[kXStep * kGroupNodes];
-        bool failed = false;
-        if (decide) {
-          if (hadjust_kind(en) == kHadjDec) {
-            const double t_adv = final_step ? t1 : t + h0;
-            if (fabs(hn) < fabs(h0) && t_adv + hn != t_adv) h0 = hn;   // rejected: retry, same k1
-            else failed = true;                                         // step size underflow
-          } else {
-            h = hn;
-            h0 = hn;
+      }
+      s.clear(LaneFlags::kEval | LaneFlags::kPost | LaneFlags::kFresh | LaneFlags::kDecide | LaneFlags::kStepping |
+              LaneFlags::kFinalStep);
+      // nothing to integrate (standard.F90:580): success, timeStep -1
+      if (__any(zero_length)) finish(zero_length, -1.0, true, GAL_STATUS_SUCCESS);
+      if (__any(failed)) {
+        // node-evolver trial loop (standard.F90:657-692)
+        bool rescued = false;
+        if (enforce) {
+          if (owner) {
+            bool any = false;
+#pragma unroll
+            for (int i = 0; i < kOwned; ++i) any |= Y0(i) < 0.0 && ((nonneg >> i) & 1u);
+            norm_flags[wave * kGroupNodes + lane] = any ? 4 : 0;
           }
-          decide = false;
-        }
-        if (__any(zero_length)) {
-          // nothing to integrate (standard.F90:580): success, timeStep -1
-          finish(zero_length, -1.0, true, GAL_STATUS_SUCCESS);
-          zero_length = false;
-        }
-        if (__any(failed)) {
-          // node-evolver trial loop (standard.F90:657-692)
-          bool rescued = false;
-          if (enforce) {
-            if (owner) {
-              bool any = false;
+          __syncthreads();
 #pragma unroll
-              for (int i = 0; i < kOwned; ++i) any |= y[i] < 0.0 && ((nonneg >> i) & 1u);
-              norm_flags[wave * kGroupNodes + lane] = any ? 4 : 0;
-            }
-            __syncthreads();
+          for (int w = 0; w < kOwnerWaves; ++w) rescued |= (norm_flags[w * kGroupNodes + lane] & 4) != 0;
+          rescued = rescued && failed;
+          if (owner && rescued) {
 #pragma unroll
-            for (int w = 0; w < kOwnerWaves; ++w) rescued |= (norm_flags[w * kGroupNodes + lane] & 4) != 0;
-            rescued = rescued && failed;
-            if (owner && rescued) {
-#pragma unroll
-              for (int i = 0; i < kOwned; ++i)
-                if (y[i] < 0.0 && ((nonneg >> i) & 1u)) y[i] = 0.0;
-            }
-            store_state(rescued);
-            if (__any(rescued)) finish(rescued, h_node / (double)(1 << trial), true, GAL_STATUS_SUCCESS);
+            for (int i = 0; i < kOwned; ++i)
+              a.y[(size_t)(v0 + i) * a.ld + node] = Y0(i) < 0.0 && ((nonneg >> i) & 1u) ? 0.0 : Y0(i);
           }
-          const bool retry = failed && !rescued;
-          bool spent = false;
-          if (retry) {
-            spent = ++trial >= 8;
-            if (!spent) {
-              if (owner) {
-#pragma unroll
-                for (int i = 0; i < kOwned; ++i) y[i] = a.y[(size_t)(v0 + i) * a.ld + node];
-              }
-              start_trial(reuse ? h_node / (double)(1 << trial) : -1.0);
-            }
+          if (__any(rescued)) finish(rescued, h_node / (double)(1 << trial), true, GAL_STATUS_SUCCESS);
+        }
+        const bool retry = failed && !rescued;
+        bool spent = false;
+        if (retry) {
+          spent = ++trial >= 8;
+          if (!spent) {
+            s.set(LaneFlags::kFetch);
+            start_trial(reuse ? h_node / (double)(1 << trial) : -1.0);
           }
-          // all trials failed: state restored, errorStatusUnderflow (standard.F90:715-718)
-          if (__any(spent)) finish(spent, 0.0, false, GAL_STATUS_UNDERFLOW);
         }
-        // Wall-time limit (node_evolver/standard.F90:693-705 and the RHS's own
-        // check, standard.F90:860-866): the nodes return errorStatusXCPU with
-        // their state as it came in.
-        if (a.wall_ticks && wall_expired && __any(active)) {
-          finish(active, 0.0, false, GAL_STATUS_XCPU);
-          eval = false;
-        }
-        stepping = active && !eval;
-        if (!__any(stepping)) {
-          time_stale = true;
-          break;
-        }
+        // all trials failed: state restored, errorStatusUnderflow (standard.F90:715-718)
+        if (__any(spent)) finish(spent, 0.0, false, GAL_STATUS_UNDERFLOW);
+      }
+      // Wall-time limit (node_evolver/standard.F90:693-705 and the RHS's own
+      // check, standard.F90:860-866): the nodes return errorStatusXCPU with
+      // their state as it came in.
+      if (a.wall_ticks && wall_expired && __any(s.has(LaneFlags::kActive))) {
+        finish(s.has(LaneFlags::kActive), 0.0, false, GAL_STATUS_XCPU);
+        s.clear(LaneFlags::kEval | LaneFlags::kFetch);
+      }
+      const bool stepping = s.has(LaneFlags::kActive) && !s.has(LaneFlags::kEval);
+      if (__any(stepping)) {
         // gsl_odeiv2_evolve_apply: clip the step to reach t1 exactly
         const double dt = t1 - t;
-        final_step = false;
-        if (stepping && ((dt >= 0.0 && h0 > dt) || (dt < 0.0 && h0 < dt))) {
-          h0 = dt;
-          final_step = true;
+        if (stepping) {
+          s.set(LaneFlags::kStepping);
+          if ((dt >= 0.0 && h0 > dt) || (dt < 0.0 && h0 < dt)) {
+            h0 = dt;
+            s.set(LaneFlags::kFinalStep);
+          }
+          if (wave == kCoolingWave) {
+            ++n_attempt;
+            n_rhs += 5;
+          }
         }
-        if (stepping) ++n_attempt;
         if (owner) {
 #pragma clang fp contract(off)
 #pragma unroll
-          for (int i = 0; i < kOwned; ++i) XY[i * kGroupNodes] = fma(h0, ck::b21 * K(0, i), y[i]);
+          for (int i = 0; i < kOwned; ++i) XY[i * kGroupNodes] = fma(h0, ck::b21 * K(0, i), Y0(i));
         }
-        continue;
+        ph = 0;
+      } else {
+        time_stale = true;
+        ph = kClaims;
       }
-      // ---- k6 is in kn: solution, error norm, controller ----------------------
+    } else {
+      // ---- k6 is in kn: solution, error norm, controller ---------------------
       double yn[kOwned];
       if (owner) {
         ErrorNorm e;
@@ -572,49 +618,62 @@ __device__ __forceinline__ void group_wave(const EvolveArgs& a, double* __restri
                          enforce && ((nonneg >> i) & 1u));
           negative |= yn[i] < 0.0 ? 1u << i : 0u;
         }
-        X[(kXNorm + wave) * kGroupNodes] = e.rmax;
+        F[(kFarNorm + wave) * kGroupNodes] = e.rmax;
         norm_flags[wave * kGroupNodes + lane] = (e.forbidden ? 1 : 0) | ((negative & fixable) ? 2 : 0);
       }
       __syncthreads();   // error norms published
-      en = ErrorNorm{};
-      need_fix = 0;
+      rmax = ErrorNorm{}.rmax;
+      int seen = 0;
 #pragma unroll
       for (int w = 0; w < kOwnerWaves; ++w) {
-        const double r = X[(kXNorm + w) * kGroupNodes];
-        en.rmax = r > en.rmax ? r : en.rmax;
-        const int fl = norm_flags[w * kGroupNodes + lane];
-        en.forbidden = en.forbidden || (fl & 1) != 0;
-        need_fix |= fl & 2;
+        const double r = F[(kFarNorm + w) * kGroupNodes];
+        rmax = r > rmax ? r : rmax;
+        seen |= norm_flags[w * kGroupNodes + lane];
       }
-      decide = stepping;
-      const bool accepted = stepping && hadjust_kind(en) != kHadjDec;
+      s.clear(LaneFlags::kForbidden | LaneFlags::kNeedFix);
+      if (seen & 1) s.set(LaneFlags::kForbidden);
+      if (seen & 2) s.set(LaneFlags::kNeedFix);
+      const bool stepping = s.has(LaneFlags::kStepping);
+      const bool accepted = stepping && hadjust_kind(norm()) != kHadjDec;
+      const bool final_step = s.has(LaneFlags::kFinalStep), need_fix = s.has(LaneFlags::kNeedFix);
       bool done = false;
+      if (stepping) s.set(LaneFlags::kDecide);
       if (accepted) {
-        ++n_accept;
+        if (wave == kCoolingWave) ++n_accept;
         t = final_step ? t1 : t + h0;
-        if (owner) {
-#pragma unroll
-          for (int i = 0; i < kOwned; ++i) y[i] = yn[i];
-        }
         done = !(sign * (t1 - t) > 0.0);
-        eval = post = !done;
-        if (done) decide = false;
+        if (done) s.clear(LaneFlags::kDecide);
+        else s.set(LaneFlags::kEval | LaneFlags::kPost);
       }
       if (__any(done)) {
-        if (__any(done && need_fix != 0)) {
+        if (__any(done && need_fix)) {
           if (owner && done) {
 #pragma unroll
-            for (int i = 0; i < kOwned; ++i) XY[i * kGroupNodes] = y[i];
+            for (int i = 0; i < kOwned; ++i) XY[i * kGroupNodes] = yn[i];
           }
           __syncthreads();
-          fix_published(done && need_fix != 0);
+          fix_published(done && need_fix, [&](int i, double v) { yn[i] = v; });
         }
-        store_state(done);
+        if (owner && done) {
+#pragma unroll
+          for (int i = 0; i < kOwned; ++i) a.y[(size_t)(v0 + i) * a.ld + node] = yn[i];
+        }
         // odeSolverSolve returns xStep = driver h (solver.F90:593)
         double h_out = h;
-        if (wave == kCoolingWave && done && !final_step) h_out = hadjust_step(en, kRkckOrder, h0);
+        if (wave == kCoolingWave && done && !final_step) h_out = hadjust_step(norm(), kRkckOrder, h0);
         finish(done, h_out, true, GAL_STATUS_SUCCESS);
       }
+      // the state that the next derivative is taken at: the new one, or again
+      // the one that the attempt started from
+      if (owner) {
+        if (accepted) {
+#pragma unroll
+          for (int i = 0; i < kOwned; ++i) Y0(i) = yn[i];
+        }
+#pragma unroll
+        for (int i = 0; i < kOwned; ++i) XY[i * kGroupNodes] = accepted ? yn[i] : y[i];
+      }
+      ph = kClaims;
     }
   }
 }

@@ -44,28 +44,33 @@ static_assert(kOwned * kOwnerWaves == kNV, "owners must tile the state");
 constexpr int kTimeVectors = (int)(sizeof(TimePart) / sizeof(double));
 constexpr int kMidVectors = 11;
 
-// Stages whose derivatives are kept (the sixth is consumed as it is produced).
-constexpr int kStages = 5;
+// Stages whose derivatives are kept: k1, k2 (whose place k5 takes once the last
+// stage input no longer needs it), k3 and k4.  k6 is consumed as it is produced.
+constexpr int kStages = 4;
 
 // LDS of a group, in vectors of 64 doubles.
 enum : int {
   kXState = 0,                              // stage state
   kXGalaxy = kXState + kNV,                 // galaxy half of the derivative
   kXHalo = kXGalaxy + kNV,                  // hot-halo half
-  kXStage = kXHalo + kNV,                   // stage derivatives k1..k5, each kNV vectors
-  kXTime = kXStage + kStages * kNV,         // TimePart of this stage and of the next
-  kXMid = kXTime + 2 * kTimeVectors,        // published at the pauses
-  kXNorm = kXMid + kMidVectors,             // each owner's error norm
-  kXStep = kXNorm + kOwnerWaves,            // step size chosen by the controller
-  kXVectors = kXStep + 1,
-  // published at the pauses
-  kMidRho0 = kXMid, kMidRhoOut, kMidEffThin, kMidEddCap, kMidMdotSph, kMidInvRMean,   // profile wave
-  kMidLambda, kMidNhPerRho, kMidNallPerNh, kMidMdot, kMidJet,                         // cooling wave
+  kXStage = kXHalo + kNV,                   // stage derivatives, each kNV vectors
+  kXStart = kXStage + kStages * kNV,        // state at the start of the step
+  kXFar = kXStart + kNV,                    // what follows, counted from here
+  kXVectors = kXFar + 2 * kTimeVectors + kMidVectors + kOwnerWaves + 1
+};
+enum : int {
+  kFarTime = 0,                             // TimePart of this stage and of the next
+  kFarMid = kFarTime + 2 * kTimeVectors,    // published within an evaluation
+  kFarNorm = kFarMid + kMidVectors,         // each owner's error norm
+  kFarStep = kFarNorm + kOwnerWaves,        // step size chosen by the controller
+  // published within an evaluation
+  kMidRho0 = kFarMid, kMidRhoOut, kMidEffThin, kMidEddCap, kMidMdotSph, kMidInvRMean,   // profile wave
+  kMidLambda, kMidNhPerRho, kMidNallPerNh, kMidMdot, kMidJet,                           // cooling wave
   kMidEnd,
   // claimed nodes, in the time part that is not in use
   kXClaimNode = 0, kXClaimT0, kXClaimT1, kXClaimStep, kXClaimPar
 };
-static_assert(kMidEnd - kXMid == kMidVectors, "count the published values");
+static_assert(kMidEnd - kFarMid == kMidVectors, "count the published values");
 static_assert(kXClaimPar + GAL_NPARAM_NODE <= kTimeVectors, "a claim must fit a time part");
 
 // The copy of the parameters that the RHS reads.
@@ -145,15 +150,16 @@ __device__ __forceinline__ void load_state(const double* __restrict__ X, double 
   for (int v = 0; v < kNV; ++v) y[v] = X[(kXState + v) * kGroupNodes];
 }
 
-// X: this lane's column of the group's LDS; xt, the vector at which this
-// stage's time part starts.
+// X: this lane's column of the group's LDS; F: the part of it from kXFar on;
+// time: this stage's time part.
 __device__ __forceinline__ void galaxy_wave_rhs(const GroupConstants& G, int mode, int ops, const NodePar& np,
-                                                double* __restrict__ X, int xt, int* __restrict__ flags, int round) {
+                                                double* __restrict__ X, double* __restrict__ F,
+                                  const double* __restrict__ time, int* __restrict__ flags, int round) {
   double y[kNV], f[kNV];
   load_state(X, y);
 #pragma unroll
   for (int v = 0; v < kNV; ++v) f[v] = 0.0;
-  const TimePart T = load_time_part(X + xt * kGroupNodes);
+  const TimePart T = load_time_part(time);
   if (mode == GAL_PHYSICS_TEST) {
     test_rates(T.time, y, f);
   } else {
@@ -161,7 +167,7 @@ __device__ __forceinline__ void galaxy_wave_rhs(const GroupConstants& G, int mod
     galaxy_rates(G.P, G.D, ops, box, np, T, y, f);
     if (!box && (ops & GAL_OPERATOR_CGM_OUTER_RADIUS)) {
       await(flags, kProfileReady, round);
-      outer_radius_rates(G.P, np, T, X[kMidRho0 * kGroupNodes], X[kMidRhoOut * kGroupNodes], y, f);
+      outer_radius_rates(G.P, np, T, F[kMidRho0 * kGroupNodes], F[kMidRhoOut * kGroupNodes], y, f);
     }
   }
 #pragma unroll
@@ -177,35 +183,35 @@ constexpr unsigned kBlackHoleVars =
               GAL_V_SPHEROID_ANGULAR_MOMENTUM, GAL_V_BH_MASS, GAL_V_BH_SPIN});
 constexpr unsigned kCoolingVars = kHaloVars & ~kBlackHoleVars;
 
-__device__ __forceinline__ void profile_wave_rhs(const GroupConstants& G, int ops, double* __restrict__ X, int xt,
-                                                 int* __restrict__ flags, int round) {
+__device__ __forceinline__ void profile_wave_rhs(const GroupConstants& G, int ops, double* __restrict__ X, double* __restrict__ F,
+                                  const double* __restrict__ time, int* __restrict__ flags, int round) {
   auto Y = [&](int v) { return X[(kXState + v) * kGroupNodes]; };
-  const TimePart T = load_time_part(X + xt * kGroupNodes);
+  const TimePart T = load_time_part(time);
   const double m_hot = Y(GAL_V_HOT_MASS), r_out = Y(GAL_V_HOT_OUTER_RADIUS), m_bh = Y(GAL_V_BH_MASS);
   const double mg_s = Y(GAL_V_SPHEROID_MASS_GAS), ms_s = Y(GAL_V_SPHEROID_MASS_STELLAR);
   const double j_s = Y(GAL_V_SPHEROID_ANGULAR_MOMENTUM), zg_s = Y(GAL_V_SPHEROID_ABUNDANCES_GAS);
   const double y_spin = Y(GAL_V_BH_SPIN), r_bh = Y(GAL_V_BH_RADIAL_POSITION);
   const GalaxyRadius galaxy = galaxy_radius(T, Y(GAL_V_SPIN_ANGULAR_MOMENTUM));
   HotProfile p = hot_profile(T, m_hot, r_out);
-  X[kMidRho0 * kGroupNodes] = p.rho0;
-  X[kMidRhoOut * kGroupNodes] = p.rho_out;
+  F[kMidRho0 * kGroupNodes] = p.rho0;
+  F[kMidRhoOut * kGroupNodes] = p.rho_out;
   signal(flags, kProfileReady, round);
   const BlackHole b = black_hole(G.P, G.D, galaxy, m_bh, after_signal(y_spin), after_signal(r_bh), mg_s);
-  X[kMidEffThin * kGroupNodes] = b.eff_thin;
-  X[kMidEddCap * kGroupNodes] = b.edd_cap;
-  X[kMidMdotSph * kGroupNodes] = b.mdot_sph;
+  F[kMidEffThin * kGroupNodes] = b.eff_thin;
+  F[kMidEddCap * kGroupNodes] = b.edd_cap;
+  F[kMidMdotSph * kGroupNodes] = b.mdot_sph;
   signal(flags, kAccretorReady, round);
   p.uo = after_signal(p.uo);
-  X[kMidInvRMean * kGroupNodes] = hot_inv_mean_radius(T, p);
+  F[kMidInvRMean * kGroupNodes] = hot_inv_mean_radius(T, p);
   signal(flags, kMeanRadiusReady, round);
   double f[kNV];
 #pragma unroll
   for (int v = 0; v < kNV; ++v) f[v] = 0.0;
   await(flags, kCoolingFunctionReady, round);
-  f[GAL_V_HOT_ENERGY_RADIATED] += radiated_energy(X[kMidLambda * kGroupNodes], X[kMidNhPerRho * kGroupNodes],
-                                                  X[kMidNallPerNh * kGroupNodes], m_hot, r_out);
+  f[GAL_V_HOT_ENERGY_RADIATED] += radiated_energy(F[kMidLambda * kGroupNodes], F[kMidNhPerRho * kGroupNodes],
+                                                  F[kMidNallPerNh * kGroupNodes], m_hot, r_out);
   await(flags, kAccretionReady, round);
-  black_hole_rates(G.P, G.D, ops, T, b, X[kMidMdot * kGroupNodes], X[kMidJet * kGroupNodes], m_bh, mg_s, ms_s, j_s,
+  black_hole_rates(G.P, G.D, ops, T, b, F[kMidMdot * kGroupNodes], F[kMidJet * kGroupNodes], m_bh, mg_s, ms_s, j_s,
                    zg_s, galaxy.r, f);
 #pragma unroll
   for (int v = 0; v < kNV; ++v)
@@ -213,30 +219,30 @@ __device__ __forceinline__ void profile_wave_rhs(const GroupConstants& G, int op
 }
 
 __device__ __forceinline__ void cooling_wave_rhs(const GroupConstants& G, const double* __restrict__ tab,
-                                                 const NodePar& np, double* __restrict__ X, int xt,
-                                                 int* __restrict__ flags, int round) {
+                                                 const NodePar& np, double* __restrict__ X, double* __restrict__ F,
+                                  const double* __restrict__ time, int* __restrict__ flags, int round) {
   auto Y = [&](int v) { return X[(kXState + v) * kGroupNodes]; };
-  const TimePart T = load_time_part(X + xt * kGroupNodes);
+  const TimePart T = load_time_part(time);
   const double m_hot = Y(GAL_V_HOT_MASS), r_out = Y(GAL_V_HOT_OUTER_RADIUS), z_hot = Y(GAL_V_HOT_ABUNDANCES);
   const double j_hot = Y(GAL_V_HOT_ANGULAR_MOMENTUM), m_bh = Y(GAL_V_BH_MASS), y_spin = Y(GAL_V_BH_SPIN);
   const CoolingTime c = cooling_time(G.D, tab, G.C, T, m_hot, z_hot, r_out);
-  X[kMidLambda * kGroupNodes] = c.lambda_cool;
-  X[kMidNhPerRho * kGroupNodes] = c.nh_per_rho;
-  X[kMidNallPerNh * kGroupNodes] = c.nall_per_nh;
+  F[kMidLambda * kGroupNodes] = c.lambda_cool;
+  F[kMidNhPerRho * kGroupNodes] = c.nh_per_rho;
+  F[kMidNallPerNh * kGroupNodes] = c.nall_per_nh;
   signal(flags, kCoolingFunctionReady, round);
   await(flags, kAccretorReady, round);   // and with it the profile
-  const double rho0 = X[kMidRho0 * kGroupNodes];
-  const HotAccretion s = hot_accretion(G.P, G.D, T, c, X[kMidEffThin * kGroupNodes], X[kMidEddCap * kGroupNodes],
-                                       X[kMidMdotSph * kGroupNodes], rho0, X[kMidRhoOut * kGroupNodes], m_hot, r_out,
+  const double rho0 = F[kMidRho0 * kGroupNodes];
+  const HotAccretion s = hot_accretion(G.P, G.D, T, c, F[kMidEffThin * kGroupNodes], F[kMidEddCap * kGroupNodes],
+                                       F[kMidMdotSph * kGroupNodes], rho0, F[kMidRhoOut * kGroupNodes], m_hot, r_out,
                                        m_bh, y_spin);
-  X[kMidMdot * kGroupNodes] = s.mdot;
-  X[kMidJet * kGroupNodes] = s.p_jet;
+  F[kMidMdot * kGroupNodes] = s.mdot;
+  F[kMidJet * kGroupNodes] = s.p_jet;
   signal(flags, kAccretionReady, round);
   double f[kNV];
 #pragma unroll
   for (int v = 0; v < kNV; ++v) f[v] = 0.0;
   await(flags, kMeanRadiusReady, round);
-  cooling_rates(G.P, np, T, s, c.inv_m_hot, rho0, X[kMidInvRMean * kGroupNodes], m_hot, z_hot, j_hot, r_out, m_bh, f);
+  cooling_rates(G.P, np, T, s, c.inv_m_hot, rho0, F[kMidInvRMean * kGroupNodes], m_hot, z_hot, j_hot, r_out, m_bh, f);
 #pragma unroll
   for (int v = 0; v < kNV; ++v)
     if ((kCoolingVars >> v) & 1u) X[(kXHalo + v) * kGroupNodes] = f[v];
