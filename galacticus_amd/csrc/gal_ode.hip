@@ -249,10 +249,9 @@ __device__ __forceinline__ void claim_nodes(const EvolveArgs& a, int n_claim, bo
 // in LDS, a lane's booleans share one register, and there is one loop with one
 // evaluation in it and one exit.
 //
-// Measured on the stiffest node of 100,000 isolated halos (3701 attempts): 20.3
+// Measured on the stiffest node of 100,000 isolated halos (3701 attempts): 18.7
 // us an attempt, 22.6 us with the state in registers and nested loops, and 43
 // us with one wave for the whole RHS, or two waves that split it in halves.
-// Evolving 100,000 of them takes 44.7 ms, and 88.2 ms that way.
 //
 template <int WAVE, bool GRAPH>
 __device__ __forceinline__ void group_wave(const EvolveArgs& a, double* __restrict__ X,
@@ -293,9 +292,9 @@ __device__ __forceinline__ void group_wave(const EvolveArgs& a, double* __restri
   int round = 0;
   int tb = 0;              // which time part is the coming stage's
   // owners
-  double sc[kOwned];
+  double abs_tol[kOwned];    // absolute tolerance times the error scale
 #pragma unroll
-  for (int i = 0; i < kOwned; ++i) sc[i] = 0.0;
+  for (int i = 0; i < kOwned; ++i) abs_tol[i] = 0.0;
   // derivative of a stage, and the state at the start of the step
   auto K = [&](int stage, int i) -> double& { return XK[((stage == 4 ? 1 : stage) * kNV + i) * kGroupNodes]; };
   auto Y0 = [&](int i) -> double& { return X0[i * kGroupNodes]; };
@@ -414,7 +413,7 @@ __device__ __forceinline__ void group_wave(const EvolveArgs& a, double* __restri
           if (t0 == t1) s.clear(LaneFlags::kEval);
           if (owner && scales_given) {
 #pragma unroll
-            for (int i = 0; i < kOwned; ++i) sc[i] = a.scale[(size_t)(v0 + i) * a.ld + node];
+            for (int i = 0; i < kOwned; ++i) abs_tol[i] = a.eps_abs * a.scale[(size_t)(v0 + i) * a.ld + node];
           }
         }
         if (__any(s.has(LaneFlags::kActive))) break;
@@ -443,10 +442,10 @@ __device__ __forceinline__ void group_wave(const EvolveArgs& a, double* __restri
       scales_of_halo(G.P, G.D, T.mass, T.r_vir, T.v_vir, galaxy_radius(T, ys[GAL_V_SPIN_ANGULAR_MOMENTUM]).r, ys, s30);
       if (s.has(LaneFlags::kFresh)) {
 #pragma unroll
-        for (int i = 0; i < kOwned; ++i) sc[i] = mode == GAL_PHYSICS_TEST ? 1.0 : s30[v0 + i];
-        if (a.scale) {
-#pragma unroll
-          for (int i = 0; i < kOwned; ++i) a.scale[(size_t)(v0 + i) * a.ld + node] = sc[i];
+        for (int i = 0; i < kOwned; ++i) {
+          const double sc = mode == GAL_PHYSICS_TEST ? 1.0 : rounded(s30[v0 + i]);
+          abs_tol[i] = a.eps_abs * sc;
+          if (a.scale) a.scale[(size_t)(v0 + i) * a.ld + node] = sc;
         }
       }
     }
@@ -468,6 +467,7 @@ __device__ __forceinline__ void group_wave(const EvolveArgs& a, double* __restri
         tn = t + kNextTime[ph] * h0;
       }
       store_time_part(time_part(G.P, G.D, G.C, np, tn), time_vectors(tb ^ 1));
+      if (ph != kTimeOnly && mode == GAL_PHYSICS_STANDARD) time_wave_rhs(X, F, flags, round);
     } else if (ph != kTimeOnly) {
       if constexpr (wave == kGalaxyWave) {
         galaxy_wave_rhs(G, mode, ops, np, X, F, time_vectors(tb), flags, round);
@@ -605,7 +605,8 @@ __device__ __forceinline__ void group_wave(const EvolveArgs& a, double* __restri
       // ---- k6 is in kn: solution, error norm, controller ---------------------
       double yn[kOwned];
       if (owner) {
-        ErrorNorm e;
+        double e_max = ErrorNorm{}.rmax;
+        bool forbidden = false;
         unsigned negative = 0u;
 #pragma unroll
         for (int i = 0; i < kOwned; ++i) {
@@ -614,20 +615,24 @@ __device__ __forceinline__ void group_wave(const EvolveArgs& a, double* __restri
           const double ye =
               h0 * fma(ck::ec6, kn[i],
                        fma(ck::ec5, K(4, i), fma(ck::ec4, K(3, i), fma(ck::ec3, K(2, i), ck::ec1 * K(0, i)))));
-          error_norm_add(e, a.eps_abs, a.eps_rel, 1.0, 0.0, h0, yn[i], ye, 0.0, sc[i],
-                         enforce && ((nonneg >> i) & 1u));
+          e_max = fmax(e_max, error_ratio(a.eps_rel, yn[i], ye, abs_tol[i]));
+          forbidden = forbidden || (enforce && ((nonneg >> i) & 1u) && yn[i] < 0.0);
           negative |= yn[i] < 0.0 ? 1u << i : 0u;
         }
-        F[(kFarNorm + wave) * kGroupNodes] = e.rmax;
-        norm_flags[wave * kGroupNodes + lane] = (e.forbidden ? 1 : 0) | ((negative & fixable) ? 2 : 0);
+        // The next derivative is taken at the new state; a lane whose attempt
+        // is rejected does not need one, so it is published without a choice.
+#pragma unroll
+        for (int i = 0; i < kOwned; ++i) XY[i * kGroupNodes] = yn[i];
+        F[(kFarNorm + wave) * kGroupNodes] = e_max;
+        norm_flags[wave * kGroupNodes + lane] = (forbidden ? 1 : 0) | ((negative & fixable) ? 2 : 0);
       }
-      __syncthreads();   // error norms published
+      __syncthreads();   // error norms and new state published
       rmax = ErrorNorm{}.rmax;
       int seen = 0;
 #pragma unroll
       for (int w = 0; w < kOwnerWaves; ++w) {
         const double r = F[(kFarNorm + w) * kGroupNodes];
-        rmax = r > rmax ? r : rmax;
+        rmax = fmax(rmax, r);
         seen |= norm_flags[w * kGroupNodes + lane];
       }
       s.clear(LaneFlags::kForbidden | LaneFlags::kNeedFix);
@@ -647,11 +652,6 @@ __device__ __forceinline__ void group_wave(const EvolveArgs& a, double* __restri
       }
       if (__any(done)) {
         if (__any(done && need_fix)) {
-          if (owner && done) {
-#pragma unroll
-            for (int i = 0; i < kOwned; ++i) XY[i * kGroupNodes] = yn[i];
-          }
-          __syncthreads();
           fix_published(done && need_fix, [&](int i, double v) { yn[i] = v; });
         }
         if (owner && done) {
@@ -663,15 +663,9 @@ __device__ __forceinline__ void group_wave(const EvolveArgs& a, double* __restri
         if (wave == kCoolingWave && done && !final_step) h_out = hadjust_step(norm(), kRkckOrder, h0);
         finish(done, h_out, true, GAL_STATUS_SUCCESS);
       }
-      // the state that the next derivative is taken at: the new one, or again
-      // the one that the attempt started from
-      if (owner) {
-        if (accepted) {
+      if (owner && accepted) {
 #pragma unroll
-          for (int i = 0; i < kOwned; ++i) Y0(i) = yn[i];
-        }
-#pragma unroll
-        for (int i = 0; i < kOwned; ++i) XY[i * kGroupNodes] = accepted ? yn[i] : y[i];
+        for (int i = 0; i < kOwned; ++i) Y0(i) = yn[i];
       }
       ph = kClaims;
     }

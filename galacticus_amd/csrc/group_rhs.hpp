@@ -9,13 +9,13 @@
 // what they wait for:
 //   galaxy wave   the galaxy half, then the CGM outer radius;
 //   profile wave  hot-halo profile, ISCO, spheroid accretion, then the mean
-//                 radius of the hot gas and its radiated energy, then the
-//                 black hole's rates and winds;
+//                 radius of the hot gas, then the spheroid's rates, the black
+//                 hole's spin and its winds;
 //   time wave     the part that depends on the time alone, of the *next*
 //                 stage (its time is known ahead of its state), and the step
-//                 controller's pow;
-//   cooling wave  cooling function and time, then cooling radius, hot-mode
-//                 accretion and jet power, then net cooling: the serial chain
+//                 controller's pow; then the radiated energy;
+//   cooling wave  cooling function and time, then cooling radius and hot-mode
+//                 accretion, then jet power and net cooling: the serial chain
 //                 that nothing takes off the path.
 // They meet in a barrier when the stage state is published and when the
 // derivatives are.  In between a value goes from the wave that computes it to
@@ -42,7 +42,7 @@ constexpr int kOwnerWaves = 3, kOwned = kNV / kOwnerWaves;
 static_assert(kOwned * kOwnerWaves == kNV, "owners must tile the state");
 
 constexpr int kTimeVectors = (int)(sizeof(TimePart) / sizeof(double));
-constexpr int kMidVectors = 11;
+constexpr int kMidVectors = 10;
 
 // Stages whose derivatives are kept: k1, k2 (whose place k5 takes once the last
 // stage input no longer needs it), k3 and k4.  k6 is consumed as it is produced.
@@ -65,7 +65,7 @@ enum : int {
   kFarStep = kFarNorm + kOwnerWaves,        // step size chosen by the controller
   // published within an evaluation
   kMidRho0 = kFarMid, kMidRhoOut, kMidEffThin, kMidEddCap, kMidMdotSph, kMidInvRMean,   // profile wave
-  kMidLambda, kMidNhPerRho, kMidNallPerNh, kMidMdot, kMidJet,                           // cooling wave
+  kMidLambda, kMidNhPerRho, kMidNallPerNh, kMidMdot,                                    // cooling wave
   kMidEnd,
   // claimed nodes, in the time part that is not in use
   kXClaimNode = 0, kXClaimT0, kXClaimT1, kXClaimStep, kXClaimPar
@@ -108,7 +108,7 @@ constexpr unsigned kHaloVars =
 // vectors, then the flag; LDS keeps one wave's operations in order, and the
 // fences keep the compiler to it.  Every wait ends: a flag is set by a wave of
 // the same workgroup that runs the same rounds, and the waits form no cycle
-// (profile -> cooling -> profile's last part, profile -> galaxy).
+// (profile -> cooling -> profile's last part; profile -> galaxy; cooling -> time).
 enum Signal : int { kProfileReady = 0, kAccretorReady, kMeanRadiusReady, kCoolingFunctionReady, kAccretionReady, kSignals };
 
 __device__ __forceinline__ void signal(int* __restrict__ flags, Signal s, int round) {
@@ -175,16 +175,17 @@ __device__ __forceinline__ void galaxy_wave_rhs(const GroupConstants& G, int mod
     if ((kGalaxyVars >> v) & 1u) X[(kXGalaxy + v) * kGroupNodes] = f[v];
 }
 
-// Of the hot-halo half, the profile wave writes the variables of the black
-// hole, its spheroid and the outflow, the cooling wave the others.
-constexpr unsigned kBlackHoleVars =
+// Of the hot-halo half, the profile wave writes the variables of the spheroid,
+// the outflow and the black hole's spin, the time wave the radiated energy and
+// the cooling wave the others.
+constexpr unsigned kSpheroidVars =
     var_bits({GAL_V_HOT_OUTFLOWED_MASS, GAL_V_HOT_OUTFLOWED_ANGULAR_MOMENTUM, GAL_V_HOT_OUTFLOWED_ABUNDANCES,
-              GAL_V_HOT_ENERGY_RADIATED, GAL_V_SPHEROID_MASS_GAS, GAL_V_SPHEROID_ABUNDANCES_GAS,
-              GAL_V_SPHEROID_ANGULAR_MOMENTUM, GAL_V_BH_MASS, GAL_V_BH_SPIN});
-constexpr unsigned kCoolingVars = kHaloVars & ~kBlackHoleVars;
+              GAL_V_SPHEROID_MASS_GAS, GAL_V_SPHEROID_ABUNDANCES_GAS, GAL_V_SPHEROID_ANGULAR_MOMENTUM, GAL_V_BH_SPIN});
+constexpr unsigned kCoolingVars = kHaloVars & ~kSpheroidVars & ~(1u << GAL_V_HOT_ENERGY_RADIATED);
 
-__device__ __forceinline__ void profile_wave_rhs(const GroupConstants& G, int ops, double* __restrict__ X, double* __restrict__ F,
-                                  const double* __restrict__ time, int* __restrict__ flags, int round) {
+__device__ __forceinline__ void profile_wave_rhs(const GroupConstants& G, int ops, double* __restrict__ X,
+                                                 double* __restrict__ F, const double* __restrict__ time,
+                                                 int* __restrict__ flags, int round) {
   auto Y = [&](int v) { return X[(kXState + v) * kGroupNodes]; };
   const TimePart T = load_time_part(time);
   const double m_hot = Y(GAL_V_HOT_MASS), r_out = Y(GAL_V_HOT_OUTER_RADIUS), m_bh = Y(GAL_V_BH_MASS);
@@ -204,23 +205,33 @@ __device__ __forceinline__ void profile_wave_rhs(const GroupConstants& G, int op
   p.uo = after_signal(p.uo);
   F[kMidInvRMean * kGroupNodes] = hot_inv_mean_radius(T, p);
   signal(flags, kMeanRadiusReady, round);
+  SpheroidShares q = spheroid_shares(G.P, G.D, ops, b, m_bh, after_signal(mg_s), ms_s, j_s, zg_s, galaxy.r);
+  q.inv_mg = after_signal(q.inv_mg);
+  q.inv_mt = after_signal(q.inv_mt);
+  q.inv_m_bh = after_signal(q.inv_m_bh);
   double f[kNV];
 #pragma unroll
   for (int v = 0; v < kNV; ++v) f[v] = 0.0;
-  await(flags, kCoolingFunctionReady, round);
-  f[GAL_V_HOT_ENERGY_RADIATED] += radiated_energy(F[kMidLambda * kGroupNodes], F[kMidNhPerRho * kGroupNodes],
-                                                  F[kMidNallPerNh * kGroupNodes], m_hot, r_out);
   await(flags, kAccretionReady, round);
-  black_hole_rates(G.P, G.D, ops, T, b, F[kMidMdot * kGroupNodes], F[kMidJet * kGroupNodes], m_bh, mg_s, ms_s, j_s,
-                   zg_s, galaxy.r, f);
+  spheroid_rates(G.P, G.D, T, b, q, F[kMidMdot * kGroupNodes], m_bh, mg_s, ms_s, j_s, zg_s, galaxy.r, f);
 #pragma unroll
   for (int v = 0; v < kNV; ++v)
-    if ((kBlackHoleVars >> v) & 1u) X[(kXHalo + v) * kGroupNodes] = f[v];
+    if ((kSpheroidVars >> v) & 1u) X[(kXHalo + v) * kGroupNodes] = f[v];
+}
+
+// The time wave's share of this stage's derivative, after the next stage's
+// time part.
+__device__ __forceinline__ void time_wave_rhs(double* __restrict__ X, double* __restrict__ F,
+                                              int* __restrict__ flags, int round) {
+  await(flags, kCoolingFunctionReady, round);
+  X[(kXHalo + GAL_V_HOT_ENERGY_RADIATED) * kGroupNodes] =
+      radiated_energy(F[kMidLambda * kGroupNodes], F[kMidNhPerRho * kGroupNodes], F[kMidNallPerNh * kGroupNodes],
+                      X[(kXState + GAL_V_HOT_MASS) * kGroupNodes], X[(kXState + GAL_V_HOT_OUTER_RADIUS) * kGroupNodes]);
 }
 
 __device__ __forceinline__ void cooling_wave_rhs(const GroupConstants& G, const double* __restrict__ tab,
                                                  const NodePar& np, double* __restrict__ X, double* __restrict__ F,
-                                  const double* __restrict__ time, int* __restrict__ flags, int round) {
+                                                 const double* __restrict__ time, int* __restrict__ flags, int round) {
   auto Y = [&](int v) { return X[(kXState + v) * kGroupNodes]; };
   const TimePart T = load_time_part(time);
   const double m_hot = Y(GAL_V_HOT_MASS), r_out = Y(GAL_V_HOT_OUTER_RADIUS), z_hot = Y(GAL_V_HOT_ABUNDANCES);
@@ -230,19 +241,23 @@ __device__ __forceinline__ void cooling_wave_rhs(const GroupConstants& G, const 
   F[kMidNhPerRho * kGroupNodes] = c.nh_per_rho;
   F[kMidNallPerNh * kGroupNodes] = c.nall_per_nh;
   signal(flags, kCoolingFunctionReady, round);
-  await(flags, kAccretorReady, round);   // and with it the profile
+  await(flags, kProfileReady, round);
   const double rho0 = F[kMidRho0 * kGroupNodes];
-  const HotAccretion s = hot_accretion(G.P, G.D, T, c, F[kMidEffThin * kGroupNodes], F[kMidEddCap * kGroupNodes],
-                                       F[kMidMdotSph * kGroupNodes], rho0, F[kMidRhoOut * kGroupNodes], m_hot, r_out,
-                                       m_bh, y_spin);
+  HotAccretion s = hot_accretion(G.P, G.D, T, c, rho0, F[kMidRhoOut * kGroupNodes], m_hot, r_out, m_bh);
+  s.bondi = after_signal(s.bondi);
+  await(flags, kAccretorReady, round);
+  const double eff_thin = F[kMidEffThin * kGroupNodes];
+  accretion_rate(s, eff_thin, F[kMidEddCap * kGroupNodes], F[kMidMdotSph * kGroupNodes]);
   F[kMidMdot * kGroupNodes] = s.mdot;
-  F[kMidJet * kGroupNodes] = s.p_jet;
   signal(flags, kAccretionReady, round);
+  const double p_jet = jet_power(G.D, after_signal(s.mdot), m_bh, y_spin);
   double f[kNV];
 #pragma unroll
   for (int v = 0; v < kNV; ++v) f[v] = 0.0;
+  f[GAL_V_BH_MASS] += black_hole_growth(s.mdot, p_jet, eff_thin, m_bh);
   await(flags, kMeanRadiusReady, round);
-  cooling_rates(G.P, np, T, s, c.inv_m_hot, rho0, F[kMidInvRMean * kGroupNodes], m_hot, z_hot, j_hot, r_out, m_bh, f);
+  cooling_rates(G.P, np, T, s, p_jet, c.inv_m_hot, rho0, F[kMidInvRMean * kGroupNodes], m_hot, z_hot, j_hot, r_out,
+                m_bh, f);
 #pragma unroll
   for (int v = 0; v < kNV; ++v)
     if ((kCoolingVars >> v) & 1u) X[(kXHalo + v) * kGroupNodes] = f[v];

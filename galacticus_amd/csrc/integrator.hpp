@@ -51,6 +51,14 @@ __device__ __forceinline__ void error_norm_add(ErrorNorm& e, double eps_abs, dou
   if (non_negative && y < 0.0) e.forbidden = true;
 }
 
+// One variable's part of the norm where only the state scales the relative
+// tolerance (a_y = 1, a_dydt = 0); abs_part is eps_abs * scale_abs.
+__device__ __forceinline__ double error_ratio(double eps_rel, double y, double yerr, double abs_part) {
+#pragma clang fp contract(off)
+  const double D0 = eps_rel * fabs(y) + abs_part;
+  return fabs(yerr) / fabs(D0);
+}
+
 // Step decision from the accumulated norm (cscal2.c:127-168): whether the
 // step is repeated, kept or kept with a longer one next, and the step size
 // that follows (a pow, which callers may leave to another wave).

@@ -87,6 +87,21 @@ __device__ __forceinline__ double rounded(double x) {
   return x;
 }
 
+// x / C for a constant C, the correctly rounded quotient, from the rounded
+// reciprocal of C and one exact remainder (Markstein, "Computation of
+// elementary functions on the IBM RISC System/6000 processor", 1990): three
+// operations where a division takes eleven.  For x that is zero, NaN or normal
+// with a normal quotient; 4e8 values of [2^-64, 1) agree with the division for
+// both constants it is used with.
+struct AtomicMassHydrogen { static constexpr double value = kAtomicMassHydrogen; };
+struct AtomicMassHelium { static constexpr double value = kAtomicMassHelium; };
+template <class C>
+__device__ __forceinline__ double over(double x) {
+  constexpr double inv = 1.0 / C::value;
+  const double q = rounded(x * inv);
+  return fma(fma(-C::value, q, x), inv, q);
+}
+
 // Cooling table descriptor (table itself in global memory).
 struct CoolingDesc {
   int n_t, n_z;
@@ -167,17 +182,29 @@ __device__ __forceinline__ void cooling_temperature_index(const CoolingDesc& c, 
   row = it;
   ht = rounded((lt - t0) / (t1 - t0));
 }
-__device__ __forceinline__ double cooling_function_ln(const double* __restrict__ tab, const CoolingDesc& c, double row,
-                                                      double ht, double lz) {
+// The table cell of a temperature and metallicity: its corners and weights.
+// The corners come from global memory (the table does not fit LDS beside the
+// integrator), some 700 cycles away when they are not in the CU's own cache.
+struct CoolingCell {
+  double r00, r01, r10, r11, ht, hz;
+};
+__device__ __forceinline__ CoolingCell cooling_cell(const double* __restrict__ tab, const CoolingDesc& c, double row,
+                                                    double ht, double lz) {
   const int it = (int)row;
   int iz = (int)((lz - c.ln_z_min) * c.inv_d_ln_z);
   iz = iz < 0 ? 0 : (iz > c.n_z - 2 ? c.n_z - 2 : iz);
-  const double z0 = c.ln_z_min + c.d_ln_z * iz, z1 = c.ln_z_min + c.d_ln_z * (iz + 1);
-  const double hz = (lz - z0) / (z1 - z0);
   const double* r0 = tab + iz * c.n_t + it;
   const double* r1 = r0 + c.n_t;
-  const double v = fma(r1[1] * ht, hz, fma(r0[1] * ht, 1.0 - hz,
-                                           fma(r0[0] * (1.0 - ht), 1.0 - hz, rounded(r1[0] * (1.0 - ht) * hz))));
+  CoolingCell cell{r0[0], r0[1], r1[0], r1[1], ht};
+  __builtin_amdgcn_sched_barrier(0);   // the loads first
+  const double z0 = c.ln_z_min + c.d_ln_z * iz, z1 = c.ln_z_min + c.d_ln_z * (iz + 1);
+  cell.hz = (lz - z0) / (z1 - z0);
+  return cell;
+}
+__device__ __forceinline__ double cooling_function(const CoolingCell& c) {
+  const double ht = c.ht, hz = c.hz;
+  const double v = fma(c.r11 * ht, hz, fma(c.r01 * ht, 1.0 - hz,
+                                           fma(c.r00 * (1.0 - ht), 1.0 - hz, rounded(c.r10 * (1.0 - ht) * hz))));
   return exp(v);
 }
 
@@ -280,9 +307,10 @@ __device__ __forceinline__ Halo halo(const double* __restrict__ P, const Derived
 //                  spin growth, satellite mass loss, star formation, stellar
 //                  feedback, bar instability, CGM accretion, outflow
 //                  reincorporation and the CGM outer radius;
-//   hot_accretion, black_hole_rates, radiated_energy, cooling_rates    the
-//                  hot-halo half: black-hole accretion, jet and winds, cooling
-//                  and heating, radiated energy.
+//   hot_accretion, accretion_rate, jet_power, black_hole_growth,
+//   spheroid_rates, radiated_energy, cooling_rates    the hot-halo half:
+//                  black-hole accretion, jet and winds, cooling and heating,
+//                  radiated energy.
 // The derivative is f_galaxy + f_halo in every caller, and a block is the
 // same code wherever it runs: one lane computing all of them and four waves
 // computing some each give the same bits.
@@ -453,14 +481,18 @@ __device__ __forceinline__ CoolingTime cooling_time(const DerivedConstants& D, c
   c.inv_m_hot = (hot_ok && m_hot > kRatioMassMin) ? inv_m : 0.0;
   const double zf = fmin(fmax(z_hot * c.inv_m_hot, 0.0), 1.0);
   const double lz = log(clamp_metallicity(cd, zf * (1.0 / kMetallicitySolar)));
-  c.lambda_cool = cooling_function_ln(tab, cd, T.table_t, T.table_ht, lz);
+  const CoolingCell cell = cooling_cell(tab, cd, T.table_t, T.table_ht, lz);
+  // the composition while the cell is on its way
+  __builtin_amdgcn_sched_barrier(0);
   constexpr double kNorm = 1.0 / (kHydrogenPrimordial + kHeliumPrimordial);
   const double X = (1.0 - zf) * kHydrogenPrimordial * kNorm;
   const double Yh = (1.0 - zf) * kHeliumPrimordial * kNorm;
-  const double nh_n = X / kAtomicMassHydrogen, nhe_n = Yh / kAtomicMassHelium;
+  const double nh_n = over<AtomicMassHydrogen>(X), nhe_n = over<AtomicMassHelium>(Yh);
   c.nh_per_rho = rounded(X * D.nh_coeff);
   const double inv_nh_n = rcp(nh_n);
-  c.nall_per_nh = (nh_n + nhe_n) * inv_nh_n + (1.0 + 2.0 * nhe_n * inv_nh_n);
+  c.nall_per_nh = rounded((nh_n + nhe_n) * inv_nh_n + (1.0 + 2.0 * nhe_n * inv_nh_n));
+  __builtin_amdgcn_sched_barrier(0);
+  c.lambda_cool = cooling_function(cell);
   c.k = rounded(D.cool_k_pre * T.t_vir * c.nall_per_nh * rcp(c.lambda_cool * c.nh_per_rho));
   c.inv_k = rcp(c.k);
   return c;
@@ -703,18 +735,20 @@ __device__ __forceinline__ void outer_radius_rates(const double* __restrict__ P,
 }
 
 // ---- the hot-halo half -----------------------------------------------------
-// hot_accretion: cooling radius, hot-mode accretion and jet power, the serial
-// chain of the RHS; black_hole_rates: what the accretion and its winds do to
-// the black hole, the spheroid and the outflow; cooling_rates: cooling against
-// heating of the hot gas.
+// hot_accretion, accretion_rate, jet_power: cooling radius, hot-mode accretion
+// and the jet, the serial chain of the RHS; black_hole_growth, spheroid_rates:
+// what the accretion and its winds do to the black hole, the spheroid and the
+// outflow; cooling_rates: cooling against heating of the hot gas.
 struct HotAccretion {
-  double r_cool, xc, mdot_hot, mdot, p_jet;
+  double r_cool, xc;
+  double bondi;         // hot-mode accretion before the Eddington limit
+  bool dense;           // whether there is gas to accrete
+  double mdot_hot, mdot;
 };
 
 __device__ __forceinline__ HotAccretion hot_accretion(const double* __restrict__ P, const DerivedConstants& D,
-                                                      const TimePart& T, const CoolingTime& c, double eff_thin,
-                                                      double edd_cap, double mdot_sph, double rho0, double rho_out,
-                                                      double m_hot, double r_out, double m_bh, double y_spin) {
+                                                      const TimePart& T, const CoolingTime& c, double rho0,
+                                                      double rho_out, double m_hot, double r_out, double m_bh) {
   const bool hot_ok = m_hot > 0.0 && r_out > 0.0;
   const double lambda_cool = c.lambda_cool, K = c.k, inv_k = c.inv_k;
   // simpleRadius (cooling_radius/simple.F90:313-387) with t_available = t_dyn
@@ -724,12 +758,11 @@ __device__ __forceinline__ HotAccretion hot_accretion(const double* __restrict__
   r_cool = (K - t_avail * rho0 > 0.0) ? 0.0 : r_cool;
   r_cool = (K - t_avail * rho_out < 0.0) ? r_out : r_cool;
   r_cool = (lambda_cool > 0.0 && hot_ok) ? r_cool : 0.0;
-  const double xc = rounded(r_cool * T.inv_r_core);
+  HotAccretion s;
+  s.r_cool = r_cool;
+  s.xc = rounded(r_cool * T.inv_r_core);
   // ---- blackHolesAccretion, hot mode -------------------------------------
-  const double spin = black_hole_spin(y_spin);
-  const bool bh_ok = m_bh > 0.0;
   constexpr double kBhlUnit = kKilo * kGigaYear / kMegaParsec * 4.0 * kPi;
-  double mdot_hot;
   {
     const double cs = T.cs;
     const double r2 = fmin(kGravity * m_bh * T.inv_cs2, r_out);
@@ -741,40 +774,77 @@ __device__ __forceinline__ HotAccretion hot_accretion(const double* __restrict__
     const double rho2 = fhot * (rho0 * rcp(1.0 + sq(r2 * T.inv_r_core)));
     double m = fmax(P[GAL_P_BH_ENHANCEMENT_HOT_HALO] * kBhlUnit * r2 * r2 * rho2 * cs, 0.0);
     m = fmin(m, fmax(m_hot * cs * rcp(r_out) * (1.0 / kMpcPerKmsToGyr), 0.0));
-    m = (m > 0.0 && eff_thin > 0.0) ? fmin(m, edd_cap) : m;
-    mdot_hot = (bh_ok && hot_ok && rho2 > 1.0) ? m : 0.0;
+    s.bondi = m;
+    s.dense = m_bh > 0.0 && hot_ok && rho2 > 1.0;
   }
-  const double mdot = mdot_sph + mdot_hot;
-  const bool acc_ok = bh_ok && mdot > 0.0;
-  // Meier (2001) jet power (Shakura_Sunyaev.F90:92-140):
-  // M^-0.3 Mdot^1.2 = (Mdot^4 / M)^0.3
+  return s;
+}
+
+__device__ __forceinline__ void accretion_rate(HotAccretion& s, double eff_thin, double edd_cap, double mdot_sph) {
+  const double m = (s.bondi > 0.0 && eff_thin > 0.0) ? fmin(s.bondi, edd_cap) : s.bondi;
+  s.mdot_hot = s.dense ? m : 0.0;
+  s.mdot = mdot_sph + s.mdot_hot;
+}
+
+// Meier (2001) jet power (Shakura_Sunyaev.F90:92-140):
+// M^-0.3 Mdot^1.2 = (Mdot^4 / M)^0.3
+__device__ __forceinline__ double jet_power(const DerivedConstants& D, double mdot, double m_bh, double y_spin) {
+  const double spin = black_hole_spin(y_spin);
+  const bool acc_ok = m_bh > 0.0 && mdot > 0.0;
   const double inv_m_bh = rcp(m_bh);
   const double lm = 0.3 * log(mdot * mdot * mdot * mdot * inv_m_bh);
   const bool kerr = spin > 0.8;
   const double e_jet = exp(kerr ? D.ln_jet_kerr + lm : D.ln_jet_schw + lm + 3.785 * spin);
   const double p_jet_k = e_jet * (1.0 + 1.1 * spin + 0.29 * spin * spin);
   const double p_jet = acc_ok ? (kerr ? p_jet_k : e_jet) : 0.0;
-  return HotAccretion{r_cool, xc, mdot_hot, mdot, rounded(p_jet)};
+  return rounded(p_jet);
 }
 
-__device__ __forceinline__ void black_hole_rates(const double* __restrict__ P, const DerivedConstants& D, int ops,
-                                                 const TimePart& T, const BlackHole& b, double mdot, double p_jet,
-                                                 double m_bh, double mg_s, double ms_s, double j_s, double zg_s,
-                                                 double r_gal, double (&f)[kNV]) {
+__device__ __forceinline__ double black_hole_growth(double mdot, double p_jet, double eff_thin, double m_bh) {
+  constexpr double kInvC2 = 1.0 / ((kSpeedLight / kKilo) * (kSpeedLight / kKilo));
+  const bool acc_ok = m_bh > 0.0 && mdot > 0.0;
+  const double eff_jet = p_jet * rcp(mdot) * kInvC2;
+  const double reduced = mdot * (1.0 - eff_thin - eff_jet);
+  return acc_ok ? reduced : 0.0;
+}
+
+// What the rates of the spheroid and the black hole's spin need beside the
+// accretion rate, ready before that is known.
+struct SpheroidShares {
+  double inv_mg, inv_mt, inv_m_bh;
+  double sink_zg, sink_j;            // metals and angular momentum lost with the accreted gas
+  double eff, eff_r, wind;           // wind efficiency, times the radius; pressure ratio times the gas mass
+  bool on;
+};
+
+__device__ __forceinline__ SpheroidShares spheroid_shares(const double* __restrict__ P, const DerivedConstants& D,
+                                                          int ops, const BlackHole& b, double m_bh, double mg_s,
+                                                          double ms_s, double j_s, double zg_s, double r_gal) {
+  SpheroidShares q;
+  q.inv_mg = rcp_ratio(mg_s);
+  q.inv_mt = rcp_ratio(mg_s + ms_s);
+  q.inv_m_bh = rcp(m_bh);
+  q.sink_zg = rounded(b.mdot_sph * (zg_s * q.inv_mg));
+  q.sink_j = rounded(b.mdot_sph * (j_s * q.inv_mt));
+  q.eff = P[GAL_P_BH_WIND_EFFICIENCY] * (P[GAL_P_BH_WIND_SCALES_WITH_RADIATIVE] != 0.0 ? b.eff_thin : 1.0);
+  q.on = (ops & GAL_OPERATOR_BLACK_HOLE_WINDS) && q.eff > 0.0;
+  q.eff_r = rounded(r_gal * q.eff);
+  q.wind = rounded(D.wind_pressure_ratio * mg_s);
+  return q;
+}
+
+__device__ __forceinline__ void spheroid_rates(const double* __restrict__ P, const DerivedConstants& D,
+                                               const TimePart& T, const BlackHole& b, const SpheroidShares& q,
+                                               double mdot, double m_bh, double mg_s, double ms_s, double j_s,
+                                               double zg_s, double r_gal, double (&f)[kNV]) {
   const bool acc_ok = m_bh > 0.0 && mdot > 0.0;
   const double mt_s = mg_s + ms_s, v_gal = T.v_vir;
-  const double inv_mg_s = rcp_ratio(mg_s), inv_mt_s = rcp_ratio(mt_s), inv_m_bh = rcp(m_bh);
-  const double eff_thin = b.eff_thin, mdot_sph = b.mdot_sph;
   {
-    constexpr double kInvC2 = 1.0 / ((kSpeedLight / kKilo) * (kSpeedLight / kKilo));
-    const double eff_jet = p_jet * rcp(mdot) * kInvC2;
-    const double reduced = mdot * (1.0 - eff_thin - eff_jet);
-    const double spin_up = b.spin_up * mdot * inv_m_bh;
-    f[GAL_V_BH_MASS] += acc_ok ? reduced : 0.0;
+    const double spin_up = b.spin_up * mdot * q.inv_m_bh;
     // spheroid%massGasSinkRate: gas, metals and angular momentum in proportion
-    f[GAL_V_SPHEROID_MASS_GAS] -= acc_ok ? mdot_sph : 0.0;
-    f[GAL_V_SPHEROID_ABUNDANCES_GAS] -= acc_ok ? mdot_sph * (zg_s * inv_mg_s) : 0.0;
-    f[GAL_V_SPHEROID_ANGULAR_MOMENTUM] -= acc_ok ? mdot_sph * (j_s * inv_mt_s) : 0.0;
+    f[GAL_V_SPHEROID_MASS_GAS] -= acc_ok ? b.mdot_sph : 0.0;
+    f[GAL_V_SPHEROID_ABUNDANCES_GAS] -= acc_ok ? q.sink_zg : 0.0;
+    f[GAL_V_SPHEROID_ANGULAR_MOMENTUM] -= acc_ok ? q.sink_j : 0.0;
     f[GAL_V_BH_SPIN] += acc_ok ? spin_up : 0.0;
   }
   // ---- blackHolesWinds (black_holes/winds.F90:102-133) with ciotti2009
@@ -782,17 +852,16 @@ __device__ __forceinline__ void black_hole_rates(const double* __restrict__ P, c
   // spheroid gas, which drives an outflow efficiencyEnergeticOutflow P / V^2
   // into the hot halo (spheroid/standard/_class.F90:673-725).
   {
-    const double eff = P[GAL_P_BH_WIND_EFFICIENCY] * (P[GAL_P_BH_WIND_SCALES_WITH_RADIATIVE] != 0.0 ? eff_thin : 1.0);
-    const bool on = (ops & GAL_OPERATOR_BLACK_HOLE_WINDS) && acc_ok && eff > 0.0;
-    const double x = D.wind_pressure_ratio * mg_s * rcp(r_gal * eff * mdot) - 0.5;
+    const bool on = q.on && acc_ok;
+    const double x = q.wind * rcp(q.eff_r * mdot) - 0.5;
     double coupled = x <= 0.0 ? 0.0 : (x >= 1.0 ? 1.0 : x * x * (3.0 - 2.0 * x));
     coupled = (mg_s > 0.0 && r_gal > 0.0) ? coupled : 0.0;
     constexpr double kC2 = (kSpeedLight / kKilo) * (kSpeedLight / kKilo);
-    const double power = eff * coupled * mdot * kC2;
+    const double power = q.eff * coupled * mdot * kC2;
     const bool drive = on && power > 0.0 && mg_s > 0.0 && mt_s > 0.0 && v_gal > 0.0;
     const double mo = drive ? P[GAL_P_SPHEROID_ENERGETIC_OUTFLOW] * power * T.inv_v * T.inv_v : 0.0;
-    const double jo = mo * inv_mt_s * j_s;
-    const double zo = mo * inv_mg_s * zg_s;
+    const double jo = mo * q.inv_mt * j_s;
+    const double zo = mo * q.inv_mg * zg_s;
     f[GAL_V_SPHEROID_MASS_GAS] -= mo;
     f[GAL_V_SPHEROID_ANGULAR_MOMENTUM] -= jo;
     f[GAL_V_SPHEROID_ABUNDANCES_GAS] -= zo;
@@ -814,7 +883,7 @@ __device__ __forceinline__ double radiated_energy(double lambda_cool, double nh_
 }
 
 __device__ __forceinline__ void cooling_rates(const double* __restrict__ P, const NodePar& np, const TimePart& T,
-                                              const HotAccretion& s, double inv_m_hot, double rho0, double inv_r_mean,
+                                              const HotAccretion& s, double p_jet, double inv_m_hot, double rho0, double inv_r_mean,
                                               double m_hot, double z_of_hot, double j_of_hot, double r_out,
                                               double m_bh, double (&f)[kNV]) {
   const bool hot_ok = m_hot > 0.0 && r_out > 0.0;
@@ -840,7 +909,7 @@ __device__ __forceinline__ void cooling_rates(const double* __restrict__ P, cons
     double cool = 4.0 * kPi * r_cool * r_cool * (rho0 * rcp(1.0 + xc * xc)) * r_cool_rate;
     cool = r_cool >= r_out ? m_hot * T.inv_t_dyn : cool;
     cool = T.v_vir > P[GAL_P_COOLING_VELOCITY_CUTOFF] ? 0.0 : cool;
-    const double heat = rounded(P[GAL_P_EFFICIENCY_RADIO_MODE] * s.p_jet * sq(T.inv_v));
+    const double heat = rounded(P[GAL_P_EFFICIENCY_RADIO_MODE] * p_jet * sq(T.inv_v));
     const bool heating = ok && heat > cool;
     const bool cooling = ok && cool > heat;
     // excess heating expels gas from the node (excessHeatDrivesOutflow); a
@@ -891,12 +960,16 @@ __device__ __forceinline__ void rhs(const double* __restrict__ P, const DerivedC
     if (ops & GAL_OPERATOR_CGM_OUTER_RADIUS) outer_radius_rates(P, np, T, p.rho0, p.rho_out, y, f);
     const CoolingTime c = cooling_time(D, tab, cd, T, m_hot, z_hot, r_out);
     const BlackHole b = black_hole(P, D, galaxy, m_bh, y_spin, y[GAL_V_BH_RADIAL_POSITION], mg_s);
-    const HotAccretion s = hot_accretion(P, D, T, c, b.eff_thin, b.edd_cap, b.mdot_sph, p.rho0, p.rho_out, m_hot,
-                                         r_out, m_bh, y_spin);
-    black_hole_rates(P, D, ops, T, b, s.mdot, s.p_jet, m_bh, mg_s, y[GAL_V_SPHEROID_MASS_STELLAR],
-                     y[GAL_V_SPHEROID_ANGULAR_MOMENTUM], y[GAL_V_SPHEROID_ABUNDANCES_GAS], galaxy.r, fh);
+    const double ms_s = y[GAL_V_SPHEROID_MASS_STELLAR], j_s = y[GAL_V_SPHEROID_ANGULAR_MOMENTUM];
+    const double zg_s = y[GAL_V_SPHEROID_ABUNDANCES_GAS];
+    HotAccretion s = hot_accretion(P, D, T, c, p.rho0, p.rho_out, m_hot, r_out, m_bh);
+    accretion_rate(s, b.eff_thin, b.edd_cap, b.mdot_sph);
+    spheroid_rates(P, D, T, b, spheroid_shares(P, D, ops, b, m_bh, mg_s, ms_s, j_s, zg_s, galaxy.r), s.mdot, m_bh,
+                   mg_s, ms_s, j_s, zg_s, galaxy.r, fh);
+    const double p_jet = jet_power(D, s.mdot, m_bh, y_spin);
+    fh[GAL_V_BH_MASS] += black_hole_growth(s.mdot, p_jet, b.eff_thin, m_bh);
     fh[GAL_V_HOT_ENERGY_RADIATED] += radiated_energy(c.lambda_cool, c.nh_per_rho, c.nall_per_nh, m_hot, r_out);
-    cooling_rates(P, np, T, s, c.inv_m_hot, p.rho0, hot_inv_mean_radius(T, p), m_hot, z_hot,
+    cooling_rates(P, np, T, s, p_jet, c.inv_m_hot, p.rho0, hot_inv_mean_radius(T, p), m_hot, z_hot,
                   y[GAL_V_HOT_ANGULAR_MOMENTUM], r_out, m_bh, fh);
   }
 #pragma unroll

@@ -31,9 +31,10 @@ TRANSCENDENTAL_WEIGHT = 20
 TRANSCENDENTALS = ("exp", "log", "log1p", "cbrt", "atan", "pow", "sinh")
 UNIT_CALLS = ("sqrt", "rsqrt", "fmin", "fmax", "fabs")
 # The functions an evaluation goes through once.
-BLOCKS = ("halo", "time_part", "cooling_temperature_index", "cooling_function_ln", "isco", "galaxy_radius",
+BLOCKS = ("halo", "time_part", "cooling_temperature_index", "cooling_cell", "cooling_function", "isco", "galaxy_radius",
           "hot_profile", "hot_inv_mean_radius", "black_hole", "cooling_time", "galaxy_rates", "outer_radius_rates",
-          "hot_accretion", "black_hole_rates", "radiated_energy", "cooling_rates")
+          "hot_accretion", "accretion_rate", "jet_power", "black_hole_growth", "spheroid_shares", "spheroid_rates",
+          "radiated_energy", "cooling_rates")
 
 
 def _function_body(src: str, signature_start: str) -> str:
