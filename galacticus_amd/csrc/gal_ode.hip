@@ -106,19 +106,22 @@ __device__ __forceinline__ int wave_claim(bool want, unsigned int* work, int n, 
   return idx;
 }
 
+template <bool SHARED>
 __device__ __forceinline__ void write_counters(const EvolveArgs& a, int node, long long na, long long nc,
                                                long long nr) {
   if (a.counters) {
-    a.counters[node] = na;
-    a.counters[(size_t)a.n + node] = nc;
-    a.counters[2 * (size_t)a.n + node] = nr;
+    store_state_word<SHARED>(a.counters + node, na);
+    store_state_word<SHARED>(a.counters + (size_t)a.n + node, nc);
+    store_state_word<SHARED>(a.counters + 2 * (size_t)a.n + node, nr);
   }
 }
 
 // What a lane of the cooling wave keeps about the node it claimed last.
 struct ClaimState {
-  int op = -1, pend = -1;              // graph mode: operation in hand, claimed ready-list entry
-  unsigned int wait_tail = ~0u;        // graph mode: appends seen while waiting on the entry
+  // graph mode: the operation in hand and its successors, the one to run after
+  // it, and the claimed entry of the ready list with what it last read
+  int op = -1, next_a = -1, next_b = -1, next = -1, pend = -1, peek = -1;
+  unsigned long long wait_progress = ~0ull;   // progress seen while waiting on the entry
   unsigned long long wait_since = 0ull;
 };
 // Claims, then the rounds of an attempt: the time part alone (new nodes), the derivative at its
@@ -153,23 +156,26 @@ enum : int { kNoClaim = -1, kExhausted = -2 };   // codes of the claim vector be
 // publish it, or why there is none, in the claim vectors of the exchange
 // area.
 template <bool GRAPH>
-__device__ __forceinline__ void claim_nodes(const EvolveArgs& a, int n_claim, bool want, ClaimState& c,
+__device__ __forceinline__ void claim_nodes(const EvolveArgs& a, int n_claim, bool want, bool idle, ClaimState& c,
                                             double* __restrict__ C) {
   auto publish = [&](int node, double t0, double t1, const double* np, size_t stride) {
     C[kXClaimNode * kGroupNodes] = (double)node;
     C[kXClaimT0 * kGroupNodes] = t0;
     C[kXClaimT1 * kGroupNodes] = t1;
-    C[kXClaimStep * kGroupNodes] = a.h_step[node];
+    C[kXClaimStep * kGroupNodes] = load_state_word<GRAPH>(a.h_step + node);
 #pragma unroll
     for (int k = 0; k < GAL_NPARAM_NODE; ++k) C[(kXClaimPar + k) * kGroupNodes] = np[k * stride];
   };
   C[kXClaimNode * kGroupNodes] = (double)kNoClaim;
   if constexpr (GRAPH) {
-    // claim an entry of the ready list, then wait for it to be written;
-    // events are applied on the spot and their successors released
+    // The operation that the lane's last one made ready, else a claimed entry
+    // of the ready list once it is written; events are applied on the spot.
+    // An entry is looked at here only by a group with nothing else to do: one
+    // with nodes under way read it during its last evaluation.
+    if (idle && c.pend >= 0) c.peek = graph_ready_entry(a.g, c.pend);
     bool again = true;
     while (again) {
-      const bool need = want && c.pend < 0;
+      const bool need = want && c.pend < 0 && c.next < 0;
       if (__any(need)) {
         const int j = wave_claim(need, a.work, a.g.n, nullptr);
         if (need) {
@@ -178,34 +184,47 @@ __device__ __forceinline__ void claim_nodes(const EvolveArgs& a, int n_claim, bo
             C[kXClaimNode * kGroupNodes] = (double)kExhausted;
           } else {
             c.pend = j;
-            c.wait_tail = ~0u;
+            c.peek = graph_ready_entry(a.g, j);
+            c.wait_progress = ~0ull;
           }
         }
       }
-      if (want && c.pend >= 0) {
-        const int k = graph_ready_entry(a.g, c.pend);
+      if (want) {
+        int k = c.next;
+        c.next = -1;
+        if (k < 0 && c.pend >= 0 && c.peek >= 0) {
+          k = c.peek;
+          c.pend = c.peek = -1;
+        }
         if (k >= 0) {
-          c.pend = -1;
           const gal_schedule_op* o = a.g.ops + k;
           const int kind = o->kind;
+          c.next_a = a.g.next_a[k];
+          c.next_b = a.g.next_b[k];
           if (kind != GAL_OP_EVOLVE) {
-            apply_event(kind, (size_t)o->a, (size_t)o->b, a.ld, a.y, a.h_step, a.g.major_ratio);
-            graph_release(a.g, k);
+            apply_event<true>(kind, (size_t)o->a, (size_t)o->b, a.ld, a.y, a.h_step, a.g.major_ratio);
+            stores_done();
+            c.next = graph_release(a.g, k, c.next_a, c.next_b);
           } else {
             c.op = k;
             publish(o->a, o->t0, o->t1, o->node_par, 1);
             want = false;
           }
-        } else {
-          const unsigned int tl = __hip_atomic_load(a.g.tail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        } else if (idle) {
+          const unsigned long long progress = graph_progress(a.g);
           const unsigned long long now = wall_clock64();
-          if (tl != c.wait_tail) {
-            c.wait_tail = tl;
+          // the list ends at what is never chained past it
+          bool over = c.pend >= a.g.n - (int)(progress >> 32);
+          if (progress != c.wait_progress) {
+            c.wait_progress = progress;
             c.wait_since = now;
           } else if (now - c.wait_since > a.stall_ticks) {
             __hip_atomic_store(a.graph_error, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            over = true;
+          }
+          if (over) {
             want = false;
-            c.pend = -1;
+            c.pend = c.peek = -1;
             C[kXClaimNode * kGroupNodes] = (double)kExhausted;
           }
         }
@@ -317,14 +336,14 @@ __device__ __forceinline__ void group_wave(const EvolveArgs& a, double* __restri
   // owners beforehand, and in graph mode its successors are released.
   auto finish = [&](bool done, double h_out, bool write_h, int status) {
     if (wave == kCoolingWave && done) {
-      if (write_h) a.h_step[node] = h_out;
-      a.status[node] = status;
-      write_counters(a, node, n_attempt, n_accept, n_rhs);
+      if (write_h) store_state_word<GRAPH>(a.h_step + node, h_out);
+      store_state_word<GRAPH>(a.status + node, status);
+      write_counters<GRAPH>(a, node, n_attempt, n_accept, n_rhs);
     }
     if constexpr (GRAPH) {
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+      stores_done();
       __syncthreads();
-      if (wave == kCoolingWave && done) graph_release(a.g, claim.op);
+      if (wave == kCoolingWave && done) claim.next = graph_release(a.g, claim.op, claim.next_a, claim.next_b);
     }
     if (done) {
       s.clear(LaneFlags::kActive);
@@ -394,7 +413,7 @@ __device__ __forceinline__ void group_wave(const EvolveArgs& a, double* __restri
       bool begun = false;
       while (__any(s.has(LaneFlags::kWant))) {
         double* C = time_vectors(tb ^ 1);
-        if (wave == kCoolingWave) claim_nodes<GRAPH>(a, n_claim, s.has(LaneFlags::kWant), claim, C);
+        if (wave == kCoolingWave) claim_nodes<GRAPH>(a, n_claim, s.has(LaneFlags::kWant), !__any(s.has(LaneFlags::kActive)), claim, C);
         __syncthreads();
         const int code = (int)C[kXClaimNode * kGroupNodes];
         begun = s.has(LaneFlags::kWant) && code >= 0;
@@ -424,7 +443,7 @@ __device__ __forceinline__ void group_wave(const EvolveArgs& a, double* __restri
       if (!__any(s.has(LaneFlags::kActive))) break;
       if (owner && s.has(LaneFlags::kFetch)) {
 #pragma unroll
-        for (int i = 0; i < kOwned; ++i) XY[i * kGroupNodes] = Y0(i) = a.y[(size_t)(v0 + i) * a.ld + node];
+        for (int i = 0; i < kOwned; ++i) XY[i * kGroupNodes] = Y0(i) = load_state_word<GRAPH>(a.y + (size_t)(v0 + i) * a.ld + node);
       }
       s.clear(LaneFlags::kFetch);
       // The time part of the derivative was computed ahead for lanes that go
@@ -445,7 +464,7 @@ __device__ __forceinline__ void group_wave(const EvolveArgs& a, double* __restri
         for (int i = 0; i < kOwned; ++i) {
           const double sc = mode == GAL_PHYSICS_TEST ? 1.0 : rounded(s30[v0 + i]);
           abs_tol[i] = a.eps_abs * sc;
-          if (a.scale) a.scale[(size_t)(v0 + i) * a.ld + node] = sc;
+          if (a.scale) store_state_word<GRAPH>(a.scale + (size_t)(v0 + i) * a.ld + node, sc);
         }
       }
     }
@@ -476,6 +495,7 @@ __device__ __forceinline__ void group_wave(const EvolveArgs& a, double* __restri
         if constexpr (wave == kCoolingWave) cooling_wave_rhs(G, a.tab, np, X, F, time_vectors(tb), flags, round);
       }
       if constexpr (wave == kCoolingWave) {
+        if (GRAPH && ph == kLast) claim.peek = graph_ready_entry(a.g, claim.pend >= 0 ? claim.pend : 0);
         if (ph == kFirst && a.wall_ticks && lane == 0) wall_expired = wall_clock64() - t_launch > a.wall_ticks;
       }
     }
@@ -553,7 +573,8 @@ __device__ __forceinline__ void group_wave(const EvolveArgs& a, double* __restri
           if (owner && rescued) {
 #pragma unroll
             for (int i = 0; i < kOwned; ++i)
-              a.y[(size_t)(v0 + i) * a.ld + node] = Y0(i) < 0.0 && ((nonneg >> i) & 1u) ? 0.0 : Y0(i);
+              store_state_word<GRAPH>(a.y + (size_t)(v0 + i) * a.ld + node,
+                                      Y0(i) < 0.0 && ((nonneg >> i) & 1u) ? 0.0 : Y0(i));
           }
           if (__any(rescued)) finish(rescued, h_node / (double)(1 << trial), true, GAL_STATUS_SUCCESS);
         }
@@ -656,7 +677,7 @@ __device__ __forceinline__ void group_wave(const EvolveArgs& a, double* __restri
         }
         if (owner && done) {
 #pragma unroll
-          for (int i = 0; i < kOwned; ++i) a.y[(size_t)(v0 + i) * a.ld + node] = yn[i];
+          for (int i = 0; i < kOwned; ++i) store_state_word<GRAPH>(a.y + (size_t)(v0 + i) * a.ld + node, yn[i]);
         }
         // odeSolverSolve returns xStep = driver h (solver.F90:593)
         double h_out = h;

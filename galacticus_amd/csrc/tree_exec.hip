@@ -57,7 +57,7 @@ __global__ void event_kernel(int n, const int* __restrict__ kind, const int* __r
                              double major_ratio) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  apply_event(kind[i], (size_t)from[i], (size_t)to[i], ld, y, h_step, major_ratio);
+  apply_event<false>(kind[i], (size_t)from[i], (size_t)to[i], ld, y, h_step, major_ratio);
 }
 
 // Compact copies of a wave's non-satellite evolve operations for the
@@ -379,7 +379,7 @@ int build_device_graph(const gal_schedule& sc, int device, hipStream_t s, Device
   g.ready0 = upload(ready, s, ok);
   ok = ok && hipMalloc(&g.npred, sizeof(int) * (size_t)n_all) == hipSuccess &&
        hipMalloc(&g.ready, sizeof(int) * ready.size()) == hipSuccess &&
-       hipMalloc(&g.err, sizeof(int)) == hipSuccess && hipMalloc(&g.tail, sizeof(unsigned int)) == hipSuccess;
+       hipMalloc(&g.err, sizeof(int)) == hipSuccess && hipMalloc(&g.tail, 2 * sizeof(unsigned int)) == hipSuccess;
   // the host vectors are released on return: the copies must have landed
   if (hipStreamSynchronize(s) != hipSuccess) return GAL_E_HIP;
   return ok ? GAL_OK : GAL_E_NOMEM;
@@ -413,7 +413,8 @@ __global__ void graph_reset_kernel(int n_all, const int* __restrict__ npred0, in
   if (i < n) ready[i] = ready0[i];
   if (i < ld) h[i] = -1.0;
   if (i == 0) {
-    *tail = r0;
+    tail[0] = r0;
+    tail[1] = 0u;
     *err = 0;
   }
 }
@@ -460,13 +461,13 @@ static int tree_evolve_graph(gal_ode_batch* h, const gal_schedule* sched_c, int 
   if (hipStreamSynchronize(s) != hipSuccess && rc == GAL_OK) rc = GAL_E_HIP;
   if (rc == GAL_OK) {
     int err = 0;
-    unsigned int appended = 0;
+    unsigned int reached[2] = {0, 0};   // appended to the ready list, and chained past it
     if (hipMemcpy(&err, dg->err, sizeof(err), hipMemcpyDeviceToHost) != hipSuccess ||
-        hipMemcpy(&appended, dg->tail, sizeof(appended), hipMemcpyDeviceToHost) != hipSuccess) {
+        hipMemcpy(reached, dg->tail, sizeof(reached), hipMemcpyDeviceToHost) != hipSuccess) {
       rc = GAL_E_HIP;
-    } else if (err != 0 || appended != (unsigned int)dg->n) {
-      fprintf(stderr, "gal_tree_evolve_d: the operation graph stopped with %u of %d operations ready\n", appended,
-              dg->n);
+    } else if (err != 0 || reached[0] + reached[1] != (unsigned int)dg->n) {
+      fprintf(stderr, "gal_tree_evolve_d: the operation graph stopped with %u of %d operations ready\n",
+              reached[0] + reached[1], dg->n);
       rc = GAL_E_HIP;
     }
   }

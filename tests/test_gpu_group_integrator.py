@@ -1,10 +1,12 @@
 """The integrator's groups of 64 nodes, partial and full.  The nodes of a
 group share barriers, flags and LDS but no arithmetic, so a node's results are
-the same to the last bit in any lane and beside any other nodes."""
+the same to the last bit in any lane and beside any other nodes; and a
+forest's operations give the same state whichever lane runs them, chained or
+claimed."""
 import numpy as np
 import pytest
 
-from galacticus_amd import params as gp, workloads as wl
+from galacticus_amd import params as gp, trees as tr, workloads as wl
 from galacticus_amd.cooling import synthetic_cie_table
 
 pytestmark = pytest.mark.gpu
@@ -52,3 +54,31 @@ def test_results_do_not_depend_on_the_group(torch_cuda, n, kind, operators, opti
         for whole, part in zip(together, run(i)):
             assert torch_cuda.equal(whole[..., torch_cuda.from_numpy(i)], part)
     assert (together[2] == 0).all()
+
+
+@pytest.mark.parametrize("trees,resolution", [(1, 5.0e10), (1, 2.0e9), (3, 2.0e10), (90, 2.0e10), (300, 1.0e11)])
+def test_chained_operations_match_the_waves(torch_cuda, trees, resolution):
+    """A single branch, where every operation is chained to the one before; a
+    tree, where mergers leave the last to arrive with the successor; and more
+    trees than a group has lanes."""
+    torch = torch_cuda
+    from galacticus_amd.evolver import NodeEvolverBatched
+    physics = gp.physics_params()
+    cosmo = tr.cosmology(physics)
+    t0, t5 = (float(wl.scale_factor_to_cosmic_time(a)) for a in (1.0, 1.0 / 6.0))
+    forest = tr.Forest.build_pch(trees, np.geomspace(2.0e11, 2.0e12, trees), t0, cosmo,
+                                 tr.pch_params(resolution, t5), seed=trees)
+    walk = tr.walk_params(t0, merging_multiplier=0.2)
+    schedule = tr.Schedule(forest, cosmo, walk)
+    print("nodes", forest.n_nodes, "operations", schedule.n_ops, flush=True)
+    y0 = forest.initial_state(cosmo, walk)
+    ev = NodeEvolverBatched(forest.n_nodes, physics, synthetic_cie_table())
+    out = []
+    for executor in ("waves", "graph", "graph"):
+        y = torch.from_numpy(y0.copy()).cuda()
+        scale = torch.zeros_like(y)
+        status = tr.evolve_forest(ev, schedule, y, scale=scale, executor=executor)
+        torch.cuda.synchronize()
+        out.append((y.cpu(), scale.cpu(), status.cpu()))
+    for other in out[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(out[0], other))
