@@ -35,6 +35,7 @@ namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));  // in a caller's buffer of floats
 
 constexpr int kIn = GAL_MLP_INPUTS, kHid = GAL_MLP_HIDDEN, kOut = GAL_MLP_OUTPUTS, kOutLd = GAL_MLP_OUT_LD;
 constexpr int kLayers = 4;
@@ -50,14 +51,40 @@ constexpr int64_t param_count() {
 constexpr int64_t kParams = param_count();
 
 // ---- bf16 ------------------------------------------------------------------
-__device__ __forceinline__ uint16_t f2bf(float f) {  // round to nearest even; NaN stays quiet NaN
-  const uint32_t u = __float_as_uint(f);
-  const uint32_t rounded = (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
-  const uint32_t quiet = (u >> 16) | 0x40u;
-  return (uint16_t)(((u & 0x7fffffffu) > 0x7f800000u) ? quiet : rounded);   // a select, not a branch
+// round to nearest even; NaN stays quiet NaN (v_cvt_pk_bf16_f32)
+__device__ __forceinline__ uint16_t f2bf(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
+// two or four values in one instruction each two
+__device__ __forceinline__ uint32_t f2bf2(float a, float b) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), bf16x2));
 }
+__device__ __forceinline__ uint2 f2bf4(f32x4 v) { return make_uint2(f2bf2(v[0], v[1]), f2bf2(v[2], v[3])); }
 __device__ __forceinline__ float bf2f(uint16_t b) { return __uint_as_float(((uint32_t)b) << 16); }
-__device__ __forceinline__ float silu(float z) { return z / (1.0f + __expf(-z)); }
+
+// SiLU, z / (1 + exp(-z)).  The network's epilogues are bound by vector
+// instructions, and an IEEE division is eleven of them with two changes of
+// the denormal mode.  The quotient from the hardware reciprocal and one
+// residual correction is four: q = z r, q + r (z - d q), where the residual
+// is exact in one fma, so the result is the correctly rounded quotient but
+// for ties within 2^-46.  That holds while d = 1 + exp(-z) and z are far
+// from the ends of the range; beyond |z| = 80 (and for infinities, where the
+// residual would be NaN) silu_far divides.  A NaN takes either to NaN.
+constexpr float kSiluNear = 80.0f;
+__device__ __forceinline__ float silu_near(float z) {
+  const float d = 1.0f + __expf(-z);
+  const float r = __builtin_amdgcn_rcpf(d);
+  const float q = z * r;
+  return fmaf(fmaf(-d, q, z), r, q);
+}
+__device__ __forceinline__ float silu_far(float z) { return z / (1.0f + __expf(-z)); }
+__device__ __forceinline__ float silu(float z) {   // both, and a select
+  const float near = silu_near(z), far = silu_far(z);
+  return fabsf(z) > kSiluNear ? far : near;
+}
+__device__ __forceinline__ float abs_max4(f32x4 z) {
+  return fmaxf(fmaxf(fabsf(z[0]), fabsf(z[1])), fmaxf(fabsf(z[2]), fabsf(z[3])));
+}
 __device__ __forceinline__ float dsilu(float z) {
   const float s = 1.0f / (1.0f + __expf(-z));
   return s * (1.0f + z * (1.0f - s));
@@ -166,17 +193,36 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs g) {
       }
 }
 
+// ---- weights in fragment order ------------------------------------------------
+// The fused kernels read a wave's MFMA operand of weights, 16 columns x 32 k
+// with eight consecutive k per lane, as one contiguous KiB: fragment
+// (c / 16, k / 32), lane 16 (k / 8 mod 4) + c mod 16, element k mod 8.  From
+// rows of 512 bytes the same operand touches 16 cache lines and uses half of
+// each.
+__host__ __device__ constexpr size_t frag_offset(int c, int k, int n_k) {
+  return ((size_t)(c / 16) * (n_k / 32) + k / 32) * 512 + ((k / 8) % 4 * 16 + c % 16) * 8 + k % 8;
+}
+
 // ---- fused inference forward ---------------------------------------------
 // The whole network for 128 rows per workgroup in one kernel: the rows'
 // activations stay in LDS from layer to layer (76 KiB, so two workgroups
 // share a CU).  Wave w computes all 128 rows x columns [64w, 64w+64) of a
 // hidden layer (8 x 4 tiles of 16 x 16); for the 32-column output layer waves
 // 0 and 1 take one column tile each.  A wave's columns are its own, so it
-// reads its weight fragments straight from the transposed bf16 weights
-// ([n][k], k contiguous) into registers, four k chunks at a time, with no LDS
-// staging and no workgroup barrier inside a layer.  The arithmetic is the
-// per-layer GEMMs' (same MFMA, same k order, same bias + SiLU epilogue and
-// bf16 rounding), so the outputs are bit-identical to them.
+// reads its weight fragments straight from memory in fragment order into
+// registers, four k chunks at a time, with no LDS staging and no workgroup
+// barrier inside a layer.  The weights are the MFMA's A operand, so a lane
+// ends with four consecutive columns of one row: it adds one bias vector,
+// rounds two values per instruction and writes 8 bytes to LDS (16 to the
+// output).  The arithmetic is the per-layer GEMMs' (same products, same k
+// order, same bias + SiLU epilogue and bf16 rounding), so the outputs are
+// bit-identical to them.
+// Bound by the epilogue's vector instructions, about 15 issue slots for each
+// activation beside 16 x 16 x 32 products that take 40 % as long.  500,000
+// rows with their output buffer took 420 us with an IEEE division, the bf16
+// rounding in integer instructions, two-byte LDS writes, weights read from
+// transposed rows (copied anew in each call) and a launch for every 131,072
+// rows; 260 us as it is here.
 constexpr int FR = 128;                 // rows per workgroup
 constexpr int LDH = kHid + 8;           // activation row stride (bf16)
 constexpr int LDX = kIn + 8;            // input row stride (bf16)
@@ -184,7 +230,7 @@ constexpr size_t kFusedLds = sizeof(uint16_t) * ((size_t)FR * LDH + (size_t)FR *
 
 struct FusedArgs {
   const uint16_t* x;                 // [n][kIn] bf16
-  const uint16_t* wt[kLayers];       // [kLdW[l]][kFanIn[l]] bf16
+  const uint16_t* wf[kLayers];       // bf16, fragment order: frag_offset(n, k, kFanIn[l])
   const float* bias[kLayers];
   float* out;                        // [n][kOutLd]
   int n;
@@ -199,7 +245,7 @@ __device__ __forceinline__ void fused_layer(const FusedArgs& a, int l, const uin
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const bool active = LAST ? wave < 2 : true;
   const int nbase = LAST ? wave * 16 : wave * 64;
-  const uint16_t* __restrict__ wt = a.wt[l];
+  const uint16_t* __restrict__ wf = a.wf[l] + (size_t)(nbase / 16) * NK * 512 + lane * 8;
   f32x4 acc[8][JT];
 #pragma unroll
   for (int i = 0; i < 8; ++i)
@@ -212,8 +258,7 @@ __device__ __forceinline__ void fused_layer(const FusedArgs& a, int l, const uin
       for (int kk = 0; kk < KG; ++kk)
 #pragma unroll
         for (int j = 0; j < JT; ++j)
-          bq[kk][j] = *reinterpret_cast<const uint4*>(wt + (size_t)(nbase + j * 16 + (lane & 15)) * K +
-                                                      (g0 + kk) * TK + (lane >> 4) * 8);
+          bq[kk][j] = *reinterpret_cast<const uint4*>(wf + (size_t)(j * NK + g0 + kk) * 512);
 #pragma unroll
       for (int kk = 0; kk < KG; ++kk) {
 #pragma unroll
@@ -223,7 +268,7 @@ __device__ __forceinline__ void fused_layer(const FusedArgs& a, int l, const uin
           const bf16x8 av = __builtin_bit_cast(bf16x8, v);
 #pragma unroll
           for (int j = 0; j < JT; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, __builtin_bit_cast(bf16x8, bq[kk][j]), acc[i][j],
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, bq[kk][j]), av, acc[i][j],
                                                                 0, 0, 0);
         }
       }
@@ -232,22 +277,53 @@ __device__ __forceinline__ void fused_layer(const FusedArgs& a, int l, const uin
   // every wave has read this layer's input before any epilogue overwrites H
   __syncthreads();
   if (!active) return;
+  // column nbase + 16 j + 4 (lane / 16) + r of row 16 i + lane mod 16
+  const int c0 = nbase + (lane >> 4) * 4;
   const float* __restrict__ bias = a.bias[l];
+  f32x4 b[JT];
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int j = 0; j < JT; ++j)
 #pragma unroll
-    for (int j = 0; j < JT; ++j)
+    for (int r = 0; r < 4; ++r) b[j][r] = bias[LAST ? min(c0 + r, kOut - 1) : c0 + j * 16 + r];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = i * 16 + (lane >> 4) * 4 + r;
-        const int col = nbase + j * 16 + (lane & 15);
-        const float z = acc[i][j][r] + bias[LAST ? (col < kOut ? col : 0) : col];
-        if (LAST) {
-          if (col < kOut && r0 + row < a.n) a.out[(size_t)(r0 + row) * kOutLd + col] = z;
-        } else {
-          H[row * LDH + col] = f2bf(silu(z));
+  for (int i = 0; i < 8; ++i) {
+    const int row = i * 16 + (lane & 15);
+    if (LAST) {
+      if (r0 + row >= a.n) continue;
+      const f32x4 z = acc[i][0] + b[0];
+      float* o = a.out + (size_t)(r0 + row) * kOutLd + c0;
+      if (c0 + 3 < kOut) {
+        *reinterpret_cast<f32x4_a4*>(o) = z;
+      } else {
+        o[0] = z[0]; o[1] = z[1]; o[2] = z[2];
+      }
+    } else {
+      float far = 0.0f;
+#pragma unroll
+      for (int j = 0; j < JT; ++j) {
+        acc[i][j] += b[j];
+        far = fmaxf(far, abs_max4(acc[i][j]));
+      }
+      uint16_t* h = H + row * LDH + c0;
+      if (__builtin_expect(__any(far > kSiluNear), 0)) {   // uniform: the rare block lies apart
+#pragma unroll
+        for (int j = 0; j < JT; ++j) {
+          f32x4 v;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) v[r] = silu(acc[i][j][r]);
+          *reinterpret_cast<uint2*>(h + j * 16) = f2bf4(v);
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < JT; ++j) {
+          f32x4 v;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) v[r] = silu_near(acc[i][j][r]);
+          *reinterpret_cast<uint2*>(h + j * 16) = f2bf4(v);
         }
       }
+    }
+  }
 }
 
 __global__ __launch_bounds__(256, 2) void mlp_forward_fused(FusedArgs a) {
@@ -266,20 +342,12 @@ __global__ __launch_bounds__(256, 2) void mlp_forward_fused(FusedArgs a) {
   __syncthreads();
   fused_layer<kIn, false>(a, 0, X, LDX, H, r0);
   __syncthreads();
-  fused_layer<kHid, false>(a, 1, H, LDH, H, r0);
-  __syncthreads();
-  fused_layer<kHid, false>(a, 2, H, LDH, H, r0);
-  __syncthreads();
+#pragma unroll 1
+  for (int l = 1; l < 3; ++l) {   // one copy of the layer's code in the instruction cache
+    fused_layer<kHid, false>(a, l, H, LDH, H, r0);
+    __syncthreads();
+  }
   fused_layer<kHid, true>(a, 3, H, LDH, H, r0);
-}
-
-// Transposed bf16 copy of one layer's weights: wt[n][k] = wbf[k][n].
-__global__ __launch_bounds__(256) void transpose_weights_kernel(const uint16_t* __restrict__ wbf, int K, int N,
-                                                                uint16_t* __restrict__ wt) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= K * N) return;
-  const int k = e / N, n = e % N;
-  wt[(size_t)n * K + k] = wbf[e];
 }
 
 // ---- training support kernels ----------------------------------------------
@@ -358,6 +426,7 @@ struct AdamArgs {
   float* m;
   float* v;
   uint16_t* wbf[kLayers];
+  uint16_t* wf[kLayers];
   float* grad_out;
   const float* pw;
   const float* pb;
@@ -370,7 +439,7 @@ struct AdamArgs {
 };
 
 // Sum the split partials into the gradient (fixed order) and take one Adam
-// step; keeps the bf16 copy of each weight in step with its fp32 master.
+// step; keeps the bf16 copies of each weight in step with its fp32 master.
 __global__ __launch_bounds__(256) void adam_kernel(AdamArgs a) {
   const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= kParams) return;
@@ -404,15 +473,21 @@ __global__ __launch_bounds__(256) void adam_kernel(AdamArgs a) {
   a.v[p] = v;
   const float w = a.param[p] - lr * (m / bc1) / (sqrtf(v / bc2) + a.eps);
   a.param[p] = w;
-  if (!is_b) a.wbf[l][(size_t)k * kLdW[l] + n] = f2bf(w);
+  if (!is_b) {
+    const uint16_t b = f2bf(w);
+    a.wbf[l][(size_t)k * kLdW[l] + n] = b;
+    a.wf[l][frag_offset(n, k, kFanIn[l])] = b;
+  }
 }
 
 __global__ void weights_to_bf16_kernel(const float* __restrict__ param, int64_t w_off, int fan_in, int fan_out,
-                                       int ldw, uint16_t* __restrict__ wbf) {
+                                       int ldw, uint16_t* __restrict__ wbf, uint16_t* __restrict__ wf) {
   const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= (int64_t)fan_in * fan_out) return;
   const int k = (int)(q / fan_out), n = (int)(q % fan_out);
-  wbf[(size_t)k * ldw + n] = f2bf(param[w_off + q]);
+  const uint16_t b = f2bf(param[w_off + q]);
+  wbf[(size_t)k * ldw + n] = b;
+  wf[frag_offset(n, k, fan_in)] = b;
 }
 
 __global__ void gather_kernel(const uint16_t* __restrict__ ds_x, const float* __restrict__ ds_t,
@@ -779,7 +854,7 @@ struct gal_mlp {
   float* d_m = nullptr;
   float* d_v = nullptr;
   uint16_t* d_wbf[kLayers] = {};
-  uint16_t* d_wt[kLayers] = {};   // transposed bf16 weights for the fused inference kernel
+  uint16_t* d_wf[kLayers] = {};   // the same in fragment order, columns as operand rows (forward)
   uint16_t* d_x = nullptr;
   float* d_t = nullptr;
   uint16_t* d_z[3] = {};
@@ -919,6 +994,7 @@ AdamArgs adam_args(gal_mlp* m, int n, float* grad_out, int apply) {
   a.param = m->d_param; a.m = m->d_m; a.v = m->d_v;
   for (int l = 0; l < kLayers; ++l) {
     a.wbf[l] = m->d_wbf[l];
+    a.wf[l] = m->d_wf[l];
     a.w_off[l] = m->w_off[l]; a.b_off[l] = m->b_off[l]; a.pw_off[l] = m->pw_off[l]; a.pb_off[l] = m->pb_off[l];
   }
   const int rps = ((n + m->splits - 1) / m->splits + TK - 1) / TK * TK;
@@ -978,19 +1054,13 @@ int infer_layers(gal_mlp* m, int n, const uint16_t* x, float* out, hipStream_t s
   return forward(m, n, x, nullptr, h, out, s);
 }
 
-// Refresh the transposed weights from the current bf16 weights.
-int prepare_fused(gal_mlp* m, hipStream_t s) {
-  // the LDS limit of the kernel on the current device (a cheap host call; no
-  // process-wide state)
+// The LDS limit of the fused kernel on the current device (a cheap host call;
+// no process-wide state).
+int prepare_fused() {
   static_assert(kFusedLds <= 163840, "fused forward LDS must fit a CU");
   HIP_TRY(hipFuncSetAttribute((const void*)mlp_forward_fused, hipFuncAttributeMaxDynamicSharedMemorySize,
                               (int)kFusedLds));
-  for (int l = 0; l < kLayers; ++l) {
-    const int e = kFanIn[l] * kLdW[l];
-    hipLaunchKernelGGL(transpose_weights_kernel, dim3((e + 255) / 256), dim3(256), 0, s, m->d_wbf[l], kFanIn[l],
-                       kLdW[l], m->d_wt[l]);
-  }
-  return hipGetLastError() == hipSuccess ? GAL_OK : GAL_E_HIP;
+  return GAL_OK;
 }
 
 // The fused one-kernel forward (after prepare_fused).
@@ -998,7 +1068,7 @@ int infer(gal_mlp* m, int n, const uint16_t* x, float* out, hipStream_t s) {
   if (n <= 0) return GAL_OK;
   FusedArgs a{};
   a.x = x;
-  for (int l = 0; l < kLayers; ++l) { a.wt[l] = m->d_wt[l]; a.bias[l] = m->d_param + m->b_off[l]; }
+  for (int l = 0; l < kLayers; ++l) { a.wf[l] = m->d_wf[l]; a.bias[l] = m->d_param + m->b_off[l]; }
   a.out = out;
   a.n = n;
   hipLaunchKernelGGL(mlp_forward_fused, dim3((n + FR - 1) / FR), dim3(256), kFusedLds, s, a);
@@ -1045,7 +1115,7 @@ int gal_mlp_create(int batch, gal_mlp** out) {
             hipMalloc(&m->d_local, sizeof(int)) == hipSuccess;
   for (int l = 0; l < kLayers && ok; ++l)
     ok = hipMalloc(&m->d_wbf[l], sizeof(uint16_t) * kFanIn[l] * kLdW[l]) == hipSuccess &&
-         hipMalloc(&m->d_wt[l], sizeof(uint16_t) * kFanIn[l] * kLdW[l]) == hipSuccess;
+         hipMalloc(&m->d_wf[l], sizeof(uint16_t) * kFanIn[l] * kLdW[l]) == hipSuccess;
   for (int l = 0; l < 3 && ok; ++l)
     ok = hipMalloc(&m->d_z[l], sizeof(uint16_t) * kHid * B) == hipSuccess &&
          hipMalloc(&m->d_h[l], sizeof(uint16_t) * kHid * B) == hipSuccess;
@@ -1062,7 +1132,8 @@ int gal_mlp_create(int batch, gal_mlp** out) {
          hipMemset(m->d_step, 0, sizeof(long long)) == hipSuccess &&
          hipMemset(m->d_dout, 0, sizeof(uint16_t) * kOutLd * B) == hipSuccess;
     for (int l = 0; l < kLayers && ok; ++l)
-      ok = hipMemset(m->d_wbf[l], 0, sizeof(uint16_t) * kFanIn[l] * kLdW[l]) == hipSuccess;
+      ok = hipMemset(m->d_wbf[l], 0, sizeof(uint16_t) * kFanIn[l] * kLdW[l]) == hipSuccess &&
+           hipMemset(m->d_wf[l], 0, sizeof(uint16_t) * kFanIn[l] * kLdW[l]) == hipSuccess;
     ok = ok && hipDeviceSynchronize() == hipSuccess;
   }
   if (!ok) {
@@ -1079,7 +1150,7 @@ int gal_mlp_destroy(gal_mlp* m) {
   if (!m) return GAL_OK;
   release_graph(m);
   hipFree(m->d_param); hipFree(m->d_m); hipFree(m->d_v);
-  for (int l = 0; l < kLayers; ++l) { hipFree(m->d_wbf[l]); hipFree(m->d_wt[l]); }
+  for (int l = 0; l < kLayers; ++l) { hipFree(m->d_wbf[l]); hipFree(m->d_wf[l]); }
   hipFree(m->d_x); hipFree(m->d_t);
   for (int l = 0; l < 3; ++l) { hipFree(m->d_z[l]); hipFree(m->d_h[l]); }
   hipFree(m->d_out); hipFree(m->d_dout); hipFree(m->d_dz[0]); hipFree(m->d_dz[1]);
@@ -1103,7 +1174,7 @@ int gal_mlp_set_params(gal_mlp* m, const float* params, int64_t n) {
   for (int l = 0; l < kLayers; ++l) {
     const int64_t cnt = (int64_t)kFanIn[l] * kFanOut[l];
     hipLaunchKernelGGL(weights_to_bf16_kernel, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, 0,
-                       (const float*)m->d_param, m->w_off[l], kFanIn[l], kFanOut[l], kLdW[l], m->d_wbf[l]);
+                       (const float*)m->d_param, m->w_off[l], kFanIn[l], kFanOut[l], kLdW[l], m->d_wbf[l], m->d_wf[l]);
   }
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipDeviceSynchronize());
@@ -1151,9 +1222,9 @@ int gal_mlp_set_loss(gal_mlp* m, const float* var_weight, const float* target_si
 int gal_mlp_forward_d(gal_mlp* m, int64_t n, const uint16_t* x, float* out, void* stream) {
   if (!m || n < 0 || (n > 0 && (!x || !out))) return GAL_E_INVALID;
   hipStream_t s = (hipStream_t)stream;
-  const int chunk = (int)std::min<int64_t>(n, kInferChunk);
+  constexpr int64_t chunk = 1 << 30;   // rows of one launch: a grid of 32-bit size
   if (n == 0) return GAL_OK;
-  GAL_TRY(prepare_fused(m, s));
+  GAL_TRY(prepare_fused());
   for (int64_t c0 = 0; c0 < n; c0 += chunk) {
     const int nc = (int)std::min<int64_t>(chunk, n - c0);
     GAL_TRY(infer(m, nc, x + c0 * kIn, out + c0 * kOutLd, s));
@@ -1303,7 +1374,7 @@ int gal_surrogate_evolve_d(gal_ode_batch* h, gal_mlp* m, const float* norm, cons
   if (!m->d_rej_count) HIP_TRY(hipMalloc(&m->d_rej_count, sizeof(int)));
   const int chunk = std::min(n, kInferChunk);
   GAL_TRY(ensure_inference(m, chunk));
-  GAL_TRY(prepare_fused(m, s));
+  GAL_TRY(prepare_fused());
   HIP_TRY(hipMemsetAsync(m->d_rej_count, 0, sizeof(int), s));
   for (int c0 = 0; c0 < n; c0 += chunk) {
     const int nc = std::min(chunk, n - c0);

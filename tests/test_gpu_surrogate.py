@@ -99,6 +99,38 @@ def test_fused_forward_equals_layer_path(torch_cuda):
         assert bool(torch.isfinite(fused[:, :31]).all())
 
 
+@pytest.mark.parametrize("n", [1, 127, 129])
+def test_activation_over_its_whole_range(torch_cuda, n):
+    """Layer 1 puts chosen pre-activations into the units, identity layers carry them to the outputs: three SiLUs
+    and roundings.  Each rounding is half a bf16 ulp (2^-9) and SiLU's relative slope is below 2 for these values
+    or its result below 1e-30; beyond |z| = 80 the kernels take the division instead of the reciprocal."""
+    torch = torch_cuda
+    from galacticus_amd.surrogate import SurrogateMLP, FAN_IN, FAN_OUT
+    v = np.array([-1e30, -1e4, -200.0, -95.0, -88.5, -87.0, -80.5, -80.0, -79.5, -40.0, -17.0, -8.0, -3.0, -1.0, -0.25,
+                  -1e-3, -1e-20, 0.0, 1e-20, 1e-3, 0.25, 1.0, 3.0, 17.0, 79.5, 80.0, 80.5, 95.0, 300.0, 1e4, 1e30],
+                 dtype=np.float32)
+    bias = np.zeros(256, dtype=np.float32)
+    bias[:31] = v
+    parts = []
+    for l, (a, b) in enumerate(zip(FAN_IN, FAN_OUT)):
+        w = np.zeros((a, b), dtype=np.float32) if l == 0 else np.eye(a, b, dtype=np.float32)
+        parts += [w.ravel(), bias if l == 0 else np.zeros(b, dtype=np.float32)]
+    m = SurrogateMLP(256, params=np.concatenate(parts))
+    x = _bits(torch, om.bf16(np.random.default_rng(3).normal(0, 1, (n, 32)).astype(np.float32)))
+    fused, layers = m.forward(x)[:, :31], m.forward(x, layers=True)[:, :31]
+    ref = v.astype(np.float64)
+    with np.errstate(over="ignore"):
+        for _ in range(3):
+            ref = ref / (1.0 + np.exp(-ref))
+    assert torch.equal(fused, layers)
+    err = np.abs(fused.cpu().numpy() - ref)
+    assert (err <= (1 + 2 + 4) * 2.0 ** -9 * np.abs(ref) + 1e-30).all(), err.max(axis=0)
+    p = m.get_params()
+    p[32 * 256] = np.nan                                       # a NaN reaches every output it takes part in
+    m.set_params(p)
+    assert bool(torch.isnan(m.forward(x)[:, :31]).all())
+
+
 def test_gradient_matches_oracle(torch_cuda):
     torch = torch_cuda
     m, p = _net()
