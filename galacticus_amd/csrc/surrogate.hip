@@ -3,18 +3,15 @@
 // and gate kernels, and the surrogate evolve that routes rejected nodes to
 // the FP64 integrator.  C ABI of include/gal_surrogate.h.
 //
-// Matrix products.  One kernel template computes C = A B for the three
-// shapes of training: activations x weights (forward), gradients x W^T
-// (backward through a layer) and activations^T x gradients (weight
-// gradients, split over the batch so that every split writes its own fp32
-// partial sum; the Adam kernel adds the partials in a fixed order, so
-// training is deterministic).  Each 256-thread workgroup owns a 64 x 64 tile
-// of C, each of its four waves a 32 x 32 quarter, built from 2 x 2
-// v_mfma_f32_16x16x32_bf16 tiles with fp32 accumulators.  Operand tiles of
-// 64 x 32 are staged in LDS as [row][k] with a padded row stride, so that
-// each lane reads its eight consecutive k values with one 16-byte load.
-// Epilogues fuse the bias, SiLU and the bf16 rounding of the activations
-// (forward) and the SiLU derivative (backward).
+// Matrix products are v_mfma_f32_16x16x32_bf16 tiles with fp32 accumulators.
+// Inference runs the four layers in one kernel (mlp_forward_fused), a training
+// step is three launches (train_rows_kernel, train_weights_kernel,
+// adam_kernel).  Weight gradients are split over the batch, every split writes
+// its own fp32 partial sum and the Adam kernel adds them in a fixed order, so
+// training is deterministic.  gemm_kernel is the plain layer by layer product
+// that the fused forward is compared with: each 256-thread workgroup owns a
+// 64 x 64 tile, each of its four waves a 32 x 32 quarter, operand tiles of
+// 64 x 32 staged in LDS as [row][k].
 #include <hip/hip_runtime.h>
 #include <cstdint>
 #include <cstdio>
@@ -85,66 +82,53 @@ __device__ __forceinline__ float silu(float z) {   // both, and a select
 __device__ __forceinline__ float abs_max4(f32x4 z) {
   return fmaxf(fmaxf(fabsf(z[0]), fabsf(z[1])), fmaxf(fabsf(z[2]), fabsf(z[3])));
 }
+// Its derivative, with the same two forms of the logistic function.
+template <bool FAR>
 __device__ __forceinline__ float dsilu(float z) {
-  const float s = 1.0f / (1.0f + __expf(-z));
+  const float d = 1.0f + __expf(-z);
+  const float r = __builtin_amdgcn_rcpf(d);
+  const float s = FAR && fabsf(z) > kSiluNear ? 1.0f / d : fmaf(fmaf(-d, r, 1.0f), r, r);
   return s * (1.0f + z * (1.0f - s));
 }
 
 // ---- MFMA GEMM ---------------------------------------------------------------
 constexpr int TM = 64, TN = 64, TK = 32, LDT = TK + 8;
-enum Epi { EPI_SILU = 0, EPI_LINEAR = 1, EPI_DSILU = 2, EPI_PARTIAL = 3 };
+enum Epi { EPI_SILU = 0, EPI_LINEAR = 1 };
 
 struct GemmArgs {
-  const uint16_t* A;  // A(m,k) = AT ? A[k*lda + m] : A[m*lda + k]
-  const uint16_t* B;  // B(k,n) = BT ? B[n*ldb + k] : B[k*ldb + n]
+  const uint16_t* A;  // [m][k], row stride lda
+  const uint16_t* B;  // [k][n], row stride ldb
   int M, N, K, lda, ldb, ldc;
   int n_valid;        // epilogue writes columns n < n_valid
-  int k_split;        // K rows per split (multiple of TK); grid.z splits
-  const float* bias;  // SILU, LINEAR
-  uint16_t* out_bf;   // SILU: activation; DSILU: gradient wrt pre-activation
-  uint16_t* z_bf;     // SILU: pre-activation (may be null)
-  const uint16_t* z_in;  // DSILU: pre-activation of this layer
-  float* out_f;       // LINEAR: output; PARTIAL: [split][M][ldc]
+  const float* bias;
+  uint16_t* out_bf;   // SILU: activation
+  float* out_f;       // LINEAR: output
 };
 
-template <bool AT, bool BT, int EPI>
+template <int EPI>
 __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs g) {
   __shared__ __attribute__((aligned(16))) uint16_t As[TM * LDT];
   __shared__ __attribute__((aligned(16))) uint16_t Bs[TN * LDT];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
   const int m0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
-  const int kbeg = blockIdx.z * g.k_split;
-  const int kend = min(g.K, kbeg + g.k_split);
   f32x4 acc[2][2];
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
-  for (int k0 = kbeg; k0 < kend; k0 += TK) {
-    if (!AT) {  // rows of A are contiguous in k
+  for (int k0 = 0; k0 < g.K; k0 += TK) {
+    {  // rows of A are contiguous in k
       const int r = tid >> 2, c = (tid & 3) * 8;
       uint4 v = zero;
-      if (m0 + r < g.M && k0 + c < kend) v = *reinterpret_cast<const uint4*>(g.A + (size_t)(m0 + r) * g.lda + k0 + c);
+      if (m0 + r < g.M && k0 + c < g.K) v = *reinterpret_cast<const uint4*>(g.A + (size_t)(m0 + r) * g.lda + k0 + c);
       *reinterpret_cast<uint4*>(As + r * LDT + c) = v;
-    } else {    // A^T: contiguous in m, transposed into LDS
-      const int kk = tid >> 3, c = (tid & 7) * 8;
-      uint4 v = zero;
-      if (k0 + kk < kend && m0 + c < g.M) v = *reinterpret_cast<const uint4*>(g.A + (size_t)(k0 + kk) * g.lda + m0 + c);
-      const uint16_t* e = reinterpret_cast<const uint16_t*>(&v);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) As[(c + j) * LDT + kk] = e[j];
     }
-    if (BT) {   // B^T rows are contiguous in k
-      const int r = tid >> 2, c = (tid & 3) * 8;
-      uint4 v = zero;
-      if (n0 + r < g.N && k0 + c < kend) v = *reinterpret_cast<const uint4*>(g.B + (size_t)(n0 + r) * g.ldb + k0 + c);
-      *reinterpret_cast<uint4*>(Bs + r * LDT + c) = v;
-    } else {    // B: contiguous in n, transposed into LDS
+    {  // B: contiguous in n, transposed into LDS
       const int kk = tid >> 3, c = (tid & 7) * 8;
       uint4 v = zero;
-      if (k0 + kk < kend && n0 + c < g.N) v = *reinterpret_cast<const uint4*>(g.B + (size_t)(k0 + kk) * g.ldb + n0 + c);
+      if (k0 + kk < g.K && n0 + c < g.N) v = *reinterpret_cast<const uint4*>(g.B + (size_t)(k0 + kk) * g.ldb + n0 + c);
       const uint16_t* e = reinterpret_cast<const uint16_t*>(&v);
 #pragma unroll
       for (int j = 0; j < 8; ++j) Bs[(c + j) * LDT + kk] = e[j];
@@ -179,17 +163,11 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs g) {
         if (m >= g.M || n >= g.n_valid) continue;
         const float c = acc[i][j][r];
         const size_t o = (size_t)m * g.ldc + n;
-        if (EPI == EPI_SILU) {
-          const float z = c + g.bias[n];
-          if (g.z_bf) g.z_bf[o] = f2bf(z);
+        const float z = c + g.bias[n];
+        if (EPI == EPI_SILU)
           g.out_bf[o] = f2bf(silu(z));
-        } else if (EPI == EPI_LINEAR) {
-          g.out_f[o] = c + g.bias[n];
-        } else if (EPI == EPI_DSILU) {
-          g.out_bf[o] = f2bf(c * dsilu(bf2f(g.z_in[o])));
-        } else {
-          g.out_f[((size_t)blockIdx.z * g.M + m) * g.ldc + n] = c;
-        }
+        else
+          g.out_f[o] = z;
       }
 }
 
@@ -354,71 +332,514 @@ __global__ __launch_bounds__(256, 2) void mlp_forward_fused(FusedArgs a) {
 // Network outputs enter sinh(); beyond +-20 they are clipped (sinh(20) = 2.4e8).
 constexpr float kOutClip = 20.0f;
 
-struct LossArgs {
-  const float* out;
+// ---- the training step: rows, weight gradients, Adam ---------------------------
+// Three launches make a step.  rows: forward, loss and the gradients with
+// respect to every pre-activation, 32 rows of the batch per workgroup, with
+// the activations in LDS and registers.  weights: all weight and bias
+// gradients as split partial sums.  Adam: the sums over the splits and the
+// update.  At 8192 rows they take 22 + 16 + 7.5 us.  A launch for each
+// product, sum and copy (18 of them, none of which fills the chip) took
+// 200 us.
+//
+// What rows leaves for weights is laid out in blocks of 32 rows,
+// [block][unit][32 rows]: a workgroup's block is written in one piece, and a
+// product over rows reads its MFMA operands (16 units x 32 rows) as contiguous
+// KiB, with no transposition through LDS.  Rows past the end of the batch are
+// zeros.
+constexpr int RB = 32;                   // rows per block: one k chunk of the weight gradients
+constexpr int kRowThreads = 512;         // wave w: hidden units [32w, 32w+32) of all 32 rows
+constexpr int LDF = kOutLd + 1;          // fp32 row stride of the output tile
+
+struct RowsArgs {
+  const uint16_t* x;                     // the rows, or the data set's rows when perm is set
   const float* target;
-  uint16_t* dout;
-  float* loss_partial;
-  int B;
+  const int* perm;
+  const long long* cursor;
+  long long ds_n;
+  int n;
+  const uint16_t* wf[kLayers];           // frag_offset(n, k, fan_in)
+  const uint16_t* wb[kLayers];           // frag_offset(k, n, padded fan_out)
+  const float* bias[kLayers];
+  uint16_t* xt;                          // [block][unit][32]: inputs,
+  uint16_t* ht[3];                       //   activations,
+  uint16_t* dzt[3];                      //   gradients wrt pre-activations,
+  uint16_t* dot;                         //   gradients wrt outputs
+  float* row_loss;
   float w[32], sigma[32];
   unsigned head_mask;
   float head_w, inv_wsum, inv_B;
 };
 
-__global__ __launch_bounds__(256) void loss_kernel(LossArgs a) {
-  __shared__ float red[256];
-  const int r = blockIdx.x * 256 + threadIdx.x;
-  float l = 0.0f;
-  if (r < a.B) {
-    const float* o = a.out + (size_t)r * kOutLd;
-    const float* t = a.target + (size_t)r * kOutLd;
-    uint16_t* d = a.dout + (size_t)r * kOutLd;
-    float mse = 0.0f, emax = 0.0f;
-    for (int v = 0; v < 30; ++v) {
-      const float res = o[v] - t[v];
-      mse += a.w[v] * res * res;
-      d[v] = f2bf(2.0f * a.w[v] * res * a.inv_wsum * a.inv_B);
-      // targets are asinh((r - m)/sigma) of the residual r: the error of the
-      // residual itself is sigma |sinh(o) - sinh(t)|
-      if ((a.head_mask >> v) & 1u)
-        emax = fmaxf(emax, a.sigma[v] * fabsf(sinhf(fminf(fmaxf(o[v], -kOutClip), kOutClip)) - sinhf(t[v])));
+// NK k chunks of a wave's 32 x 32 tile: rows of A (LDS) times its weights.
+template <int NK>
+__device__ __forceinline__ void rows_product(const uint16_t* __restrict__ A, int lda, const uint4 (&w)[NK][2],
+                                             f32x4 (&acc)[2][2]) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int kk = 0; kk < NK; ++kk)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const uint4 v = *reinterpret_cast<const uint4*>(A + (i * 16 + (lane & 15)) * lda + kk * TK + (lane >> 4) * 8);
+      const bf16x8 av = __builtin_bit_cast(bf16x8, v);
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, __builtin_bit_cast(bf16x8, w[kk][j]), acc[i][j],
+                                                            0, 0, 0);
     }
-    // a sample whose target was clipped carries a flag in column 31: its true
-    // error is at least 1 (asinh units), so the head learns to reject it
-    if (t[31] != 0.0f) emax = fmaxf(emax, 1.0f);
-    const float rh = o[GAL_MLP_HEAD] - logf(emax + 1.0e-7f);
-    l = mse * a.inv_wsum + a.head_w * rh * rh;
-    d[GAL_MLP_HEAD] = f2bf(2.0f * a.head_w * rh * a.inv_B);
-    d[31] = 0;
-  }
-  red[threadIdx.x] = l;
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) a.loss_partial[blockIdx.x] = red[0];
 }
 
-// Column sums of a bf16 gradient, one fp32 partial per batch split.  A
-// workgroup covers 64 columns of one split: each wave reads whole 128-byte
-// row segments (64 consecutive columns) of every fourth row, and the four
-// waves' sums are added in LDS in a fixed order (deterministic).
-__global__ __launch_bounds__(256) void colsum_kernel(const uint16_t* __restrict__ dz, int B, int N, int ld,
-                                                     int rows_per_split, float* __restrict__ partial) {
-  __shared__ float red[4][64];
-  const int col = threadIdx.x & 63, q = threadIdx.x >> 6;
-  const int n = blockIdx.x * 64 + col;
-  const int s = blockIdx.y;
-  const int r0 = s * rows_per_split, r1 = min(B, r0 + rows_per_split);
-  float acc = 0.0f;
-  if (n < N) {
-#pragma unroll 8
-    for (int r = r0 + q; r < r1; r += 4) acc += bf2f(dz[(size_t)r * ld + n]);
+// A wave's weight fragments of two adjacent 16-column tiles.
+template <int NK>
+__device__ __forceinline__ void rows_weights(const uint16_t* __restrict__ w, int tile, uint4 (&q)[NK][2]) {
+#pragma unroll
+  for (int kk = 0; kk < NK; ++kk)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      q[kk][j] = *reinterpret_cast<const uint4*>(w + (size_t)((tile + j) * NK + kk) * 512 + (threadIdx.x & 63) * 8);
+}
+
+__device__ __forceinline__ uint2 zero_past(uint2 v, int valid) {  // keep the first `valid` of four bf16
+  if (valid < 4) {
+    v.y = valid < 3 ? 0u : v.y & 0xffffu;
+    v.x = valid < 1 ? 0u : (valid < 2 ? v.x & 0xffffu : v.x);
   }
-  red[q][col] = acc;
+  return v;
+}
+
+// Four consecutive rows of one unit to the LDS tile (when a later layer reads
+// it) and to the block for the weight gradients.
+__device__ __forceinline__ void rows_store(uint2 v, uint16_t* __restrict__ tile, uint16_t* __restrict__ block, int row,
+                                           int unit, int valid_rows) {
+  if (tile) {
+    tile[(row + 0) * LDH + unit] = (uint16_t)v.x;
+    tile[(row + 1) * LDH + unit] = (uint16_t)(v.x >> 16);
+    tile[(row + 2) * LDH + unit] = (uint16_t)v.y;
+    tile[(row + 3) * LDH + unit] = (uint16_t)(v.y >> 16);
+  }
+  *reinterpret_cast<uint2*>(block + (size_t)unit * RB + row) = zero_past(v, valid_rows - row);
+}
+
+// Bias, SiLU and rounding of a hidden layer; z (bf16) stays for the backward.
+template <bool FAR>
+__device__ __forceinline__ void rows_activate(const f32x4 (&acc)[2][2], uint16_t* __restrict__ tile,
+                                              uint16_t* __restrict__ block, int valid_rows) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      f32x4 h;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) h[r] = FAR ? silu(acc[i][j][r]) : silu_near(acc[i][j][r]);
+      rows_store(f2bf4(h), tile, block, i * 16 + (lane >> 4) * 4, wave * 32 + j * 16 + (lane & 15), valid_rows);
+    }
+}
+
+__device__ __forceinline__ void rows_hidden(f32x4 (&acc)[2][2], const float (&bias)[2], uint2 (&z)[2][2],
+                                            uint16_t* __restrict__ tile, uint16_t* __restrict__ block,
+                                            int valid_rows) {
+  float far = 0.0f;
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      acc[i][j] += bias[j];
+      z[i][j] = f2bf4(acc[i][j]);
+      far = fmaxf(far, abs_max4(acc[i][j]));
+    }
+  if (__builtin_expect(__any(far > kSiluNear), 0))
+    rows_activate<true>(acc, tile, block, valid_rows);
+  else
+    rows_activate<false>(acc, tile, block, valid_rows);
+}
+
+// Gradient wrt a hidden layer's pre-activation.
+template <bool FAR>
+__device__ __forceinline__ void rows_chain(const f32x4 (&acc)[2][2], const f32x4 (&z)[2][2],
+                                           uint16_t* __restrict__ tile, uint16_t* __restrict__ block,
+                                           int valid_rows) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      f32x4 d;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) d[r] = acc[i][j][r] * dsilu<FAR>(z[i][j][r]);
+      rows_store(f2bf4(d), tile, block, i * 16 + (lane >> 4) * 4, wave * 32 + j * 16 + (lane & 15), valid_rows);
+    }
+}
+
+__device__ __forceinline__ void rows_gradient(const f32x4 (&acc)[2][2], const uint2 (&zq)[2][2],
+                                              uint16_t* __restrict__ tile, uint16_t* __restrict__ block,
+                                              int valid_rows) {
+  f32x4 z[2][2];
+  float far = 0.0f;
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const uint2 q = zq[i][j];
+      z[i][j] = f32x4{bf2f((uint16_t)q.x), bf2f((uint16_t)(q.x >> 16)), bf2f((uint16_t)q.y),
+                      bf2f((uint16_t)(q.y >> 16))};
+      far = fmaxf(far, abs_max4(z[i][j]));
+    }
+  if (__builtin_expect(__any(far > kSiluNear), 0))
+    rows_chain<true>(acc, z, tile, block, valid_rows);
+  else
+    rows_chain<false>(acc, z, tile, block, valid_rows);
+}
+
+// [unit][32 rows] of an LDS tile of 32 rows x 32 columns (threads 0..127).
+__device__ __forceinline__ void rows_transpose(const uint16_t* __restrict__ tile, uint16_t* __restrict__ block,
+                                               int valid_rows) {
+  const int u = threadIdx.x >> 2, r = (threadIdx.x & 3) * 8;
+  if (u >= 32) return;
+  uint32_t q[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const uint32_t lo = r + 2 * e < valid_rows ? tile[(r + 2 * e) * LDX + u] : 0u;
+    const uint32_t hi = r + 2 * e + 1 < valid_rows ? tile[(r + 2 * e + 1) * LDX + u] : 0u;
+    q[e] = lo | hi << 16;
+  }
+  *reinterpret_cast<uint4*>(block + u * RB + r) = make_uint4(q[0], q[1], q[2], q[3]);
+}
+
+// Bound by the serial chain of layers: eight waves share a layer's 256 units,
+// and each asks for the next layer's weights before it starts on this one's
+// products, so that memory is waited for once.  A workgroup's 570 KB of
+// weights come from the L2; 32 rows make 256 workgroups of a batch of 8192.
+__global__ __launch_bounds__(kRowThreads, 2) void train_rows_kernel(RowsArgs a) {
+  __shared__ __attribute__((aligned(16))) uint16_t X[RB * LDX];
+  __shared__ __attribute__((aligned(16))) uint16_t H[2][RB * LDH];
+  __shared__ float O[RB * LDF], R[RB * LDF];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const size_t blk = blockIdx.x;
+  const int r0 = blockIdx.x * RB;
+  const int valid = min(RB, a.n - r0);
+  uint16_t* const hb[3] = {a.ht[0] + blk * kHid * RB, a.ht[1] + blk * kHid * RB, a.ht[2] + blk * kHid * RB};
+  uint16_t* const db[3] = {a.dzt[0] + blk * kHid * RB, a.dzt[1] + blk * kHid * RB, a.dzt[2] + blk * kHid * RB};
+
+  // this thread's row of the batch: sixteen threads to a row
+  const int row = tid >> 4, c = tid & 15;
+  float2 t = make_float2(0.0f, 0.0f);
+  uint4 xv = make_uint4(0u, 0u, 0u, 0u);
+  if (row < valid) {
+    long long src = r0 + row;
+    if (a.perm) {
+      src += *a.cursor;
+      if (src >= a.ds_n) src %= a.ds_n;
+      src = a.perm[src];
+    }
+    if (c < 4) xv = *reinterpret_cast<const uint4*>(a.x + src * kIn + c * 8);
+    t.x = a.target[src * kOutLd + 2 * c];
+    t.y = a.target[src * kOutLd + 2 * c + 1];
+  }
+  // loads return in order: what is small and needed soon goes first
+  float b[3][2];
+#pragma unroll
+  for (int l = 0; l < 3; ++l)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) b[l][j] = a.bias[l][wave * 32 + j * 16 + (lane & 15)];
+  const int out_col = (wave & 1) * 16 + (lane & 15);           // of waves 0..3
+  const float b_out = a.bias[3][min(out_col, kOut - 1)];
+  const float2 vw = make_float2(a.w[2 * c], a.w[2 * c + 1]);
+  const float2 vs = make_float2(a.sigma[2 * c], a.sigma[2 * c + 1]);
+  uint4 w1[1][2], w2[8][2], w3[8][2], w4[8];
+  rows_weights(a.wf[0], wave * 2, w1);
+  rows_weights(a.wf[1], wave * 2, w2);
+  if (c < 4) *reinterpret_cast<uint4*>(X + row * LDX + c * 8) = xv;
   __syncthreads();
-  if (q == 0 && n < N) partial[(size_t)s * ld + n] = (red[0][col] + red[1][col]) + (red[2][col] + red[3][col]);
+  rows_transpose(X, a.xt + blk * kIn * RB, valid);
+  f32x4 acc[2][2];
+  uint2 z1[2][2], z2[2][2], z3[2][2];
+  rows_product(X, LDX, w1, acc);
+  rows_hidden(acc, b[0], z1, H[0], hb[0], valid);
+  __syncthreads();
+  rows_weights(a.wf[2], wave * 2, w3);
+  rows_product(H[0], LDH, w2, acc);
+  rows_hidden(acc, b[1], z2, H[1], hb[1], valid);
+  __syncthreads();
+  if (wave < 4) {  // the output layer: one 16 x 16 tile for each of four waves
+#pragma unroll
+    for (int kk = 0; kk < 8; ++kk)
+      w4[kk] = *reinterpret_cast<const uint4*>(a.wf[3] + (size_t)((wave & 1) * 8 + kk) * 512 + lane * 8);
+  }
+  rows_weights(a.wb[3], wave * 2, w1);
+  rows_product(H[1], LDH, w3, acc);
+  rows_hidden(acc, b[2], z3, H[0], hb[2], valid);
+  __syncthreads();
+  rows_weights(a.wb[2], wave * 2, w2);
+  if (wave < 4) {
+    const int i = wave >> 1;
+    f32x4 o = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int kk = 0; kk < 8; ++kk) {
+      const uint4 v = *reinterpret_cast<const uint4*>(H[0] + (i * 16 + (lane & 15)) * LDH + kk * TK + (lane >> 4) * 8);
+      o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, v), __builtin_bit_cast(bf16x8, w4[kk]), o,
+                                                  0, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) O[(i * 16 + (lane >> 4) * 4 + r) * LDF + out_col] = o[r] + b_out;
+  }
+  __syncthreads();
+  // The loss and its gradient, two variables per thread.  The error head's
+  // target is the row's largest error; the squares are added in the order of
+  // the variables by one thread per row.
+  {
+    const int v = 2 * c;
+    const float2 o = make_float2(O[row * LDF + v], O[row * LDF + v + 1]);
+    const float2 res = make_float2(o.x - t.x, o.y - t.y);
+    R[row * LDF + v] = res.x;
+    R[row * LDF + v + 1] = res.y;
+    const float t31 = __shfl(t.y, (lane & 48) | 15);
+    uint16_t* d = X + row * LDX;
+    float emax = 0.0f;
+    // targets are asinh((r - m)/sigma) of the residual r: the error of the
+    // residual itself is sigma |sinh(o) - sinh(t)|
+    if (c < 15) {
+      if ((a.head_mask >> v) & 1u)
+        emax = fmaxf(emax, vs.x * fabsf(sinhf(fminf(fmaxf(o.x, -kOutClip), kOutClip)) - sinhf(t.x)));
+      if ((a.head_mask >> (v + 1)) & 1u)
+        emax = fmaxf(emax, vs.y * fabsf(sinhf(fminf(fmaxf(o.y, -kOutClip), kOutClip)) - sinhf(t.y)));
+      d[v] = f2bf(2.0f * vw.x * res.x * a.inv_wsum * a.inv_B);
+      d[v + 1] = f2bf(2.0f * vw.y * res.y * a.inv_wsum * a.inv_B);
+    }
+#pragma unroll
+    for (int m = 8; m > 0; m >>= 1) emax = fmaxf(emax, __shfl_xor(emax, m));
+    // a sample whose target was clipped carries a flag in column 31: its true
+    // error is at least 1 (asinh units), so the head learns to reject it
+    if (t31 != 0.0f) emax = fmaxf(emax, 1.0f);
+    if (c == 15) {
+      const float rh = o.x - logf(emax + 1.0e-7f);
+      R[row * LDF + GAL_MLP_HEAD] = rh;
+      d[GAL_MLP_HEAD] = f2bf(2.0f * a.head_w * rh * a.inv_B);
+      d[31] = 0;
+    }
+  }
+  __syncthreads();
+  rows_transpose(X, a.dot + blk * kOutLd * RB, valid);
+  if (tid >= kRowThreads - RB) {  // the last wave's lanes: one per row
+    const int rr = tid - (kRowThreads - RB);
+    float mse = 0.0f;
+#pragma unroll
+    for (int v = 0; v < 30; ++v) {
+      const float res = R[rr * LDF + v];
+      mse += a.w[v] * res * res;
+    }
+    const float rh = R[rr * LDF + GAL_MLP_HEAD];
+    if (rr < valid) a.row_loss[r0 + rr] = mse * a.inv_wsum + a.head_w * rh * rh;
+  }
+  rows_product(X, LDX, w1, acc);
+  rows_gradient(acc, z3, H[1], db[2], valid);
+  __syncthreads();
+  rows_weights(a.wb[1], wave * 2, w3);
+  rows_product(H[1], LDH, w2, acc);
+  rows_gradient(acc, z2, H[0], db[1], valid);
+  __syncthreads();
+  rows_product(H[0], LDH, w3, acc);
+  rows_gradient(acc, z1, nullptr, db[0], valid);
+}
+
+// Weight gradients act^T . grad and bias gradients (column sums of grad) of
+// all layers, over one split of the rows each: partial[split][k][n].  A wave
+// owns a 32 x 32 tile, and a workgroup's four tiles share operands through
+// the L1.  A block of 32 rows is one k chunk, whose fragments are contiguous.
+// Consecutive workgroups take the same part of consecutive splits: with a
+// multiple of eight splits an XCD's L2 holds the splits it works on.
+constexpr int kWeightParts = 36;                       // workgroups per split for the products: 2 + 16 + 16 + 2
+constexpr int kBiasParts = 4;                         // and for the column sums, a layer each
+
+struct WeightArgs {
+  const uint16_t* act[kLayers];
+  const uint16_t* grad[kLayers];
+  float* pw[kLayers];
+  float* pb[kLayers];
+  int n, splits, rows_per_split;         // rows_per_split: a multiple of RB
+  // the step's loss, counters and learning rate (one further workgroup)
+  const float* row_loss;
+  float* loss_partial;
+  float inv_B;
+  float* loss;                           // null: a training step's loss_hist
+  float* loss_hist;
+  int hist_cap;
+  long long* step;
+  long long* cursor;
+  int* local;
+  int advance;
+  float lr0, lr_min, beta1, beta2;
+  int64_t total_steps;
+  float* rates;                          // lr and the two bias corrections of the step
+};
+
+// Sum of the rows' losses, 256 rows to a partial sum, and a training step's
+// counters.
+__device__ void finish_step(const WeightArgs& a) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int nb = (a.n + 255) / 256;
+  constexpr int G = 4;   // partial sums under way in a wave
+  for (int b0 = wave * G; b0 < nb; b0 += 4 * G) {
+    float v[G][4];
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int r = (b0 + g) * 256 + q * 64 + lane;
+        v[g][q] = a.row_loss[min(r, a.n - 1)];
+        if (r >= a.n) v[g][q] = 0.0f;
+      }
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      float s = (v[g][0] + v[g][2]) + (v[g][1] + v[g][3]);
+#pragma unroll
+      for (int m = 32; m > 0; m >>= 1) s += __shfl_xor(s, m);
+      if (lane == 0 && b0 + g < nb) a.loss_partial[b0 + g] = s;
+    }
+  }
+  __threadfence_block();
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    float s = 0.0f;
+#pragma unroll 8
+    for (int b = 0; b < nb; ++b) s += a.loss_partial[b];
+    if (a.loss) *a.loss = s * a.inv_B;
+    if (a.advance) {
+      const int ls = *a.local;
+      if (ls < a.hist_cap) a.loss_hist[ls] = s * a.inv_B;
+      *a.local = ls + 1;
+      *a.cursor += a.n;
+    }
+  }
+  if (a.advance && threadIdx.x == 64) {
+    const long long step = *a.step + 1;
+    *a.step = step;
+    const double t = (double)step;
+    const double frac = fmin(t, (double)a.total_steps) / (double)a.total_steps;
+    a.rates[0] = (float)(a.lr_min + 0.5 * (a.lr0 - a.lr_min) * (1.0 + cos(kPi * frac)));
+    a.rates[1] = (float)(1.0 - pow((double)a.beta1, t));
+    a.rates[2] = (float)(1.0 - pow((double)a.beta2, t));
+  }
+}
+
+__global__ __launch_bounds__(256) void train_weights_kernel(WeightArgs a) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (blockIdx.x == 0) {  // first: its chain of loads and sums is the longest
+    finish_step(a);
+    return;
+  }
+  const int part = (blockIdx.x - 1) / a.splits, split = (blockIdx.x - 1) % a.splits;
+  const int nblk = (a.n + RB - 1) / RB, per = a.rows_per_split / RB;
+  const int b0 = split * per, b1 = min(nblk, b0 + per);
+  if (part >= kWeightParts) {
+    // a unit per lane; the sums of the rows q, q + 4, ... are kept apart
+    int u = (part - kWeightParts) * 256 + threadIdx.x;
+    const int l = min(u / kHid, 3);
+    u -= l * kHid;
+    const int units = l == 3 ? kOutLd : kHid;
+    if (u >= units) return;
+    const uint16_t* g = a.grad[0];
+    float* pb = a.pb[0];
+    if (l == 1) { g = a.grad[1]; pb = a.pb[1]; }
+    if (l == 2) { g = a.grad[2]; pb = a.pb[2]; }
+    if (l == 3) { g = a.grad[3]; pb = a.pb[3]; }
+    float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 4
+    for (int b = b0; b < b1; ++b) {
+      const uint4* e = reinterpret_cast<const uint4*>(g + ((size_t)b * units + u) * RB);
+#pragma unroll
+      for (int i = 0; i < RB / 8; ++i) {
+        const uint4 v = e[i];
+        s[0] += bf2f((uint16_t)v.x);
+        s[1] += __uint_as_float(v.x & 0xffff0000u);
+        s[2] += bf2f((uint16_t)v.y);
+        s[3] += __uint_as_float(v.y & 0xffff0000u);
+        s[0] += bf2f((uint16_t)v.z);
+        s[1] += __uint_as_float(v.z & 0xffff0000u);
+        s[2] += bf2f((uint16_t)v.w);
+        s[3] += __uint_as_float(v.w & 0xffff0000u);
+      }
+    }
+    pb[(size_t)split * units + u] = (s[0] + s[1]) + (s[2] + s[3]);
+    return;
+  }
+  // the wave's tile: rows [mt, mt+32) x columns [nt, nt+32) of layer l
+  const uint16_t *A, *G;
+  float* pw;
+  int mt, nt, M, N;
+  if (part < 32) {
+    const int p = part & 15;
+    A = part < 16 ? a.act[1] : a.act[2];
+    G = part < 16 ? a.grad[1] : a.grad[2];
+    pw = part < 16 ? a.pw[1] : a.pw[2];
+    M = kHid; N = kHid;
+    mt = (p >> 2) * 64 + (wave >> 1) * 32;
+    nt = (p & 3) * 64 + (wave & 1) * 32;
+  } else if (part < 34) {
+    A = a.act[0]; G = a.grad[0]; pw = a.pw[0];
+    M = kIn; N = kHid;
+    mt = 0;
+    nt = (part & 1) * 128 + wave * 32;
+  } else {
+    A = a.act[3]; G = a.grad[3]; pw = a.pw[3];
+    M = kHid; N = kOutLd;
+    mt = (part & 1) * 128 + wave * 32;
+    nt = 0;
+  }
+  f32x4 acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  const int at = (lane & 15) * RB + (lane >> 4) * 8;
+  const uint16_t* pa = A + (size_t)mt * RB + at;
+  const uint16_t* pg = G + (size_t)nt * RB + at;
+  // four k chunks' operands in flight at a time
+  constexpr int KU = 4;
+  int b = b0;
+  for (; b + KU <= b1; b += KU) {
+    uint4 av[KU][2], gv[KU][2];
+#pragma unroll
+    for (int u = 0; u < KU; ++u)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        av[u][i] = *reinterpret_cast<const uint4*>(pa + ((size_t)(b + u) * M + i * 16) * RB);
+        gv[u][i] = *reinterpret_cast<const uint4*>(pg + ((size_t)(b + u) * N + i * 16) * RB);
+      }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < KU; ++u)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, av[u][i]),
+                                                              __builtin_bit_cast(bf16x8, gv[u][j]), acc[i][j], 0, 0, 0);
+  }
+  for (; b < b1; ++b) {
+    uint4 av[2], gv[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      av[i] = *reinterpret_cast<const uint4*>(pa + ((size_t)b * M + i * 16) * RB);
+      gv[i] = *reinterpret_cast<const uint4*>(pg + ((size_t)b * N + i * 16) * RB);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, av[i]),
+                                                            __builtin_bit_cast(bf16x8, gv[j]), acc[i][j], 0, 0, 0);
+  }
+  float* out = pw + ((size_t)split * M + mt + (lane >> 4) * 4) * N + nt + (lane & 15);
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) out[(size_t)(i * 16 + r) * N + j * 16] = acc[i][j][r];
 }
 
 struct AdamArgs {
@@ -427,14 +848,14 @@ struct AdamArgs {
   float* v;
   uint16_t* wbf[kLayers];
   uint16_t* wf[kLayers];
+  uint16_t* wb[kLayers];
   float* grad_out;
   const float* pw;
   const float* pb;
   int64_t w_off[kLayers], b_off[kLayers], pw_off[kLayers], pb_off[kLayers];
   int splits;
-  float lr0, lr_min, beta1, beta2, eps;
-  int64_t total_steps;
-  const long long* step;
+  float beta1, beta2, eps;
+  const float* rates;   // WeightArgs::rates
   int apply;
 };
 
@@ -456,19 +877,18 @@ __global__ __launch_bounds__(256) void adam_kernel(AdamArgs a) {
   }
   float g = 0.0f;
   if (is_b) {
+#pragma unroll 16
     for (int s = 0; s < a.splits; ++s) g += a.pb[a.pb_off[l] + (int64_t)s * kLdW[l] + n];
   } else {
+#pragma unroll 16
     for (int s = 0; s < a.splits; ++s) g += a.pw[a.pw_off[l] + ((int64_t)s * kFanIn[l] + k) * kLdW[l] + n];
   }
   if (a.grad_out) a.grad_out[p] = g;
   if (!a.apply) return;
-  const double t = (double)(*a.step + 1);
-  const double frac = fmin(t, (double)a.total_steps) / (double)a.total_steps;
-  const float lr = (float)(a.lr_min + 0.5 * (a.lr0 - a.lr_min) * (1.0 + cos(kPi * frac)));
-  const float bc1 = (float)(1.0 - pow((double)a.beta1, t));
-  const float bc2 = (float)(1.0 - pow((double)a.beta2, t));
-  const float m = a.beta1 * a.m[p] + (1.0f - a.beta1) * g;
-  const float v = a.beta2 * a.v[p] + (1.0f - a.beta2) * g * g;
+  const float lr = a.rates[0], bc1 = a.rates[1], bc2 = a.rates[2];
+  // which product is rounded is written out: a last bit here grows over the steps
+  const float m = fmaf(g, 1.0f - a.beta1, a.beta1 * a.m[p]);
+  const float v = fmaf(g, g * (1.0f - a.beta2), a.beta2 * a.v[p]);
   a.m[p] = m;
   a.v[p] = v;
   const float w = a.param[p] - lr * (m / bc1) / (sqrtf(v / bc2) + a.eps);
@@ -477,34 +897,20 @@ __global__ __launch_bounds__(256) void adam_kernel(AdamArgs a) {
     const uint16_t b = f2bf(w);
     a.wbf[l][(size_t)k * kLdW[l] + n] = b;
     a.wf[l][frag_offset(n, k, kFanIn[l])] = b;
+    a.wb[l][frag_offset(k, n, kLdW[l])] = b;
   }
 }
 
 __global__ void weights_to_bf16_kernel(const float* __restrict__ param, int64_t w_off, int fan_in, int fan_out,
-                                       int ldw, uint16_t* __restrict__ wbf, uint16_t* __restrict__ wf) {
+                                       int ldw, uint16_t* __restrict__ wbf, uint16_t* __restrict__ wf,
+                                       uint16_t* __restrict__ wb) {
   const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= (int64_t)fan_in * fan_out) return;
   const int k = (int)(q / fan_out), n = (int)(q % fan_out);
   const uint16_t b = f2bf(param[w_off + q]);
   wbf[(size_t)k * ldw + n] = b;
   wf[frag_offset(n, k, fan_in)] = b;
-}
-
-__global__ void gather_kernel(const uint16_t* __restrict__ ds_x, const float* __restrict__ ds_t,
-                              const int* __restrict__ perm, long long ds_n, const long long* __restrict__ cursor,
-                              int B, uint16_t* __restrict__ x, float* __restrict__ t) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= B) return;
-  const long long c = (*cursor + r) % ds_n;
-  const long long src = perm[c];
-  const uint4* xs = reinterpret_cast<const uint4*>(ds_x + src * kIn);
-  uint4* xd = reinterpret_cast<uint4*>(x + (size_t)r * kIn);
-#pragma unroll
-  for (int j = 0; j < kIn * 2 / 16; ++j) xd[j] = xs[j];
-  const uint4* ts = reinterpret_cast<const uint4*>(ds_t + src * kOutLd);
-  uint4* td = reinterpret_cast<uint4*>(t + (size_t)r * kOutLd);
-#pragma unroll
-  for (int j = 0; j < kOutLd * 4 / 16; ++j) td[j] = ts[j];
+  wb[frag_offset(k, n, ldw)] = b;
 }
 
 __global__ void reset_train_kernel(long long* cursor, int* local) {
@@ -512,25 +918,6 @@ __global__ void reset_train_kernel(long long* cursor, int* local) {
     *cursor = 0;
     *local = 0;
   }
-}
-
-__global__ void advance_kernel(long long* step, long long* cursor, int* local, const float* __restrict__ loss_partial,
-                               int nb, float inv_B, float* loss_hist, int hist_cap, int B) {
-  if (threadIdx.x != 0) return;
-  float s = 0.0f;
-  for (int i = 0; i < nb; ++i) s += loss_partial[i];
-  const int ls = *local;
-  if (ls < hist_cap) loss_hist[ls] = s * inv_B;
-  *local = ls + 1;
-  *step += 1;
-  *cursor += B;
-}
-
-__global__ void loss_sum_kernel(const float* __restrict__ loss_partial, int nb, float inv_B, float* loss) {
-  if (threadIdx.x != 0) return;
-  float s = 0.0f;
-  for (int i = 0; i < nb; ++i) s += loss_partial[i];
-  *loss = s * inv_B;
 }
 
 // ---- node encoding ------------------------------------------------------------
@@ -848,20 +1235,21 @@ __global__ __launch_bounds__(256) void apply_kernel(GateArgs a) {
 // ============================================================================
 struct gal_mlp {
   int device = 0;
-  int batch = 0, splits = 0, rows_per_split = 0;
+  int batch = 0, splits = 0;
   int64_t w_off[kLayers] = {}, b_off[kLayers] = {}, pw_off[kLayers] = {}, pb_off[kLayers] = {};
   float* d_param = nullptr;
   float* d_m = nullptr;
   float* d_v = nullptr;
   uint16_t* d_wbf[kLayers] = {};
   uint16_t* d_wf[kLayers] = {};   // the same in fragment order, columns as operand rows (forward)
-  uint16_t* d_x = nullptr;
-  float* d_t = nullptr;
-  uint16_t* d_z[3] = {};
-  uint16_t* d_h[3] = {};
-  float* d_out = nullptr;
-  uint16_t* d_dout = nullptr;
-  uint16_t* d_dz[2] = {};
+  uint16_t* d_wb[kLayers] = {};   // and rows as operand rows (backward)
+  // blocks of 32 rows, [block][unit][32], of the batch under way
+  uint16_t* d_xt = nullptr;
+  uint16_t* d_ht[3] = {};
+  uint16_t* d_dzt[3] = {};
+  uint16_t* d_dot = nullptr;
+  float* d_row_loss = nullptr;
+  float* d_rates = nullptr;
   float* d_pw = nullptr;
   float* d_pb = nullptr;
   float* d_loss_partial = nullptr;
@@ -881,9 +1269,10 @@ struct gal_mlp {
   const int* ds_perm = nullptr;
   hipStream_t stream = nullptr;
   hipEvent_t ev_in = nullptr, ev_out = nullptr;
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t exec = nullptr;
-  bool graph_valid = false;
+  // the captured step, and kGraphSteps of them: the GPU idles for 8 us between
+  // two graphs and not at all within one
+  hipGraph_t graph[2] = {};
+  hipGraphExec_t exec[2] = {};
   int inf_rows = 0;
   uint16_t* d_ix = nullptr;
   uint16_t* d_ih[2] = {};
@@ -897,15 +1286,13 @@ namespace {
 
 constexpr int kInferChunk = 1 << 17;
 
-template <bool AT, bool BT, int EPI>
-int gemm(const GemmArgs& g, int splits, hipStream_t s) {
+template <int EPI>
+int gemm(const GemmArgs& g, hipStream_t s) {
   // Operand loads are 16-byte vectors along the contiguous dimension.
-  if ((!AT && (g.K % 8 || g.lda % 8)) || (AT && (g.M % 8 || g.lda % 8)) || (BT && (g.K % 8 || g.ldb % 8)) ||
-      (!BT && (g.N % 8 || g.ldb % 8)) || g.k_split % TK)
-    return GAL_E_INVALID;
-  const dim3 grid((g.N + TN - 1) / TN, (g.M + TM - 1) / TM, splits);
+  if (g.K % 8 || g.lda % 8 || g.N % 8 || g.ldb % 8) return GAL_E_INVALID;
+  const dim3 grid((g.N + TN - 1) / TN, (g.M + TM - 1) / TM);
   if (grid.y > 65535u) return GAL_E_INVALID;
-  hipLaunchKernelGGL((gemm_kernel<AT, BT, EPI>), grid, dim3(256), 0, s, g);
+  hipLaunchKernelGGL(gemm_kernel<EPI>, grid, dim3(256), 0, s, g);
   return hipGetLastError() == hipSuccess ? GAL_OK : GAL_E_HIP;
 }
 
@@ -913,7 +1300,6 @@ GemmArgs gemm_args(const uint16_t* A, const uint16_t* B, int M, int N, int K, in
   GemmArgs g{};
   g.A = A; g.B = B; g.M = M; g.N = N; g.K = K; g.lda = lda; g.ldb = ldb; g.ldc = ldc;
   g.n_valid = N;
-  g.k_split = ((K + TK - 1) / TK) * TK;
   return g;
 }
 
@@ -923,70 +1309,76 @@ GemmArgs gemm_args(const uint16_t* A, const uint16_t* B, int M, int N, int K, in
     if (rc_ != GAL_OK) return rc_; \
   } while (0)
 
-// Forward through the four layers for n rows of x; training keeps the
-// pre-activations and activations of each hidden layer.
-int forward(gal_mlp* m, int n, const uint16_t* x, uint16_t* const z[3], uint16_t* const h[3], float* out,
-            hipStream_t s) {
+// Forward through the four layers for n rows of x, one launch each.
+int forward(gal_mlp* m, int n, const uint16_t* x, uint16_t* const h[3], float* out, hipStream_t s) {
   const uint16_t* in = x;
   for (int l = 0; l < 3; ++l) {
     GemmArgs g = gemm_args(in, m->d_wbf[l], n, kFanOut[l], kFanIn[l], kFanIn[l], kLdW[l], kFanOut[l]);
     g.bias = m->d_param + m->b_off[l];
     g.out_bf = h[l];
-    g.z_bf = z ? z[l] : nullptr;
-    GAL_TRY((gemm<false, false, EPI_SILU>(g, 1, s)));
+    GAL_TRY((gemm<EPI_SILU>(g, s)));
     in = h[l];
   }
   GemmArgs g = gemm_args(in, m->d_wbf[3], n, kOutLd, kHid, kHid, kLdW[3], kOutLd);
   g.n_valid = kOut;
   g.bias = m->d_param + m->b_off[3];
   g.out_f = out;
-  return gemm<false, false, EPI_LINEAR>(g, 1, s);
+  return gemm<EPI_LINEAR>(g, s);
 }
 
-// Backward pass from the output gradient already in d_dout; writes the
-// per-split partial gradients of every layer.
-int backward(gal_mlp* m, int n, const uint16_t* x, hipStream_t s) {
-  const int rps = ((n + m->splits - 1) / m->splits + TK - 1) / TK * TK;
-  const int splits = (n + rps - 1) / rps;
-  const uint16_t* grad = m->d_dout;  // gradient wrt this layer's output
-  int ld_grad = kOutLd;
-  int pp = 0;
-  for (int l = kLayers - 1; l >= 0; --l) {
-    const uint16_t* act_in = l == 0 ? x : m->d_h[l - 1];
-    // weight gradient: act_in^T (fan_in x n) . grad (n x ldW)
-    GemmArgs gw = gemm_args(act_in, grad, kFanIn[l], kLdW[l], n, kFanIn[l], ld_grad, kLdW[l]);
-    gw.k_split = rps;
-    gw.out_f = m->d_pw + m->pw_off[l];
-    GAL_TRY((gemm<true, false, EPI_PARTIAL>(gw, splits, s)));
-    hipLaunchKernelGGL(colsum_kernel, dim3((kLdW[l] + 63) / 64, splits), dim3(256), 0, s, grad, n, kLdW[l], ld_grad,
-                       rps, m->d_pb + m->pb_off[l]);
-    if (l == 0) break;
-    // gradient wrt the pre-activation of layer l-1: (grad . W_l^T) * silu'(z_{l-1})
-    GemmArgs gx = gemm_args(grad, m->d_wbf[l], n, kHid, kLdW[l], ld_grad, kLdW[l], kHid);
-    gx.z_in = m->d_z[l - 1];
-    gx.out_bf = m->d_dz[pp];
-    GAL_TRY((gemm<false, true, EPI_DSILU>(gx, 1, s)));
-    grad = m->d_dz[pp];
-    ld_grad = kHid;
-    pp ^= 1;
-  }
-  m->rows_per_split = rps;
-  return hipGetLastError() == hipSuccess ? GAL_OK : GAL_E_HIP;
-}
+// Rows of a split of n rows: a multiple of the weight gradients' k chunk.
+int split_rows(const gal_mlp* m, int n) { return ((n + m->splits - 1) / m->splits + RB - 1) / RB * RB; }
 
-LossArgs loss_args(gal_mlp* m, int n, const float* target) {
-  LossArgs a{};
-  a.out = m->d_out;
+// Forward, loss and gradients of n rows: the weights' partial sums.  With perm
+// the rows are the batch at the cursor of the permuted data set, and the step's
+// counters, loss and learning rate move on.
+int grad_pass(gal_mlp* m, int n, const uint16_t* x, const float* target, const int* perm, float* loss,
+              hipStream_t s) {
+  RowsArgs a{};
+  a.x = x;
   a.target = target;
-  a.dout = m->d_dout;
-  a.loss_partial = m->d_loss_partial;
-  a.B = n;
+  a.perm = perm;
+  a.cursor = m->d_cursor;
+  a.ds_n = m->ds_n;
+  a.n = n;
+  WeightArgs g{};
+  for (int l = 0; l < kLayers; ++l) {
+    a.wf[l] = m->d_wf[l];
+    a.wb[l] = m->d_wb[l];
+    a.bias[l] = m->d_param + m->b_off[l];
+    g.act[l] = l ? m->d_ht[l - 1] : m->d_xt;
+    g.grad[l] = l < 3 ? m->d_dzt[l] : m->d_dot;
+    g.pw[l] = m->d_pw + m->pw_off[l];
+    g.pb[l] = m->d_pb + m->pb_off[l];
+  }
+  a.xt = m->d_xt;
+  for (int l = 0; l < 3; ++l) { a.ht[l] = m->d_ht[l]; a.dzt[l] = m->d_dzt[l]; }
+  a.dot = m->d_dot;
+  a.row_loss = m->d_row_loss;
   for (int v = 0; v < 32; ++v) { a.w[v] = m->var_w[v]; a.sigma[v] = m->sigma[v]; }
   a.head_mask = m->head_mask;
   a.head_w = m->head_w;
   a.inv_wsum = m->inv_wsum;
   a.inv_B = 1.0f / (float)n;
-  return a;
+  hipLaunchKernelGGL(train_rows_kernel, dim3((n + RB - 1) / RB), dim3(kRowThreads), 0, s, a);
+  g.n = n;
+  g.rows_per_split = split_rows(m, n);
+  g.splits = (n + g.rows_per_split - 1) / g.rows_per_split;
+  g.row_loss = m->d_row_loss;
+  g.loss_partial = m->d_loss_partial;
+  g.inv_B = a.inv_B;
+  g.loss = loss;
+  g.loss_hist = m->d_loss_hist;
+  g.hist_cap = m->loss_hist_cap;
+  g.step = m->d_step;
+  g.cursor = m->d_cursor;
+  g.local = m->d_local;
+  g.advance = perm != nullptr;
+  g.lr0 = m->lr0; g.lr_min = m->lr_min; g.beta1 = m->beta1; g.beta2 = m->beta2;
+  g.total_steps = m->total_steps;
+  g.rates = m->d_rates;
+  hipLaunchKernelGGL(train_weights_kernel, dim3(g.splits * (kWeightParts + kBiasParts) + 1), dim3(256), 0, s, g);
+  return hipGetLastError() == hipSuccess ? GAL_OK : GAL_E_HIP;
 }
 
 AdamArgs adam_args(gal_mlp* m, int n, float* grad_out, int apply) {
@@ -995,44 +1387,59 @@ AdamArgs adam_args(gal_mlp* m, int n, float* grad_out, int apply) {
   for (int l = 0; l < kLayers; ++l) {
     a.wbf[l] = m->d_wbf[l];
     a.wf[l] = m->d_wf[l];
+    a.wb[l] = m->d_wb[l];
     a.w_off[l] = m->w_off[l]; a.b_off[l] = m->b_off[l]; a.pw_off[l] = m->pw_off[l]; a.pb_off[l] = m->pb_off[l];
   }
-  const int rps = ((n + m->splits - 1) / m->splits + TK - 1) / TK * TK;
+  const int rps = split_rows(m, n);
   a.splits = (n + rps - 1) / rps;
   a.grad_out = grad_out;
   a.pw = m->d_pw; a.pb = m->d_pb;
-  a.lr0 = m->lr0; a.lr_min = m->lr_min; a.beta1 = m->beta1; a.beta2 = m->beta2; a.eps = m->eps;
-  a.total_steps = m->total_steps;
-  a.step = m->d_step;
+  a.beta1 = m->beta1; a.beta2 = m->beta2; a.eps = m->eps;
+  a.rates = m->d_rates;
   a.apply = apply;
   return a;
 }
 
-int grad_pass(gal_mlp* m, int n, const uint16_t* x, const float* target, hipStream_t s) {
-  GAL_TRY(forward(m, n, x, m->d_z, m->d_h, m->d_out, s));
-  hipLaunchKernelGGL(loss_kernel, dim3((n + 255) / 256), dim3(256), 0, s, loss_args(m, n, target));
-  return backward(m, n, x, s);
-}
-
 int record_train_step(gal_mlp* m, hipStream_t s) {
   const int B = m->batch;
-  hipLaunchKernelGGL(gather_kernel, dim3((B + 255) / 256), dim3(256), 0, s, m->ds_x, m->ds_t, m->ds_perm, m->ds_n,
-                     (const long long*)m->d_cursor, B, m->d_x, m->d_t);
-  GAL_TRY(grad_pass(m, B, m->d_x, m->d_t, s));
+  GAL_TRY(grad_pass(m, B, m->ds_x, m->ds_t, m->ds_perm, nullptr, s));
   hipLaunchKernelGGL(adam_kernel, dim3((unsigned)((kParams + 255) / 256)), dim3(256), 0, s,
                      adam_args(m, B, nullptr, 1));
-  hipLaunchKernelGGL(advance_kernel, dim3(1), dim3(64), 0, s, m->d_step, m->d_cursor, m->d_local,
-                     (const float*)m->d_loss_partial, (B + 255) / 256, 1.0f / (float)B, m->d_loss_hist,
-                     m->loss_hist_cap, B);
   return hipGetLastError() == hipSuccess ? GAL_OK : GAL_E_HIP;
 }
 
+constexpr int kGraphSteps = 8;
+
 void release_graph(gal_mlp* m) {
-  if (m->exec) hipGraphExecDestroy(m->exec);
-  if (m->graph) hipGraphDestroy(m->graph);
-  m->exec = nullptr;
-  m->graph = nullptr;
-  m->graph_valid = false;
+  for (int k = 0; k < 2; ++k) {
+    if (m->exec[k]) hipGraphExecDestroy(m->exec[k]);
+    if (m->graph[k]) hipGraphDestroy(m->graph[k]);
+    m->exec[k] = nullptr;
+    m->graph[k] = nullptr;
+  }
+}
+
+// Capture `steps` training steps as graph k unless that is there.
+int ensure_graph(gal_mlp* m, int k, int steps) {
+  if (m->exec[k]) return GAL_OK;
+  HIP_TRY(hipStreamBeginCapture(m->stream, hipStreamCaptureModeThreadLocal));
+  int rc = GAL_OK;
+  for (int i = 0; i < steps && rc == GAL_OK; ++i) rc = record_train_step(m, m->stream);
+  hipGraph_t g = nullptr;
+  const hipError_t e = hipStreamEndCapture(m->stream, &g);
+  if (rc != GAL_OK || e != hipSuccess) {
+    if (g) hipGraphDestroy(g);
+    hipGetLastError();
+    return rc != GAL_OK ? rc : GAL_E_HIP;
+  }
+  const hipError_t ie = hipGraphInstantiate(&m->exec[k], g, nullptr, nullptr, 0);
+  if (ie != hipSuccess) {
+    m->exec[k] = nullptr;
+    hipGraphDestroy(g);
+    HIP_TRY(ie);
+  }
+  m->graph[k] = g;
+  return GAL_OK;
 }
 
 int ensure_inference(gal_mlp* m, int rows) {
@@ -1048,10 +1455,10 @@ int ensure_inference(gal_mlp* m, int rows) {
   return GAL_OK;
 }
 
-// Per-layer GEMM path (the training kernels' forward).
+// Per-layer GEMM path.
 int infer_layers(gal_mlp* m, int n, const uint16_t* x, float* out, hipStream_t s) {
   uint16_t* h[3] = {m->d_ih[0], m->d_ih[1], m->d_ih[0]};
-  return forward(m, n, x, nullptr, h, out, s);
+  return forward(m, n, x, h, out, s);
 }
 
 // The LDS limit of the fused kernel on the current device (a cheap host call;
@@ -1099,14 +1506,14 @@ int gal_mlp_create(int batch, gal_mlp** out) {
     m->pb_off[l] = pb;
     pb += (int64_t)m->splits * kLdW[l];
   }
-  const size_t B = (size_t)batch;
+  const size_t B = (size_t)(batch + RB - 1) / RB * RB;
   bool ok = hipMalloc(&m->d_param, sizeof(float) * kParams) == hipSuccess &&
             hipMalloc(&m->d_m, sizeof(float) * kParams) == hipSuccess &&
             hipMalloc(&m->d_v, sizeof(float) * kParams) == hipSuccess &&
-            hipMalloc(&m->d_x, sizeof(uint16_t) * kIn * B) == hipSuccess &&
-            hipMalloc(&m->d_t, sizeof(float) * kOutLd * B) == hipSuccess &&
-            hipMalloc(&m->d_out, sizeof(float) * kOutLd * B) == hipSuccess &&
-            hipMalloc(&m->d_dout, sizeof(uint16_t) * kOutLd * B) == hipSuccess &&
+            hipMalloc(&m->d_xt, sizeof(uint16_t) * kIn * B) == hipSuccess &&
+            hipMalloc(&m->d_dot, sizeof(uint16_t) * kOutLd * B) == hipSuccess &&
+            hipMalloc(&m->d_row_loss, sizeof(float) * B) == hipSuccess &&
+            hipMalloc(&m->d_rates, sizeof(float) * 3) == hipSuccess &&
             hipMalloc(&m->d_pw, sizeof(float) * pw) == hipSuccess &&
             hipMalloc(&m->d_pb, sizeof(float) * pb) == hipSuccess &&
             hipMalloc(&m->d_loss_partial, sizeof(float) * ((B + 255) / 256)) == hipSuccess &&
@@ -1115,11 +1522,11 @@ int gal_mlp_create(int batch, gal_mlp** out) {
             hipMalloc(&m->d_local, sizeof(int)) == hipSuccess;
   for (int l = 0; l < kLayers && ok; ++l)
     ok = hipMalloc(&m->d_wbf[l], sizeof(uint16_t) * kFanIn[l] * kLdW[l]) == hipSuccess &&
-         hipMalloc(&m->d_wf[l], sizeof(uint16_t) * kFanIn[l] * kLdW[l]) == hipSuccess;
+         hipMalloc(&m->d_wf[l], sizeof(uint16_t) * kFanIn[l] * kLdW[l]) == hipSuccess &&
+         hipMalloc(&m->d_wb[l], sizeof(uint16_t) * kFanIn[l] * kLdW[l]) == hipSuccess;
   for (int l = 0; l < 3 && ok; ++l)
-    ok = hipMalloc(&m->d_z[l], sizeof(uint16_t) * kHid * B) == hipSuccess &&
-         hipMalloc(&m->d_h[l], sizeof(uint16_t) * kHid * B) == hipSuccess;
-  for (int l = 0; l < 2 && ok; ++l) ok = hipMalloc(&m->d_dz[l], sizeof(uint16_t) * kHid * B) == hipSuccess;
+    ok = hipMalloc(&m->d_ht[l], sizeof(uint16_t) * kHid * B) == hipSuccess &&
+         hipMalloc(&m->d_dzt[l], sizeof(uint16_t) * kHid * B) == hipSuccess;
   // the training stream is created on the first training call: every stream
   // holds a hardware queue for the rest of the process, and inference-only
   // handles never need one
@@ -1129,11 +1536,11 @@ int gal_mlp_create(int batch, gal_mlp** out) {
     ok = hipMemset(m->d_param, 0, sizeof(float) * kParams) == hipSuccess &&
          hipMemset(m->d_m, 0, sizeof(float) * kParams) == hipSuccess &&
          hipMemset(m->d_v, 0, sizeof(float) * kParams) == hipSuccess &&
-         hipMemset(m->d_step, 0, sizeof(long long)) == hipSuccess &&
-         hipMemset(m->d_dout, 0, sizeof(uint16_t) * kOutLd * B) == hipSuccess;
+         hipMemset(m->d_step, 0, sizeof(long long)) == hipSuccess;
     for (int l = 0; l < kLayers && ok; ++l)
       ok = hipMemset(m->d_wbf[l], 0, sizeof(uint16_t) * kFanIn[l] * kLdW[l]) == hipSuccess &&
-           hipMemset(m->d_wf[l], 0, sizeof(uint16_t) * kFanIn[l] * kLdW[l]) == hipSuccess;
+           hipMemset(m->d_wf[l], 0, sizeof(uint16_t) * kFanIn[l] * kLdW[l]) == hipSuccess &&
+           hipMemset(m->d_wb[l], 0, sizeof(uint16_t) * kFanIn[l] * kLdW[l]) == hipSuccess;
     ok = ok && hipDeviceSynchronize() == hipSuccess;
   }
   if (!ok) {
@@ -1150,10 +1557,9 @@ int gal_mlp_destroy(gal_mlp* m) {
   if (!m) return GAL_OK;
   release_graph(m);
   hipFree(m->d_param); hipFree(m->d_m); hipFree(m->d_v);
-  for (int l = 0; l < kLayers; ++l) { hipFree(m->d_wbf[l]); hipFree(m->d_wf[l]); }
-  hipFree(m->d_x); hipFree(m->d_t);
-  for (int l = 0; l < 3; ++l) { hipFree(m->d_z[l]); hipFree(m->d_h[l]); }
-  hipFree(m->d_out); hipFree(m->d_dout); hipFree(m->d_dz[0]); hipFree(m->d_dz[1]);
+  for (int l = 0; l < kLayers; ++l) { hipFree(m->d_wbf[l]); hipFree(m->d_wf[l]); hipFree(m->d_wb[l]); }
+  hipFree(m->d_xt); hipFree(m->d_dot); hipFree(m->d_row_loss); hipFree(m->d_rates);
+  for (int l = 0; l < 3; ++l) { hipFree(m->d_ht[l]); hipFree(m->d_dzt[l]); }
   hipFree(m->d_pw); hipFree(m->d_pb); hipFree(m->d_loss_partial);
   hipFree(m->d_step); hipFree(m->d_cursor); hipFree(m->d_local); hipFree(m->d_loss_hist);
   hipFree(m->d_ix); hipFree(m->d_ih[0]); hipFree(m->d_ih[1]); hipFree(m->d_iout);
@@ -1174,7 +1580,7 @@ int gal_mlp_set_params(gal_mlp* m, const float* params, int64_t n) {
   for (int l = 0; l < kLayers; ++l) {
     const int64_t cnt = (int64_t)kFanIn[l] * kFanOut[l];
     hipLaunchKernelGGL(weights_to_bf16_kernel, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, 0,
-                       (const float*)m->d_param, m->w_off[l], kFanIn[l], kFanOut[l], kLdW[l], m->d_wbf[l], m->d_wf[l]);
+                       (const float*)m->d_param, m->w_off[l], kFanIn[l], kFanOut[l], kLdW[l], m->d_wbf[l], m->d_wf[l], m->d_wb[l]);
   }
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipDeviceSynchronize());
@@ -1249,13 +1655,10 @@ int gal_mlp_gradient_d(gal_mlp* m, int n, const uint16_t* x, const float* target
                        void* stream) {
   if (!m || n < 1 || n > m->batch || !x || !target) return GAL_E_INVALID;
   hipStream_t s = (hipStream_t)stream;
-  GAL_TRY(grad_pass(m, n, x, target, s));
+  GAL_TRY(grad_pass(m, n, x, target, nullptr, loss, s));
   if (grad)
     hipLaunchKernelGGL(adam_kernel, dim3((unsigned)((kParams + 255) / 256)), dim3(256), 0, s,
                        adam_args(m, n, grad, 0));
-  if (loss)
-    hipLaunchKernelGGL(loss_sum_kernel, dim3(1), dim3(64), 0, s, (const float*)m->d_loss_partial, (n + 255) / 256,
-                       1.0f / (float)n, loss);
   HIP_TRY(hipGetLastError());
   return GAL_OK;
 }
@@ -1286,22 +1689,11 @@ int gal_mlp_train_d(gal_mlp* m, int n_steps, int use_graph, float* loss_trace, v
   hipLaunchKernelGGL(reset_train_kernel, dim3(1), dim3(64), 0, m->stream, m->d_cursor, m->d_local);
   HIP_TRY(hipGetLastError());
   if (use_graph) {
-    if (!m->graph_valid) {
-      release_graph(m);
-      HIP_TRY(hipStreamBeginCapture(m->stream, hipStreamCaptureModeThreadLocal));
-      const int rc = record_train_step(m, m->stream);
-      hipGraph_t g = nullptr;
-      const hipError_t e = hipStreamEndCapture(m->stream, &g);
-      if (rc != GAL_OK || e != hipSuccess) {
-        if (g) hipGraphDestroy(g);
-        hipGetLastError();
-        return rc != GAL_OK ? rc : GAL_E_HIP;
-      }
-      m->graph = g;
-      HIP_TRY(hipGraphInstantiate(&m->exec, m->graph, nullptr, nullptr, 0));
-      m->graph_valid = true;
-    }
-    for (int i = 0; i < n_steps; ++i) HIP_TRY(hipGraphLaunch(m->exec, m->stream));
+    const int many = n_steps / kGraphSteps, rest = n_steps % kGraphSteps;
+    if (many) GAL_TRY(ensure_graph(m, 1, kGraphSteps));
+    if (rest) GAL_TRY(ensure_graph(m, 0, 1));
+    for (int i = 0; i < many; ++i) HIP_TRY(hipGraphLaunch(m->exec[1], m->stream));
+    for (int i = 0; i < rest; ++i) HIP_TRY(hipGraphLaunch(m->exec[0], m->stream));
   } else {
     for (int i = 0; i < n_steps; ++i) GAL_TRY(record_train_step(m, m->stream));
   }

@@ -370,7 +370,7 @@ def train_surrogate(evolver: NodeEvolverBatched, pairs: PairSet, epochs: int = 2
     torch.cuda.synchronize()
     t_start = time.perf_counter()
     perm = torch.empty(n, dtype=torch.int32, device=dev)
-    mlp.set_dataset(x, target, perm)   # fixed buffers: one captured step graph serves every epoch
+    mlp.set_dataset(x, target, perm)   # fixed buffers: the captured step graphs serve every epoch
     for _ in range(epochs):
         perm.copy_(torch.randperm(n, device=dev, generator=gen))
         losses.append(mlp.train_steps(steps_per_epoch, use_graph=use_graph))

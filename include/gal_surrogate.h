@@ -123,8 +123,8 @@ int gal_mlp_gradient_d(gal_mlp* m, int n, const uint16_t* x, const float* target
 int gal_mlp_set_dataset(gal_mlp* m, int64_t n, const uint16_t* x, const float* target, const int* perm);
 
 /* n_steps Adam steps on consecutive batches of the permuted dataset,
-   starting from its first row.  use_graph != 0 replays one captured
-   hipGraph per step.  loss_trace: device fp32[n_steps] or NULL. */
+   starting from its first row.  use_graph != 0 replays captured
+   hipGraphs of eight steps and of one.  loss_trace: device fp32[n_steps] or NULL. */
 int gal_mlp_train_d(gal_mlp* m, int n_steps, int use_graph, float* loss_trace, void* stream);
 
 /* ---- node encoding and the surrogate evolve ---------------------------- */

@@ -154,6 +154,52 @@ def test_gradient_matches_oracle(torch_cuda):
             o += size
 
 
+@pytest.mark.parametrize("batch,n", [(512, 1), (512, 31), (512, 33), (8192, 8192), (9001, 8999)])
+def test_gradient_at_block_edges(torch_cuda, batch, n):
+    """Row counts around the 32-row blocks and splits with a ragged end, after a full batch has filled the buffers:
+    rows past the end count for nothing.  Bars as above."""
+    torch = torch_cuda
+    m, p = _net(batch)
+    rng = np.random.default_rng(n)
+    x = om.bf16(rng.normal(0, 1, (batch, 32)).astype(np.float32))
+    t = rng.normal(0, 1, (batch, 32)).astype(np.float32)
+    xb, tb = _bits(torch, x), torch.from_numpy(t).cuda()
+    m.gradient(xb, tb)
+    g, loss = m.gradient(xb[:n], tb[:n])
+    g = g.cpu().numpy()
+    w, sigma, hv = _loss_config()
+    out, cache = om.forward_bf16(p, x[:n])
+    lref, g_out = om.loss_grad(out, t[:n], w, sigma, hv.astype(bool), 0.1)
+    gref = om.backward_bf16(p, cache, g_out)
+    assert abs(float(loss) - lref) <= 1e-2 * abs(lref)
+    o = 0
+    for a, b in zip(om.FAN_IN, om.FAN_OUT):
+        for size in (a * b, b):
+            assert np.linalg.norm(g[o:o + size] - gref[o:o + size]) <= 3e-2 * np.linalg.norm(gref[o:o + size]), (o, size)
+            o += size
+
+
+def test_batches_wrap_around_the_data_set(torch_cuda):
+    """Batches that run over the data set's end continue at its first row: the same weights as from a data set with
+    those rows written out."""
+    torch = torch_cuda
+    rng = np.random.default_rng(8)
+    x = _bits(torch, om.bf16(rng.normal(0, 1, (700, 32)).astype(np.float32)))
+    t = torch.from_numpy(rng.normal(0, 1, (700, 32)).astype(np.float32)).cuda()
+    perm = torch.from_numpy(rng.permutation(700).astype(np.int32)).cuda()
+    order = perm[torch.arange(4 * 500, device="cuda") % 700]
+    res = []
+    rows = order.long()
+    for data in ((x, t, perm),
+                 (x[rows].contiguous(), t[rows].contiguous(), torch.arange(2000, dtype=torch.int32, device="cuda"))):
+        m, _ = _net(batch=500, seed=3)
+        m.set_adam(lr=1e-3, total_steps=12)
+        m.set_dataset(*data)
+        losses = m.train_steps(4)
+        res.append((losses.cpu().numpy(), m.get_params()))
+    assert np.array_equal(res[0][0], res[1][0]) and np.array_equal(res[0][1], res[1][1])
+
+
 def test_gradient_finite_difference_on_gpu(torch_cuda):
     torch = torch_cuda
     m, p = _net()
