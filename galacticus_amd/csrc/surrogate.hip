@@ -182,29 +182,35 @@ __host__ __device__ constexpr size_t frag_offset(int c, int k, int n_k) {
 }
 
 // ---- fused inference forward ---------------------------------------------
-// The whole network for 128 rows per workgroup in one kernel: the rows'
-// activations stay in LDS from layer to layer (76 KiB, so two workgroups
-// share a CU).  Wave w computes all 128 rows x columns [64w, 64w+64) of a
-// hidden layer (8 x 4 tiles of 16 x 16); for the 32-column output layer waves
-// 0 and 1 take one column tile each.  A wave's columns are its own, so it
+// The whole network for FR rows per workgroup in one kernel: the rows'
+// activations stay in LDS from layer to layer.  Wave w computes all rows x
+// columns [64w, 64w+64) of a hidden layer, and one of the two column tiles of
+// half the rows of the output layer.  A wave's columns are its own, so it
 // reads its weight fragments straight from memory in fragment order into
-// registers, four k chunks at a time, with no LDS staging and no workgroup
+// registers, KG k chunks at a time, with no LDS staging and no workgroup
 // barrier inside a layer.  The weights are the MFMA's A operand, so a lane
 // ends with four consecutive columns of one row: it adds one bias vector,
 // rounds two values per instruction and writes 8 bytes to LDS (16 to the
 // output).  The arithmetic is the per-layer GEMMs' (same products, same k
 // order, same bias + SiLU epilogue and bf16 rounding), so the outputs are
 // bit-identical to them.
-// Bound by the epilogue's vector instructions, about 15 issue slots for each
-// activation beside 16 x 16 x 32 products that take 40 % as long.  500,000
-// rows with their output buffer took 420 us with an IEEE division, the bf16
-// rounding in integer instructions, two-byte LDS writes, weights read from
-// transposed rows (copied anew in each call) and a launch for every 131,072
-// rows; 260 us as it is here.
-constexpr int FR = 128;                 // rows per workgroup
+//
+// Bound by the epilogue's vector instructions, ten for each activation, beside
+// 16 x 16 x 32 products that take a third as long; four waves on a SIMD hide
+// some of the products and waits under them.  500,000 rows with their output
+// buffer: 254 us with 64 rows per workgroup, 260 us with 128 rows and two waves
+// on a SIMD (interleaving one half's products with the other half's epilogue
+// within each wave: 264), and 420 us with an IEEE division, the bf16 rounding
+// in integer instructions, two-byte LDS writes and weights read from
+// transposed rows that each call copied anew.
+//
+// Few rows are bound by the chain of the four layers instead, and 32 rows per
+// workgroup make it shorter and the workgroups more: 1000 rows 9 us against 14
+// (128 rows: 22), 20,000 rows 18 against 22.  From 32,768 rows on they would no
+// longer all be on the chip at once, and 60,000 rows take 42 us against 40.
 constexpr int LDH = kHid + 8;           // activation row stride (bf16)
 constexpr int LDX = kIn + 8;            // input row stride (bf16)
-constexpr size_t kFusedLds = sizeof(uint16_t) * ((size_t)FR * LDH + (size_t)FR * LDX);
+constexpr int kFewRows = 32768;
 
 struct FusedArgs {
   const uint16_t* x;                 // [n][kIn] bf16
@@ -214,22 +220,24 @@ struct FusedArgs {
   int n;
 };
 
-template <int K, bool LAST>
+template <int FR, int KG_MAX, int K, bool LAST>
 __device__ __forceinline__ void fused_layer(const FusedArgs& a, int l, const uint16_t* __restrict__ A, int lda,
                                             uint16_t* __restrict__ H, int r0) {
   constexpr int NK = K / TK;
-  constexpr int KG = NK < 4 ? NK : 4;                    // k chunks per register group
+  constexpr int KG = NK < KG_MAX ? NK : KG_MAX;                    // k chunks per register group
   constexpr int JT = LAST ? 1 : 4;                       // column tiles per wave
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const bool active = LAST ? wave < 2 : true;
-  const int nbase = LAST ? wave * 16 : wave * 64;
+  // the wave's number as a scalar: so are its addresses, but for the lane
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nbase = LAST ? (wave & 1) * 16 : wave * 64;
+  constexpr int IT = LAST ? FR / 32 : FR / 16;           // row tiles per wave
+  const int ibase = LAST ? (wave >> 1) * IT : 0;
   const uint16_t* __restrict__ wf = a.wf[l] + (size_t)(nbase / 16) * NK * 512 + lane * 8;
-  f32x4 acc[8][JT];
+  f32x4 acc[IT][JT];
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < IT; ++i)
 #pragma unroll
     for (int j = 0; j < JT; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  if (active) {
+  {
     for (int g0 = 0; g0 < NK; g0 += KG) {
       uint4 bq[KG][JT];
 #pragma unroll
@@ -240,8 +248,8 @@ __device__ __forceinline__ void fused_layer(const FusedArgs& a, int l, const uin
 #pragma unroll
       for (int kk = 0; kk < KG; ++kk) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const uint4 v = *reinterpret_cast<const uint4*>(A + (i * 16 + (lane & 15)) * lda + (g0 + kk) * TK +
+        for (int i = 0; i < IT; ++i) {
+          const uint4 v = *reinterpret_cast<const uint4*>(A + ((ibase + i) * 16 + (lane & 15)) * lda + (g0 + kk) * TK +
                                                           (lane >> 4) * 8);
           const bf16x8 av = __builtin_bit_cast(bf16x8, v);
 #pragma unroll
@@ -254,7 +262,6 @@ __device__ __forceinline__ void fused_layer(const FusedArgs& a, int l, const uin
   }
   // every wave has read this layer's input before any epilogue overwrites H
   __syncthreads();
-  if (!active) return;
   // column nbase + 16 j + 4 (lane / 16) + r of row 16 i + lane mod 16
   const int c0 = nbase + (lane >> 4) * 4;
   const float* __restrict__ bias = a.bias[l];
@@ -264,8 +271,8 @@ __device__ __forceinline__ void fused_layer(const FusedArgs& a, int l, const uin
 #pragma unroll
     for (int r = 0; r < 4; ++r) b[j][r] = bias[LAST ? min(c0 + r, kOut - 1) : c0 + j * 16 + r];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int row = i * 16 + (lane & 15);
+  for (int i = 0; i < IT; ++i) {
+    const int row = (ibase + i) * 16 + (lane & 15);
     if (LAST) {
       if (r0 + row >= a.n) continue;
       const f32x4 z = acc[i][0] + b[0];
@@ -304,10 +311,10 @@ __device__ __forceinline__ void fused_layer(const FusedArgs& a, int l, const uin
   }
 }
 
-__global__ __launch_bounds__(256, 2) void mlp_forward_fused(FusedArgs a) {
-  extern __shared__ __attribute__((aligned(16))) uint16_t fused_lds[];
-  uint16_t* H = fused_lds;
-  uint16_t* X = H + FR * LDH;
+template <int FR, int KG>
+__global__ __launch_bounds__(256, 4) void mlp_forward_fused(FusedArgs a) {
+  __shared__ __attribute__((aligned(16))) uint16_t H[FR * LDH];
+  __shared__ __attribute__((aligned(16))) uint16_t X[FR * LDX];
   const int tid = threadIdx.x;
   const int r0 = blockIdx.x * FR;
   const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
@@ -318,14 +325,14 @@ __global__ __launch_bounds__(256, 2) void mlp_forward_fused(FusedArgs a) {
     *reinterpret_cast<uint4*>(X + r * LDX + c) = v;
   }
   __syncthreads();
-  fused_layer<kIn, false>(a, 0, X, LDX, H, r0);
+  fused_layer<FR, KG, kIn, false>(a, 0, X, LDX, H, r0);
   __syncthreads();
 #pragma unroll 1
   for (int l = 1; l < 3; ++l) {   // one copy of the layer's code in the instruction cache
-    fused_layer<kHid, false>(a, l, H, LDH, H, r0);
+    fused_layer<FR, KG, kHid, false>(a, l, H, LDH, H, r0);
     __syncthreads();
   }
-  fused_layer<kHid, true>(a, 3, H, LDH, H, r0);
+  fused_layer<FR, KG, kHid, true>(a, 3, H, LDH, H, r0);
 }
 
 // ---- training support kernels ----------------------------------------------
@@ -427,7 +434,7 @@ __device__ __forceinline__ void rows_store(uint2 v, uint16_t* __restrict__ tile,
 template <bool FAR>
 __device__ __forceinline__ void rows_activate(const f32x4 (&acc)[2][2], uint16_t* __restrict__ tile,
                                               uint16_t* __restrict__ block, int valid_rows) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 #pragma unroll
   for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -462,7 +469,7 @@ template <bool FAR>
 __device__ __forceinline__ void rows_chain(const f32x4 (&acc)[2][2], const f32x4 (&z)[2][2],
                                            uint16_t* __restrict__ tile, uint16_t* __restrict__ block,
                                            int valid_rows) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 #pragma unroll
   for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -517,7 +524,7 @@ __global__ __launch_bounds__(kRowThreads, 2) void train_rows_kernel(RowsArgs a) 
   __shared__ __attribute__((aligned(16))) uint16_t X[RB * LDX];
   __shared__ __attribute__((aligned(16))) uint16_t H[2][RB * LDH];
   __shared__ float O[RB * LDF], R[RB * LDF];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const size_t blk = blockIdx.x;
   const int r0 = blockIdx.x * RB;
   const int valid = min(RB, a.n - r0);
@@ -726,7 +733,7 @@ __device__ void finish_step(const WeightArgs& a) {
 }
 
 __global__ __launch_bounds__(256) void train_weights_kernel(WeightArgs a) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (blockIdx.x == 0) {  // first: its chain of loads and sums is the longest
     finish_step(a);
     return;
@@ -1461,16 +1468,7 @@ int infer_layers(gal_mlp* m, int n, const uint16_t* x, float* out, hipStream_t s
   return forward(m, n, x, h, out, s);
 }
 
-// The LDS limit of the fused kernel on the current device (a cheap host call;
-// no process-wide state).
-int prepare_fused() {
-  static_assert(kFusedLds <= 163840, "fused forward LDS must fit a CU");
-  HIP_TRY(hipFuncSetAttribute((const void*)mlp_forward_fused, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)kFusedLds));
-  return GAL_OK;
-}
-
-// The fused one-kernel forward (after prepare_fused).
+// The fused one-kernel forward.
 int infer(gal_mlp* m, int n, const uint16_t* x, float* out, hipStream_t s) {
   if (n <= 0) return GAL_OK;
   FusedArgs a{};
@@ -1478,7 +1476,10 @@ int infer(gal_mlp* m, int n, const uint16_t* x, float* out, hipStream_t s) {
   for (int l = 0; l < kLayers; ++l) { a.wf[l] = m->d_wf[l]; a.bias[l] = m->d_param + m->b_off[l]; }
   a.out = out;
   a.n = n;
-  hipLaunchKernelGGL(mlp_forward_fused, dim3((n + FR - 1) / FR), dim3(256), kFusedLds, s, a);
+  if (n <= kFewRows)
+    hipLaunchKernelGGL((mlp_forward_fused<32, 4>), dim3((n + 31) / 32), dim3(256), 0, s, a);
+  else
+    hipLaunchKernelGGL((mlp_forward_fused<64, 2>), dim3((n + 63) / 64), dim3(256), 0, s, a);
   return hipGetLastError() == hipSuccess ? GAL_OK : GAL_E_HIP;
 }
 
@@ -1630,7 +1631,6 @@ int gal_mlp_forward_d(gal_mlp* m, int64_t n, const uint16_t* x, float* out, void
   hipStream_t s = (hipStream_t)stream;
   constexpr int64_t chunk = 1 << 30;   // rows of one launch: a grid of 32-bit size
   if (n == 0) return GAL_OK;
-  GAL_TRY(prepare_fused());
   for (int64_t c0 = 0; c0 < n; c0 += chunk) {
     const int nc = (int)std::min<int64_t>(chunk, n - c0);
     GAL_TRY(infer(m, nc, x + c0 * kIn, out + c0 * kOutLd, s));
@@ -1766,7 +1766,6 @@ int gal_surrogate_evolve_d(gal_ode_batch* h, gal_mlp* m, const float* norm, cons
   if (!m->d_rej_count) HIP_TRY(hipMalloc(&m->d_rej_count, sizeof(int)));
   const int chunk = std::min(n, kInferChunk);
   GAL_TRY(ensure_inference(m, chunk));
-  GAL_TRY(prepare_fused());
   HIP_TRY(hipMemsetAsync(m->d_rej_count, 0, sizeof(int), s));
   for (int c0 = 0; c0 < n; c0 += chunk) {
     const int nc = std::min(chunk, n - c0);

@@ -105,7 +105,7 @@ int gal_mlp_set_loss(gal_mlp* m, const float* var_weight, const float* target_si
                      double head_weight);
 
 /* Inference: x (device bf16, n x 32) -> out (device fp32, n x 32; column 31
-   is not written).  One fused kernel runs all four layers for 128 rows per
+   is not written).  One fused kernel runs all four layers for a tile of rows per
    workgroup, activations kept in LDS. */
 int gal_mlp_forward_d(gal_mlp* m, int64_t n, const uint16_t* x, float* out, void* stream);
 

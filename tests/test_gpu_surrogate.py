@@ -131,6 +131,19 @@ def test_activation_over_its_whole_range(torch_cuda, n):
     assert bool(torch.isnan(m.forward(x)[:, :31]).all())
 
 
+@pytest.mark.parametrize("n", [31, 33, 32767, 32768, 32769, 32769 + 64])
+def test_fused_forward_at_tile_edges(torch_cuda, n):
+    """Both row tiles of the fused forward (few rows and many), full and ragged: bit-identical to the layer path, and
+    the row after the last is left alone."""
+    torch = torch_cuda
+    m, _ = _net()
+    x = _bits(torch, om.bf16(np.random.default_rng(n).normal(0, 1, (n, 32)).astype(np.float32)))
+    out = torch.full((n + 1, 32), 7.0, device="cuda")
+    m.forward(x, out=out)
+    assert torch.equal(out[:n, :31], m.forward(x, layers=True)[:, :31])
+    assert bool((out[n] == 7.0).all()) and bool((out[:, 31] == 7.0).all())
+
+
 def test_gradient_matches_oracle(torch_cuda):
     torch = torch_cuda
     m, p = _net()
