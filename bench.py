@@ -46,14 +46,12 @@ METRIC = "node-Gyr evolved/sec: FP64 batched RK vs MLP+fallback at ≤1% M* erro
 FP64_PEAK_TFLOPS = 78.6
 
 # HBM bytes per evolve launch on the 1e5-node isolated-halo batch, by launch
-# shape, from rocprofv3 --pmc FETCH_SIZE and --pmc WRITE_SIZE runs of this
-# script (profiles/evolve_kernel_hbm_traffic_isolated_halos_1e5.md), each
-# counter scaled by what it reads for one elementwise kernel that reads and
-# writes 1 GiB (FETCH_SIZE x 2.0000, WRITE_SIZE x 1.0000).
-HBM_TRAFFIC_1E5 = {
-    (64, 1, 2): (241314.75 * 2.0 + 223554.75 * 1.0) * 1024,
-    (64, 2, 2): (1922487.5 * 2.0 + 3820465.0 * 1.0) * 1024,
-}
+# shape, from rocprofv3 --pmc FETCH_SIZE and --pmc WRITE_SIZE runs
+# (profiles/evolve_kernel_hbm_traffic_isolated_halos_1e5.md), each counter
+# scaled by what it reads for one elementwise kernel that reads and writes
+# 1 GiB (FETCH_SIZE x 2.0000, WRITE_SIZE x 1.0000).  The shapes run one kernel.
+_TRAFFIC = (240854.06 * 2.0 + 213911.25 * 1.0) * 1024
+HBM_TRAFFIC_1E5 = {(64, 1, 2): _TRAFFIC, (64, 2, 2): _TRAFFIC}
 
 
 _T_START = time.perf_counter()
@@ -1053,9 +1051,7 @@ def main():
             "workload": "batched plain RK: isolated-halo node ODE systems (FP64 Cash-Karp, rel 1e-3, abs 1e-6 x scale)",
             "n_nodes": n, "n_vars": 30, "node_gyr": node_gyr, "seed": args.seed,
             "halo_mass": "log-uniform 1e9-1e13 Msun", "f_hot": "uniform 0.05-0.17", "metallicity": "log-uniform 1e-4-0.02",
-            "dt_gyr": "uniform 0.1-2", "cooling_table": "200x50 FP64", "parallelism": ("single GPU, one node per lane"
-                                                                   + (", the RHS split over two waves"
-                                                                      if launch[2] == 2 else "")),
+            "dt_gyr": "uniform 0.1-2", "cooling_table": "200x50 FP64", "parallelism": "single GPU, one node per lane, the RHS split over four waves",
             "launch": {"nodes_per_workgroup": launch[0], "workgroups_per_cu": launch[1], "rhs_waves": launch[2],
                        "streams": n_streams,
                        "claim_order": ("planned for every batch of a round before its evolves launch" if plan_ahead
