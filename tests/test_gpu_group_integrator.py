@@ -1,8 +1,10 @@
 """The integrator's groups of 64 nodes, partial and full.  The nodes of a
 group share barriers, flags and LDS but no arithmetic, so a node's results are
-the same to the last bit in any lane and beside any other nodes; and a
-forest's operations give the same state whichever lane runs them, chained or
-claimed."""
+the same to the last bit in any lane and beside any other nodes; a forest's
+operations give the same state whichever lane runs them, chained or claimed;
+and the four waves of a group compute the right-hand side that one lane does."""
+from fractions import Fraction
+
 import numpy as np
 import pytest
 
@@ -82,3 +84,78 @@ def test_chained_operations_match_the_waves(torch_cuda, trees, resolution):
         out.append((y.cpu(), scale.cpu(), status.cpu()))
     for other in out[1:]:
         assert all(torch.equal(a, b) for a, b in zip(out[0], other))
+
+
+_fma = np.vectorize(lambda a, b, c: float(Fraction(a) * Fraction(b) + Fraction(c)), otypes=[float])
+
+
+def _cash_karp_step(rhs, t, y, h):
+    """The state after one Cash-Karp step of the derivative rhs(t, y): the tableau in doubles, and each sum with one
+    rounding per term in the integrator's order."""
+    k1 = rhs(t, y)
+    k2 = rhs(_fma(1 / 5, h, t), _fma(h, (1 / 5) * k1, y))
+    k3 = rhs(_fma(3 / 10, h, t), _fma(h, _fma(9 / 40, k2, (3 / 40) * k1), y))
+    k4 = rhs(_fma(3 / 5, h, t), _fma(h, _fma(6 / 5, k3, _fma(3 / 10, k1, (-9 / 10) * k2)), y))
+    k5 = rhs(t + h, _fma(h, _fma(35 / 27, k4, _fma(-70 / 27, k3, _fma(5 / 2, k2, (-11 / 54) * k1))), y))
+    k6 = rhs(_fma(7 / 8, h, t),
+             _fma(h, _fma(253 / 4096, k5, _fma(44275 / 110592, k4, _fma(575 / 13824, k3, _fma(
+                 1631 / 55296, k1, (175 / 512) * k2)))), y))
+    return _fma(h, _fma(512 / 1771, k6, _fma(125 / 594, k4, _fma(37 / 378, k1, (250 / 621) * k3))), y)
+
+
+_FIXABLE = [wl.V[v] for v in ("HOT_MASS", "HOT_OUTER_RADIUS", "DISK_MASS_GAS", "DISK_MASS_STELLAR",
+                              "DISK_ANGULAR_MOMENTUM", "SPHEROID_MASS_GAS", "SPHEROID_MASS_STELLAR",
+                              "SPHEROID_ANGULAR_MOMENTUM")]
+
+
+def _one_step_batch(kind, n):
+    """Intervals from 2^-10 to 2^-4 Gyr, the long ones a large part of what changes fast, from times whose sums with
+    them are exact."""
+    physics = gp.physics_params()
+    if kind == "box":
+        physics, b = wl.closed_box()[:2]
+        b = wl.NodeBatch(*(np.repeat(a[..., :1], n, axis=-1) for a in (b.y, b.node_par, b.t_start, b.t_end, b.h_step)))
+    else:
+        b = (wl.satellite_halos if kind == "satellite" else wl.isolated_halos)(n, seed=47, params=physics)
+    if kind == "test":
+        physics = gp.physics_params(physicsMode=gp.PHYSICS_TEST)
+    h = np.round(np.geomspace(2.0 ** -10, 2.0 ** -4, n) * 2.0 ** 20) / 2.0 ** 20
+    t0 = np.round(b.t_start * 2.0 ** 30) / 2.0 ** 30
+    assert ((t0 + h) - t0 == h).all()
+    return physics, b, t0, h
+
+
+@pytest.mark.parametrize("kind,operators", [("isolated", k) for k in range(16)] + [("satellite", k) for k in range(16)] +
+                         [("box", None), ("test", None)])
+def test_four_waves_compute_the_derivative_of_one_lane(torch_cuda, kind, operators):
+    """One accepted step (tolerances that accept any) against the same step put together on the host from derivatives
+    that rhs_device computes, one lane to a node: equal to the last bit.  Nodes that the step leaves negative where
+    the post-step fixes apply, or not finite, are left out."""
+    torch = torch_cuda
+    from galacticus_amd.evolver import NodeEvolverBatched
+    n = 70
+    physics, b, t0, h = _one_step_batch(kind, n)
+    if operators is not None:
+        physics[gp.P["nodeOperators"]] = operators
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    par = d(b.node_par)
+    single = NodeEvolverBatched(n, physics, synthetic_cie_table())
+
+    def rhs(t, y):
+        bad = ~np.isfinite(y)
+        k = single.rhs_device(d(t), d(np.where(bad, 1.0, y)), par).cpu().numpy()
+        lost.update(np.nonzero((bad | ~np.isfinite(k)).any(axis=0))[0].tolist())
+        return np.where(np.isfinite(k), k, 0.0)
+
+    lost = set()
+    expected = _cash_karp_step(rhs, t0, b.y, h)
+    keep = (expected[_FIXABLE] >= 0.0).all(axis=0)
+    keep[list(lost)] = False
+    y, h_step, status, _, counters = _evolve(torch, physics, {"odeToleranceAbsolute": 1.0e12,
+                                                              "odeToleranceRelative": 1.0e12},
+                                             b.y, b.node_par, t0, t0 + h, np.full(n, -1.0))
+    changed = (expected != b.y)[:, keep].any(axis=1).sum()
+    print(kind, operators, "nodes compared", int(keep.sum()), "variables that change", int(changed), flush=True)
+    assert keep.sum() >= n // 2
+    assert (status == 0).all() and (counters.numpy()[:, keep] == np.array([[1], [1], [6]])).all()
+    assert np.array_equal(y.numpy()[:, keep], expected[:, keep])
