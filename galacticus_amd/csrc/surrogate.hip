@@ -211,6 +211,12 @@ __host__ __device__ constexpr size_t frag_offset(int c, int k, int n_k) {
 constexpr int LDH = kHid + 8;           // activation row stride (bf16)
 constexpr int LDX = kIn + 8;            // input row stride (bf16)
 constexpr int kFewRows = 32768;
+constexpr int kManyRows = 64;           // rows per workgroup of more than kFewRows
+constexpr int kFusedThreads = 256;
+// Rows of one launch: a launch of 2^32 threads or more is refused.
+constexpr int64_t kLaunchRows = int64_t{1} << 29;
+static_assert((kLaunchRows + kManyRows - 1) / kManyRows * kFusedThreads < (int64_t{1} << 32),
+              "a launch must have fewer than 2^32 threads");
 
 struct FusedArgs {
   const uint16_t* x;                 // [n][kIn] bf16
@@ -312,13 +318,13 @@ __device__ __forceinline__ void fused_layer(const FusedArgs& a, int l, const uin
 }
 
 template <int FR, int KG>
-__global__ __launch_bounds__(256, 4) void mlp_forward_fused(FusedArgs a) {
+__global__ __launch_bounds__(kFusedThreads, 4) void mlp_forward_fused(FusedArgs a) {
   __shared__ __attribute__((aligned(16))) uint16_t H[FR * LDH];
   __shared__ __attribute__((aligned(16))) uint16_t X[FR * LDX];
   const int tid = threadIdx.x;
   const int r0 = blockIdx.x * FR;
   const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
-  for (int e = tid; e < FR * (kIn / 8); e += 256) {
+  for (int e = tid; e < FR * (kIn / 8); e += kFusedThreads) {
     const int r = e / (kIn / 8), c = (e % (kIn / 8)) * 8;
     uint4 v = zero;
     if (r0 + r < a.n) v = *reinterpret_cast<const uint4*>(a.x + (size_t)(r0 + r) * kIn + c);
@@ -1477,9 +1483,10 @@ int infer(gal_mlp* m, int n, const uint16_t* x, float* out, hipStream_t s) {
   a.out = out;
   a.n = n;
   if (n <= kFewRows)
-    hipLaunchKernelGGL((mlp_forward_fused<32, 4>), dim3((n + 31) / 32), dim3(256), 0, s, a);
+    hipLaunchKernelGGL((mlp_forward_fused<32, 4>), dim3((n + 31) / 32), dim3(kFusedThreads), 0, s, a);
   else
-    hipLaunchKernelGGL((mlp_forward_fused<64, 2>), dim3((n + 63) / 64), dim3(256), 0, s, a);
+    hipLaunchKernelGGL((mlp_forward_fused<kManyRows, 2>), dim3((n + kManyRows - 1) / kManyRows), dim3(kFusedThreads), 0, s,
+                       a);
   return hipGetLastError() == hipSuccess ? GAL_OK : GAL_E_HIP;
 }
 
@@ -1629,10 +1636,9 @@ int gal_mlp_set_loss(gal_mlp* m, const float* var_weight, const float* target_si
 int gal_mlp_forward_d(gal_mlp* m, int64_t n, const uint16_t* x, float* out, void* stream) {
   if (!m || n < 0 || (n > 0 && (!x || !out))) return GAL_E_INVALID;
   hipStream_t s = (hipStream_t)stream;
-  constexpr int64_t chunk = 1 << 30;   // rows of one launch: a grid of 32-bit size
   if (n == 0) return GAL_OK;
-  for (int64_t c0 = 0; c0 < n; c0 += chunk) {
-    const int nc = (int)std::min<int64_t>(chunk, n - c0);
+  for (int64_t c0 = 0; c0 < n; c0 += kLaunchRows) {
+    const int nc = (int)std::min<int64_t>(kLaunchRows, n - c0);
     GAL_TRY(infer(m, nc, x + c0 * kIn, out + c0 * kOutLd, s));
   }
   return GAL_OK;

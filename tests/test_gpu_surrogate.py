@@ -144,6 +144,34 @@ def test_fused_forward_at_tile_edges(torch_cuda, n):
     assert bool((out[n] == 7.0).all()) and bool((out[:, 31] == 7.0).all())
 
 
+def test_forward_of_more_rows_than_a_launch_takes(torch_cuda):
+    """2^30 rows, 192 GiB of inputs and outputs: a launch takes fewer than 2^32 threads, so they go in several.  The
+    rows at the start, round the middle and at the end equal the same rows on their own."""
+    torch = torch_cuda
+    n, need = 1 << 30, (1 << 30) * (32 * 2 + 32 * 4)
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < need + (16 << 30):
+        pytest.skip("less than 208 GiB of device memory free")
+    m, _ = _net()
+    places = [slice(0, 100), slice(n // 2 - 100, n // 2 + 100), slice(n - 100, n)]
+    rng = np.random.default_rng(12)
+    rows = [_bits(torch, om.bf16(rng.normal(0, 1, (s.stop - s.start, 32)).astype(np.float32))) for s in places]
+    x = out = None
+    try:
+        x = torch.zeros((n, 32), dtype=torch.int16, device="cuda")
+        out = torch.empty((n, 32), dtype=torch.float32, device="cuda")
+        for s, r in zip(places, rows):
+            x[s] = r
+            out[s] = 7.0
+        m.forward(x, out=out)
+        for s, r in zip(places, rows):
+            assert torch.equal(out[s][:, :31], m.forward(r)[:, :31])
+            assert bool((out[s][:, 31] == 7.0).all())
+    finally:
+        del x, out
+        torch.cuda.empty_cache()
+
+
 def test_gradient_matches_oracle(torch_cuda):
     torch = torch_cuda
     m, p = _net()
