@@ -33,8 +33,8 @@ sys.path.insert(0, ROOT)
 # concurrent forests): with 8 queues the four forest streams shared queues
 # (64 trees in 0.29 s), with 16 they did not (0.17 s).  Read when the HIP
 # runtime starts, so it is set before torch is.
-# Up to 32 evolve streams, each on a queue of its own: 32 queues (the most
-# this pool allows).  With 22, the 20 timed batches ran at 14.5 ms per step
+# Up to 32 evolve streams, each on a queue of its own: 32 queues.
+# With 22, the 20 timed batches ran at 14.5 ms per step
 # instead of 11.1; with 20, two of them shared a queue (19.6 ms).  A process
 # keeps a queue for every stream it ever used, and beyond about 24 the
 # hardware scheduler time-slices them, which makes persistent tree launches
@@ -45,13 +45,22 @@ if int(os.environ.get("GPU_MAX_HW_QUEUES", "4")) < 32:
 METRIC = "node-Gyr evolved/sec: FP64 batched RK vs MLP+fallback at ≤1% M* error"
 FP64_PEAK_TFLOPS = 78.6
 
-# HBM bytes per evolve launch on the 1e5-node isolated-halo batch, by launch
-# shape, from rocprofv3 --pmc FETCH_SIZE and --pmc WRITE_SIZE runs
+# The launch of the integrator: groups of 64 nodes, one group of four waves to
+# a CU.  It has no other (launch shapes set on a handle are kept and reported
+# there, and change nothing).
+KERNEL_LAUNCH = {"nodes_per_workgroup": 64, "workgroups_per_cu": 1, "rhs_waves": 4}
+
+# HBM bytes per evolve launch on the 1e5-node isolated-halo batch, from
+# rocprofv3 --pmc FETCH_SIZE and --pmc WRITE_SIZE runs
 # (profiles/evolve_kernel_hbm_traffic_isolated_halos_1e5.md), each counter
 # scaled by what it reads for one elementwise kernel that reads and writes
-# 1 GiB (FETCH_SIZE x 2.0000, WRITE_SIZE x 1.0000).  The shapes run one kernel.
-_TRAFFIC = (240854.06 * 2.0 + 213911.25 * 1.0) * 1024
-HBM_TRAFFIC_1E5 = {(64, 1, 2): _TRAFFIC, (64, 2, 2): _TRAFFIC}
+# 1 GiB (FETCH_SIZE x 2.0000, WRITE_SIZE x 1.0000).
+HBM_TRAFFIC_1E5 = (240854.06 * 2.0 + 213911.25 * 1.0) * 1024
+
+
+def hbm_traffic(n, seed):
+    """Bytes per launch where they were counted: the standard batch."""
+    return HBM_TRAFFIC_1E5 if n == 100000 and seed == 0 else None
 
 
 _T_START = time.perf_counter()
@@ -227,8 +236,6 @@ def surrogate_leg(physics, table, tol_abs, tol_rel, args):
     h0 = -torch.ones(n, dtype=torch.float64, device=test.t0.device)
     holder = {}
 
-    launch = ev.autotune(test.y0, test.node_par, test.t0, test.t1, h0)
-
     def run_rk():
         y, h = test.y0.clone(), h0.clone()
         ev.evolve_device(y, test.node_par, test.t0, test.t1, h)
@@ -261,13 +268,12 @@ def surrogate_leg(physics, table, tol_abs, tol_rel, args):
     chain = chained_histories(ev, se, physics, args)
     forest = surrogate_in_forest(se, physics, table, tol_abs, tol_rel)
     rk_rate, sur_rate = gyr / t_rk, gyr / t_sur
-    piped = pipelined_surrogate(ev, mlp, norm, gate, test, h0, launch, physics, table, tol_abs, tol_rel, args)
+    piped = pipelined_surrogate(ev, mlp, norm, gate, test, h0, physics, table, tol_abs, tol_rel, args)
     log(f"surrogate: RK {rk_rate:.4g} node-Gyr/s, surrogate+fallback {sur_rate:.4g} ({sur_rate / rk_rate:.2f}x), "
         f"rejected {n_rej / n:.3f}, median M* error {float(ms_err.median()):.2e}")
     log(f"surrogate pipelined: RK {piped['rk_s_per_batch'] * 1e3:.2f} ms/batch "
-        f"({piped['rk_streams']} streams, launch {piped['rk_launch']}), surrogate+fallback "
-        f"{piped['surrogate_s_per_batch'] * 1e3:.2f} ms/batch ({piped['surrogate_streams']} streams, "
-        f"launch {piped['surrogate_launch']}) "
+        f"({piped['rk_streams']} streams), surrogate+fallback "
+        f"{piped['surrogate_s_per_batch'] * 1e3:.2f} ms/batch ({piped['surrogate_streams']} streams) "
         f"({piped['rk_s_per_batch'] / piped['surrogate_s_per_batch']:.2f}x)")
     args.trained_surrogate = se
     return {
@@ -281,7 +287,7 @@ def surrogate_leg(physics, table, tol_abs, tol_rel, args):
                      "data_generation_s": gen_s, "loss_first": rep.loss_first, "loss_last": rep.loss_last,
                      "roofline": {"bound": "mfma", "achieved": rep.tflops, "peak": 2500.0, "unit": "TFLOP/s",
                                   "frac": rep.tflops / 2500.0, "flop_per_sample": sg.FLOPS_TRAIN_PER_ROW}},
-        "inference": {"intervals": n, "node_gyr": gyr, "launch": list(launch), "rk_node_gyr_per_s": rk_rate,
+        "inference": {"intervals": n, "node_gyr": gyr, "launch": KERNEL_LAUNCH, "rk_node_gyr_per_s": rk_rate,
                       "surrogate_node_gyr_per_s": sur_rate, "speedup": sur_rate / rk_rate,
                       "rejected_fraction": n_rej / n, "statuses_ok": bool((st == 0).all()),
                       "gate": dataclasses_asdict(gate),
@@ -300,19 +306,15 @@ def dataclasses_asdict(x):
     return dataclasses.asdict(x)
 
 
-PIPELINE_SHAPES = ((64, 1, 1), (64, 2, 1), (64, 4, 1), (64, 1, 2), (64, 2, 2))
-
-
-def pipelined_surrogate(ev, mlp, norm, gate, test, h0, launch, physics, table, tol_abs, tol_rel, args):
+def pipelined_surrogate(ev, mlp, norm, gate, test, h0, physics, table, tol_abs, tol_rel, args):
     """Throughput of both paths as bench's main leg measures the integrator:
     independent copies of the evaluation batch alternate over streams, each
     stream with its own integrator handle (and network handle), so one
     batch's tail of stiff nodes overlaps the next batch's start.  Each path
-    runs with the number of streams and the integrator launch shape that are
-    fastest for it in this overlapped regime (the fallback batch is a sparse
-    subset of stiff intervals, whose best configuration differs from the full
-    batch's): every combination gets one timed pass, the fastest is timed
-    afresh (median of three passes)."""
+    runs with the number of streams that is fastest for it in this overlapped
+    regime (the fallback batch is a sparse subset of stiff intervals, whose
+    best number differs from the full batch's): the median of three passes for
+    each, and the fastest is timed afresh in the same way."""
     import torch
     from galacticus_amd import surrogate as sg
     from galacticus_amd.evolver import NodeEvolverBatched
@@ -351,28 +353,23 @@ def pipelined_surrogate(ev, mlp, norm, gate, test, h0, launch, physics, table, t
             torch.cuda.synchronize()
             return (time.perf_counter() - t) / batches
 
-        per_config = {}
+        def median_pass(used):
+            return float(np.median([timed_pass(used) for _ in range(3)]))
+
+        by_streams = {}
         for used in counts:
-            for shape in PIPELINE_SHAPES:
-                for e in evs:
-                    e.set_launch(*shape)
-                for j in range(used):      # warm-up (allocations of first use)
-                    launch_one(j % batches, used)
-                torch.cuda.synchronize()
-                per_config[(used, shape)] = timed_pass(used)
-        used, best = min(per_config, key=per_config.get)
-        for e in evs:
-            e.set_launch(*best)
-        out[f"{name}_s_per_batch"] = float(np.median([timed_pass(used) for _ in range(3)]))
-        out[f"{name}_launch"] = list(best)
+            for j in range(used):      # warm-up (allocations of first use)
+                launch_one(j % batches, used)
+            torch.cuda.synchronize()
+            by_streams[used] = median_pass(used)
+        used = min(by_streams, key=by_streams.get)
+        out[f"{name}_s_per_batch"] = median_pass(used)
         out[f"{name}_streams"] = used
-        out[f"{name}_s_per_batch_by_config"] = {f"{u} streams, {a},{b},{c}": v
-                                                  for (u, (a, b, c)), v in per_config.items()}
+        out[f"{name}_s_per_batch_by_streams"] = {str(u): v for u, v in by_streams.items()}
         if name == "surrogate":
             out["rejected_fraction_last_batch"] = int((accepted[0] == 0).sum()) / n
         out[f"{name}_statuses_ok"] = all(bool((st == 0).all()) for st in status)
         del ys, hs
-    ev.set_launch(*launch)
     out.update({"stream_counts": counts, "batches": batches, "intervals_per_batch": n})
     for m in mlps[1:]:
         m.close()
@@ -509,7 +506,7 @@ def _forest_run(physics, table, tol_abs, tol_rel, n_trees, log_m, z_start, label
     out = {"workload": label, "nodes": forest.n_nodes, "operations": sched.n_ops, "waves": sched.n_waves,
            "evolve_intervals": int(k[0]), "promotions": int(k[1]), "halo_mergers": int(k[2]),
            "galaxy_mergers": int(k[3]), "node_gyr": gyr, "executor": "operation graph, one persistent launch",
-           "launch": list(ev.launch()), "gpu_seconds": gpu_s, "gpu_seconds_first_call": times[0],
+           "launch": KERNEL_LAUNCH, "gpu_seconds": gpu_s, "gpu_seconds_first_call": times[0],
            "node_gyr_per_s": gyr / gpu_s,
            "host_build_seconds": build_s, "host_schedule_seconds": sched_s, "statuses_ok": bool((st == 0).all())}
     log(f"trees ({label}): {forest.n_nodes} nodes, {sched.n_ops} operations in {sched.n_waves} waves, "
@@ -813,7 +810,8 @@ def main():
                     help="order each overlapped batch's claims inside its own evolve call instead of planning all "
                          "batches before the evolves launch")
     ap.add_argument("--launch", default="auto",
-                    help="launch shape 'nodes_per_workgroup,workgroups_per_cu[,rhs_waves]', or 'auto' to time them")
+                    help="launch shape 'nodes_per_workgroup,workgroups_per_cu[,rhs_waves]' to set on the handles "
+                         "(the integrator runs alike at every one), or 'auto' for theirs")
     ap.add_argument("--no-cpu", action="store_true", help="skip the CPU baseline leg")
     ap.add_argument("--cpu-seconds", type=float, default=15.0)
     ap.add_argument("--no-surrogate", action="store_true", help="skip the surrogate training/inference legs")
@@ -893,10 +891,9 @@ def main():
         log(f"copy calibration: {n_el * 8} bytes read and written by one elementwise kernel")
         del src, dst
     # One stream per evolver handle, created once: the runtime maps streams
-    # to its hardware queues in creation order, so tuning and the timed region
+    # to its hardware queues in creation order, so warm-up and the timed region
     # share the same queues.
     streams = stream_pool(n_streams)
-    tuning = {}
     plan_ahead = not args.no_plan
 
     def overlapped_round(items, before=None, after=None):
@@ -930,41 +927,18 @@ def main():
                 if after:
                     after(k)
 
-    shapes = ((64, 1, 1), (64, 2, 1), (64, 4, 1), (64, 1, 2), (64, 2, 2))
     if args.launch != "auto":
-        v = tuple(int(x) for x in args.launch.split(","))
-        shapes = (v if len(v) == 3 else v + (1,),)
-    if args.launch == "auto":
-        single = ev.autotune(y0, npar, t0, t1, h0)
-        tuning["single_launch_choice"] = list(single)
-    if len(shapes) > 1:
-        # The library's autotuner times single launches; the timed region
-        # overlaps independent batches on n_streams streams, where a shape
-        # with more resident lanes can win although it loses alone.  Time
-        # each shape on one round of n_streams concurrent batches and keep
-        # the fastest per batch.
-        best = None
-        for shape in shapes:
-            for e in evs:
-                e.set_launch(*shape)
-            yt = [y0.clone() for _ in range(n_streams)]
-            ht = [h0.clone() for _ in range(n_streams)]
-            torch.cuda.synchronize()
-            t_a = time.perf_counter()
-            overlapped_round([(j, yt[j], ht[j], None, None, None) for j in range(n_streams)])
-            torch.cuda.synchronize()
-            ms = (time.perf_counter() - t_a) * 1e3 / n_streams
-            tuning[f"{shape[0]},{shape[1]},{shape[2]}"] = ms
-            if best is None or ms < best[0]:
-                best = (ms, shape)
-            del yt, ht
-        launch = best[1]
-    else:
-        launch = shapes[0]
-    for e in evs:
-        e.set_launch(*launch)
-    log(f"launch: {launch[0]} nodes per workgroup, {launch[1]} workgroups per CU, {launch[2]} waves per group, "
-        f"{n_streams} streams (tuning {tuning})")
+        shape = tuple(int(x) for x in args.launch.split(","))
+        for e in evs:
+            e.set_launch(*(shape if len(shape) == 3 else shape + (1,)))
+    # every handle's first launch, with what it allocates, is untimed
+    yt = [y0.clone() for _ in range(n_streams)]
+    ht = [h0.clone() for _ in range(n_streams)]
+    torch.cuda.synchronize()
+    overlapped_round([(j, yt[j], ht[j], None, None, None) for j in range(n_streams)])
+    torch.cuda.synchronize()
+    del yt, ht
+    log(f"launch: {KERNEL_LAUNCH}, {n_streams} streams")
     total = args.warmup + args.steps
     ys = [y0.clone() for _ in range(total)]
     hs = [h0.clone() for _ in range(total)]
@@ -1052,11 +1026,9 @@ def main():
             "n_nodes": n, "n_vars": 30, "node_gyr": node_gyr, "seed": args.seed,
             "halo_mass": "log-uniform 1e9-1e13 Msun", "f_hot": "uniform 0.05-0.17", "metallicity": "log-uniform 1e-4-0.02",
             "dt_gyr": "uniform 0.1-2", "cooling_table": "200x50 FP64", "parallelism": "single GPU, one node per lane, the RHS split over four waves",
-            "launch": {"nodes_per_workgroup": launch[0], "workgroups_per_cu": launch[1], "rhs_waves": launch[2],
-                       "streams": n_streams,
-                       "claim_order": ("planned for every batch of a round before its evolves launch" if plan_ahead
-                                       else "inside each evolve call"),
-                       "tuning_ms_per_step": tuning},
+            "launch": dict(KERNEL_LAUNCH, streams=n_streams,
+                           claim_order=("planned for every batch of a round before its evolves launch" if plan_ahead
+                                        else "inside each evolve call")),
         },
         "single_launch": {
             "ms": single_launch_ms,
@@ -1072,7 +1044,7 @@ def main():
             "peak": FP64_PEAK_TFLOPS,
             "unit": "TFLOP/s",
             "frac": achieved_tflops / FP64_PEAK_TFLOPS,
-            "traffic": HBM_TRAFFIC_1E5.get(tuple(launch)) if n == 100000 and args.seed == 0 else None,
+            "traffic": hbm_traffic(n, args.seed),
             "traffic_unit": "bytes per launch (rocprofv3 counters, calibrated)",
             "flop_per_rhs_evaluation": gflops.rhs_flops(),
             "flop_per_attempt_combination": gflops.combination_flops(),
