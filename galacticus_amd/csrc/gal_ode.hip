@@ -1040,9 +1040,7 @@ int gal_ode_batch_set_cooling_table(gal_ode_batch* h, const double* ln_lambda, i
 int gal_ode_batch_set_launch(gal_ode_batch* h, int nodes_per_block, int blocks_per_cu) {
   if (!h) return GAL_E_INVALID;
   if (nodes_per_block != 64) return GAL_E_INVALID;
-  // one workgroup per CU keeps every lane vector in LDS; two keep state and
-  // scales in the HBM workspace; three or four keep the stage derivatives
-  // there (the LDS of a CU is 160 KiB)
+  // kept and reported only: launch_evolve has one shape
   if (blocks_per_cu < 1 || blocks_per_cu > 4) return GAL_E_INVALID;
   h->nodes_per_block = nodes_per_block;
   h->blocks_per_cu = blocks_per_cu;
@@ -1079,6 +1077,7 @@ int gal_ode_batch_get_launch(gal_ode_batch* h, int* nodes_per_block, int* blocks
 extern "C++" {
 template <bool GRAPH = false>
 static int launch_evolve(gal_ode_batch* h, const EvolveArgs& args, hipStream_t s) {
+  // a combination that is documented as refused; the kernel would run alike
   if (h->rhs_waves == 2 && h->blocks_per_cu > 2) return GAL_E_INVALID;
   // one group of nodes fills a CU, and a lone group per CU is claimed from
   // until the last node is out
@@ -1200,60 +1199,16 @@ int gal_ode_hadjust_d(int n, int dim, int ord, double eps_abs, double eps_rel, d
 int gal_ode_batch_autotune(gal_ode_batch* h, int n, int ld, double* y, const double* node_par,
                            const double* t_start, const double* t_end, double* h_step, double* scale, int* status,
                            void* stream, int* best_nodes_per_block, int* best_blocks_per_cu) {
-  // Times each admissible launch shape on copies of the inputs (the caller's
-  // arrays are untouched), keeps the fastest and leaves it set on the handle.
-  if (!h || n <= 0 || ld < n) return GAL_E_INVALID;
-  hipStream_t s = (hipStream_t)stream;
-  double *wy = nullptr, *wh = nullptr, *wsc = nullptr;
-  int* wst = nullptr;
-  const size_t nn = (size_t)ld;
-  if (hipMalloc(&wy, sizeof(double) * GAL_NVAR * nn) != hipSuccess ||
-      hipMalloc(&wh, sizeof(double) * nn) != hipSuccess ||
-      hipMalloc(&wsc, sizeof(double) * GAL_NVAR * nn) != hipSuccess ||
-      hipMalloc(&wst, sizeof(int) * nn) != hipSuccess) {
-    hipFree(wy); hipFree(wh); hipFree(wsc); hipFree(wst);
-    return GAL_E_NOMEM;
-  }
-  // (nodes per workgroup, workgroups per CU, waves per group of nodes); the
-  // kernel runs alike at every admitted shape, so one stands for all
-  const int shapes[][3] = {{64, 1, 2}};
-  float best = 1e30f;
-  int bn = h->nodes_per_block, bb = h->blocks_per_cu, bw = h->rhs_waves;
-  hipEvent_t e0, e1;
-  hipEventCreate(&e0);
-  hipEventCreate(&e1);
-  int rc = GAL_OK;
-  for (auto& sh : shapes) {
-    if (gal_ode_batch_set_launch(h, sh[0], sh[1]) != GAL_OK || gal_ode_batch_set_rhs_waves(h, sh[2]) != GAL_OK)
-      continue;
-    for (int rep = 0; rep < 2 && rc == GAL_OK; ++rep) {
-      hipMemcpyAsync(wy, y, sizeof(double) * GAL_NVAR * nn, hipMemcpyDeviceToDevice, s);
-      hipMemcpyAsync(wh, h_step, sizeof(double) * nn, hipMemcpyDeviceToDevice, s);
-      if (scale && (h->flags & GAL_FLAG_SCALES_PROVIDED))
-        hipMemcpyAsync(wsc, scale, sizeof(double) * GAL_NVAR * nn, hipMemcpyDeviceToDevice, s);
-      hipEventRecord(e0, s);
-      rc = gal_ode_batch_evolve_d(h, n, ld, wy, node_par, t_start, t_end, wh, wsc, wst, nullptr, stream);
-      hipEventRecord(e1, s);
-      hipEventSynchronize(e1);
-      float ms = 0.0f;
-      hipEventElapsedTime(&ms, e0, e1);
-      if (rep == 1 && ms < best) {
-        best = ms;
-        bn = sh[0];
-        bb = sh[1];
-        bw = sh[2];
-      }
-    }
-  }
-  hipEventDestroy(e0);
-  hipEventDestroy(e1);
-  hipFree(wy); hipFree(wh); hipFree(wsc); hipFree(wst);
-  (void)status;
-  gal_ode_batch_set_launch(h, bn, bb);
-  gal_ode_batch_set_rhs_waves(h, bw);
-  if (best_nodes_per_block) *best_nodes_per_block = bn;
-  if (best_blocks_per_cu) *best_blocks_per_cu = bb;
-  return rc;
+  // The kernel runs alike at every admitted shape: there is nothing to time.
+  if (!h || n <= 0 || n > h->n_max || ld < n || !h->have_physics || !h->have_table) return GAL_E_INVALID;
+  if (!y || !node_par || !t_start || !t_end || !h_step) return GAL_E_INVALID;
+  (void)scale; (void)status; (void)stream;
+  h->nodes_per_block = 64;
+  h->blocks_per_cu = 1;
+  h->rhs_waves = 2;
+  if (best_nodes_per_block) *best_nodes_per_block = h->nodes_per_block;
+  if (best_blocks_per_cu) *best_blocks_per_cu = h->blocks_per_cu;
+  return GAL_OK;
 }
 
 }  // extern "C"

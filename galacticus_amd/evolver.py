@@ -212,17 +212,15 @@ class NodeEvolverBatched:
         return dydt
 
     def autotune(self, y, node_par, t_start, t_end, h_step, stream=None):
-        """Time the launch shapes on copies of the inputs; keeps the fastest."""
-        import torch
+        """Set the default launch shape and return it: the integrator runs
+        alike at every one (gal_ode_batch_autotune)."""
         n = int(t_start.shape[0])
         self._check_shapes(n, y, node_par, t_end, h_step)
         bn, bb = ctypes.c_int(), ctypes.c_int()
-        scale = torch.empty_like(y)
-        status = torch.empty(n, dtype=torch.int32, device=y.device)
         s = ctypes.c_void_p(0 if stream is None else stream.cuda_stream)
         _lib.check(self.L.gal_ode_batch_autotune(self.handle, n, int(y.shape[1]), _ptr(y), _ptr(node_par),
-                                                 _ptr(t_start), _ptr(t_end), _ptr(h_step), _ptr(scale),
-                                                 _ptr(status), s, ctypes.byref(bn), ctypes.byref(bb)),
+                                                 _ptr(t_start), _ptr(t_end), _ptr(h_step), _ptr(None), _ptr(None), s,
+                                                 ctypes.byref(bn), ctypes.byref(bb)),
                    "gal_ode_batch_autotune")
         return self.launch()
 

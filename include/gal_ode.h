@@ -359,9 +359,11 @@ int gal_ode_batch_set_rhs_waves(gal_ode_batch *h, int waves);
    autotune).  No counterpart in the reference. */
 int gal_ode_batch_get_launch(gal_ode_batch *h, int *nodes_per_block, int *blocks_per_cu, int *rhs_waves);
 
-/* Return the autotuned launch, measured on this handle (nodes_per_block,
-   blocks_per_cu; the waves per group are left set on the handle, see
-   gal_ode_batch_get_launch) after a call to gal_ode_batch_autotune. */
+/* Set and return the default launch (64 nodes per workgroup, one workgroup
+   per CU, two waves per group): the integrator runs alike at every one, so
+   nothing is timed or allocated.  The arguments are those of
+   gal_ode_batch_evolve_d and have to describe a batch that it would take;
+   scale and status may be NULL. */
 int gal_ode_batch_autotune(gal_ode_batch *h, int n, int ld, double *y,
                            const double *node_par, const double *t_start,
                            const double *t_end, double *h_step,

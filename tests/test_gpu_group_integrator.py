@@ -159,3 +159,27 @@ def test_four_waves_compute_the_derivative_of_one_lane(torch_cuda, kind, operato
     assert keep.sum() >= n // 2
     assert (status == 0).all() and (counters.numpy()[:, keep] == np.array([[1], [1], [6]])).all()
     assert np.array_equal(y.numpy()[:, keep], expected[:, keep])
+
+
+def test_autotune_takes_no_memory_and_runs_nothing(torch_cuda):
+    """With one launch shape there is nothing to time: a leading dimension whose copies no device holds is accepted,
+    and the arrays stay as they are.  What cannot be evolved is refused."""
+    import ctypes
+    torch = torch_cuda
+    from galacticus_amd import _lib
+    from galacticus_amd.evolver import NodeEvolverBatched
+    b = wl.isolated_halos(64, seed=1)
+    ev = NodeEvolverBatched(64, gp.physics_params(), synthetic_cie_table())
+    arrays = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (b.y, b.node_par, b.t_start, b.t_end, b.h_step)]
+    before = [a.clone() for a in arrays]
+    blocks = ctypes.c_int(), ctypes.c_int()
+    pointers = [ctypes.c_void_p(a.data_ptr()) for a in arrays]
+    call = lambda n, ld, p: ev.L.gal_ode_batch_autotune(ev.handle, n, ld, *p, None, None, None,
+                                                        ctypes.byref(blocks[0]), ctypes.byref(blocks[1]))
+    ev.set_launch(64, 4, 1)
+    assert call(64, 2 ** 31 - 1, pointers) == _lib.GAL_OK
+    torch.cuda.synchronize()
+    assert (blocks[0].value, blocks[1].value) == (64, 1) and ev.launch() == (64, 1, 2)
+    assert all(torch.equal(a, o) for a, o in zip(arrays, before))
+    for n, ld, p in ((0, 64, pointers), (65, 65, pointers), (64, 63, pointers), (64, 64, [None] + pointers[1:])):
+        assert call(n, ld, p) == -1        # GAL_E_INVALID
