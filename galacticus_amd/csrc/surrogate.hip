@@ -933,6 +933,11 @@ __global__ void weights_to_bf16_kernel(const float* __restrict__ param, int64_t 
   wb[frag_offset(k, n, ldw)] = b;
 }
 
+// A kernel and not a memset, which a caller's graph replays wrongly.
+__global__ void reset_count_kernel(int* count) {
+  if (threadIdx.x == 0) *count = 0;
+}
+
 __global__ void reset_train_kernel(long long* cursor, int* local) {
   if (threadIdx.x == 0) {
     *cursor = 0;
@@ -1779,7 +1784,8 @@ int gal_surrogate_evolve_d(gal_ode_batch* h, gal_mlp* m, const float* norm, cons
   if (!m->d_rej_count) HIP_TRY(hipMalloc(&m->d_rej_count, sizeof(int)));
   const int chunk = std::min(n, kInferChunk);
   GAL_TRY(ensure_inference(m, chunk));
-  HIP_TRY(hipMemsetAsync(m->d_rej_count, 0, sizeof(int), s));
+  hipLaunchKernelGGL(reset_count_kernel, dim3(1), dim3(64), 0, s, m->d_rej_count);
+  HIP_TRY(hipGetLastError());
   for (int c0 = 0; c0 < n; c0 += chunk) {
     const int nc = std::min(chunk, n - c0);
     GAL_TRY(gal_surrogate_encode_d(h, nc, ld, y + c0, nullptr, node_par + c0, t_start + c0, t_end + c0, norm,

@@ -393,6 +393,55 @@ def test_rejected_nodes_get_the_integrator_result(torch_cuda, cooling_table):
     assert torch.equal(y, y_ref) and torch.equal(h, h_ref) and torch.equal(st, st_ref)
 
 
+def test_surrogate_evolve_captured_in_a_hip_graph(torch_cuda, cooling_table):
+    """The call that only enqueues records into a caller's graph (claim order by node index): replays on other nodes,
+    with other numbers rejected, equal eager calls bit for bit, with eager work between them."""
+    torch = torch_cuda
+    from galacticus_amd.evolver import NodeEvolverBatched
+    from galacticus_amd.surrogate import SurrogateEvolver, GateConfig, PairSet, encode
+    p, b, t1, ev, mlp, norm, d = _surrogate_setup(torch, cooling_table)
+    x, _, _ = encode(ev, PairSet(d(b.y), None, d(b.node_par), d(b.t_start), d(t1)), norm=norm, with_target=False)
+    head = float(mlp.forward(x)[:, 30].median())
+    ev = NodeEvolverBatched(b.n, p, cooling_table, cost_order=False)
+    se = SurrogateEvolver(ev, mlp, norm, GateConfig(error_max=math.exp(head), mass_tolerance=1e9, metal_tolerance=1e9,
+                                                    negative_tolerance=1e9))
+    orders = [np.random.default_rng(k).permutation(b.n)[:b.n // 2] for k in range(4)]
+    batches = [[d(a[..., o]) for a in (b.y, b.node_par, b.t_start, t1, b.h_step)] for o in orders]
+
+    def evolve(args, scale, status, accepted, stream=None):
+        y, par, t_a, t_b, h = args
+        se.evolve_device(y, par, t_a, t_b, h, scale=scale, status=status, accepted=accepted, stream=stream,
+                         count_rejected=False)
+        return y, h, scale, status, accepted
+
+    n = b.n // 2
+    buffers = lambda: (torch.zeros((30, n), dtype=torch.float64, device="cuda"),
+                       torch.zeros(n, dtype=torch.int32, device="cuda"),
+                       torch.zeros(n, dtype=torch.int32, device="cuda"))
+    eager = [[t.clone() for t in evolve([a.clone() for a in args], *buffers())] for args in batches]
+    rejected = [int((e[4] == 0).sum()) for e in eager]
+    print("rejected", rejected, flush=True)
+    assert len(set(rejected)) > 1 and 0 < min(rejected) and max(rejected) < n
+    held, out = [a.clone() for a in batches[0]], buffers()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        evolve(held, *out, stream=side)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        evolve(held, *out, stream=torch.cuda.current_stream())
+    for args, expected in zip(batches, eager):
+        for a, o in zip(held, args):
+            a.copy_(o)
+        g.replay()
+        torch.cuda.synchronize()
+        for got, ref in zip((held[0], held[4], *out), expected):
+            assert torch.equal(got, ref)
+        mlp.forward(x)
+
+
 @pytest.mark.parametrize("centre,spread", [(0.01, 1.0e-3), (-0.05, 0.01), (1.5, 0.1)],
                          ids=["small-growth", "shrink", "large-growth"])
 def test_accepted_nodes_get_the_decoded_network_output(torch_cuda, cooling_table, centre, spread):
