@@ -55,7 +55,7 @@ KERNEL_LAUNCH = {"nodes_per_workgroup": 64, "workgroups_per_cu": 1, "rhs_waves":
 # (profiles/evolve_kernel_hbm_traffic_isolated_halos_1e5.md), each counter
 # scaled by what it reads for one elementwise kernel that reads and writes
 # 1 GiB (FETCH_SIZE x 2.0000, WRITE_SIZE x 1.0000).
-HBM_TRAFFIC_1E5 = (240854.06 * 2.0 + 213911.25 * 1.0) * 1024
+HBM_TRAFFIC_1E5 = (241462.80 * 2.0 + 223397.97 * 1.0) * 1024
 
 
 def hbm_traffic(n, seed):
