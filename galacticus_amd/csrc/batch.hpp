@@ -18,7 +18,7 @@ struct gal_ode_batch {
   int n_cus = 0;
   int nodes_per_block = 64;
   int blocks_per_cu = 1;
-  int rhs_waves = 2;          // waves per group of 64 nodes (2: the RHS split over two SIMDs)
+  int rhs_waves = 2;          // these three are kept and reported: the integrator has one launch shape
   double wall_limit_s = 0.0;  // per-launch wall-time limit (0: none)
   double wall_clock_hz = 0.0; // frequency of the device's realtime counter
   double graph_stall_s = 60.0;  // operation-graph executor: give up after this long without progress

@@ -260,7 +260,9 @@ __device__ __forceinline__ void claim_nodes(const EvolveArgs& a, int n_claim, bo
 // One instance of this per wave of the group: a lone wave issues one
 // instruction every 4.6 cycles whatever it is (a dependent FP64 FMA costs no
 // more than an independent one, and a move of half a constant as much as
-// either), so the instruction count of each wave is what there is to save.
+// either), so what there is to save is instructions on the chain that crosses
+// the waves.  An attempt's six evaluations are some 14.6 of its 18.7 us; the
+// rest is between them, where each owner forms ten variables one by one.
 // With a loop of its own a wave keeps the constants of its own transcendental
 // functions in registers across the integration.  Between two evaluations
 // every value that is carried round the loop and set on more than one path
@@ -726,8 +728,10 @@ __global__ void reset_counter_kernel(unsigned int* w) {
   if (threadIdx.x == 0 && blockIdx.x == 0) *w = 0u;
 }
 
-// One lane per node and some 3500 instructions a node with 60 doubles in and
-// out: a million nodes take 116 us, 4.8 TB/s, and 100,000 17 us.  The whole RHS
+// One lane per node and 2600 instructions a wave (2164 vector, 401 scalar)
+// with 38 doubles of a node in and 30 out: a million nodes take 116 us, 4.7
+// TB/s, and 100,000 17 us, in which a wave issues vector instructions for 31 %
+// of its time and waits for memory or an issue slot for 63 %.  The whole RHS
 // in one lane wants more than 200 registers, so two waves share a SIMD: with
 // 128 registers a wave (four to a SIMD) it spills and takes 210 us, with 168
 // 149 us.  Single waves as workgroups spread a small batch over more CUs than

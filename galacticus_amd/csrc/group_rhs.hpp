@@ -4,9 +4,11 @@
 // A node's Cash-Karp attempts are a serial chain of RHS evaluations, and a
 // wave64 FP64 instruction takes its issue cycles whether one lane or all 64
 // are active, so the time of a stiff node -- and of every launch, which lasts
-// as long as its stiffest node -- is the number of instructions in the
-// longest wave's share of an RHS.  The blocks of physics.hpp are dealt out by
-// what they wait for:
+// as long as its stiffest node -- is the chain of instructions from one
+// barrier to the next, through whichever waves it crosses: the waves issue
+// vector instructions in 35 % of their time and wait, for each other, LDS and
+// the cooling table, in 45 %.  The blocks of physics.hpp are dealt out by what
+// they wait for:
 //   galaxy wave   the galaxy half, then the CGM outer radius;
 //   profile wave  hot-halo profile, ISCO, spheroid accretion, then the mean
 //                 radius of the hot gas, then the spheroid's rates, the black
@@ -24,8 +26,11 @@
 // for 6300 cycles of work in the busiest wave.
 //
 // All exchange goes through LDS vectors of 64 doubles, one per lane
-// (conflict-free); a vector is written by one wave and read by the others on
-// the far side of a barrier.
+// (conflict-free), each written by one wave.  The stage state, the time parts,
+// the halves of the derivative, the error norms, the step size and the claims
+// are read on the far side of a barrier.  The kMid vectors are written and
+// read within one evaluation, with no barrier between: a wave reads one only
+// after it has awaited the signal that is named beside it.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -63,9 +68,13 @@ enum : int {
   kFarMid = kFarTime + 2 * kTimeVectors,    // published within an evaluation
   kFarNorm = kFarMid + kMidVectors,         // each owner's error norm
   kFarStep = kFarNorm + kOwnerWaves,        // step size chosen by the controller
-  // published within an evaluation
-  kMidRho0 = kFarMid, kMidRhoOut, kMidEffThin, kMidEddCap, kMidMdotSph, kMidInvRMean,   // profile wave
-  kMidLambda, kMidNhPerRho, kMidNallPerNh, kMidMdot,                                    // cooling wave
+  // published within an evaluation, by the profile wave:
+  kMidRho0 = kFarMid, kMidRhoOut,             // kProfileReady
+  kMidEffThin, kMidEddCap, kMidMdotSph,       // kAccretorReady
+  kMidInvRMean,                               // kMeanRadiusReady
+  // and by the cooling wave:
+  kMidLambda, kMidNhPerRho, kMidNallPerNh,    // kCoolingFunctionReady
+  kMidMdot,                                   // kAccretionReady
   kMidEnd,
   // claimed nodes, in the time part that is not in use
   kXClaimNode = 0, kXClaimT0, kXClaimT1, kXClaimStep, kXClaimPar
