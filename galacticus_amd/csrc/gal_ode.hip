@@ -729,8 +729,8 @@ __global__ void reset_counter_kernel(unsigned int* w) {
 }
 
 // One lane per node and 2600 instructions a wave (2164 vector, 401 scalar)
-// with 38 doubles of a node in and 30 out: a million nodes take 116 us, 4.7
-// TB/s, and 100,000 17 us, in which a wave issues vector instructions for 31 %
+// with 38 doubles of a node in and 30 out: a million nodes take 116 to 132 us,
+// 4.1 to 4.7 TB/s, and 100,000 17 us, in which a wave issues vector instructions for 31 %
 // of its time and waits for memory or an issue slot for 63 %.  The whole RHS
 // in one lane wants more than 200 registers, so two waves share a SIMD: with
 // 128 registers a wave (four to a SIMD) it spills and takes 210 us, with 168
